@@ -306,6 +306,14 @@ __device__ __forceinline__ void buf_store2(buf_rsrc r, int voff, float2 v) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, voff, 0, 0);
 }
 
+__device__ __forceinline__ void buf_store1(buf_rsrc r, int voff, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, voff, 0, 0);
+}
+__device__ __forceinline__ void buf_store4(buf_rsrc r, int voff, float4 v) {
+  using u4 = __attribute__((ext_vector_type(4))) unsigned;
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, 0, 0);
+}
+
 // Workgroup barrier that is also a compiler fence: no load or store is moved
 // across it, so twiddle and spectrum loads stay inside their pass instead of
 // being hoisted (and held in VGPRs) across the whole kernel.

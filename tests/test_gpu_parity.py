@@ -383,6 +383,50 @@ def test_cfar_complex_input_and_edges(mx, orc):
     assert bad == 0
 
 
+@pytest.mark.parametrize("Nx", [3, 4, 5, 231, 233, 256, 467])
+@pytest.mark.parametrize("Ny,win,guard", [(1, (5, 13), (3, 3)), (2, (7, 21), (3, 5)), (8, (7, 21), (3, 5)),
+                                          (9, (3, 5), (1, 3)), (67, (5, 13), (3, 5)), (131, (7, 21), (3, 5))])
+def test_cfar_strips(mx, orc, Ny, Nx, win, guard):
+    """Strips of 256 columns walked row by row: maps narrower and wider than a
+    strip by a few columns, shorter than the window, than a band and just
+    past one, rows at every 4-byte alignment, f32 and c64 input, with and
+    without the averages, the power written for c64, strided outputs."""
+    rng = np.random.default_rng(1000 * Ny + Nx)
+    C = 2
+    D = crandn(rng, C, Ny, Nx).astype(np.complex64)
+    D[0, 0, 0] *= 60
+    D[-1, -1, -1] *= 60
+    mask = np.ones(win)
+    cy, cx, gy, gx = win[0] // 2, win[1] // 2, guard[0] // 2, guard[1] // 2
+    mask[cy - gy:cy + gy + 1, cx - gx:cx + gx + 1] = 0
+    pwr = np.abs(D.astype(complex)) ** 2
+    pw32 = pwr.astype(np.float32)
+    ref, ref32 = orc.cfar(pwr, mask), orc.cfar(pw32.astype(np.float64), mask)
+
+    def ba_ok(ba, r):
+        some = ~np.isnan(r["ba"])   # a cell without any training cell has no average
+        assert np.array_equal(~np.isnan(host(ba)), some)
+        assert rel(host(ba)[some], r["ba"][some]) < RTOL
+
+    buf = torch.zeros((C, Ny, Nx + 2), dtype=torch.float32, device="cuda")
+    view = buf[:, :, 1:Nx + 1]   # rows at 4, 12, ... bytes past a 16-byte boundary
+    view.copy_(dev(pw32, torch.float32))
+    dets, ba, _ = mx.cfar(view, win=win, guard=guard, want_ba=True)
+    ba_ok(ba, ref32)
+    assert dets_match(host(dets), ref32)[0] == 0
+    wide = torch.zeros((C, Ny, Nx, 2), dtype=torch.int32, device="cuda")
+    mx.cfar(view, win=win, guard=guard, dets=wide[..., 0])
+    assert dets_match(host(wide[..., 0]), ref32)[0] == 0 and int(wide[..., 1].abs().sum()) == 0
+    cbuf = torch.zeros((C, Ny, Nx + 1), dtype=torch.complex64, device="cuda")
+    cview = cbuf[:, :, 1:]
+    cview.copy_(dev(D))
+    pw_out = torch.empty((C, Ny, Nx), dtype=torch.float32, device="cuda")
+    dets, ba, _ = mx.cfar(cview, win=win, guard=guard, pw=pw_out, want_ba=True)
+    assert rel(host(pw_out), pwr) < RTOL
+    ba_ok(ba, ref)
+    assert dets_match(host(dets), ref)[0] == 0
+
+
 @pytest.mark.parametrize("C,Ny,Nx,win,guard,aligned", [
     (2, 512, 3001, (7, 21), (3, 5), True),    # the large cube's window, ragged last tile
     (3, 40, 777, (5, 13), (3, 5), True),      # fewer rows than one tile band
