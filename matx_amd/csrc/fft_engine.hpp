@@ -9,10 +9,9 @@
 //   a_m *= W_{Ls*R}^{m*k}                           (W_n = e^{-2 pi i/n} forward)
 //   b = DFT_R(a)
 //   Y[(j-k)*R + q*Ls + k] = b_q                     q = 0..R-1
-// After the last pass Y is in natural order.  Twiddles come from tables built
-// on the host in double precision and rounded once to float (one table per
-// (Ls, R) pass, k-major with stride R so a thread reads its R entries as one
-// contiguous run).
+// After the last pass Y is in natural order.  The twiddles are folded into the
+// butterflies (dft_tw below); their factors come from tables built on the host
+// in double precision and rounded once to float.
 #pragma once
 
 #include "mxr_internal.hpp"
@@ -198,11 +197,12 @@ __host__ __device__ constexpr RadixSeq reversed(RadixSeq s) {
   for (int i = 0; i < s.n; ++i) o.r[i] = s.r[s.n - 1 - i];
   return o;
 }
-// Offset (in float2) of pass p's twiddle table inside a sequence's table.
+// Offset (in float2) of pass p's twiddle table inside a sequence's table: Ls
+// rows of R/2 factors per pass.
 __host__ __device__ constexpr int64_t tw_offset(RadixSeq s, int p) {
   int64_t off = 0, Ls = 1;
   for (int i = 0; i < p; ++i) {
-    off += (Ls > 1) ? Ls * s.r[i] : 0;
+    off += (Ls > 1) ? Ls * s.r[i] / 2 : 0;
     Ls *= s.r[i];
   }
   return off;
@@ -219,65 +219,122 @@ __host__ __device__ constexpr int pass_ls(RadixSeq s, int p) {
 __device__ __forceinline__ int lds_pad(int i) { return i + (i >> 4); }
 __host__ __device__ constexpr int lds_padded_len(int n) { return n + (n >> 4) + 1; }
 
-// --------------------------------------------------------- pass helpers
-template <int R, bool INV>
-__device__ __forceinline__ void apply_twiddles(float2 (&a)[R], const float2 *__restrict__ tw, int k) {
-  // tw points at the pass table; entries k*R + m, m = 1..R-1 (entry 0 holds
-  // 1 and is skipped).  Two twiddles per 16-byte load.
-  const float4 *t4 = reinterpret_cast<const float4 *>(tw + (int64_t)k * R);
+// ------------------------------------------------ twiddled butterflies
+// DFT_R of (x_j w^j), w = e^{-+2 pi i k/(Ls R)}, as a tree of two-point
+// butterflies a +- f b whose factor f is kept as (c, t) with f = c (1 -+ i t),
+// c = cos, t = tan: u + i v = b (1 -+ i t) takes two fused multiply-adds and
+// a +- c (u + i v) four, where a complex product and two complex sums take
+// eight.  A radix-16 butterfly is 32 of them, 192 instructions in place of
+// 152 for the plain butterfly, 60 for its twiddle products and 44 for deriving
+// eleven of the fifteen twiddles from four, and each input is rounded by one
+// operation less; a row of factors is half the size of a row of twiddles.
+// Measured: the 2048-point blocks of conv1d's FFT method (16 x 1048576, 209
+// taps) 98 -> 67 us, 8192 chirp-z transforms of 1000 points 94 -> 77 us.
+// pc4096_kernel, which had a row of four twiddles per butterfly and derived the
+// rest, gains from it only with its rows kept in registers for the inverse
+// passes (133 us a 16 x 128 x 9000 cube with the rows loaded four times, 127
+// with them kept; 132 before).
+//
+// The factors of one k (w_n = e^{-2 pi i/n}; the tree's other factors are
+// these times -i, a swap):
+//   R = 4:  w^2, w
+//   R = 8:  w^4, w^2; w, w w_8
+//   R = 16: w^8, w^4; w^2, w^2 w_8; w, w w_16; w w_8, w w_16^3
+// stored two to a float4, group h of row k at [h * Ls + k], so that lanes with
+// neighbouring k read neighbouring 16-byte words.  All angles lie in [0, pi)
+// and only the first factor's reaches pi/2, where c is kept at TW_MIN_COS: the
+// factor is then off by that much, a sixteenth of a rounding.
+constexpr double TW_MIN_COS = 1.0 / (1 << 28);
+
+template <int R>
+struct TwRow {
+  float4 g[R / 4];
+};
+template <int R>
+__device__ __forceinline__ TwRow<R> load_tw(const float4 *__restrict__ tw, int ls, int k) {
+  TwRow<R> r;
 #pragma unroll
-  for (int h = 0; h < R / 2; ++h) {
-    float4 w = t4[h];
-    if (h > 0) a[2 * h] = cmul(a[2 * h], make_float2(w.x, INV ? -w.y : w.y));
-    a[2 * h + 1] = cmul(a[2 * h + 1], make_float2(w.z, INV ? -w.w : w.w));
+  for (int h = 0; h < R / 4; ++h) r.g[h] = tw[h * ls + k];
+  return r;
+}
+
+// p = a + f b, m = a - f b; ROT: f times W_4 (-i forward, +i inverse)
+template <bool INV, bool ROT>
+__device__ __forceinline__ void tbf(float2 a, float2 b, float c, float t, float2 &p, float2 &m) {
+  const float u = fmaf(INV ? -t : t, b.y, b.x), v = fmaf(INV ? t : -t, b.x, b.y);
+  if constexpr (!ROT) {
+    p = make_float2(fmaf(c, u, a.x), fmaf(c, v, a.y));
+    m = make_float2(fmaf(-c, u, a.x), fmaf(-c, v, a.y));
+  } else if constexpr (!INV) {
+    p = make_float2(fmaf(c, v, a.x), fmaf(-c, u, a.y));
+    m = make_float2(fmaf(-c, v, a.x), fmaf(c, u, a.y));
+  } else {
+    p = make_float2(fmaf(-c, v, a.x), fmaf(c, u, a.y));
+    m = make_float2(fmaf(c, v, a.x), fmaf(-c, u, a.y));
   }
 }
 
-// Host: build the twiddle table of a radix sequence for length N in double
-// precision, rounded once to float.  Layout per pass p (Ls > 1):
-// entry k*R + m = exp(-2 pi i m k / (Ls R)).
-void build_twiddles(int N, RadixSeq s, float2 *out);
+// DFT_4 of (a0, f a1, f^2 a2, f^3 a3) in place; f^2 = (c2, t2), times W_4 with
+// ROT2, f = (c1, t1)
+template <bool INV, bool ROT2>
+__device__ __forceinline__ void dft4_tw(float2 &a0, float2 &a1, float2 &a2, float2 &a3, float c2, float t2,
+                                        float c1, float t1) {
+  float2 u0, u1, v0, v1;
+  tbf<INV, ROT2>(a0, a2, c2, t2, u0, u1);
+  tbf<INV, ROT2>(a1, a3, c2, t2, v0, v1);
+  tbf<INV, false>(u0, v0, c1, t1, a0, a2);
+  tbf<INV, true>(u1, v1, c1, t1, a1, a3);
+}
+
+template <bool INV>
+__device__ __forceinline__ void dft_tw(float2 (&a)[4], const TwRow<4> &w) {
+  dft4_tw<INV, false>(a[0], a[1], a[2], a[3], w.g[0].x, w.g[0].y, w.g[0].z, w.g[0].w);
+}
+
+template <bool INV>
+__device__ __forceinline__ void dft_tw(float2 (&a)[8], const TwRow<8> &w) {
+  // 8 = 2 x 4: DFT_4 of the even and of the odd inputs with w^2, then pairs
+  // with w w_8^r
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+    dft4_tw<INV, false>(a[q], a[q + 2], a[q + 4], a[q + 6], w.g[0].x, w.g[0].y, w.g[0].z, w.g[0].w);
+  float2 y[8];
+  tbf<INV, false>(a[0], a[1], w.g[1].x, w.g[1].y, y[0], y[4]);
+  tbf<INV, false>(a[2], a[3], w.g[1].z, w.g[1].w, y[1], y[5]);
+  tbf<INV, true>(a[4], a[5], w.g[1].x, w.g[1].y, y[2], y[6]);
+  tbf<INV, true>(a[6], a[7], w.g[1].z, w.g[1].w, y[3], y[7]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a[i] = y[i];
+}
+
+template <bool INV>
+__device__ __forceinline__ void dft_tw(float2 (&a)[16], const TwRow<16> &w) {
+  // 16 = 4 x 4: DFT_4 over inputs q + 4m with w^4, then over q with w w_16^r
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    dft4_tw<INV, false>(a[q], a[q + 4], a[q + 8], a[q + 12], w.g[0].x, w.g[0].y, w.g[0].z, w.g[0].w);
+  dft4_tw<INV, false>(a[0], a[1], a[2], a[3], w.g[1].x, w.g[1].y, w.g[2].x, w.g[2].y);
+  dft4_tw<INV, false>(a[4], a[5], a[6], a[7], w.g[1].z, w.g[1].w, w.g[2].z, w.g[2].w);
+  dft4_tw<INV, true>(a[8], a[9], a[10], a[11], w.g[1].x, w.g[1].y, w.g[3].x, w.g[3].y);
+  dft4_tw<INV, true>(a[12], a[13], a[14], a[15], w.g[1].z, w.g[1].w, w.g[3].z, w.g[3].w);
+  float2 y[16];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) y[r + 4 * q] = a[4 * r + q];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) a[i] = y[i];
+}
+
+// Host: the factors of row k of a pass (Ls, R), R/2 of them in the order above.
+void tw_factors(int R, int64_t Ls, int64_t k, float2 *out);
 
 // Per-device cache of twiddle tables keyed by (N, reversed?).  Returns a
 // device pointer owned by the library.
 const float2 *twiddles_device(int N, bool reversed_seq);
 
-// v[m] *= W^{mk}, m = 1..15, from one power-base row (W^k, W^2k, W^4k,
-// W^8k): the other powers are products of at most four of them (at most
-// three extra roundings).  inv conjugates (inverse transform).
-__device__ __forceinline__ void tw_from_base(float2 (&v)[16], float4 b0, float4 b1, bool inv) {
-  float2 w1 = make_float2(b0.x, b0.y), w2 = make_float2(b0.z, b0.w);
-  float2 w4 = make_float2(b1.x, b1.y), w8 = make_float2(b1.z, b1.w);
-  if (inv) {
-    w1.y = -w1.y;
-    w2.y = -w2.y;
-    w4.y = -w4.y;
-    w8.y = -w8.y;
-  }
-  float2 w[16];
-  w[1] = w1;
-  w[2] = w2;
-  w[4] = w4;
-  w[8] = w8;
-  w[3] = cmul(w2, w1);
-  w[5] = cmul(w4, w1);
-  w[6] = cmul(w4, w2);
-  w[7] = cmul(w[6], w1);
-  w[9] = cmul(w8, w1);
-  w[10] = cmul(w8, w2);
-  w[11] = cmul(w[10], w1);
-  w[12] = cmul(w8, w4);
-  w[13] = cmul(w[12], w1);
-  w[14] = cmul(w[12], w2);
-  w[15] = cmul(w[14], w1);
-#pragma unroll
-  for (int m = 1; m < 16; ++m) v[m] = cmul(v[m], w[m]);
-}
-
-// Per-device cache of radix-16 power-base rows for the pass with sub-length
-// Ls of an N-point transform: row k (k < Ls) holds W^k, W^2k, W^4k, W^8k with
-// W = e^{-2 pi i / (16 Ls)}, each from double precision rounded once.
-const float4 *pow_base_device(int N, int Ls);
+// Per-device cache of the table of one radix-16 pass with sub-length Ls.
+const float4 *tw16_device(int Ls);
 
 // Raw buffer access (MUBUF) for the block kernels: a resource covering
 // `bytes` bytes from `base`.  The hardware range check returns zeros for
@@ -298,6 +355,11 @@ __device__ __forceinline__ buf_rsrc make_rsrc(const void *base, int bytes) {
 __device__ __forceinline__ float2 buf_load2(buf_rsrc r, int voff) {
   return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
 }
+// with a scalar part of the offset (for offsets known to be in range: it is
+// not checked), which an instruction takes without an address register
+__device__ __forceinline__ float2 buf_load2s(buf_rsrc r, int voff, int soff) {
+  return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+}
 __device__ __forceinline__ float4 buf_load4(buf_rsrc r, int voff) {
   return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
 }
@@ -312,6 +374,21 @@ __device__ __forceinline__ void buf_store1(buf_rsrc r, int voff, float v) {
 __device__ __forceinline__ void buf_store4(buf_rsrc r, int voff, float4 v) {
   using u4 = __attribute__((ext_vector_type(4))) unsigned;
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, 0, 0);
+}
+
+// Two-point butterflies across a pair of neighbouring lanes: the even lane
+// holds a[m] and gets a[m] + b[m], the odd lane holds b[m] and gets
+// a[m] - b[m].
+template <int N>
+__device__ __forceinline__ void pair_dft2(float2 (&v)[N], bool odd) {
+  const int sg = odd ? 0x80000000 : 0;
+  auto one = [&](float x) {
+    const int i = __float_as_int(x);
+    const int o = __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, true);  // quad_perm [1, 0, 3, 2]
+    return __int_as_float(o) + __int_as_float(i ^ sg);
+  };
+#pragma unroll
+  for (int m = 0; m < N; ++m) v[m] = make_float2(one(v[m].x), one(v[m].y));
 }
 
 // Workgroup barrier that is also a compiler fence: no load or store is moved
@@ -398,9 +475,10 @@ struct Pass {
       if constexpr (LS > 1) {
         int t, j;
         LY::template bfly<R>(threadIdx.x + u * NT, t, j);
-        apply_twiddles<R, INV>(v[u], tw, j & (LS - 1));
+        dft_tw<INV>(v[u], load_tw<R>(reinterpret_cast<const float4 *>(tw), LS, j & (LS - 1)));
+      } else {
+        dft<R, INV>(v[u]);
       }
-      dft<R, INV>(v[u]);
     }
   }
   // f(u, q, t, i) for the output positions store<LS> visits, value

@@ -92,6 +92,22 @@ __host__ __device__ inline void batch_offsets(const BatchIdx &bi, int64_t flat,
   *ob = b;
 }
 
+// The same for a flat index and batch extents below 2^31 (32-bit divisions: a
+// 64-bit one is some seventy dependent scalar instructions ahead of a
+// workgroup's first load).
+__device__ inline void batch_offsets32(const BatchIdx &bi, uint32_t flat, int64_t *oa, int64_t *ob) {
+  int64_t a = 0, b = 0;
+  for (int d = bi.nd - 1; d >= 0; --d) {
+    const uint32_t s = (uint32_t)bi.shape[d], q = flat / s;
+    const uint32_t i = flat - q * s;
+    flat = q;
+    a += (int64_t)i * bi.sa[d];
+    b += (int64_t)i * bi.sb[d];
+  }
+  *oa = a;
+  *ob = b;
+}
+
 // -------------------------------------------------------- device complex
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(WgT<M>::NT) void pc_wgrad_kernel(WgArgs a) {
 
 // M = 8192: the transforms of the 8192-point pulse-compression kernel
 // (radix 2 x 16 x 16 x 16, 512 threads, the radix-2 pass folded into the
-// load, power-base twiddles for Ls = 2, 32, 512), so the x spectrum, the gy
+// load, factor tables for Ls = 2, 32, 512), so the x spectrum, the gy
 // spectrum and the running product take 16 bins each per thread (bins
 // j + 512q).  Those three live sets need more than the 128 VGPRs of two
 // workgroups per CU, so it runs one (up to 256 VGPRs, no spills).
@@ -135,8 +135,8 @@ struct Wg8192Args {
 // the workgroup's previous LDS reads are done.  Post: LDS is free (the last
 // exchange ends with a barrier).
 template <class LoadF>
-__device__ __forceinline__ void fwd8192_regs(float2 (&v)[16], LoadF &&ld, const float4 *pA,
-                                             const float4 *pB, const float4 *pC, float2 *lds) {
+__device__ __forceinline__ void fwd8192_regs(float2 (&v)[16], LoadF &&ld, const float4 *bA,
+                                             const float4 *bB, const float4 *bC, float2 *lds) {
   constexpr int NT = 512;
   using LY = Layout<8192, 1, false>;
   const int j = threadIdx.x;
@@ -161,19 +161,14 @@ __device__ __forceinline__ void fwd8192_regs(float2 (&v)[16], LoadF &&ld, const 
 #pragma unroll
     for (int m = 0; m < 16; ++m) v[m] = odd ? csub(a[m], b[m]) : cadd(a[m], b[m]);
   }
-  float4 t0 = pA[0], t1 = pA[1];
-  tw_from_base(v, t0, t1, false);  // Ls = 2
-  dft16<false>(v);
-  t0 = pB[0];
-  t1 = pB[1];
+  TwRow<16> tw = load_tw<16>(bA, 2, j & 1);
+  dft_tw<false>(v, tw);  // Ls = 2
+  tw = load_tw<16>(bB, 32, j & 31);
   xchg(2);
-  tw_from_base(v, t0, t1, false);  // Ls = 32
-  dft16<false>(v);
-  t0 = pC[0];
-  t1 = pC[1];
+  dft_tw<false>(v, tw);  // Ls = 32
+  tw = load_tw<16>(bC, 512, j);
   xchg(32);
-  tw_from_base(v, t0, t1, false);  // Ls = 512
-  dft16<false>(v);
+  dft_tw<false>(v, tw);  // Ls = 512
 }
 
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
@@ -182,7 +177,6 @@ void wgrad8192_kernel(Wg8192Args p) {
   __shared__ float2 lds[LY::LDS_ELEMS];
   const WgArgs &a = p.a;
   const int j = threadIdx.x;
-  const float4 *pA = p.bA + (j & 1) * 2, *pB = p.bB + (j & 31) * 2, *pC = p.bC + j * 2;
   float2 acc[16];
 #pragma unroll
   for (int q = 0; q < 16; ++q) acc[q] = make_float2(0.f, 0.f);
@@ -201,9 +195,9 @@ void wgrad8192_kernel(Wg8192Args p) {
       int gi = lo + i;
       if (gi >= n32) gi -= n32;
       return gi < seff ? xr[gi] : make_float2(0.f, 0.f);
-    }, pA, pB, pC, lds);
-    fwd8192_regs(Gv, [&](int i) { return i < lim ? gr[lo + i] : make_float2(0.f, 0.f); }, pA, pB,
-                 pC, lds);
+    }, p.bA, p.bB, p.bC, lds);
+    fwd8192_regs(Gv, [&](int i) { return i < lim ? gr[lo + i] : make_float2(0.f, 0.f); }, p.bA,
+                 p.bB, p.bC, lds);
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       acc[q].x += X[q].x * Gv[q].x + X[q].y * Gv[q].y;  // X conj(G)
@@ -329,7 +323,7 @@ static mxr_status wgrad_run(const WgradJob &j, hipStream_t s) {
     a.partial = ws;
     a.twf = twf;
     if constexpr (M == 8192) {
-      Wg8192Args p{a, pow_base_device(8192, 2), pow_base_device(8192, 32), pow_base_device(8192, 512)};
+      Wg8192Args p{a, tw16_device(2), tw16_device(32), tw16_device(512)};
       MXR_REQUIRE(p.bA && p.bB && p.bC, MXR_OUT_OF_MEMORY,
                   "pc waveform gradient: twiddle table allocation failed");
       ProfScope ps("wgrad8192_kernel", s);

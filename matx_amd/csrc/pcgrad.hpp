@@ -6,6 +6,10 @@
 
 namespace mxr {
 
+// The 4096- and 8192-point kernels address a row's samples with 32-bit byte
+// offsets; longer rows take the general kernels.
+constexpr int64_t PC_BUF_MAX_N = 1 << 27;
+
 // One call: every row of x ([rows, S], row offsets bi.sa) against its lags
 // gy ([rows, nout], offsets bi.sb) over the overlap-save blocks (M, V, nblk)
 // of the forward plan; w ([L]) is the raw waveform the forward windowed and

@@ -60,6 +60,15 @@ struct OlsBlock {
   const float2 *wc;  // M-point spectrum, scaled by 1/M
 };
 
+// Group g of a call: block g mod nblk of row g / nblk.
+__device__ __forceinline__ OlsBlock pc_block(const PcArgs &a, int64_t g) {
+  const uint32_t row = (uint32_t)g / (uint32_t)a.nblk, blk = (uint32_t)g - row * (uint32_t)a.nblk;
+  int64_t ox, oy;
+  batch_offsets32(a.bi, row, &ox, &oy);
+  return OlsBlock{a.x + ox, a.y + oy, (int)blk * (int)a.V, (int)a.n, (int)a.seff,
+                  (int)a.nout, (int)a.V, a.wc};
+}
+
 // Body shared by the per-call kernel and the ragged-batch kernels.  Pre: the
 // workgroup's previous use of lds is finished (barrier passed).
 template <int M>
@@ -198,12 +207,7 @@ __global__ __launch_bounds__(256) void pc_ols_multi_kernel(PcArgs a) {
   __shared__ OlsBlock obs[TB];
   if (threadIdx.x < TB) {
     const int64_t g0 = (int64_t)blockIdx.x * TB;
-    const int64_t g = g0 + threadIdx.x < a.groups ? g0 + threadIdx.x : g0;
-    const int64_t row = g / a.nblk;
-    int64_t ox, oy;
-    batch_offsets(a.bi, row, &ox, &oy);
-    OlsBlock ob{a.x + ox, a.y + oy, (int)((g % a.nblk) * a.V), (int)a.n, (int)a.seff,
-                (int)a.nout, (int)a.V, a.wc};
+    OlsBlock ob = pc_block(a, g0 + threadIdx.x < a.groups ? g0 + threadIdx.x : g0);
     if (g0 + threadIdx.x >= a.groups) {  // past the last group: idle transform
       ob.seff = 0;
       ob.nout = ob.lo;
@@ -238,38 +242,32 @@ void pc_ols_kernel(PcArgs a) {
 }
 
 // Dedicated M = 4096 block kernel (plan radix 16 x 16 x 16, 256 threads, one
-// radix-16 butterfly per thread per pass).  Twiddles are built in registers
-// from four base powers W^k, W^2k, W^4k, W^8k per pass (one 32-byte row of a
-// compact table, W = e^{-2 pi i / (16 Ls)}): W^{mk} for the other m is a
-// product of at most four of them (at most three extra roundings).  The base
-// rows are fetched before each LDS exchange, so their latency hides behind
-// the exchange and its barriers instead of stalling the butterfly after it;
-// the inverse passes reuse the forward rows conjugated.
+// radix-16 butterfly per thread per pass).
 struct Pc4096Args {
   PcArgs a;
-  const float4 *base1;  // [16][2] float4: power-base rows of pass Ls = 16
-  const float4 *base2;  // [256][2] float4: power-base rows of pass Ls = 256
+  const float4 *base1;  // factors of pass Ls = 16
+  const float4 *base2;  // factors of pass Ls = 256
 };
 
 
 // One M = 4096 overlap-save block (256 threads); lds holds 4096 padded
 // elements.  Pre: the workgroup's previous use of lds is finished.
-// Thread j owns butterfly j of every radix-16 pass: its twiddles of the
-// Ls = 16 and Ls = 256 passes come from power-base rows (j & 15) and j
-// (W^k, W^2k, W^4k, W^8k), fetched before each LDS exchange so their
-// latency hides behind it (the inverse passes re-fetch them from cache and
-// conjugate; keeping them live costs more registers than the reload).  A block that
-// does not wrap reads x through a raw buffer resource ending at the row's
-// last sample (the hardware returns zeros past it) and writes its kept lags
-// through one ending at its last kept lag (stores past it are dropped), so
-// the block needs no per-element tests.  spec(i) gives spectrum bin i (the
-// block's 1/M included); thread j reads bins j + 256 q only.
+// Thread j owns butterfly j of every radix-16 pass: its factors of the
+// Ls = 16 and Ls = 256 passes are rows j & 15 and j, loaded once, ahead of the
+// samples' arrival, and kept for the inverse passes.  A block that does not
+// wrap reads x through a raw buffer resource ending at the row's last sample
+// (the hardware returns zeros past it) and writes its kept lags through one
+// ending at its last kept lag (stores past it are dropped), so the block needs
+// no per-element tests; a wrapping block reads through one over the whole row.
+// The spectrum's sixteen loads share one address register.  spec(q) gives bin
+// j + 256 q (the block's 1/M included).
 // Loads samples m0 .. m0 + NV - 1 of thread j of block ob
 // (x[lo + j + 256 m]) into v[0 .. NV).
 template <int NV>
 __device__ __forceinline__ void load_block4096(const OlsBlock &ob, float2 (&v)[NV], int m0 = 0) {
   constexpr int NT = 256;
-  const int j = threadIdx.x;
+  int j = threadIdx.x;
+  asm volatile("" : "+v"(j));  // the 16 offsets are formed here, not kept in registers by a caller's loop
   const float2 *__restrict__ xr = ob.xr;
   const int lo = ob.lo, n32 = ob.n, seff32 = ob.seff;
   if (lo + 4096 <= n32) {
@@ -279,11 +277,11 @@ __device__ __forceinline__ void load_block4096(const OlsBlock &ob, float2 (&v)[N
 #pragma unroll
     for (int m = 0; m < NV; ++m) v[m] = buf_load2(rx, (j + (m0 + m) * NT) * 8);
   } else {  // the block wraps around the circular period n (full fft_conv)
+    const buf_rsrc rx = make_rsrc(xr, seff32 * 8);
 #pragma unroll
     for (int m = 0; m < NV; ++m) {
-      int gi = lo + j + (m0 + m) * NT;
-      if (gi >= n32) gi -= n32;
-      v[m] = gi < seff32 ? xr[gi] : make_float2(0.f, 0.f);
+      const int gi = lo + j + (m0 + m) * NT;
+      v[m] = buf_load2(rx, (int)min((uint32_t)gi, (uint32_t)(gi - n32)) * 8);
     }
   }
 }
@@ -319,47 +317,33 @@ __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)
     for (int m = 0; m < 16; ++m) v[m] = lds[rbase + m * (NT + NT / 16)];
     wg_barrier();
   };
-  const float4 *b1p = base1 + (j & 15) * 2;
-  const float4 *b2p = base2 + j * 2;
-  float4 t0, t1;
+  TwRow<16> t1 = load_tw<16>(base1, 16, j & 15), t2 = load_tw<16>(base2, 256, j);
 
   // forward pass 0 (Ls = 1) on the samples as loaded
   dft16<false>(v);
-  t0 = b1p[0];
-  t1 = b1p[1];
   xchg(1);
-  tw_from_base(v, t0, t1, false);  // forward pass 1 (Ls = 16)
-  dft16<false>(v);
-  t0 = b2p[0];
-  t1 = b2p[1];
+  dft_tw<false>(v, t1);  // forward pass 1 (Ls = 16)
   // the spectrum bins this thread multiplies, fetched before the exchange
   // so that their cache latency hides behind it and the last forward pass
   float2 sp[16];
   if constexpr (!LATE_SPEC) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) sp[q] = spec(j + q * 256);
+    for (int q = 0; q < 16; ++q) sp[q] = spec(q);
   }
   xchg(16);
-  tw_from_base(v, t0, t1, false);  // forward pass 2 (Ls = 256)
-  dft16<false>(v);
+  dft_tw<false>(v, t2);  // forward pass 2 (Ls = 256)
   if constexpr (LATE_SPEC) {
     wg_barrier();  // the spectrum is complete
 #pragma unroll
-    for (int q = 0; q < 16; ++q) sp[q] = spec(j + q * 256);
+    for (int q = 0; q < 16; ++q) sp[q] = spec(q);
   }
 #pragma unroll
   for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], sp[q]);
   dft16<true>(v);            // inverse pass 0 (Ls = 1)
-  t0 = b1p[0];
-  t1 = b1p[1];
   xchg(1);
-  tw_from_base(v, t0, t1, true);   // inverse pass 1 (Ls = 16)
-  dft16<true>(v);
-  t0 = b2p[0];
-  t1 = b2p[1];
+  dft_tw<true>(v, t1);   // inverse pass 1 (Ls = 16)
   xchg(16);
-  tw_from_base(v, t0, t1, true);   // inverse pass 2 (Ls = 256)
-  dft16<true>(v);
+  dft_tw<true>(v, t2);   // inverse pass 2 (Ls = 256)
   // lags lo + j + 256 q below lo + lim are kept (the spectrum carries the 1/M)
   const int lim = (ob.nout - lo) < ob.V ? (ob.nout - lo) : ob.V;
   const buf_rsrc ry = make_rsrc(ob.yr + lo, lim * 8);
@@ -380,26 +364,20 @@ __device__ __forceinline__ void ols_block4096(const OlsBlock ob, const float4 *b
 // The block's spectrum from its buffer (ob.wc).
 __device__ __forceinline__ void ols_block4096(const OlsBlock ob, const float4 *base1,
                                               const float4 *base2, float2 *lds) {
-  ols_block4096(ob, base1, base2, lds, [&](int i) { return ob.wc[i]; });
+  const buf_rsrc rw = make_rsrc(ob.wc, 4096 * 8);
+  ols_block4096(ob, base1, base2, lds, [&](int q) { return buf_load2s(rw, (int)threadIdx.x * 8, q * 2048); });
 }
 
-__device__ __forceinline__ OlsBlock pc4096_block(const PcArgs &a, int64_t g) {
-  const int64_t row = g / a.nblk;
-  int64_t ox, oy;
-  batch_offsets(a.bi, row, &ox, &oy);
-  return OlsBlock{a.x + ox, a.y + oy, (int)((g % a.nblk) * a.V), (int)a.n, (int)a.seff,
-                  (int)a.nout, (int)a.V, a.wc};
-}
-
-// One workgroup per block.  (A persistent form that loads the next block's
-// samples during the current block's inverse passes needs more registers
-// than four workgroups per CU allow, and measured 11 % slower.)
+// One workgroup per block.  (Resident workgroups that load the next block's
+// samples during the last inverse pass measure 5 to 10 % slower: the memory
+// counter is shared by loads and stores, so the next block's first wait for a
+// load also waits for this block's stores to land.)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void pc4096_kernel(Pc4096Args pa) {
   using LY = Layout<4096, 1, false>;
   __shared__ float2 lds[LY::LDS_ELEMS];
   const PcArgs &a = pa.a;
-  ols_block4096(pc4096_block(a, xcd_remap(blockIdx.x, a.groups)), pa.base1, pa.base2, lds);
+  ols_block4096(pc_block(a, xcd_remap(blockIdx.x, a.groups)), pa.base1, pa.base2, lds);
 }
 
 // Small grids (fft_conv on a few hundred pulses, where one workgroup per
@@ -427,17 +405,12 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
   constexpr int NT = 256;
   if (threadIdx.x < NT) {
     const PcArgs &a = q.p.a;
-    const int64_t g = xcd_remap(blockIdx.x, a.groups);
-    const int64_t row = g / a.nblk;
-    int64_t ox, oy;
-    batch_offsets(a.bi, row, &ox, &oy);
-    const OlsBlock ob{a.x + ox, a.y + oy, (int)((g % a.nblk) * a.V), (int)a.n, (int)a.seff,
-                      (int)a.nout, (int)a.V, nullptr};
+    const OlsBlock ob = pc_block(a, xcd_remap(blockIdx.x, a.groups));
     float2 v[16];
     load_block4096(ob, v, 0);
     // barriers: 4 in the forward exchanges, 1 for the spectrum, 4 in the
     // inverse exchanges
-    auto spec = [&](int i) { return wsp[i]; };
+    auto spec = [&](int q) { return wsp[(int)threadIdx.x + q * 256]; };
     filter_block4096<decltype(spec), true>(ob, v, q.p.base1, q.p.base2, lds, spec);
     return;
   }
@@ -458,18 +431,13 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
     const int i = j + m * NT;
     v[m] = keep_if(q.w[(int64_t)(i < q.L ? i : 0) * q.wstride], i < q.L);
   }
-  const float4 *b1p = q.p.base1 + (j & 15) * 2;
-  const float4 *b2p = q.p.base2 + j * 2;
   dft16<false>(v);
-  float4 t0 = b1p[0], t1 = b1p[1];
+  TwRow<16> tw = load_tw<16>(q.p.base1, 16, j & 15);
   xchg(1);
-  tw_from_base(v, t0, t1, false);
-  dft16<false>(v);
-  t0 = b2p[0];
-  t1 = b2p[1];
+  dft_tw<false>(v, tw);
+  tw = load_tw<16>(q.p.base2, 256, j);
   xchg(16);
-  tw_from_base(v, t0, t1, false);
-  dft16<false>(v);
+  dft_tw<false>(v, tw);
   // the exchange above ended with a barrier after every read of wsp
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
@@ -482,19 +450,19 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
 }
 
 // Dedicated M = 8192 block kernel: radix sequence 2 x 16 x 16 x 16 over 512
-// threads (one radix-16 butterfly per thread per pass) with the power-base
-// twiddles of the 4096-point kernel for the passes Ls = 2, 32, 512
+// threads (one radix-16 butterfly per thread per pass) with the factor
+// tables of the passes Ls = 2, 32, 512
 // (conjugated for the inverse).  The forward radix-2 pass (Ls = 1, no
 // twiddles) is folded into the load: radix-16 butterfly j of the next pass
 // takes X1[j + 512m] = x[j0] +- x[j0 + 4096] with j0 = j/2 + 256m and the
-// sign given by j's parity, so every thread reads its 16 input pairs straight
-// from HBM (its neighbour reads the same pairs for the other sign, from L1).
+// sign given by j's parity: the two threads of a pair load one of the two
+// samples each and swap them (DPP).
 // The inverse radix-2 pass pairs bins k and k + 4096, which the forward's
 // last pass leaves in one thread (slots q and q + 8), so it runs in
 // registers before the first inverse exchange: five LDS exchanges per block.
 struct Pc8192Args {
   PcArgs a;
-  const float4 *bA, *bB, *bC;  // power-base rows for Ls = 2, 32, 512
+  const float4 *bA, *bB, *bC;  // factors of passes Ls = 2, 32, 512
 };
 
 __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *bA, const float4 *bB,
@@ -520,64 +488,46 @@ __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *b
     for (int m = 0; m < 16; ++m) v[m] = lds[rbase + 544 * m];
     wg_barrier();
   };
-  auto ldx = [&](int i) {
-    int gi = lo + i;
-    if (gi >= n32) gi -= n32;
-    return gi < seff32 ? xr[gi] : make_float2(0.f, 0.f);
-  };
-  const float4 *pA = bA + (j & 1) * 2;
-  const float4 *pB = bB + (j & 31) * 2;
-  const float4 *pC = bC + j * 2;
 
-  // forward radix-2 pass folded into the load; a block that does not wrap
-  // reads through a raw buffer resource ending at the row's last sample
-  // (zeros past it from the hardware range check)
+  // forward radix-2 pass: the two lanes of a pair load one half each (a block
+  // that does not wrap through a raw buffer resource ending at the row's last
+  // sample, zeros past it) and form sum and difference
   {
-    const int jh = j >> 1;
-    const bool odd = (j & 1) != 0;
-    float2 a[16], b[16];
+    const int i0 = (j >> 1) + (j & 1) * 4096;
     if (lo + 8192 <= n32) {
       int avail = seff32 - lo;
       avail = avail < 0 ? 0 : (avail > 8192 ? 8192 : avail);
       const buf_rsrc rx = make_rsrc(xr + lo, avail * 8);
 #pragma unroll
-      for (int m = 0; m < 16; ++m) {
-        a[m] = buf_load2(rx, (jh + 256 * m) * 8);
-        b[m] = buf_load2(rx, (jh + 256 * m + 4096) * 8);
-      }
+      for (int m = 0; m < 16; ++m) v[m] = buf_load2(rx, (i0 + 256 * m) * 8);
     } else {
+      const buf_rsrc rx = make_rsrc(xr, seff32 * 8);
 #pragma unroll
       for (int m = 0; m < 16; ++m) {
-        a[m] = ldx(jh + 256 * m);
-        b[m] = ldx(jh + 256 * m + 4096);
+        const int gi = lo + i0 + 256 * m;
+        v[m] = buf_load2(rx, (int)min((uint32_t)gi, (uint32_t)(gi - n32)) * 8);
       }
     }
-#pragma unroll
-    for (int m = 0; m < 16; ++m) v[m] = odd ? csub(a[m], b[m]) : cadd(a[m], b[m]);
+    pair_dft2(v, (j & 1) != 0);
   }
-  float4 t0 = pA[0], t1 = pA[1];
-  tw_from_base(v, t0, t1, false);  // forward pass Ls = 2
-  dft16<false>(v);
-  t0 = pB[0];
-  t1 = pB[1];
+  TwRow<16> tw = load_tw<16>(bA, 2, j & 1);
+  dft_tw<false>(v, tw);  // forward pass Ls = 2
+  tw = load_tw<16>(bB, 32, j & 31);
   xchg(2);
-  tw_from_base(v, t0, t1, false);  // forward pass Ls = 32
-  dft16<false>(v);
-  t0 = pC[0];
-  t1 = pC[1];
+  dft_tw<false>(v, tw);  // forward pass Ls = 32
+  tw = load_tw<16>(bC, 512, j);
   // the spectrum bins this thread multiplies, fetched before the exchange
+  const buf_rsrc rw = make_rsrc(ob.wc, 8192 * 8);
   float2 sp[16];
 #pragma unroll
-  for (int q = 0; q < 16; ++q) sp[q] = ob.wc[j + q * 512];
+  for (int q = 0; q < 16; ++q) sp[q] = buf_load2s(rw, j * 8, q * 4096);
   xchg(32);
-  tw_from_base(v, t0, t1, false);  // forward pass Ls = 512: bins j + 512q
-  dft16<false>(v);
+  dft_tw<false>(v, tw);  // forward pass Ls = 512: bins j + 512q
 #pragma unroll
   for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], sp[q]);
   // inverse radix-2 pass (Ls = 1) on bins j + 512q, j + 512q + 4096; its
   // outputs 2 (j + 512 q) and the next sit at pad(2 j) + 1088 q and + 1
-  t0 = pA[0];
-  t1 = pA[1];
+  tw = load_tw<16>(bA, 2, j & 1);
   const int e0 = lds_pad(2 * j);
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
@@ -588,18 +538,13 @@ __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *b
 #pragma unroll
   for (int m = 0; m < 16; ++m) v[m] = lds[rbase + 544 * m];
   wg_barrier();
-  tw_from_base(v, t0, t1, true);  // inverse pass Ls = 2
-  dft16<true>(v);
-  t0 = pB[0];
-  t1 = pB[1];
+  dft_tw<true>(v, tw);  // inverse pass Ls = 2
+  tw = load_tw<16>(bB, 32, j & 31);
   xchg(2);
-  tw_from_base(v, t0, t1, true);  // inverse pass Ls = 32
-  dft16<true>(v);
-  t0 = pC[0];
-  t1 = pC[1];
+  dft_tw<true>(v, tw);  // inverse pass Ls = 32
+  tw = load_tw<16>(bC, 512, j);
   xchg(32);
-  tw_from_base(v, t0, t1, true);  // inverse pass Ls = 512: lags j + 512q
-  dft16<true>(v);
+  dft_tw<true>(v, tw);  // inverse pass Ls = 512: lags j + 512q
   // lags lo + j + 512 q below lo + lim are kept (stores past lim dropped by
   // the range check; the spectrum carries the 1/M)
   const int lim = (ob.nout - lo) < ob.V ? (ob.nout - lo) : ob.V;
@@ -612,13 +557,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void pc8192_kernel(Pc8192Args pa) {
   using LY = Layout<8192, 1, false>;
   __shared__ float2 lds[LY::LDS_ELEMS];
-  const PcArgs &a = pa.a;
-  const int64_t g = xcd_remap(blockIdx.x, a.groups);
-  const int64_t row = g / a.nblk;
-  int64_t ox, oy;
-  batch_offsets(a.bi, row, &ox, &oy);
-  const OlsBlock ob{a.x + ox, a.y + oy, (int)((g % a.nblk) * a.V), (int)a.n, (int)a.seff,
-                    (int)a.nout, (int)a.V, a.wc};
+  const OlsBlock ob = pc_block(pa.a, xcd_remap(blockIdx.x, pa.a.groups));
   ols_block8192(ob, pa.bA, pa.bB, pa.bC, lds);
 }
 
@@ -717,10 +656,10 @@ __device__ __forceinline__ int item_job_lane(const int *item_job, int64_t it) {
 }
 
 __device__ __forceinline__ OlsBlock job_block(const PcJob &jb, int64_t it) {
-  const int64_t local = it - jb.item0;
-  const int64_t row = local / jb.nblk;
-  const int b = (int)(local % jb.nblk);
-  const int c = (int)(row / jb.P), p = (int)(row % jb.P);
+  const uint32_t local = (uint32_t)(it - jb.item0);
+  const uint32_t row = local / (uint32_t)jb.nblk;
+  const int b = (int)(local - row * (uint32_t)jb.nblk);
+  const int c = (int)(row / (uint32_t)jb.P), p = (int)(row - (uint32_t)c * (uint32_t)jb.P);
   return OlsBlock{jb.x + c * jb.x_cs + p * jb.x_ps, jb.y + c * jb.y_cs + p * jb.y_ps, b * jb.V,
                   jb.n, jb.seff, jb.nout, jb.V, jb.wc};
 }
@@ -853,7 +792,7 @@ mxr_status launch_pc_batch(int M, const PcJob *d_jobs, const int *d_item_job, in
   ProfScope ps("pc_batch_kernel", s);
   switch (M) {
     case 4096: {
-      const float4 *b1 = pow_base_device(4096, 16), *b2 = pow_base_device(4096, 256);
+      const float4 *b1 = tw16_device(16), *b2 = tw16_device(256);
       MXR_REQUIRE(b1 && b2, MXR_OUT_OF_MEMORY, "ragged batch: twiddle table allocation failed");
       if (persist) pc4096_batch_kernel<true><<<dim3(grid), dim3(256), 0, s>>>(d_jobs, d_item_job, items, b1, b2);
       else pc4096_batch_kernel<false><<<dim3(grid), dim3(256), 0, s>>>(d_jobs, d_item_job, items, b1, b2);
@@ -875,8 +814,7 @@ mxr_status launch_pc_batch(int M, const PcJob *d_jobs, const int *d_item_job, in
           d_jobs, d_item_job, items, twf, twi);                                                       \
     break;
     case 8192: {
-      const float4 *bA = pow_base_device(8192, 2), *bB = pow_base_device(8192, 32),
-                   *bC = pow_base_device(8192, 512);
+      const float4 *bA = tw16_device(2), *bB = tw16_device(32), *bC = tw16_device(512);
       MXR_REQUIRE(bA && bB && bC, MXR_OUT_OF_MEMORY, "ragged batch: twiddle table allocation failed");
       if (persist) pc8192_batch_kernel<true><<<dim3(grid), dim3(512), 0, s>>>(d_jobs, d_item_job, items, bA, bB, bC);
       else pc8192_batch_kernel<false><<<dim3(grid), dim3(512), 0, s>>>(d_jobs, d_item_job, items, bA, bB, bC);
@@ -1008,9 +946,10 @@ constexpr int64_t PC_WF_FUSE_MAX_GROUPS = 512;
 template <int M>
 mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
   if constexpr (M == 4096) {
-    if (wa && pa && pa->groups > 0 && pa->bpw == 1 && pa->groups <= PC_WF_FUSE_MAX_GROUPS &&
-        !wa->window && !wa->normalize && !wa->writeback && wa->L >= 1 && wa->L <= 4096) {
-      Pc4096WfArgs q{{*pa, pow_base_device(4096, 16), pow_base_device(4096, 256)}, wa->w, wa->wstride,
+    if (wa && pa && pa->groups > 0 && pa->bpw == 1 && pa->n <= PC_BUF_MAX_N &&
+        pa->groups <= PC_WF_FUSE_MAX_GROUPS && !wa->window && !wa->normalize && !wa->writeback &&
+        wa->L >= 1 && wa->L <= 4096) {
+      Pc4096WfArgs q{{*pa, tw16_device(16), tw16_device(256)}, wa->w, wa->wstride,
                      (int)wa->L, wa->conj, wa->out_scale};
       MXR_REQUIRE(q.p.base1 && q.p.base2, MXR_OUT_OF_MEMORY,
                   "pulse compression: twiddle table allocation failed");
@@ -1027,9 +966,8 @@ mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
   MXR_HIP_TRY(hipGetLastError());
   if (!pa || pa->groups <= 0) return MXR_SUCCESS;
   if constexpr (M == 8192) {
-    if (pa->bpw == 1) {
-      Pc8192Args p8{*pa, pow_base_device(8192, 2), pow_base_device(8192, 32),
-                    pow_base_device(8192, 512)};
+    if (pa->bpw == 1 && pa->n <= PC_BUF_MAX_N) {
+      Pc8192Args p8{*pa, tw16_device(2), tw16_device(32), tw16_device(512)};
       MXR_REQUIRE(p8.bA && p8.bB && p8.bC, MXR_OUT_OF_MEMORY,
                   "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc8192_kernel", s);
@@ -1039,8 +977,8 @@ mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
     }
   }
   if constexpr (M == 4096) {
-    if (pa->bpw == 1) {
-      Pc4096Args p4{*pa, pow_base_device(4096, 16), pow_base_device(4096, 256)};
+    if (pa->bpw == 1 && pa->n <= PC_BUF_MAX_N) {
+      Pc4096Args p4{*pa, tw16_device(16), tw16_device(256)};
       MXR_REQUIRE(p4.base1 && p4.base2, MXR_OUT_OF_MEMORY, "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc4096_kernel", s);
       pc4096_kernel<<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
@@ -1079,13 +1017,13 @@ mxr_status dispatch_pc(int M, const WfArgs *wa, const PcArgs *pa, hipStream_t s)
 }  // namespace
 
 // Builds every table the block kernels of size M read (forward and reversed
-// pass twiddles, the power-base rows of the dedicated 4096 and 8192 kernels),
+// pass twiddles, the factor tables of the dedicated 4096 and 8192 kernels),
 // so that later launches allocate nothing (and can be graph-captured).
 mxr_status pc_tables_prepare(int M, const char *fn) {
   bool ok = twiddles_device(M, false) && twiddles_device(M, true);
-  if (M == 4096) ok = ok && pow_base_device(4096, 16) && pow_base_device(4096, 256);
+  if (M == 4096) ok = ok && tw16_device(16) && tw16_device(256);
   if (M == 8192)
-    ok = ok && pow_base_device(8192, 2) && pow_base_device(8192, 32) && pow_base_device(8192, 512);
+    ok = ok && tw16_device(2) && tw16_device(32) && tw16_device(512);
   MXR_REQUIRE(ok, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   return MXR_SUCCESS;
 }

@@ -99,26 +99,33 @@ int max_lds_per_block() {
   return v;
 }
 
-void build_twiddles(int N, RadixSeq s, float2 *out) {
+void tw_factors(int R, int64_t Ls, int64_t k, float2 *out) {
+  // exponent num/16 of w_R beside the power of w: w^pw w_16^num
+  struct F {
+    int pw, num;
+  };
+  static const F f4[] = {{2, 0}, {1, 0}}, f8[] = {{4, 0}, {2, 0}, {1, 0}, {1, 2}},
+                 f16[] = {{8, 0}, {4, 0}, {2, 0}, {2, 2}, {1, 0}, {1, 1}, {1, 2}, {1, 3}};
+  const F *f = R == 4 ? f4 : (R == 8 ? f8 : f16);
   const double two_pi = 6.283185307179586476925286766559;
-  int64_t Ls = 1;
-  for (int p = 0; p < s.n; ++p) {
-    const int R = s.r[p];
-    if (Ls > 1) {
-      float2 *t = out + tw_offset(s, p);
-      const int64_t len = Ls * R;
-      for (int64_t k = 0; k < Ls; ++k) {
-        for (int m = 0; m < R; ++m) {
-          // reduce m*k modulo len before scaling: the angle index stays exact
-          const int64_t e = (m * k) % len;
-          const double a = -two_pi * (double)e / (double)len;
-          t[k * R + m] = make_float2((float)std::cos(a), (float)std::sin(a));
-        }
-      }
-    }
-    Ls *= R;
+  for (int i = 0; i < R / 2; ++i) {
+    const double ang = two_pi * ((double)(f[i].pw * k) / (double)(Ls * R) + f[i].num / 16.0);
+    double c = std::cos(ang);
+    if (std::fabs(c) < TW_MIN_COS) c = TW_MIN_COS;
+    out[i] = make_float2((float)c, (float)(std::sin(ang) / c));
   }
-  (void)N;
+}
+
+// The table of one pass: factors 2h, 2h + 1 of row k at float2 index 2 (h Ls + k).
+static void tw_pass(int R, int64_t Ls, float2 *out) {
+  float2 f[8];
+  for (int64_t k = 0; k < Ls; ++k) {
+    tw_factors(R, Ls, k, f);
+    for (int h = 0; h < R / 4; ++h) {
+      out[2 * (h * Ls + k)] = f[2 * h];
+      out[2 * (h * Ls + k) + 1] = f[2 * h + 1];
+    }
+  }
 }
 
 // --------------------------------------------------------- device caches
@@ -155,7 +162,8 @@ const float2 *twiddles_device(int N, bool rev) {
   if (rev) s = reversed(s);
   const int64_t sz = tw_size(s) < 2 ? 2 : tw_size(s);
   std::vector<float2> host((size_t)sz, make_float2(1.f, 0.f));
-  build_twiddles(N, s, host.data());
+  for (int p = 0; p < s.n; ++p)
+    if (pass_ls(s, p) > 1) tw_pass(s.r[p], pass_ls(s, p), host.data() + tw_offset(s, p));
   float2 *d = nullptr;
   if (hipMalloc(&d, sizeof(float2) * sz) != hipSuccess) return nullptr;
   // a synchronous copy: tables are built once per (device, size), before use
@@ -211,29 +219,17 @@ namespace {
 std::map<TwKey, float4 *> g_pb;
 }
 
-const float4 *pow_base_device(int N, int Ls) {
+const float4 *tw16_device(int Ls) {
   const int dev = device_id();
   std::lock_guard<std::mutex> g(g_tw_mu);
-  TwKey key{dev, N, Ls};
+  TwKey key{dev, 16, Ls};
   auto it = g_pb.find(key);
   if (it != g_pb.end()) return it->second;
-  const double two_pi = 6.283185307179586476925286766559;
-  const int64_t len = (int64_t)16 * Ls;
-  std::vector<float4> host((size_t)Ls * 2);
-  for (int64_t k = 0; k < Ls; ++k) {
-    float2 w[4];
-    const int pw[4] = {1, 2, 4, 8};
-    for (int i = 0; i < 4; ++i) {
-      const int64_t e = (pw[i] * k) % len;
-      const double ang = -two_pi * (double)e / (double)len;
-      w[i] = make_float2((float)std::cos(ang), (float)std::sin(ang));
-    }
-    host[2 * k] = make_float4(w[0].x, w[0].y, w[1].x, w[1].y);
-    host[2 * k + 1] = make_float4(w[2].x, w[2].y, w[3].x, w[3].y);
-  }
+  std::vector<float2> host((size_t)Ls * 8);
+  tw_pass(16, Ls, host.data());
   float4 *d = nullptr;
-  if (hipMalloc(&d, sizeof(float4) * host.size()) != hipSuccess) return nullptr;
-  if (hipMemcpy(d, host.data(), sizeof(float4) * host.size(), hipMemcpyHostToDevice) != hipSuccess) {
+  if (hipMalloc(&d, sizeof(float2) * host.size()) != hipSuccess) return nullptr;
+  if (hipMemcpy(d, host.data(), sizeof(float2) * host.size(), hipMemcpyHostToDevice) != hipSuccess) {
     (void)hipFree(d);
     return nullptr;
   }
@@ -314,7 +310,7 @@ static void clear_workspaces() {
 CacheClearRegistrar g_reg_ws(clear_workspaces);
 
 // Plans (pulse-compression and ragged) keep raw pointers to the twiddle and
-// power-base tables; while any plan is alive mxr_clear_caches leaves the
+// factor tables; while any plan is alive mxr_clear_caches leaves the
 // tables in place (a few hundred KiB), so a live plan never reads freed memory.
 namespace {
 int g_live_plans = 0;  // guarded by g_tw_mu

@@ -183,3 +183,38 @@ def test_pulse_compression_plan(mx, orc):
     with pytest.raises(mx.MatxError):
         plan(dev(np.zeros((2, S - 1), np.complex64)))   # wrong row length
     plan.close()
+
+
+@pytest.mark.parametrize("S,L,n,C", [(16384, 1000, 16384, 3), (16379, 1000, 16384, 3), (9000, 1000, 32768, 5),
+                                     (32768, 3001, 32768, 1), (30001, 3001, 32768, 3), (4096, 900, 4096, 1)])
+def test_pulse_compression_wrapping_blocks(mx, S, L, n, C):
+    """All n lags of a plan whose overlap-save blocks run past the period
+    (samples from the row's start again) or past the row's last sample, for
+    blocks of 4096 and 8192 points, against numpy's FP64 FFT."""
+    rng = np.random.default_rng(S + L)
+    x = (rng.standard_normal((C, S)) + 1j * rng.standard_normal((C, S))).astype(np.complex64)
+    w = (rng.standard_normal(L) + 1j * rng.standard_normal(L)).astype(np.complex64)
+    plan = mx.ops.PulseCompressionPlan(S, L, n, n, window=False, normalize=False)
+    plan.set_waveform(dev(w))
+    ref = np.fft.ifft(np.fft.fft(x.astype(complex), n) * np.conj(np.fft.fft(w.astype(complex), n)))
+    assert rel(host(plan(dev(x))), ref) < RTOL
+    plan.close()
+
+
+@pytest.mark.parametrize("L", [700, 3000])
+@pytest.mark.parametrize("log2n", [27, 28])
+def test_pulse_compression_long_period(mx, L, log2n):
+    """The largest period of the block kernels' 32-bit byte offsets and the one
+    past it (the general kernel), on short rows: both give the lags of a short
+    period that already covers every nonzero one."""
+    rng = np.random.default_rng(L)
+    S, nout = 9001, 9001 - L + 1
+    x = dev((rng.standard_normal((2, S)) + 1j * rng.standard_normal((2, S))).astype(np.complex64))
+    w = dev((rng.standard_normal(L) + 1j * rng.standard_normal(L)).astype(np.complex64))
+    y = []
+    for n in (16384, 1 << log2n):
+        plan = mx.ops.PulseCompressionPlan(S, L, n, nout)
+        plan.set_waveform(w)
+        y.append(host(plan(x)))
+        plan.close()
+    assert rel(y[1], y[0]) < RTOL
