@@ -22,6 +22,7 @@
 #include "fft_engine.hpp"
 #include "mxr_cache.hpp"
 #include "pcgrad.hpp"
+#include "ragged.hpp"
 
 namespace mxr {
 
@@ -121,92 +122,105 @@ __global__ __launch_bounds__(WgT<M>::NT) void pc_wgrad_kernel(WgArgs a) {
 }
 
 // M = 8192: the transforms of the 8192-point pulse-compression kernel
-// (radix 2 x 16 x 16 x 16, 512 threads, the radix-2 pass folded into the
-// load, factor tables for Ls = 2, 32, 512), so the x spectrum, the gy
-// spectrum and the running product take 16 bins each per thread (bins
-// j + 512q).  Those three live sets need more than the 128 VGPRs of two
-// workgroups per CU, so it runs one (up to 256 VGPRs, no spills).
+// (radix 2 x 16 x 16 x 16, the radix-2 pass folded into the load).  Threads
+// 0-511 transform the block of x and threads 512-1023 that of gy, side by
+// side in an LDS buffer each (bins j + 512q of thread j); then each half
+// multiplies and accumulates one half of the bins, the other transform's
+// through LDS.
+// One 16-wave workgroup per CU at 128 VGPRs; with both transforms in the same
+// 512 threads one after the other, the two spectra and the running product
+// took 242 VGPRs, eight waves per CU: 2610 us against 2207 on 16 x 512 x 32768.
+// The next block's samples are loaded before the last pass (nothing is stored
+// in the walk, so no wait for a load waits for a store).
 struct Wg8192Args {
   WgArgs a;
-  const float4 *bA, *bB, *bC;
+  const float4 *bA, *bB, *bC;  // factors of passes Ls = 2, 32, 512
 };
 
-// Forward 8192-point transform of ld(i); bins j + 512q end in v[q].  Pre:
-// the workgroup's previous LDS reads are done.  Post: LDS is free (the last
-// exchange ends with a barrier).
-template <class LoadF>
-__device__ __forceinline__ void fwd8192_regs(float2 (&v)[16], LoadF &&ld, const float4 *bA,
-                                             const float4 *bB, const float4 *bC, float2 *lds) {
-  constexpr int NT = 512;
-  using LY = Layout<8192, 1, false>;
-  const int j = threadIdx.x;
-  auto xchg = [&](int ls_out) {
-    const int k = j & (ls_out - 1), base = (j - k) * 16 + k;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) lds[LY::addr(0, base + q * ls_out)] = v[q];
-    wg_barrier();
-#pragma unroll
-    for (int m = 0; m < 16; ++m) v[m] = lds[LY::addr(0, j + m * NT)];
-    wg_barrier();
-  };
-  {
-    const int jh = j >> 1;
-    const bool odd = (j & 1) != 0;
-    float2 a[16], b[16];
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      a[m] = ld(jh + 256 * m);
-      b[m] = ld(jh + 256 * m + 4096);
-    }
-#pragma unroll
-    for (int m = 0; m < 16; ++m) v[m] = odd ? csub(a[m], b[m]) : cadd(a[m], b[m]);
-  }
-  TwRow<16> tw = load_tw<16>(bA, 2, j & 1);
-  dft_tw<false>(v, tw);  // Ls = 2
-  tw = load_tw<16>(bB, 32, j & 31);
-  xchg(2);
-  dft_tw<false>(v, tw);  // Ls = 32
-  tw = load_tw<16>(bC, 512, j);
-  xchg(32);
-  dft_tw<false>(v, tw);  // Ls = 512
-}
-
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4)))
 void wgrad8192_kernel(Wg8192Args p) {
   using LY = Layout<8192, 1, false>;
-  __shared__ float2 lds[LY::LDS_ELEMS];
+  __shared__ float2 lds2[2][LY::LDS_ELEMS];
   const WgArgs &a = p.a;
-  const int j = threadIdx.x;
-  float2 acc[16];
+  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 9);
+  const int j = threadIdx.x & 511;
+  float2 *const lds = lds2[half];
+  const int rbase = lds_pad(j);
+  float2 acc[8], v[16];
 #pragma unroll
-  for (int q = 0; q < 16; ++q) acc[q] = make_float2(0.f, 0.f);
-  for (int64_t it = blockIdx.x; it < a.items; it += gridDim.x) {
-    // (the previous item's last exchange ended with a barrier)
-    const int64_t row = it / a.nblk;
-    const int lo = (int)(it % a.nblk) * a.V;
+  for (int q = 0; q < 8; ++q) acc[q] = make_float2(0.f, 0.f);
+  auto xchg = [&](int ls_out) {
+    const int k = j & (ls_out - 1), wbase = lds_pad((j - k) * 16 + k);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) lds[wbase + (ls_out == 2 ? 2 * q + (q >= 8) : 34 * q)] = v[q];
+    wg_barrier();
+#pragma unroll
+    for (int m = 0; m < 16; ++m) v[m] = lds[rbase + 544 * m];
+    wg_barrier();
+  };
+  // samples i0 + 256 m of item it's block of x (wrapping at n, zero from seff
+  // on) or of gy (zero from the block's last kept lag on)
+  auto fetch = [&](int64_t it, float2 (&u)[16]) {
+    const uint32_t row = (uint32_t)it / (uint32_t)a.nblk;
+    const int lo = (int)((uint32_t)it - row * (uint32_t)a.nblk) * a.V;
     int64_t ox, oy;
-    batch_offsets(a.bi, row, &ox, &oy);
-    const float2 *xr = a.x + ox;
-    const float2 *gr = a.gy + oy;
-    const int n32 = a.n, seff = a.seff;
-    const int lim = (a.nout - lo) < a.V ? (a.nout - lo) : a.V;
-    float2 X[16], Gv[16];
-    fwd8192_regs(X, [&](int i) {
-      int gi = lo + i;
-      if (gi >= n32) gi -= n32;
-      return gi < seff ? xr[gi] : make_float2(0.f, 0.f);
-    }, p.bA, p.bB, p.bC, lds);
-    fwd8192_regs(Gv, [&](int i) { return i < lim ? gr[lo + i] : make_float2(0.f, 0.f); }, p.bA,
-                 p.bB, p.bC, lds);
+    batch_offsets32(a.bi, row, &ox, &oy);
+    int jo = j;
+    asm volatile("" : "+v"(jo));  // the offsets are formed here, not kept across the walk
+    const int i0 = (jo >> 1) + (jo & 1) * 4096;
+    if (half || lo + 8192 <= a.n) {
+      const float2 *src = half ? a.gy + oy + lo : a.x + ox + lo;
+      int len = half ? ((a.nout - lo) < a.V ? (a.nout - lo) : a.V) : a.seff - lo;
+      len = len < 0 ? 0 : (len > 8192 ? 8192 : len);
+      const buf_rsrc r = make_rsrc(src, len * 8);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      acc[q].x += X[q].x * Gv[q].x + X[q].y * Gv[q].y;  // X conj(G)
-      acc[q].y += X[q].y * Gv[q].x - X[q].x * Gv[q].y;
+      for (int m = 0; m < 16; ++m) u[m] = buf_load2(r, (i0 + 256 * m) * 8);
+    } else {
+      const buf_rsrc r = make_rsrc(a.x + ox, a.seff * 8);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        const int gi = lo + i0 + 256 * m;
+        u[m] = buf_load2(r, (int)min((uint32_t)gi, (uint32_t)(gi - a.n)) * 8);
+      }
     }
-  }
-  float2 *pp = a.partial + (int64_t)blockIdx.x * 8192;
+  };
+  // the grid has at most one workgroup per item
+  int64_t it = blockIdx.x;
+  fetch(it, v);
+  for (;;) {
+    pair_dft2(v, (j & 1) != 0);
+    TwRow<16> tw = load_tw<16>(opaque(p.bA), 2, j & 1);
+    dft_tw<false>(v, tw);  // Ls = 2
+    tw = load_tw<16>(opaque(p.bB), 32, j & 31);
+    xchg(2);
+    dft_tw<false>(v, tw);  // Ls = 32
+    tw = load_tw<16>(opaque(p.bC), 512, j);
+    xchg(32);
+    it += gridDim.x;
+    float2 nx[16];
+    const bool more = it < a.items;
+    if (more) fetch(it, nx);
+    dft_tw<false>(v, tw);  // Ls = 512: bins j + 512q
+    // the x half takes bins q < 8, the gy half the others: each leaves the
+    // other's bins in its own buffer
 #pragma unroll
-  for (int q = 0; q < 16; ++q) pp[j + 512 * q] = acc[q];
+    for (int q = 0; q < 8; ++q) lds[j + 512 * q] = half ? v[q] : v[q + 8];
+    wg_barrier();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float2 o = lds2[half ^ 1][j + 512 * q];
+      const float2 x = half ? o : v[q], g = half ? v[q + 8] : o;
+      acc[q].x += x.x * g.x + x.y * g.y;  // X conj(G)
+      acc[q].y += x.y * g.x - x.x * g.y;
+    }
+    if (!more) break;
+    wg_barrier();  // the buffers are free again
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = nx[q];
+  }
+  float2 *pp = a.partial + (int64_t)blockIdx.x * 8192 + half * 4096;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) pp[j + 512 * q] = acc[q];
 }
 
 // spec[k] = sum over workgroups g of partial[g][k], in order, in double.
@@ -298,8 +312,10 @@ static mxr_status wgrad_run(const WgradJob &j, hipStream_t s) {
   if (items > 0) {
     int per_cu = 1, cus = 0;
     hipError_t oe;
-    if constexpr (M == 8192)
-      oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad8192_kernel, 512, 0);
+    // the dedicated kernel's 32-bit block numbers and byte offsets
+    const bool w8 = M == 8192 && j.n <= PC_BUF_MAX_N && items < (1ll << 31);
+    if (w8)
+      oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad8192_kernel, 1024, 0);
     else
       oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pc_wgrad_kernel<M>, T::NT, 0);
     if (oe != hipSuccess || per_cu < 1) per_cu = 1;
@@ -322,12 +338,12 @@ static mxr_status wgrad_run(const WgradJob &j, hipStream_t s) {
     a.V = (int)j.V;
     a.partial = ws;
     a.twf = twf;
-    if constexpr (M == 8192) {
+    if (w8) {
       Wg8192Args p{a, tw16_device(2), tw16_device(32), tw16_device(512)};
       MXR_REQUIRE(p.bA && p.bB && p.bC, MXR_OUT_OF_MEMORY,
                   "pc waveform gradient: twiddle table allocation failed");
       ProfScope ps("wgrad8192_kernel", s);
-      wgrad8192_kernel<<<dim3((unsigned)grid), dim3(512), 0, s>>>(p);
+      wgrad8192_kernel<<<dim3((unsigned)grid), dim3(1024), 0, s>>>(p);
     } else {
       ProfScope ps("pc_wgrad_kernel", s);
       pc_wgrad_kernel<M><<<dim3((unsigned)grid), dim3(T::NT), 0, s>>>(a);
