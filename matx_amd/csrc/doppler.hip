@@ -4,11 +4,12 @@
 // CFARDetections, examples/simple_radar_pipeline.h:321-357,398).
 //
 // A workgroup owns a tile of TR consecutive range bins of one channel across
-// all P pulses.  It loads the tile with coalesced TR-wide row reads into LDS,
-// evaluates the canceller and the window while feeding the first Stockham
-// pass, runs the remaining passes down the LDS columns (element (pulse i,
-// range t) at i*TR + t, so consecutive lanes touch consecutive words), and
-// writes the range-Doppler map and/or its power with TR-wide coalesced rows.
+// all P pulses.  Each thread loads a strip of pulses of one range bin (TR-wide
+// coalesced row reads), applies the canceller and the window in registers and
+// leaves the Doppler-input rows in LDS; the Stockham passes run down the LDS
+// columns (range bins of a row side by side, so consecutive lanes touch
+// consecutive words), and the last one writes the range-Doppler map and/or its
+// power with TR-wide coalesced rows.
 // HBM traffic per tile: P*TR*8 bytes in, nd*TR*(4 and/or 8) bytes out.
 #include "fft_engine.hpp"
 #include "mxr_cache.hpp"
@@ -29,93 +30,115 @@ struct DopCfg {
   static constexpr int TR = ND <= 128 ? 32 : (ND <= 512 ? 16 : 8);
 };
 
-// Coalesced load of a pulse tile: rows p < P of TR range bins from r0 into
-// lds[p * TR + t] (zero past R), 16 loads in flight per lane.
-template <int ND, int TR = DopCfg<ND>::TR, int NT = DopCfg<ND>::NT>
-__device__ __forceinline__ void load_pulse_tile(const float2 *yc, int64_t ys_p, int64_t ys_r,
-                                                int P, int R, int r0, float2 *lds) {
-  constexpr int RPI = NT / TR;  // pulses covered by one sweep of the workgroup
-  constexpr int BATCH = 16;
-  const int t = threadIdx.x % TR, p0 = threadIdx.x / TR;
-  const int r = r0 + t;
-  const bool rok = r < R;
-  const float2 *col = yc + (int64_t)r * ys_r;
-  for (int pb = 0; pb < P; pb += RPI * BATCH) {
-    float2 v[BATCH];
+// LDS layout of a tile: rows of TR range bins, padded below 32 bins (see
+// Layout); ND >= 32 where there is anything to pad.
+template <int ND, int TR>
+using DopLayout = Layout<ND, TR, true, (TR < 32 && ND >= 32)>;
+
+// Doppler-input rows win[i] * canceller(y)[i] of TR range bins from r0 into LDS
+// (element (i, t) at the layout's place; zero from rows_t on).  A thread forms
+// a strip of consecutive rows of one column: it loads the strip's pulses and
+// one on either side, all in flight together, and applies the canceller and
+// the window in registers, one LDS write an element (staging the pulses and
+// reading three per row back takes three more LDS accesses an element and a
+// barrier).  With y32 the loads go through a buffer resource over the channel,
+// which reads pulses outside it as zeros; columns past R then hold whatever
+// follows the row (never stored).
+template <int ND, int TR, int NT, class A>
+__device__ __forceinline__ void load_canceller(const A &a, int c, int r0, float2 *lds, const float *win) {
+  using LY = DopLayout<ND, TR>;
+  constexpr int SR = ND * TR >= NT ? ND * TR / NT : 1;  // rows per strip
+  constexpr int NS = ND / SR;                           // strips per column
+  const int t = threadIdx.x % TR, s = threadIdx.x / TR;
+  if (NS * TR < NT && s >= NS) return;
+  const int i0 = s * SR, pb = i0 + a.p_off - 1;  // pulse held in v[0]
+  float2 v[SR + 2];
+  if (a.y32) {
+    const buf_rsrc ry = make_rsrc(a.y + (int64_t)c * a.ys_c, ((a.P - 1) * (int)a.ys_p + a.R) * 8);
+    const int step = (int)a.ys_p * 8;
+    int off = pb * step + (r0 + t) * 8;
 #pragma unroll
-    for (int u = 0; u < BATCH; ++u) {
-      const int p = pb + p0 + u * RPI;
-      v[u] = (rok && p < P) ? col[(int64_t)p * ys_p] : make_float2(0.f, 0.f);
-    }
+    for (int u = 0; u < SR + 2; ++u, off += step) v[u] = buf_load2(ry, off);
+  } else {
+    const float2 *col = a.y + (int64_t)c * a.ys_c + (int64_t)min(r0 + t, a.R - 1) * a.ys_r;
 #pragma unroll
-    for (int u = 0; u < BATCH; ++u) {
-      const int p = pb + p0 + u * RPI;
-      if (p < P) lds[p * TR + t] = v[u];
+    for (int u = 0; u < SR + 2; ++u) {
+      const int p = pb + u;
+      v[u] = keep_if(col[(int64_t)min(max(p, 0), a.P - 1) * a.ys_p], p >= 0 && p < a.P);
     }
+  }
+#pragma unroll
+  for (int u = 0; u < SR; ++u) {
+    const int i = i0 + u;
+    const float2 m = v[u + 1];
+    const float2 x = a.no_tpc ? m
+                              : make_float2(v[u].x + v[u + 2].x - 2.0f * m.x, v[u].y + v[u + 2].y - 2.0f * m.y);
+    lds[LY::addr(t, i)] = keep_if(cscale(x, win[i]), i < a.rows_t);
   }
 }
 
-// One tile: TR range bins from r0 of channel c.  lds holds rows_buf * TR
-// elements, win ND floats.  Pre: the workgroup's previous use of both is
-// finished.
-template <int ND, int TR = DopCfg<ND>::TR, int NT = DopCfg<ND>::NT>
-__device__ __forceinline__ void doppler_tile(const DopArgs &a, int c, int r0, int rows_buf,
-                                             float2 *lds, float *win) {
-  using LY = Layout<ND, TR, true>;
-  using SQ = Seq<ND, false>;
-  constexpr int K = SQ::n;
+template <int ND, int NT, class A>
+__device__ __forceinline__ void load_window(const A &a, float *win) {
   for (int i = threadIdx.x; i < ND; i += NT) {
     float h = 0.f;
     if (i < a.rows_t)
       h = a.taps ? a.taps[(int64_t)i * a.taps_s] : (i < a.win_rows ? hamming_f32(i, a.win_rows) : 1.0f);
     win[i] = h;
   }
-  load_pulse_tile<ND, TR, NT>(a.y + (int64_t)c * a.ys_c, a.ys_p, a.ys_r, a.P, a.R, r0, lds);
-  wg_barrier();
+}
 
-  auto tpc = [&](int t, int i) -> float2 {
-    if (i >= a.rows_t) return make_float2(0.f, 0.f);
-    const int p = i + a.p_off;
-    float2 m = lds[p * TR + t];
-    if (a.no_tpc) return cscale(m, win[i]);
-    float2 s = p >= 1 ? lds[(p - 1) * TR + t] : make_float2(0.f, 0.f);
-    float2 u = p + 1 < a.P ? lds[(p + 1) * TR + t] : make_float2(0.f, 0.f);
-    float2 v = make_float2(s.x + u.x - 2.0f * m.x, s.y + u.y - 2.0f * m.y);
-    return cscale(v, win[i]);
-  };
-  auto store_out = [&](int t, int k, float2 v) {
+// One tile: TR range bins from r0 of channel c.  lds holds the layout's
+// elements, win ND floats.  Pre: the workgroup's previous use of both is
+// finished.
+template <int ND, int TR = DopCfg<ND>::TR, int NT = DopCfg<ND>::NT>
+__device__ __forceinline__ void doppler_tile(const DopArgs &a, int c, int r0, float2 *lds, float *win) {
+  using LY = DopLayout<ND, TR>;
+  using SQ = Seq<ND, false>;
+  constexpr int K = SQ::n;
+  load_window<ND, NT>(a, win);
+  __syncthreads();
+  load_canceller<ND, TR, NT>(a, c, r0, lds, win);
+  wg_barrier();
+  lds_passes<LY, SQ, ND, NT, TR, false, 0, K - 1>(lds, a.tw);
+  constexpr int RL = SQ::template R<K - 1>;
+  constexpr int LSL = SQ::template LS<K - 1>;
+  Pass<LY, RL, ND, NT, TR> pl;
+  pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
+  pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
+  if (a.out32) {  // columns past R are dropped by the range check
+    constexpr int FAR = 0x7ffffff0;
+    if (a.pw) {
+      const buf_rsrc rp = make_rsrc(a.pw + (int64_t)c * a.ps_c, ((ND - 1) * (int)a.ps_k + a.R) * 4);
+      pl.template store<LSL>([&](int t, int k, float2 v) {
+        buf_store1(rp, r0 + t < a.R ? (k * (int)a.ps_k + r0 + t) * 4 : FAR, cabs2(v));
+      });
+    }
+    if (a.rd) {
+      const buf_rsrc rr = make_rsrc(a.rd + (int64_t)c * a.rs_c, ((ND - 1) * (int)a.rs_k + a.R) * 8);
+      pl.template store<LSL>([&](int t, int k, float2 v) {
+        buf_store2(rr, r0 + t < a.R ? (k * (int)a.rs_k + r0 + t) * 8 : FAR, v);
+      });
+    }
+    return;
+  }
+  pl.template store<LSL>([&](int t, int k, float2 v) {
     const int r = r0 + t;
     if (r >= a.R) return;
     if (a.rd) a.rd[(int64_t)c * a.rs_c + (int64_t)k * a.rs_k + (int64_t)r * a.rs_r] = v;
     if (a.pw) a.pw[(int64_t)c * a.ps_c + (int64_t)k * a.ps_k + (int64_t)r * a.ps_r] = cabs2(v);
-  };
-
-  constexpr int R0 = SQ::template R<0>;
-  Pass<LY, R0, ND, NT, TR> p0;
-  p0.load(tpc);
-  if constexpr (K == 1) {
-    p0.template compute<1, false>(nullptr);
-    p0.template store<1>(store_out);
-  } else {
-    wg_barrier();  // every canceller read is done before the tile is overwritten
-    p0.template compute<1, false>(nullptr);
-    p0.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
-    wg_barrier();
-    lds_passes<LY, SQ, ND, NT, TR, false, 1, K - 1>(lds, a.tw);
-    constexpr int RL = SQ::template R<K - 1>;
-    constexpr int LSL = SQ::template LS<K - 1>;
-    Pass<LY, RL, ND, NT, TR> pl;
-    pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
-    pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
-    pl.template store<LSL>(store_out);
-  }
+  });
 }
 
+// Neighbouring tiles share cache lines when rows are not line-aligned (and a
+// tile narrower than a line always does): they go to one XCD's L2.
 template <int ND>
-__global__ __launch_bounds__(DopCfg<ND>::NT) void doppler_kernel(DopArgs a, int rows_buf) {
-  extern __shared__ float2 lds[];  // rows_buf * TR
-  __shared__ float win[ND];
-  doppler_tile<ND>(a, blockIdx.y, blockIdx.x * DopCfg<ND>::TR, rows_buf, lds, win);
+__global__ __launch_bounds__(DopCfg<ND>::NT) void doppler_kernel(DopArgs a) {
+  __shared__ float2 lds[DopLayout<ND, DopCfg<ND>::TR>::LDS_ELEMS];
+  __shared__ __align__(16) float win[ND];
+  const uint32_t tiles = (uint32_t)(a.R + DopCfg<ND>::TR - 1) / DopCfg<ND>::TR;
+  const uint32_t g = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t c = g / tiles;
+  doppler_tile<ND>(a, (int)c, (int)(g - c * tiles) * DopCfg<ND>::TR, lds, win);
 }
 
 // Ragged batch: the (job, channel, tile) items of every job of one Doppler
@@ -140,14 +163,13 @@ __global__ __launch_bounds__(DopBatchCfg<ND>::NT) void doppler_batch_kernel(cons
                                                                           const int *item_job,
                                                                           int64_t items) {
   constexpr int TR = DopBatchCfg<ND>::TR;
-  __shared__ float2 lds[ND * TR];
-  __shared__ float win[ND];
+  __shared__ float2 lds[DopLayout<ND, TR>::LDS_ELEMS];
+  __shared__ __align__(16) float win[ND];
   auto item = [&](int64_t it) {
     const int ji = item_job ? __builtin_amdgcn_readfirstlane(item_job[it]) : 0;
     const DopJob jb = uniform_copy(&jobs[ji]);
-    const int64_t local = it - jb.item0;
-    doppler_tile<ND, TR, DopBatchCfg<ND>::NT>(jb.a, (int)(local / jb.tiles), (int)(local % jb.tiles) * TR,
-                                             ND, lds, win);
+    const uint32_t local = (uint32_t)(it - jb.item0), c = local / (uint32_t)jb.tiles;
+    doppler_tile<ND, TR, DopBatchCfg<ND>::NT>(jb.a, (int)c, (int)(local - c * (uint32_t)jb.tiles) * TR, lds, win);
   };
   if constexpr (!PERSIST) {
     item(blockIdx.x);
@@ -210,17 +232,11 @@ int doppler_batch_tile(int nd) {
 template <int ND>
 static mxr_status launch_doppler(const DopArgs &a, hipStream_t s) {
   constexpr int TR = DopCfg<ND>::TR;
-  const int rows_buf = a.P > ND ? a.P : ND;
-  const size_t lds = (size_t)rows_buf * TR * sizeof(float2);
-  MXR_REQUIRE(lds + ND * sizeof(float) <= (size_t)max_lds_per_block(), MXR_NOT_SUPPORTED,
-              "doppler: %d pulses x %d range bins do not fit in LDS", rows_buf, TR);
-  if (lds + ND * sizeof(float) > 65536)
-    MXR_HIP_TRY(hipFuncSetAttribute((const void *)doppler_kernel<ND>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  dim3 grid((a.R + TR - 1) / TR, a.C);
+  const int64_t G = (int64_t)((a.R + TR - 1) / TR) * a.C;
+  MXR_REQUIRE(G < (1ll << 31), MXR_INVALID_SIZE, "doppler: too many tiles");
   {
     ProfScope ps("doppler_kernel", s);
-    doppler_kernel<ND><<<grid, dim3(DopCfg<ND>::NT), lds, s>>>(a, rows_buf);
+    doppler_kernel<ND><<<dim3((unsigned)G), dim3(DopCfg<ND>::NT), 0, s>>>(a);
   }
   MXR_HIP_TRY(hipGetLastError());
   return MXR_SUCCESS;
@@ -293,6 +309,9 @@ static mxr_status doppler_run(const mxr_tensor *pow_out, const mxr_tensor *rd_ou
   }
   MXR_REQUIRE(nd >= 2 && nd <= 1024 && (nd & (nd - 1)) == 0, MXR_NOT_SUPPORTED,
               "doppler: FFT size %lld must be a power of two in [2, 1024]", (long long)nd);
+  a.y32 = rows32(P, R, y->stride[1], y->stride[2], 8);
+  a.out32 = (!rd_out || rows32(nd, R, rd_out->stride[1], rd_out->stride[2], 8)) &&
+            (!pow_out || rows32(nd, R, pow_out->stride[1], pow_out->stride[2], 4));
   a.tw = twiddles_device((int)nd, false);
   MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "doppler: twiddle table allocation failed");
   switch (nd) {
@@ -362,30 +381,34 @@ struct DopGradArgs {
   int skip_zero;   // test each tile's gpow for all zeros first
   int C, P, R, tiles;
   int rows_t, p_off, no_tpc, win_rows;
-  const float2 *tw;
+  int y32, gp32, gy32;  // rows32 of each
+  const float2 *tw, *twi;  // tables of the forward and of the reversed sequence
 };
 
-// Adjoint tiles: as the forward's, except at 512 Doppler bins, where two
-// transforms per tile favour occupancy: 8 range bins (32 KiB) measured 17 %
-// faster than 16 and 2x faster than 4.
+// Adjoint tiles: as the forward's, except at 512 Doppler bins, where 8 range
+// bins and 256 threads (four workgroups per CU) measure 1057 us on
+// 16 x 512 x 28673, 8 x 512 threads 1133, 16 x 512 1084, 16 x 256 1133.
 template <int ND>
 struct DopAdjCfg {
   static constexpr int TR = ND == 512 ? 8 : DopCfg<ND>::TR;
+  static constexpr int NT = ND == 512 ? 256 : DopCfg<ND>::NT;
 };
 
 template <int ND>
-__global__ __launch_bounds__(DopCfg<ND>::NT) void doppler_adj_kernel(DopGradArgs a) {
-  constexpr int NT = DopCfg<ND>::NT;
+__global__ __launch_bounds__(DopAdjCfg<ND>::NT) void doppler_adj_kernel(DopGradArgs a) {
+  constexpr int NT = DopAdjCfg<ND>::NT;
   constexpr int TR = DopAdjCfg<ND>::TR;
   static_assert(TR <= 64 && 64 % TR == 0, "range tile must divide a wave");
-  using LY = Layout<ND, TR, true>;
+  using LY = DopLayout<ND, TR>;
   using SQ = Seq<ND, false>;
+  using SI = Seq<ND, true>;
   constexpr int K = SQ::n;
-  extern __shared__ float2 lds[];  // max(P, ND) * TR: y tile, then D, then gu
-  __shared__ float win[ND];
-  const int c = blockIdx.y;
-  const int r0 = blockIdx.x * TR;
-  float *part = a.partial ? a.partial + ((int64_t)c * a.tiles + blockIdx.x) * a.P : nullptr;
+  __shared__ float2 lds[LY::LDS_ELEMS];  // the windowed canceller rows, then D, then gu
+  __shared__ __align__(16) float win[ND];
+  const uint32_t g0 = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+  const int c = (int)(g0 / (uint32_t)a.tiles), tile = (int)(g0 - (uint32_t)c * (uint32_t)a.tiles);
+  const int r0 = tile * TR;
+  float *part = a.partial ? a.partial + ((int64_t)c * a.tiles + tile) * a.P : nullptr;
   float2 *gyc = a.gy ? a.gy + (int64_t)c * a.gys_c : nullptr;
   const float *gpc = a.gp + (int64_t)c * a.gs_c;
   if (a.skip_zero) {
@@ -408,89 +431,90 @@ __global__ __launch_bounds__(DopCfg<ND>::NT) void doppler_adj_kernel(DopGradArgs
       return;
     }
   }
-  for (int i = threadIdx.x; i < ND; i += NT) {
-    float h = 0.f;
-    if (i < a.rows_t)
-      h = a.taps ? a.taps[(int64_t)i * a.taps_s] : (i < a.win_rows ? hamming_f32(i, a.win_rows) : 1.0f);
-    win[i] = h;
-  }
-  load_pulse_tile<ND, TR>(a.y + (int64_t)c * a.ys_c, a.ys_p, a.ys_r, a.P, a.R, r0, lds);
+  load_window<ND, NT>(a, win);
+  __syncthreads();
+  load_canceller<ND, TR, NT>(a, c, r0, lds, win);
   wg_barrier();
 
-  // forward: first pass fed by the windowed canceller, the rest in LDS; the
-  // last forward pass stores gD = 2 gpow D.  The gpow values of the last
-  // pass's outputs are fetched before its LDS reads (column clamped, zeroed
-  // past R by a mask, so the loads issue back to back).
+  // forward passes; the last one's outputs are the first inverse pass's
+  // inputs (the inverse runs the reversed radix sequence), so gD = 2 gpow D
+  // is formed in registers between them.  The gpow values are fetched before
+  // the last pass's LDS reads.
   constexpr int RL = SQ::template R<K - 1>;
   constexpr int LSL = SQ::template LS<K - 1>;
   using PL = Pass<LY, RL, ND, NT, TR>;
-  float gpv[PL::BPT][RL];
-  auto fetch_gp = [&]() {
-    PL::template outputs<LSL>([&](int u, int q, int t, int k) {
-      const int r = r0 + t;
-      const float g = gpc[(int64_t)k * a.gs_k + (int64_t)min(r, a.R - 1) * a.gs_r];
-      gpv[u][q] = __int_as_float(__float_as_int(g) & (r < a.R ? -1 : 0));
-    });
-  };
-  auto store_gd = [&](PL &pl) {
-    PL::template outputs<LSL>([&](int u, int q, int t, int k) {
-      lds[LY::addr(t, k)] = cscale(pl.v[u][q], 2.0f * gpv[u][q]);
-    });
-  };
-  constexpr int R0 = SQ::template R<0>;
-  Pass<LY, R0, ND, NT, TR> p0;
-  if constexpr (K == 1) fetch_gp();
-  p0.load([&](int t, int i) -> float2 {
-    if (i >= a.rows_t) return make_float2(0.f, 0.f);
-    const int p = i + a.p_off;
-    const float2 m = lds[p * TR + t];
-    if (a.no_tpc) return cscale(m, win[i]);
-    const float2 s = p >= 1 ? lds[(p - 1) * TR + t] : make_float2(0.f, 0.f);
-    const float2 u = p + 1 < a.P ? lds[(p + 1) * TR + t] : make_float2(0.f, 0.f);
-    return cscale(make_float2(s.x + u.x - 2.0f * m.x, s.y + u.y - 2.0f * m.y), win[i]);
-  });
-  wg_barrier();  // every canceller read is done before the tile is overwritten
-  p0.template compute<1, false>(nullptr);
-  if constexpr (K == 1) {
-    store_gd(p0);
-  } else {
-    p0.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
-    wg_barrier();
-    lds_passes<LY, SQ, ND, NT, TR, false, 1, K - 1>(lds, a.tw);
+  lds_passes<LY, SQ, ND, NT, TR, false, 0, K - 1>(lds, a.tw);
+  {
+    float gpv[PL::BPT][RL];
+    if (a.gp32) {
+      const buf_rsrc rg = make_rsrc(gpc, ((ND - 1) * (int)a.gs_k + a.R) * 4);
+      PL::template outputs<LSL>([&](int u, int q, int t, int k) {
+        gpv[u][q] = buf_load1(rg, (k * (int)a.gs_k + r0 + t) * 4);
+      });
+    } else {
+      PL::template outputs<LSL>([&](int u, int q, int t, int k) {
+        gpv[u][q] = gpc[(int64_t)k * a.gs_k + (int64_t)min(r0 + t, a.R - 1) * a.gs_r];
+      });
+    }
     PL pl;
-    fetch_gp();
     pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
     wg_barrier();
     pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
-    store_gd(pl);
+    PL::template outputs<LSL>([&](int u, int q, int t, int k) {
+      // a column past R holds no data: its gradient stays finite
+      pl.v[u][q] = keep_if(cscale(pl.v[u][q], 2.0f * gpv[u][q]), r0 + t < a.R);
+    });
+    // gu = F^H gD, unscaled
+    pl.template compute<1, true>(nullptr);
+    pl.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
   }
   wg_barrier();
-  // gu = F^H gD: the same passes with conjugate twiddles, unscaled
-  lds_passes<LY, SQ, ND, NT, TR, true, 0, K>(lds, a.tw);
+  lds_passes<LY, SI, ND, NT, TR, true, 1, K>(lds, a.twi);
 
-  // window, canceller transpose, coalesced store; tap-gradient partials
+  // window, canceller transpose, coalesced store: a thread takes a strip of
+  // rows of one column, as in the load
   auto s_at = [&](int t, int i) -> float2 {
-    return (i >= 0 && i < a.rows_t) ? cscale(lds[LY::addr(t, i)], win[i]) : make_float2(0.f, 0.f);
+    const int ic = min(max(i, 0), ND - 1);
+    return keep_if(cscale(lds[LY::addr(t, ic)], win[ic]), i >= 0 && i < a.rows_t);
   };
-  const float2 *yc = a.y + (int64_t)c * a.ys_c;
-  for (int base = 0; base < a.P * TR; base += NT) {  // uniform trip count (shuffles)
-    const int idx = base + threadIdx.x;
-    const int p = idx / TR, t = idx % TR, r = r0 + t;
-    const bool ok = p < a.P && r < a.R;
-    float contrib = 0.f;
-    if (ok && gyc) {
-      const int i = p - a.p_off;
-      float2 g;
-      if (a.no_tpc) {
-        g = s_at(t, i);
+  if (gyc) {
+    constexpr int SR = ND * TR >= NT ? ND * TR / NT : 1;
+    constexpr int NS = ND / SR;
+    const int t = threadIdx.x % TR, st = threadIdx.x / TR, r = r0 + t;
+    auto grad = [&](float2 lo, float2 mid, float2 hi) {
+      return a.no_tpc ? mid : make_float2(lo.x + hi.x - 2.0f * mid.x, lo.y + hi.y - 2.0f * mid.y);
+    };
+    if (r < a.R && (NS * TR >= NT || st < NS)) {
+      const int p0 = st * SR;
+      float2 w[SR + 2];
+#pragma unroll
+      for (int u = 0; u < SR + 2; ++u) w[u] = s_at(t, p0 - a.p_off - 1 + u);
+      if (a.gy32) {  // rows past P are dropped by the range check
+        const buf_rsrc rg = make_rsrc(gyc, ((a.P - 1) * (int)a.gys_p + a.R) * 8);
+        const int step = (int)a.gys_p * 8;
+        int off = p0 * step + r * 8;
+#pragma unroll
+        for (int u = 0; u < SR; ++u, off += step) buf_store2(rg, off, grad(w[u], w[u + 1], w[u + 2]));
       } else {
-        const float2 lo = s_at(t, i - 1), mid = s_at(t, i), hi = s_at(t, i + 1);
-        g = make_float2(lo.x + hi.x - 2.0f * mid.x, lo.y + hi.y - 2.0f * mid.y);
+#pragma unroll
+        for (int u = 0; u < SR; ++u)
+          if (p0 + u < a.P)
+            gyc[(int64_t)(p0 + u) * a.gys_p + (int64_t)r * a.gys_r] = grad(w[u], w[u + 1], w[u + 2]);
       }
-      gyc[(int64_t)p * a.gys_p + (int64_t)r * a.gys_r] = g;
+      // a canceller without its end rows leaves up to two pulses past ND
+      for (int p = ND + st; p < a.P; p += NS) {
+        const int i = p - a.p_off;
+        gyc[(int64_t)p * a.gys_p + (int64_t)r * a.gys_r] = grad(s_at(t, i - 1), s_at(t, i), s_at(t, i + 1));
+      }
     }
-    if (part) {  // no canceller here: row p of gu pairs with pulse p
-      if (ok) {
+  }
+  if (part) {  // tap-gradient partials; no canceller here: row p of gu pairs with pulse p
+    const float2 *yc = a.y + (int64_t)c * a.ys_c;
+    for (int base = 0; base < a.P * TR; base += NT) {  // uniform trip count (shuffles)
+      const int idx = base + threadIdx.x;
+      const int p = idx / TR, t = idx % TR, r = r0 + t;
+      float contrib = 0.f;
+      if (p < a.P && r < a.R) {
         const float2 gu = lds[LY::addr(t, p)];
         const float2 yv = yc[(int64_t)p * a.ys_p + (int64_t)r * a.ys_r];
         contrib = gu.x * yv.x + gu.y * yv.y;
@@ -505,14 +529,8 @@ __global__ __launch_bounds__(DopCfg<ND>::NT) void doppler_adj_kernel(DopGradArgs
 template <int ND>
 static mxr_status launch_doppler_adj(DopGradArgs a, const mxr_tensor *gtaps, hipStream_t s) {
   constexpr int TR = DopAdjCfg<ND>::TR;
-  const int rows_buf = a.P > ND ? a.P : ND;
-  const size_t lds = (size_t)rows_buf * TR * sizeof(float2);
-  MXR_REQUIRE(lds + ND * sizeof(float) <= (size_t)max_lds_per_block(), MXR_NOT_SUPPORTED,
-              "doppler adjoint: %d pulses x %d range bins do not fit in LDS", rows_buf, TR);
-  if (lds + ND * sizeof(float) > 65536)
-    MXR_HIP_TRY(hipFuncSetAttribute((const void *)doppler_adj_kernel<ND>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   a.tiles = (a.R + TR - 1) / TR;
+  MXR_REQUIRE((int64_t)a.tiles * a.C < (1ll << 31), MXR_INVALID_SIZE, "doppler adjoint: too many tiles");
   a.partial = nullptr;
   if (gtaps) {
     a.partial = (float *)stream_workspace("doppler_taps_partial",
@@ -521,7 +539,7 @@ static mxr_status launch_doppler_adj(DopGradArgs a, const mxr_tensor *gtaps, hip
   }
   {
     ProfScope ps("doppler_adj_kernel", s);
-    doppler_adj_kernel<ND><<<dim3(a.tiles, a.C), dim3(DopCfg<ND>::NT), lds, s>>>(a);
+    doppler_adj_kernel<ND><<<dim3((unsigned)(a.tiles * a.C)), dim3(DopAdjCfg<ND>::NT), 0, s>>>(a);
   }
   MXR_HIP_TRY(hipGetLastError());
   if (gtaps) {
@@ -533,8 +551,13 @@ static mxr_status launch_doppler_adj(DopGradArgs a, const mxr_tensor *gtaps, hip
   return MXR_SUCCESS;
 }
 
-static mxr_status dispatch_doppler_adj(int64_t nd, const DopGradArgs &a, const mxr_tensor *gtaps,
-                                       hipStream_t s) {
+static mxr_status dispatch_doppler_adj(int64_t nd, DopGradArgs a, const mxr_tensor *gtaps, hipStream_t s) {
+  a.tw = twiddles_device((int)nd, false);
+  a.twi = twiddles_device((int)nd, true);
+  MXR_REQUIRE(a.tw && a.twi, MXR_OUT_OF_MEMORY, "doppler adjoint: twiddle table allocation failed");
+  a.y32 = rows32(a.P, a.R, a.ys_p, a.ys_r, 8);
+  a.gp32 = rows32(nd, a.R, a.gs_k, a.gs_r, 4);
+  a.gy32 = a.gy && rows32(a.P, a.R, a.gys_p, a.gys_r, 8);
   switch (nd) {
     case 2: return launch_doppler_adj<2>(a, gtaps, s);
     case 4: return launch_doppler_adj<4>(a, gtaps, s);
@@ -601,8 +624,6 @@ static mxr_status doppler_adjoint_impl(const mxr_tensor *gy, const mxr_tensor *g
   a.p_off = tpc_mode == MXR_CONV_VALID ? 1 : 0;
   a.no_tpc = tpc_mode == MXR_TPC_NONE;
   a.win_rows = (int)win_rows;
-  a.tw = twiddles_device((int)nd, false);
-  MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   return dispatch_doppler_adj(nd, a, nullptr, stream);
 }
 
@@ -666,8 +687,6 @@ static mxr_status doppler_taps_adjoint_impl(const mxr_tensor *gtaps, const mxr_t
   a.no_tpc = 1;
   a.win_rows = 0;
   a.skip_zero = 1;
-  a.tw = twiddles_device((int)nd, false);
-  MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   return dispatch_doppler_adj(nd, a, gtaps, s);
 }
 

@@ -352,6 +352,9 @@ __device__ __forceinline__ buf_rsrc make_rsrc(const void *base, int bytes) {
   void *ub = reinterpret_cast<void *>(((uint64_t)hi << 32) | lo);
   return __builtin_amdgcn_make_buffer_rsrc(ub, (short)0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
 }
+__device__ __forceinline__ float buf_load1(buf_rsrc r, int voff) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
+}
 __device__ __forceinline__ float2 buf_load2(buf_rsrc r, int voff) {
   return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
 }
@@ -405,12 +408,16 @@ __device__ __forceinline__ void wg_barrier() {
 //      consecutive lanes take consecutive butterflies of one transform.
 // COL: element i of transform (column) t at i*TB + t; consecutive lanes take
 //      consecutive columns, so every LDS access is unit stride across lanes.
-template <int N, int TB, bool COL>
+// PAD (COL): one spare row every 16, so that the rows 16 apart that the first
+//      radix-16 pass writes together fall into different banks when a row is
+//      shorter than the 32 lanes served at once.
+template <int N, int TB, bool COL, bool PAD = false>
 struct Layout {
   static constexpr int TSTRIDE = lds_padded_len(N);
-  static constexpr int LDS_ELEMS = COL ? N * TB : TB * TSTRIDE;
+  static constexpr int LDS_ELEMS = COL ? (N + (PAD ? N / 16 : 0)) * TB : TB * TSTRIDE;
   __device__ static __forceinline__ int addr(int t, int i) {
-    if constexpr (COL) return i * TB + t;
+    if constexpr (COL && PAD) return (i + (i >> 4)) * TB + t;
+    else if constexpr (COL) return i * TB + t;
     else return t * TSTRIDE + lds_pad(i);
   }
   template <int R>

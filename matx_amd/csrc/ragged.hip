@@ -364,6 +364,8 @@ static mxr_status ragged_create(mxr_ragged_plan *out, const mxr_ragged_job *jobs
       dj.a.p_off = 0;
       dj.a.win_rows = (int)j.P;
       dj.a.no_tpc = 1;
+      dj.a.y32 = rows32(j.P, R, dj.a.ys_p, 1, 8);
+      dj.a.out32 = rows32(nd, R, j.pw_ks, 1, 4);
       dj.a.tw = tw;
       dj.tiles = (int)((R + TR - 1) / TR);
       dj.item0 = cl.items;

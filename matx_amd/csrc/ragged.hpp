@@ -22,8 +22,19 @@ struct DopArgs {
   int no_tpc;    // input is already the canceller output
   const float *taps;  // optional real window replacing hamming(win_rows)
   int64_t taps_s;
+  int y32, out32;  // input / outputs: unit range stride, rows that follow one
+                   // another, a channel within 32-bit byte offsets (rows32)
   const float2 *tw;
 };
+
+// Whether a channel of `rows` rows of n elements (stride s_row, s_el) may be
+// addressed through one buffer resource with byte offsets from its first
+// element: an offset before the first or past the last row then falls
+// outside the resource.  The pulse-axis kernels reach up to 1024 + 16 rows
+// past either end.
+inline bool rows32(int64_t rows, int64_t n, int64_t s_row, int64_t s_el, int64_t esz) {
+  return s_el == 1 && s_row >= n && rows >= 1 && (rows + 1040) * s_row * esz < (1ll << 31);
+}
 
 // Waveform spectrum: Wc = conj?(fft_M(pad_M(w2))), w2 = w1/||w1|| (optional),
 // w1 = w .* hamming(L) (optional); optionally writes w2 back to w.

@@ -82,6 +82,48 @@ def np_doppler_adjoint(gp, y, nd, tpc, win_rows):
     return gy
 
 
+@pytest.mark.parametrize("nd,P,tpc", [(2, 4, "valid"), (8, 10, "valid"), (16, 3, "same"), (32, 34, "valid"),
+                                      (64, 41, "none"), (128, 130, "valid"), (256, 256, "same"),
+                                      (512, 514, "valid"), (512, 300, "same"), (1024, 1026, "valid")])
+@pytest.mark.parametrize("form", ["rows", "range_strided", "pulse_fast"])
+def test_doppler_strips(mx, nd, P, tpc, form):
+    """The pulse-axis pass and its adjoint where a strip, a tile or the pulses
+    end: rows of every alignment that follow one another (one buffer resource
+    a channel), every second range bin of a wider cube, and pulses fastest in
+    memory (the general addressing); two pulses more than Doppler bins."""
+    rng = np.random.default_rng(nd + P)
+    C, R = 2, 37
+    y = crandn(rng, C, P, R)
+
+    def view(a):
+        t = dev(a, torch.complex64 if np.iscomplexobj(a) else torch.float32)
+        if form == "rows":
+            buf = torch.full(a.shape[:2] + (R + 3,), float("nan"), dtype=t.dtype, device="cuda")
+            v = buf[:, :, 1:R + 1]
+        elif form == "range_strided":
+            v = torch.zeros(a.shape[:2] + (2 * R,), dtype=t.dtype, device="cuda")[:, :, ::2]
+        else:
+            v = torch.zeros((a.shape[0], R, a.shape[1]), dtype=t.dtype, device="cuda").permute(0, 2, 1)
+        v.copy_(t)
+        return v
+
+    rows = P - 2 if tpc == "valid" else P
+    win_rows = P if tpc == "none" else P - 2
+    gp = rng.standard_normal((C, nd, R)).astype(np.float32)
+    hw = np.ones(rows)
+    hw[:win_rows] = hamming(win_rows)
+    yc = y.astype(complex)
+    yp = np.pad(yc, ((0, 0), (1, 1), (0, 0)))
+    t = yc if tpc == "none" else (yp[:, :-2] - 2 * yp[:, 1:-1] + yp[:, 2:])
+    t = t[:, 1:-1] if tpc == "valid" else t
+    ref = np.abs(np.fft.fft(t * hw[None, :, None], nd, axis=1)) ** 2
+    pw, gy = view(np.zeros((C, nd, R), np.float32)), view(np.zeros((C, P, R), np.complex64))
+    mx.doppler(view(y), nd, tpc=tpc, win_rows=win_rows, pw=pw)
+    assert rel(host(pw), ref) < RTOL
+    mx.ops.doppler_adjoint(view(gp), view(y), nd, tpc=tpc, win_rows=win_rows, gy=gy)
+    assert rel(host(gy), np_doppler_adjoint(gp, y, nd, tpc, win_rows)) < RTOL
+
+
 @pytest.mark.parametrize("C,P,R,nd,tpc", [
     (2, 128, 300, 128, "same"), (2, 128, 300, 128, "valid"), (3, 20, 77, 32, "none"),
     (1, 130, 50, 128, "valid"), (2, 512, 40, 512, "valid"), (1, 64, 1000, 1024, "same"),
