@@ -11,31 +11,41 @@
 // columns and emits detections for the OUT = 64 - 2*HXA inner columns (HXA =
 // HX rounded up to even, so OUT is a multiple of 4 and every output quad
 // starts on a 16-byte boundary of the detection rows); neighbouring tiles
-// overlap by 2*HXA columns, which the XCD-local L2 serves.  The narrowest
-// halo matters: at 16 x 8001 range bins and two resident workgroups per CU,
-// 52 outputs per tile fill 4.8 rounds of the machine where 48 need 5.2.
+// overlap by 2*HXA columns, which the XCD-local L2 serves.
 //
-//  1. load: lane = range column, wave = a strip of Doppler-input rows; each
-//     lane reads its strip's pulses plus one on either side (512-byte
-//     coalesced rows), forms the canceller output and the window in
-//     registers and writes one LDS element per row (element (row i, column
-//     t) at i*TB + t).
-//  2. Stockham passes down the LDS columns (lane = column: unit-stride LDS);
-//     the last pass writes |X|^2 over the first half of the tile.
-//  3. CFAR: a thread owns 4 adjacent output columns on every 32nd Doppler
-//     row (16 lanes per row).  It reads each of its power rows with 16-byte LDS loads and forms
-//     the positive partial sums L (left of the hole), M (hole columns), Rt
-//     (right of the hole) of its 4 columns once per row; lr = L + Rt and
-//     full = lr + M go back to LDS, and each cell's noise sum adds full over
+//  1. load: lane = range column, wave = a strip of Doppler-input rows i and
+//     the strip ND/2 rows below it; each lane reads its strips' pulses plus
+//     one on either side (512-byte coalesced rows) and forms the canceller
+//     output and the window in registers.
+//  2. The transform is split by its first radix-2 stage (decimation in
+//     frequency): the even Doppler bins are the ND/2-point transform of
+//     row i + row i + ND/2, the odd ones that of the difference at frequencies
+//     half a bin up, which only changes the butterflies' factors (the table's
+//     row k holds those of k + 1/2).  Both run through one LDS buffer of half
+//     the tile, one after the other, while the other half waits in registers.
+//     So a workgroup holds 36 KiB of LDS instead of 67 and four of them share
+//     a CU, each in another phase: with the whole tile in LDS, two workgroups
+//     of eight waves per CU loaded, transformed and summed almost in turn.
+//  3. CFAR on the power rows in LDS: a thread owns 4 adjacent output columns
+//     of a band of Doppler rows and walks down it.  Per row it forms the
+//     positive partial sums L (left of the hole), M (hole columns), Rt (right
+//     of the hole) of its 4 columns; lr = L + Rt and full = lr + M of the last
+//     2HY+1 rows stay in registers, and each cell's noise sum adds full over
 //     the window rows outside the hole's Doppler extent and lr over the rows
 //     inside it.  One 16-byte detection quad per row.  Sums never subtract,
-//     so a strong cell in the hole cannot cancel (the same decomposition as
-//     the stand-alone CFAR kernel).
+//     so a strong cell in the hole cannot cancel (the same decomposition, in
+//     the same order, as the stand-alone CFAR kernel).
+//
+// 16 x 128 pulses x 8001 range bins, 5 x 13 window: 56.6 us with the whole tile
+// in LDS, 50.4 with the halves, 47.9 with the channel's loads through a buffer
+// resource (zeros outside it) and one branch a detection row; 38 us is its HBM
+// traffic at a large copy's rate, 31 us its VALU issue.
 #include <cmath>
 #include <cstdlib>
 
 #include "fft_engine.hpp"
 #include "mxr_cache.hpp"
+#include "ragged.hpp"
 
 namespace mxr {
 
@@ -61,7 +71,8 @@ struct DcArgs {
   int no_tpc;    // y already holds the canceller output
   int tiles;     // range tiles per channel
   int vec_out;   // every output row is 16-byte aligned
-  const float2 *tw;
+  int y32;       // rows32 of y, below DC_FAR bytes
+  const float2 *tw, *twh;  // ND/2-point tables: k and k + 1/2
   // threshold factor per in-bounds cell count n: alpha(n) (exact form) or
   // alpha(n)/n, alpha(n) = n*(pfa^(-1/n) - 1) evaluated in float on the host
   float thr[DC_MAXCELL + 1];
@@ -79,8 +90,9 @@ __device__ __forceinline__ void st32(T *base, uint32_t byte_off, T v) {
 }
 
 constexpr int DC_TB = 64;   // computed range columns per tile
-constexpr int DC_NT = 512;  // threads per workgroup
+constexpr int DC_NT = 256;  // threads per workgroup
 constexpr int DC_PS = 64;   // power-tile row stride (floats)
+constexpr int DC_FAR = 1 << 30;  // a byte offset past every channel with y32
 
 template <int HX>
 struct DcGeom {
@@ -116,170 +128,160 @@ __device__ __forceinline__ void dc_win4(const float *u, float (&o)[4]) {
   }
 }
 
-// Two 512-thread workgroups per CU (LDS bound): 4 waves per SIMD, so at most
-// 128 VGPRs.
+// One H-point transform down the LDS columns, from LDS to registers: the last
+// pass's butterflies end in pl (bin j + q H/RL of butterfly j).  HALF: at
+// frequencies k + 1/2.  Pre: the rows are in LDS, visible to all threads.
+// Post: LDS is free.
+template <class LY, int H, bool HALF, class PL>
+__device__ __forceinline__ void dc_transform(PL &pl, float2 *lds, const float2 *tw) {
+  using SQ = Seq<H, false>;
+  constexpr int K = SQ::n;
+  static_assert(K <= 2, "half transforms of at most two passes");
+  if constexpr (K == 2) {
+    constexpr int R0 = SQ::template R<0>;
+    Pass<LY, R0, H, DC_NT, DC_TB> p0;
+    p0.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
+    wg_barrier();
+    if constexpr (HALF) p0.template compute_tw<1, false>(tw);
+    else p0.template compute<1, false>(nullptr);
+    p0.template store<1>([&](int t, int i, float2 x) { lds[LY::addr(t, i)] = x; });
+    wg_barrier();
+  }
+  pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
+  wg_barrier();
+}
+
+// Four 256-thread workgroups per CU: 4 waves per SIMD, at most 128 VGPRs
+// (three for windows over two rows either side, whose sums take more).
 template <int ND, int HY, int HX, int EY, int EX, bool EXACT>
-__global__ __launch_bounds__(DC_NT) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(DC_NT) __attribute__((amdgpu_waves_per_eu(HY > 2 ? 3 : 4)))
 void dopcfar_kernel(DcArgs a) {
-  constexpr int TB = DC_TB, NT = DC_NT, NW = NT / 64;
+  constexpr int TB = DC_TB, NT = DC_NT, NW = NT / 64, H = ND / 2;
   constexpr int HXA = DcGeom<HX>::HXA, OUT = DcGeom<HX>::OUT;
   static_assert(OUT >= 16, "window too wide for a 64-column tile");
-  static_assert(ND >= NW, "Doppler size below one row per wave");
+  static_assert(H >= NW, "Doppler size below two rows per wave");
   constexpr int PS = DC_PS;
-  constexpr int SR = ND / NW;  // Doppler-input rows per wave in the load phase
-  using LY = Layout<ND, TB, true>;
-  using SQ = Seq<ND, false>;
+  constexpr int SR = H / NW;  // rows of a wave's strip
+  using LY = Layout<H, TB, true>;
+  using SQ = Seq<H, false>;
   constexpr int K = SQ::n;
   constexpr int NCELL = (2 * HY + 1) * (2 * HX + 1);
   static_assert(NCELL <= DC_MAXCELL, "window area");
-  // the complex tile; after the transform it holds the power rows (stride
-  // PS, HY zero rows either side) followed by the CFAR's full-sum rows
-  // (stride OUT)
-  constexpr int LDS2 = ND * TB > ((ND + 2 * HY) * (PS + OUT) + 1) / 2 ? ND * TB
-                                                                      : ((ND + 2 * HY) * (PS + OUT) + 1) / 2;
+  // the complex half tile; after the transforms the power rows (stride PS,
+  // HY zero rows either side)
+  constexpr int LDS2 = H * TB > ((ND + 2 * HY) * PS + 1) / 2 ? H * TB : ((ND + 2 * HY) * PS + 1) / 2;
   __shared__ __align__(16) float2 lds[LDS2];
-  static_assert((ND + 2 * HY) * (PS + OUT) <= 2 * LDS2, "power and full-sum rows must fit the tile");
   __shared__ float2 coef[ND];  // Doppler-input row i = coef.x*(y[p-1]+y[p+1]) + coef.y*y[p]
   __shared__ float thr_tab[NCELL + 1];
 
-  const int G = a.tiles * a.C;
-  const int g = (int)xcd_remap(blockIdx.x, G);
-  const int c = g / a.tiles, tile = g - c * a.tiles;
+  const uint32_t G = (uint32_t)(a.tiles * a.C);
+  const uint32_t g = (uint32_t)xcd_remap(blockIdx.x, G);
+  const int c = (int)(g / (uint32_t)a.tiles), tile = (int)(g - (uint32_t)c * (uint32_t)a.tiles);
   const int r0 = tile * OUT - HXA;  // range bin of tile column 0
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-  // canceller [1,-2,1] and window folded into two coefficients per row:
-  // rows past the canceller output are zero, NONE passes y[p] windowed
-  for (int i = threadIdx.x; i < ND; i += NT) {
-    float h = 0.f;
-    if (i < a.rows_t) h = i < a.win_rows ? hamming_f32(i, a.win_rows) : 1.0f;
-    coef[i] = a.no_tpc ? make_float2(0.f, h) : make_float2(h, -2.0f * h);
-  }
-  for (int n = threadIdx.x; n <= NCELL; n += NT) thr_tab[n] = a.thr[n];
-  __syncthreads();
-
-  // ---- 1. canceller + window in registers, one LDS write per element.
-  // Indices are clamped into the cube so every load is unconditional; the
-  // values outside it are replaced by zeros afterwards.
+  // ---- 1. canceller + window in registers, zeros outside the cube: from the
+  // range check of a buffer resource over the channel (a column outside it
+  // reads past the end), or, where a channel is too large for its 32-bit
+  // offsets, from masks on clamped indices.
+  float2 ev[SR], od[SR];  // rows i + (i + H), rows i - (i + H)
   {
     const int r = r0 + lane;
     const bool rok = r >= 0 && r < a.R;
-    const int rc = min(max(r, 0), a.R - 1);
     const float2 *chan = a.y + (int64_t)c * a.ys_c;
     const int i0 = wv * SR;
-    const int pb = i0 + a.p_off - 1;  // pulse held in v[0]
-    float2 v[SR + 2];
+    float2 va[SR + 2], vb[SR + 2];
+    if (a.y32) {
+      const buf_rsrc ry = make_rsrc(chan, ((a.P - 1) * a.ys_p + a.R) * 8);
+      const int step = a.ys_p * 8;
+      const int v0 = (rok ? r * 8 : DC_FAR) + (i0 + a.p_off - 1) * step;  // pulse held in va[0]
 #pragma unroll
-    for (int u = 0; u < SR + 2; ++u) {
-      const int p = pb + u;
-      const int pc = min(max(p, 0), a.P - 1);
-      const float2 t = ld32(chan, (uint32_t)(rc + pc * a.ys_p) * 8u);
-      const bool in = rok && p >= 0 && p < a.P;
-      v[u] = make_float2(in ? t.x : 0.f, in ? t.y : 0.f);
+      for (int u = 0; u < SR + 2; ++u) va[u] = buf_load2(ry, v0 + u * step);
+#pragma unroll
+      for (int u = 0; u < SR + 2; ++u) vb[u] = buf_load2(ry, v0 + (u + H) * step);
+    } else {
+      const int rc = min(max(r, 0), a.R - 1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float2(&v)[SR + 2] = h ? vb : va;
+        const int pb = i0 + h * H + a.p_off - 1;
+#pragma unroll
+        for (int u = 0; u < SR + 2; ++u) {
+          const float2 x = ld32(chan, (uint32_t)(rc + min(max(pb + u, 0), a.P - 1) * a.ys_p) * 8u);
+          v[u] = keep_if(x, rok && pb + u >= 0 && pb + u < a.P);
+        }
+      }
     }
+    // canceller [1,-2,1] and window folded into two coefficients per row:
+    // rows past the canceller output are zero, NONE passes y[p] windowed
+    for (int i = threadIdx.x; i < ND; i += NT) {
+      float w = 0.f;
+      if (i < a.rows_t) w = i < a.win_rows ? hamming_f32(i, a.win_rows) : 1.0f;
+      coef[i] = a.no_tpc ? make_float2(0.f, w) : make_float2(w, -2.0f * w);
+    }
+    for (int n = threadIdx.x; n <= NCELL; n += NT) thr_tab[n] = a.thr[n];
+    wg_barrier();
 #pragma unroll
     for (int u = 0; u < SR; ++u) {
-      const int i = i0 + u;
-      const float2 cf = coef[i];
-      const float2 x = make_float2(cf.x * (v[u].x + v[u + 2].x) + cf.y * v[u + 1].x,
-                                   cf.x * (v[u].y + v[u + 2].y) + cf.y * v[u + 1].y);
-      lds[LY::addr(lane, i)] = x;
+      const float2 ca = coef[i0 + u], cb = coef[i0 + u + H];
+      const float2 x = make_float2(ca.x * (va[u].x + va[u + 2].x) + ca.y * va[u + 1].x,
+                                   ca.x * (va[u].y + va[u + 2].y) + ca.y * va[u + 1].y);
+      const float2 z = make_float2(cb.x * (vb[u].x + vb[u + 2].x) + cb.y * vb[u + 1].x,
+                                   cb.x * (vb[u].y + vb[u + 2].y) + cb.y * vb[u + 1].y);
+      ev[u] = cadd(x, z);
+      od[u] = csub(x, z);
     }
+#pragma unroll
+    for (int u = 0; u < SR; ++u) lds[LY::addr(lane, i0 + u)] = ev[u];
   }
   wg_barrier();
 
-  // ---- 2. Doppler FFT down the columns; the last pass leaves |X|^2 in LDS
-  // as rows 0..ND-1 of a power tile with HY zero rows above and below (the
-  // CFAR's zero padding along Doppler)
-  float *const pwt = reinterpret_cast<float *>(lds) + HY * PS;  // row 0
-  if constexpr (K > 1) lds_passes<LY, SQ, ND, NT, TB, false, 0, K - 1>(lds, a.tw);
-  {
-    constexpr int RL = SQ::template R<K - 1>;
-    constexpr int LSL = SQ::template LS<K - 1>;
-    Pass<LY, RL, ND, NT, TB> pl;
-    pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
-    wg_barrier();  // the power map overwrites the tile
-    for (int i = threadIdx.x; i < 2 * HY * TB; i += NT) {
-      const int row = i / TB < HY ? i / TB - HY : ND + i / TB - HY;
-      pwt[row * PS + (i % TB)] = 0.f;
-    }
-    pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
-    pl.template store<LSL>([&](int t, int k, float2 x) { pwt[k * PS + t] = cabs2(x); });
+  // ---- 2. the two half transforms; |X|^2 stays in registers until LDS is free
+  constexpr int RL = SQ::template R<K - 1>;
+  constexpr int LSL = SQ::template LS<K - 1>;
+  using PL = Pass<LY, RL, H, NT, TB>;
+  float pe[PL::BPT][RL];
+  float *const pwt = reinterpret_cast<float *>(lds) + HY * PS;  // power row 0
+  PL pl;
+  dc_transform<LY, H, false>(pl, lds, a.tw);
+#pragma unroll
+  for (int u = 0; u < SR; ++u) lds[LY::addr(lane, wv * SR + u)] = od[u];
+  pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
+#pragma unroll
+  for (int u = 0; u < PL::BPT; ++u)
+#pragma unroll
+    for (int q = 0; q < RL; ++q) pe[u][q] = cabs2(pl.v[u][q]);
+  wg_barrier();
+  // the half-bin table holds the first pass too
+  constexpr int H0 = K == 2 ? SQ::template R<0> / 2 : 0;
+  dc_transform<LY, H, true>(pl, lds, a.twh);
+  for (int i = threadIdx.x; i < 2 * HY * TB; i += NT) {  // the CFAR's zero padding along Doppler
+    const int row = i / TB < HY ? i / TB - HY : ND + i / TB - HY;
+    pwt[row * PS + (i % TB)] = 0.f;
   }
+  PL::template outputs<LSL>([&](int u, int q, int t, int k) { pwt[2 * k * PS + t] = pe[u][q]; });
+  pl.template compute_tw<LSL, false>(a.twh + H0);
+  PL::template outputs<LSL>([&](int u, int q, int t, int k) { pwt[(2 * k + 1) * PS + t] = cabs2(pl.v[u][q]); });
   wg_barrier();
 
-  // ---- 3. CFAR over the inner columns, in two steps over the same cells.
-  // A thread owns one output column quad (tile columns tc0..tc0+3) on the
-  // rows k = kb + KS*it.
-  //  3a. per row: the positive partial sums of the row segment, lr = left +
-  //      right of the hole and full = lr + hole columns (each row's sums are
-  //      formed once; full goes to the free upper part of the tile, lr
-  //      replaces the power row once every thread has read its row);
-  //  3b. per cell: noise = sum over the window rows of full (rows outside the
-  //      hole's Doppler extent) or lr (rows inside it), then the threshold.
-  // The cell under test and the row's own lr stay in registers in between.
-  constexpr int NQO = OUT / 4;                // output column quads per row
+  // ---- 3. CFAR over the inner columns: a thread owns one output column quad
+  // (tile columns tc0..tc0+3) of a band of RB Doppler rows.
   // 16 lanes per row (quads q < NQO active): the lanes of one 16-lane LDS
   // access group read one row, so their 16-byte reads never collide in a
   // bank (rows of different lanes 256 bytes apart would)
+  constexpr int NQO = OUT / 4;  // output column quads per row
   constexpr int GQ = 16;
   static_assert(NQO <= GQ, "output quads per row");
-  constexpr int KS = NT / GQ;                 // row step between a thread's rows
-  constexpr int QIT = (ND + KS - 1) / KS;     // rows per thread (at most)
-  constexpr int NQ = 1 + 2 * HXA / 4;         // power quads read per row segment
+  constexpr int NB = NT / GQ;                      // bands
+  constexpr int RB = ND >= NB ? ND / NB : 1;       // rows per band
+  constexpr int NQ = 1 + 2 * HXA / 4;              // power quads read per row segment
   constexpr int NV = 4 * NQ;
-  constexpr int FS = OUT;                     // full-sum row stride (floats)
-  float *const fsum = reinterpret_cast<float *>(lds) + (ND + 2 * HY) * PS + HY * FS;  // row 0
-  const int q = threadIdx.x % GQ, kb = threadIdx.x / GQ;
-  const bool act = q < NQO;
-  const int tc0 = HXA + 4 * q;                // first tile column of the quad
-  float cut[QIT][4], lrk[QIT][4];
-  // zero rows of the full sums (the CFAR's zero padding along Doppler)
-  for (int i = threadIdx.x; i < 2 * HY * NQO; i += NT) {
-    const int row = i / NQO < HY ? i / NQO - HY : ND + i / NQO - HY;
-    *reinterpret_cast<float4 *>(fsum + row * FS + 4 * (i % NQO)) = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-#pragma unroll
-  for (int it = 0; it < QIT; ++it) {
-    const int k = kb + KS * it;
-    if (!act || k >= ND) continue;
-    float u[NV];
-    const float *row = pwt + k * PS + tc0 - HXA;
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) {
-      const float4 z = *reinterpret_cast<const float4 *>(row + 4 * m);
-      u[4 * m] = z.x;
-      u[4 * m + 1] = z.y;
-      u[4 * m + 2] = z.z;
-      u[4 * m + 3] = z.w;
-    }
-    // u[HXA + j + d] is tile column tc0 + j + d
-    float L[4], Mh[4], Rt[4], fl[4];
-    dc_win4<HX - EX>(u + HXA - HX, L);
-    dc_win4<2 * EX + 1>(u + HXA - EX, Mh);
-    dc_win4<HX - EX>(u + HXA + EX + 1, Rt);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      lrk[it][j] = L[j] + Rt[j];
-      fl[j] = lrk[it][j] + Mh[j];
-      cut[it][j] = u[HXA + j];
-    }
-    *reinterpret_cast<float4 *>(fsum + k * FS + 4 * q) = make_float4(fl[0], fl[1], fl[2], fl[3]);
-  }
-  wg_barrier();  // every power row has been read
-  // lr in place of the power rows (columns 0..OUT-1; the zero rows stay zero)
-#pragma unroll
-  for (int it = 0; it < QIT; ++it) {
-    const int k = kb + KS * it;
-    if (!act || k >= ND) continue;
-    *reinterpret_cast<float4 *>(pwt + k * PS + 4 * q) =
-        make_float4(lrk[it][0], lrk[it][1], lrk[it][2], lrk[it][3]);
-  }
-  wg_barrier();
-
-  const int gr0 = r0 + tc0;  // range bin of the quad (a multiple of 4, >= 0)
-  if (!act || gr0 >= a.R) return;  // no barrier follows
+  constexpr int RING = 2 * HY + 1;
+  const int q = threadIdx.x % GQ, k0 = threadIdx.x / GQ * RB;
+  const int tc0 = HXA + 4 * q;  // first tile column of the quad
+  const int gr0 = r0 + tc0;     // range bin of the quad (a multiple of 4, >= 0)
+  if (q >= NQO || k0 >= ND || gr0 >= a.R) return;  // no barrier follows
   const int R = a.R;
   // in-bounds cell count = ro*co - rh*chh; away from the first and last HY
   // Doppler rows ro = 2HY+1 and rh = 2EY+1, so it depends on the column only
@@ -293,36 +295,51 @@ void dopcfar_kernel(DcArgs a) {
     nrm_int[j] = (2 * HY + 1) * co[j] - (2 * EY + 1) * chh[j];
     thr_int[j] = thr_tab[min(max(nrm_int[j], 0), NCELL)];
   }
-  const bool vec = a.vec_out && gr0 + 3 < R;
+  // one scalar branch a row: a wave whose every quad is whole and aligned
+  const bool vec = __all(a.vec_out && gr0 + 3 < R);
   int *const dets_c = a.dets + (int64_t)c * a.ds_c;
   float *const ba_c = EXACT ? a.ba + (int64_t)c * a.bs_c : nullptr;
   float *const pw_c = a.pw ? a.pw + (int64_t)c * a.ps_c : nullptr;
 
+  float full[RING][4], lr[RING][4], ctr[RING][4];
 #pragma unroll
-  for (int it = 0; it < QIT; ++it) {
-    const int kc = kb + KS * it;  // Doppler row of the cells under test
-    if (kc >= ND) continue;
+  for (int ly = 0; ly < RB + 2 * HY; ++ly) {  // power row k0 - HY + ly
+    float u[NV];
+    const float *row = pwt + (k0 - HY + ly) * PS + tc0 - HXA;
+#pragma unroll
+    for (int m = 0; m < NQ; ++m) {
+      const float4 z = *reinterpret_cast<const float4 *>(row + 4 * m);
+      u[4 * m] = z.x;
+      u[4 * m + 1] = z.y;
+      u[4 * m + 2] = z.z;
+      u[4 * m + 3] = z.w;
+    }
+    // u[HXA + j + d] is tile column tc0 + j + d
+    float L[4], Mh[4], Rt[4];
+    dc_win4<HX - EX>(u + HXA - HX, L);
+    dc_win4<2 * EX + 1>(u + HXA - EX, Mh);
+    dc_win4<HX - EX>(u + HXA + EX + 1, Rt);
+    const int sl = ly % RING;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      lr[sl][j] = L[j] + Rt[j];
+      full[sl][j] = lr[sl][j] + Mh[j];
+      ctr[sl][j] = u[HXA + j];
+    }
+    if (ly < 2 * HY) continue;
+    const int kc = k0 + ly - 2 * HY;  // Doppler row of the cells under test
     float sm[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sm[j] = 0.f;
-#pragma unroll
     for (int dy = -HY; dy <= HY; ++dy) {
-      float t[4];
-      if (dy == 0) {
+      const int kk = (ly - HY + dy) % RING;
+      const bool inner = dy >= -EY && dy <= EY;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) t[j] = lrk[it][j];
-      } else {
-        const bool inner = dy >= -EY && dy <= EY;
-        const float *src = inner ? pwt + (kc + dy) * PS + 4 * q : fsum + (kc + dy) * FS + 4 * q;
-        const float4 z = *reinterpret_cast<const float4 *>(src);
-        t[0] = z.x;
-        t[1] = z.y;
-        t[2] = z.z;
-        t[3] = z.w;
+      for (int j = 0; j < 4; ++j) {
+        const float t = inner ? lr[kk][j] : full[kk][j];
+        sm[j] = dy == -HY ? t : sm[j] + t;
       }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sm[j] = dy == -HY ? t[j] : sm[j] + t[j];
     }
+    const float(&cv)[4] = ctr[(ly - HY) % RING];
     float thr[4];
     int nrm[4];
 #pragma unroll
@@ -330,7 +347,10 @@ void dopcfar_kernel(DcArgs a) {
       thr[j] = thr_int[j];
       nrm[j] = nrm_int[j];
     }
-    if (kc < HY || kc + HY >= ND) {  // rows whose window leaves the map
+    // rows whose window leaves the map: only a band's first and last HY
+    const int sr = ly - 2 * HY;
+    const bool may = RB < 2 * HY || sr < HY || sr >= RB - HY;
+    if (may && (kc < HY || kc + HY >= ND)) {
       const int ro = min(kc + HY, ND - 1) - max(kc - HY, 0) + 1;
       const int rh = min(kc + EY, ND - 1) - max(kc - EY, 0) + 1;
 #pragma unroll
@@ -339,7 +359,6 @@ void dopcfar_kernel(DcArgs a) {
         thr[j] = thr_tab[min(max(nrm[j], 0), NCELL)];
       }
     }
-    const float *cv = cut[it];
     int det[4];
     float bav[4];
 #pragma unroll
@@ -351,11 +370,11 @@ void dopcfar_kernel(DcArgs a) {
         det[j] = cv[j] > thr[j] * sm[j] ? 1 : 0;
       }
     }
-    const uint32_t od = (uint32_t)(kc * a.ds_k + gr0) * 4u;
+    const uint32_t od_ = (uint32_t)(kc * a.ds_k + gr0) * 4u;
     const uint32_t ob = EXACT ? (uint32_t)(kc * a.bs_k + gr0) * 4u : 0u;
     const uint32_t op = pw_c ? (uint32_t)(kc * a.ps_k + gr0) * 4u : 0u;
     if (vec) {
-      *reinterpret_cast<int4 *>(reinterpret_cast<char *>(dets_c) + od) =
+      *reinterpret_cast<int4 *>(reinterpret_cast<char *>(dets_c) + od_) =
           make_int4(det[0], det[1], det[2], det[3]);
       if constexpr (EXACT)
         *reinterpret_cast<float4 *>(reinterpret_cast<char *>(ba_c) + ob) =
@@ -367,7 +386,7 @@ void dopcfar_kernel(DcArgs a) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if (gr0 + j >= R) break;
-        st32(dets_c, od + 4u * j, det[j]);
+        st32(dets_c, od_ + 4u * j, det[j]);
         if constexpr (EXACT) st32(ba_c, ob + 4u * j, bav[j]);
         if (pw_c) st32(pw_c, op + 4u * j, cv[j]);
       }
@@ -525,6 +544,7 @@ mxr_status doppler_cfar_impl(const mxr_tensor *dets, const mxr_tensor *ba_out,
   auto al16 = [](const mxr_tensor *t) {
     return !t || ((uintptr_t)t->data % 16 == 0 && t->stride[1] % 4 == 0 && t->stride[0] % 4 == 0);
   };
+  a.y32 = rows32(P, R, y->stride[1], y->stride[2], 8) && (P + 1040) * y->stride[1] * 8 < DC_FAR;
   a.vec_out = al16(dets) && al16(ba_out) && al16(pow_out);
   if (fusable) {
     const int ncell = wy * wx;
@@ -534,8 +554,9 @@ mxr_status doppler_cfar_impl(const mxr_tensor *dets, const mxr_tensor *ba_out,
       const float alpha = nf * (std::pow(pp->pfa, -1.0f / nf) - 1.0f);
       a.thr[n] = ba_out ? alpha : alpha / nf;
     }
-    a.tw = twiddles_device((int)nd, false);
-    MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "doppler_cfar: twiddle table allocation failed");
+    a.tw = twiddles_device((int)nd / 2, false);
+    a.twh = twiddles_half_device((int)nd / 2);
+    MXR_REQUIRE(a.tw && a.twh, MXR_OUT_OF_MEMORY, "doppler_cfar: twiddle table allocation failed");
     const int hy = wy / 2, hx = wx / 2, ey = gy / 2, ex = gx / 2;
     st = MXR_NOT_SUPPORTED;
 #define MXR_DC_CASE(HY_, HX_, EY_, EX_) \

@@ -326,8 +326,14 @@ __device__ __forceinline__ void dft_tw(float2 (&a)[16], const TwRow<16> &w) {
   for (int i = 0; i < 16; ++i) a[i] = y[i];
 }
 
-// Host: the factors of row k of a pass (Ls, R), R/2 of them in the order above.
-void tw_factors(int R, int64_t Ls, int64_t k, float2 *out);
+// Host: the factors of row k (or k + 1/2) of a pass (Ls, R), R/2 of them in
+// the order above.
+void tw_factors(int R, int64_t Ls, double k, float2 *out);
+
+// A transform at frequencies k + 1/2: the same passes with the factors of
+// k + 1/2 in place of those of k, the first pass (Ls = 1) included.  Table of
+// N's sequence: pass p's rows follow those of the passes before it.
+const float2 *twiddles_half_device(int N);
 
 // Per-device cache of twiddle tables keyed by (N, reversed?).  Returns a
 // device pointer owned by the library.
@@ -486,6 +492,17 @@ struct Pass {
       } else {
         dft<R, INV>(v[u]);
       }
+    }
+  }
+  // the same with factors in the first pass too (half-bin tables)
+  template <int LS, bool INV>
+  __device__ __forceinline__ void compute_tw(const float2 *__restrict__ tw) {
+#pragma unroll
+    for (int u = 0; u < BPT; ++u) {
+      if (!active(u)) continue;
+      int t, j;
+      LY::template bfly<R>(threadIdx.x + u * NT, t, j);
+      dft_tw<INV>(v[u], load_tw<R>(reinterpret_cast<const float4 *>(tw), LS, j & (LS - 1)));
     }
   }
   // f(u, q, t, i) for the output positions store<LS> visits, value

@@ -99,7 +99,7 @@ int max_lds_per_block() {
   return v;
 }
 
-void tw_factors(int R, int64_t Ls, int64_t k, float2 *out) {
+void tw_factors(int R, int64_t Ls, double k, float2 *out) {
   // exponent num/16 of w_R beside the power of w: w^pw w_16^num
   struct F {
     int pw, num;
@@ -109,7 +109,7 @@ void tw_factors(int R, int64_t Ls, int64_t k, float2 *out) {
   const F *f = R == 4 ? f4 : (R == 8 ? f8 : f16);
   const double two_pi = 6.283185307179586476925286766559;
   for (int i = 0; i < R / 2; ++i) {
-    const double ang = two_pi * ((double)(f[i].pw * k) / (double)(Ls * R) + f[i].num / 16.0);
+    const double ang = two_pi * (f[i].pw * k / (double)(Ls * R) + f[i].num / 16.0);
     double c = std::cos(ang);
     if (std::fabs(c) < TW_MIN_COS) c = TW_MIN_COS;
     out[i] = make_float2((float)c, (float)(std::sin(ang) / c));
@@ -117,10 +117,10 @@ void tw_factors(int R, int64_t Ls, int64_t k, float2 *out) {
 }
 
 // The table of one pass: factors 2h, 2h + 1 of row k at float2 index 2 (h Ls + k).
-static void tw_pass(int R, int64_t Ls, float2 *out) {
+static void tw_pass(int R, int64_t Ls, float2 *out, double shift = 0.0) {
   float2 f[8];
   for (int64_t k = 0; k < Ls; ++k) {
-    tw_factors(R, Ls, k, f);
+    tw_factors(R, Ls, (double)k + shift, f);
     for (int h = 0; h < R / 4; ++h) {
       out[2 * (h * Ls + k)] = f[2 * h];
       out[2 * (h * Ls + k) + 1] = f[2 * h + 1];
@@ -219,14 +219,8 @@ namespace {
 std::map<TwKey, float4 *> g_pb;
 }
 
-const float4 *tw16_device(int Ls) {
-  const int dev = device_id();
-  std::lock_guard<std::mutex> g(g_tw_mu);
-  TwKey key{dev, 16, Ls};
-  auto it = g_pb.find(key);
-  if (it != g_pb.end()) return it->second;
-  std::vector<float2> host((size_t)Ls * 8);
-  tw_pass(16, Ls, host.data());
+// Uploads a table built once per key (g_tw_mu held).
+static const float4 *upload_table(const TwKey &key, const std::vector<float2> &host) {
   float4 *d = nullptr;
   if (hipMalloc(&d, sizeof(float2) * host.size()) != hipSuccess) return nullptr;
   if (hipMemcpy(d, host.data(), sizeof(float2) * host.size(), hipMemcpyHostToDevice) != hipSuccess) {
@@ -235,6 +229,32 @@ const float4 *tw16_device(int Ls) {
   }
   g_pb[key] = d;
   return d;
+}
+
+const float2 *twiddles_half_device(int N) {
+  const int dev = device_id();
+  std::lock_guard<std::mutex> g(g_tw_mu);
+  TwKey key{dev, -N, 0};
+  auto it = g_pb.find(key);
+  if (it != g_pb.end()) return reinterpret_cast<const float2 *>(it->second);
+  const RadixSeq s = radix_seq(N);
+  if (s.n < 1) return nullptr;
+  const int64_t first = s.r[0] / 2;  // the first pass's one row
+  std::vector<float2> host((size_t)(first + tw_size(s)));
+  tw_pass(s.r[0], 1, host.data(), 0.5);
+  for (int p = 1; p < s.n; ++p) tw_pass(s.r[p], pass_ls(s, p), host.data() + first + tw_offset(s, p), 0.5);
+  return reinterpret_cast<const float2 *>(upload_table(key, host));
+}
+
+const float4 *tw16_device(int Ls) {
+  const int dev = device_id();
+  std::lock_guard<std::mutex> g(g_tw_mu);
+  TwKey key{dev, 16, Ls};
+  auto it = g_pb.find(key);
+  if (it != g_pb.end()) return it->second;
+  std::vector<float2> host((size_t)Ls * 8);
+  tw_pass(16, Ls, host.data());
+  return upload_table(key, host);
 }
 
 // Per (device, stream, tag) scratch buffers that only grow: partial sums of

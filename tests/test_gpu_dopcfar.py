@@ -161,6 +161,21 @@ def test_fused_pipeline_full_range(mx, orc):
     assert host(dets).sum() > 0
 
 
+@pytest.mark.parametrize("nd,P", [(8, 6), (32, 34), (64, 40), (128, 130)])
+def test_doppler_cfar_rows_sharing_memory(mx, nd, P):
+    """Pulses that share memory (every pulse the same row, stride 0; every pulse
+    one sample on) take the kernel's clamped loads and give the bits of a
+    compact copy, which takes the buffer loads."""
+    rng = np.random.default_rng(nd)
+    C, R = 2, 301
+    base = dev((rng.standard_normal((C, R + P)) + 1j * rng.standard_normal((C, R + P))).astype(np.complex64))
+    for view in (base[:, None, :R].expand(C, P, R), base.as_strided((C, P, R), (R + P, 1, 1))):
+        a = mx.doppler_cfar(view, nd, tpc="valid", want_ba=True, want_pow=True)
+        b = mx.doppler_cfar(view.contiguous(), nd, tpc="valid", want_ba=True, want_pow=True)
+        for u, v in zip(a, b):
+            assert np.array_equal(host(u), host(v), equal_nan=True)
+
+
 def test_pulse_compression_plan(mx, orc):
     """The plan (spectrum once, block kernel per cube) gives the per-call
     entry's result and the oracle's, across two waveforms and batch shapes."""
