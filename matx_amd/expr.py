@@ -150,13 +150,13 @@ def run(out: torch.Tensor, e, stream=None) -> torch.Tensor:
     """``(out = e).run(exec)``: evaluate e into the view out, one kernel."""
     e = wrap(e)
     prog, views, consts = lower(e, tuple(out.shape))
-    descs = [L.desc(v) for v in views]
-    arr = (ctypes.POINTER(L.mxr_tensor) * max(1, len(descs)))(*[ctypes.pointer(d) for d in descs])
+    descs = [L.arg(v) for v in views]
+    arr = (ctypes.c_char_p * max(1, len(descs)))(*descs)
     instrs = (mxr_ew_instr * len(prog))(*[mxr_ew_instr(*p) for p in prog])
     cvals = (ctypes.c_float * max(2, 2 * len(consts)))(
         *[v for c in consts for v in (c.real, c.imag)])
-    L.check(L.lib().mxr_ew_eval(ctypes.byref(L.desc(out)), arr, len(descs), instrs, len(prog),
-                                cvals, len(consts), L.stream_handle(stream)))
+    L.check(L.lib().mxr_ew_eval(L.arg(out), arr, len(descs), instrs, len(prog),
+                                cvals, len(consts), L.raw_stream(stream)))
     return out
 
 
@@ -164,6 +164,5 @@ def sum(x: torch.Tensor, out=None, stream=None) -> torch.Tensor:  # noqa: A001
     """``sum(x)`` to a rank-0 tensor (include/matx/operators/sum.h)."""
     if out is None:
         out = torch.empty((), dtype=x.dtype, device=x.device)
-    L.check(L.lib().mxr_sum(ctypes.byref(L.desc(out)), ctypes.byref(L.desc(x)),
-                            L.stream_handle(stream)))
+    L.check(L.lib().mxr_sum(L.arg(out), L.arg(x), L.raw_stream(stream)))
     return out

@@ -41,9 +41,9 @@ def _fft(x, n, axis, norm, out, inverse, stream):
         shape = list(x.shape)
         shape[ax] = n
         out = torch.empty(shape, dtype=torch.complex64, device=x.device)
-    L.check(L.lib().mxr_fft_c2c(L.ref(L.desc(out)), L.ref(L.desc(x)), n,
+    L.check(L.lib().mxr_fft_c2c(L.arg(out), L.arg(x), n,
                                 L.INVERSE if inverse else L.FORWARD,
-                                _NORMS[norm], ax, L.stream_handle(stream)))
+                                _NORMS[norm], ax, L.raw_stream(stream)))
     return out
 
 
@@ -67,8 +67,8 @@ def rfft(x, n: int = 0, axis: int = -1, norm: str = "backward", out=None, stream
         shape = list(x.shape)
         shape[ax] = n // 2 + 1
         out = torch.empty(shape, dtype=torch.complex64, device=x.device)
-    L.check(L.lib().mxr_fft_r2c(L.ref(L.desc(out)), L.ref(L.desc(x)), n, _NORMS[norm], ax,
-                                L.stream_handle(stream)))
+    L.check(L.lib().mxr_fft_r2c(L.arg(out), L.arg(x), n, _NORMS[norm], ax,
+                                L.raw_stream(stream)))
     return out
 
 
@@ -81,8 +81,8 @@ def irfft(x, n: int = 0, axis: int = -1, norm: str = "backward", out=None, strea
         shape = list(x.shape)
         shape[ax] = n
         out = torch.empty(shape, dtype=torch.float32, device=x.device)
-    L.check(L.lib().mxr_fft_c2r(L.ref(L.desc(out)), L.ref(L.desc(x)), n, _NORMS[norm], ax,
-                                L.stream_handle(stream)))
+    L.check(L.lib().mxr_fft_c2r(L.arg(out), L.arg(x), n, _NORMS[norm], ax,
+                                L.raw_stream(stream)))
     return out
 
 
@@ -123,8 +123,8 @@ def fft_conv(x, w, n: int, conj: bool = True, nout: int | None = None, out=None,
     nout = n if nout is None else nout
     if out is None:
         out = torch.empty(x.shape[:-1] + (nout,), dtype=torch.complex64, device=x.device)
-    L.check(L.lib().mxr_fft_conv(L.ref(L.desc(out)), L.ref(L.desc(x)), L.ref(L.desc(w)),
-                                 int(n), 1 if conj else 0, L.stream_handle(stream)))
+    L.check(L.lib().mxr_fft_conv(L.arg(out), L.arg(x), L.arg(w),
+                                 int(n), 1 if conj else 0, L.raw_stream(stream)))
     return out
 
 
@@ -139,8 +139,8 @@ def pulse_compress(x, w, n: int, nout: int | None = None, window: bool = True,
         out = torch.empty(x.shape[:-1] + (nout,), dtype=torch.complex64, device=x.device)
     flags = (L.PC_WINDOW if window else 0) | (L.PC_NORMALIZE if normalize else 0) | \
             (L.PC_WRITEBACK if writeback else 0)
-    L.check(L.lib().mxr_pulse_compress(L.ref(L.desc(out)), L.ref(L.desc(x)), L.ref(L.desc(w)),
-                                       int(n), flags, L.stream_handle(stream)))
+    L.check(L.lib().mxr_pulse_compress(L.arg(out), L.arg(x), L.arg(w),
+                                       int(n), flags, L.raw_stream(stream)))
     return out
 
 
@@ -161,15 +161,15 @@ class PulseCompressionPlan:
         self._h = h
 
     def set_waveform(self, w, stream=None):
-        L_.check(L_.lib().mxr_pc_plan_set_waveform(self._h, L_.ref(L_.desc(w)),
-                                                   L_.stream_handle(stream)))
+        L_.check(L_.lib().mxr_pc_plan_set_waveform(self._h, L_.arg(w),
+                                                   L_.raw_stream(stream)))
         self._w = w  # keep the waveform alive until the spectrum is computed
 
     def __call__(self, x, out=None, stream=None):
         if out is None:
             out = torch.empty(x.shape[:-1] + (self.nout,), dtype=torch.complex64, device=x.device)
-        L_.check(L_.lib().mxr_pc_plan_execute(self._h, L_.ref(L_.desc(out)), L_.ref(L_.desc(x)),
-                                              L_.stream_handle(stream)))
+        L_.check(L_.lib().mxr_pc_plan_execute(self._h, L_.arg(out), L_.arg(x),
+                                              L_.raw_stream(stream)))
         return out
 
     def waveform_grad(self, gy, x, w, out=None, stream=None):
@@ -177,9 +177,9 @@ class PulseCompressionPlan:
         over every row (mxr_pc_plan_waveform_grad); gy = dL/dy."""
         if out is None:
             out = torch.empty((self.L,), dtype=torch.complex64, device=x.device)
-        L_.check(L_.lib().mxr_pc_plan_waveform_grad(self._h, L_.ref(L_.desc(out)),
-                                                    L_.ref(L_.desc(gy)), L_.ref(L_.desc(x)),
-                                                    L_.ref(L_.desc(w)), L_.stream_handle(stream)))
+        L_.check(L_.lib().mxr_pc_plan_waveform_grad(self._h, L_.arg(out),
+                                                    L_.arg(gy), L_.arg(x),
+                                                    L_.arg(w), L_.raw_stream(stream)))
         return out
 
     def close(self):
@@ -207,8 +207,8 @@ def doppler(y, nd: int, tpc: str = "same", win_rows: int | None = None, rd=None,
         pw = torch.empty((C, nd, R), dtype=torch.float32, device=y.device)
     if rd is None and want_rd:
         rd = torch.empty((C, nd, R), dtype=torch.complex64, device=y.device)
-    L.check(L.lib().mxr_doppler(L.ref(L.desc(pw)), L.ref(L.desc(rd)), L.ref(L.desc(y)), mode,
-                                int(win_rows), int(nd), L.stream_handle(stream)))
+    L.check(L.lib().mxr_doppler(L.arg(pw), L.arg(rd), L.arg(y), mode,
+                                int(win_rows), int(nd), L.raw_stream(stream)))
     return pw, rd
 
 
@@ -223,8 +223,8 @@ def doppler_adjoint(gpow, y, nd: int, tpc: str = "same", win_rows: int | None = 
     win_rows = (P - 2 if mode != L.TPC_NONE else rows) if win_rows is None else win_rows
     if gy is None:
         gy = torch.empty_like(y)
-    L.check(L.lib().mxr_doppler_adjoint(L.ref(L.desc(gy)), L.ref(L.desc(gpow)), L.ref(L.desc(y)),
-                                        mode, int(win_rows), int(nd), L.stream_handle(stream)))
+    L.check(L.lib().mxr_doppler_adjoint(L.arg(gy), L.arg(gpow), L.arg(y),
+                                        mode, int(win_rows), int(nd), L.raw_stream(stream)))
     return gy
 
 
@@ -239,8 +239,8 @@ def cfar(inp, win=(5, 13), guard=(3, 3), pfa: float = 1e-5, dets=None, ba=None, 
     if ba is None and want_ba:
         ba = torch.empty(inp.shape, dtype=torch.float32, device=inp.device)
     p = L.mxr_cfar_params(win[0], win[1], guard[0], guard[1], float(pfa))
-    L.check(L.lib().mxr_cfar(L.ref(L.desc(dets)), L.ref(L.desc(ba)), L.ref(L.desc(pw)),
-                             L.ref(L.desc(inp)), L.ctypes.byref(p), L.stream_handle(stream)))
+    L.check(L.lib().mxr_cfar(L.arg(dets), L.arg(ba), L.arg(pw),
+                             L.arg(inp), L.ctypes.byref(p), L.raw_stream(stream)))
     return dets, ba, pw
 
 
@@ -262,9 +262,9 @@ def doppler_cfar(y, nd: int, tpc: str = "same", win_rows: int | None = None, win
     if pw is None and want_pow:
         pw = torch.empty((C, nd, R), dtype=torch.float32, device=y.device)
     p = L.mxr_cfar_params(win[0], win[1], guard[0], guard[1], float(pfa))
-    L.check(L.lib().mxr_doppler_cfar(L.ref(L.desc(dets)), L.ref(L.desc(ba)), L.ref(L.desc(pw)),
-                                     L.ref(L.desc(y)), mode, int(win_rows), int(nd),
-                                     L.ctypes.byref(p), L.stream_handle(stream)))
+    L.check(L.lib().mxr_doppler_cfar(L.arg(dets), L.arg(ba), L.arg(pw),
+                                     L.arg(y), mode, int(win_rows), int(nd),
+                                     L.ctypes.byref(p), L.raw_stream(stream)))
     return dets, ba, pw
 
 
@@ -274,9 +274,9 @@ def fft_conv_adjoint(gy, x, w, n: int, conj: bool = True, want_gx: bool = True,
     waveform per row: returns (gx, gw) for gy = dL/dRe(y) + i dL/dIm(y)."""
     gx = torch.empty_like(x) if want_gx else None
     gw = torch.empty_like(w) if want_gw else None
-    L.check(L.lib().mxr_fft_conv_adjoint(L.ref(L.desc(gx)), L.ref(L.desc(gw)), L.ref(L.desc(gy)),
-                                         L.ref(L.desc(x)), L.ref(L.desc(w)), int(n),
-                                         1 if conj else 0, L.stream_handle(stream)))
+    L.check(L.lib().mxr_fft_conv_adjoint(L.arg(gx), L.arg(gw), L.arg(gy),
+                                         L.arg(x), L.arg(w), int(n),
+                                         1 if conj else 0, L.raw_stream(stream)))
     return gx, gw
 
 
@@ -284,8 +284,8 @@ def autocorr_adjoint(gy, s, n: int, stream=None):
     """Gradient w.r.t. s of r = fft_conv(s, s, n) (rows' matched filters to
     themselves) for gy = dL/dRe(r) + i dL/dIm(r)."""
     gs = torch.empty_like(s)
-    L.check(L.lib().mxr_autocorr_adjoint(L.ref(L.desc(gs)), L.ref(L.desc(gy)), L.ref(L.desc(s)),
-                                         int(n), L.stream_handle(stream)))
+    L.check(L.lib().mxr_autocorr_adjoint(L.arg(gs), L.arg(gy), L.arg(s),
+                                         int(n), L.raw_stream(stream)))
     return gs
 
 
@@ -295,8 +295,8 @@ def doppler_taps(x, taps, nd: int, want_rd: bool = False, want_pow: bool = True,
     C, P, R = x.shape
     pw = torch.empty((C, nd, R), dtype=torch.float32, device=x.device) if want_pow else None
     rd = torch.empty((C, nd, R), dtype=torch.complex64, device=x.device) if want_rd else None
-    L.check(L.lib().mxr_doppler_taps(L.ref(L.desc(pw)), L.ref(L.desc(rd)), L.ref(L.desc(x)),
-                                     L.ref(L.desc(taps)), int(nd), L.stream_handle(stream)))
+    L.check(L.lib().mxr_doppler_taps(L.arg(pw), L.arg(rd), L.arg(x),
+                                     L.arg(taps), int(nd), L.raw_stream(stream)))
     return pw, rd
 
 
@@ -306,17 +306,17 @@ def doppler_taps_adjoint(gpow, x, taps, nd: int, want_gx: bool = False, want_gta
     returns (gx, gtaps) for gpow = dL/dpow."""
     gx = torch.empty_like(x) if want_gx else None
     gt = torch.empty_like(taps) if want_gtaps else None
-    L.check(L.lib().mxr_doppler_taps_adjoint(L.ref(L.desc(gt)), L.ref(L.desc(gx)),
-                                             L.ref(L.desc(gpow)), L.ref(L.desc(x)),
-                                             L.ref(L.desc(taps)), int(nd),
-                                             L.stream_handle(stream)))
+    L.check(L.lib().mxr_doppler_taps_adjoint(L.arg(gt), L.arg(gx),
+                                             L.arg(gpow), L.arg(x),
+                                             L.arg(taps), int(nd),
+                                             L.raw_stream(stream)))
     return gx, gt
 
 
 def isl(r, stream=None):
     """Integrated sidelobe level of each row of r ([B, n] c64): [B] f32."""
     out = torch.empty((r.shape[0],), dtype=torch.float32, device=r.device)
-    L.check(L.lib().mxr_isl(L.ref(L.desc(out)), L.ref(L.desc(r)), L.stream_handle(stream)))
+    L.check(L.lib().mxr_isl(L.arg(out), L.arg(r), L.raw_stream(stream)))
     return out
 
 
@@ -325,22 +325,22 @@ def phase_isl(phi, n: int, out=None, stream=None):
     f32), one kernel: equal to isl(fft_conv(s, s, n)) with s = polar(1, phi)."""
     if out is None:
         out = torch.empty((phi.shape[0],), dtype=torch.float32, device=phi.device)
-    L.check(L.lib().mxr_phase_isl(L.ref(L.desc(out)), L.ref(L.desc(phi)), int(n),
-                                  L.stream_handle(stream)))
+    L.check(L.lib().mxr_phase_isl(L.arg(out), L.arg(phi), int(n),
+                                  L.raw_stream(stream)))
     return out
 
 
 def phase_isl_adjoint(gisl, phi, n: int, stream=None):
     gphi = torch.empty_like(phi)
-    L.check(L.lib().mxr_phase_isl_adjoint(L.ref(L.desc(gphi)), L.ref(L.desc(gisl)), L.ref(L.desc(phi)),
-                                          int(n), L.stream_handle(stream)))
+    L.check(L.lib().mxr_phase_isl_adjoint(L.arg(gphi), L.arg(gisl), L.arg(phi),
+                                          int(n), L.raw_stream(stream)))
     return gphi
 
 
 def isl_adjoint(gisl, r, stream=None):
     gr = torch.empty_like(r)
-    L.check(L.lib().mxr_isl_adjoint(L.ref(L.desc(gr)), L.ref(L.desc(gisl)), L.ref(L.desc(r)),
-                                    L.stream_handle(stream)))
+    L.check(L.lib().mxr_isl_adjoint(L.arg(gr), L.arg(gisl), L.arg(r),
+                                    L.raw_stream(stream)))
     return gr
 
 
@@ -349,16 +349,16 @@ def psl(pw, targets, ml: int = 2, q: int = 8, out=None, stream=None):
     targets ([T, 3] int32: channel, range bin, Doppler bin): [T] f32."""
     if out is None:
         out = torch.empty((targets.shape[0],), dtype=torch.float32, device=pw.device)
-    L.check(L.lib().mxr_psl(L.ref(L.desc(out)), L.ref(L.desc(pw)), L.ref(L.desc(targets)),
-                            int(ml), int(q), L.stream_handle(stream)))
+    L.check(L.lib().mxr_psl(L.arg(out), L.arg(pw), L.arg(targets),
+                            int(ml), int(q), L.raw_stream(stream)))
     return out
 
 
 def psl_adjoint(gpsl, pw, targets, ml: int = 2, q: int = 8, stream=None):
     gp = torch.empty_like(pw, memory_format=torch.contiguous_format)
-    L.check(L.lib().mxr_psl_adjoint(L.ref(L.desc(gp)), L.ref(L.desc(gpsl)), L.ref(L.desc(pw)),
-                                    L.ref(L.desc(targets)), int(ml), int(q),
-                                    L.stream_handle(stream)))
+    L.check(L.lib().mxr_psl_adjoint(L.arg(gp), L.arg(gpsl), L.arg(pw),
+                                    L.arg(targets), int(ml), int(q),
+                                    L.raw_stream(stream)))
     return gp
 
 
@@ -366,9 +366,9 @@ def psl_taps_adjoint(gpsl, pw, x, taps, targets, ml: int = 2, q: int = 8, stream
     """d(sum_t gpsl_t psl_t)/dtaps for pw = doppler_taps(x, taps)'s power,
     from the target columns alone: [P] f32."""
     gt = torch.empty_like(taps)
-    L.check(L.lib().mxr_psl_taps_adjoint(L.ref(L.desc(gt)), L.ref(L.desc(gpsl)), L.ref(L.desc(pw)),
-                                         L.ref(L.desc(x)), L.ref(L.desc(taps)), L.ref(L.desc(targets)),
-                                         int(ml), int(q), L.stream_handle(stream)))
+    L.check(L.lib().mxr_psl_taps_adjoint(L.arg(gt), L.arg(gpsl), L.arg(pw),
+                                         L.arg(x), L.arg(taps), L.arg(targets),
+                                         int(ml), int(q), L.raw_stream(stream)))
     return gt
 
 
@@ -399,11 +399,11 @@ def _conv1d(x, f, mode, method, is_corr, out, stream):
         out = torch.empty(x.shape[:-1] + (olen,), device=x.device,
                           dtype=torch.complex64 if cplx else torch.float32)
     if method == "direct":
-        L.check(L.lib().mxr_conv1d(L.ref(L.desc(out)), L.ref(L.desc(x)), L.ref(L.desc(f)), m,
-                                   L.stream_handle(stream)))
+        L.check(L.lib().mxr_conv1d(L.arg(out), L.arg(x), L.arg(f), m,
+                                   L.raw_stream(stream)))
     elif method == "fft":
-        L.check(L.lib().mxr_conv1d_fft(L.ref(L.desc(out)), L.ref(L.desc(x)), L.ref(L.desc(f)), m,
-                                       1 if is_corr else 0, L.stream_handle(stream)))
+        L.check(L.lib().mxr_conv1d_fft(L.arg(out), L.arg(x), L.arg(f), m,
+                                       1 if is_corr else 0, L.raw_stream(stream)))
     else:
         raise ValueError(f"conv1d: method must be 'direct' or 'fft', got {method!r}")
     return out
@@ -420,6 +420,6 @@ def conv2d(x, f, mode="full", out=None, stream=None):
     if out is None:
         out = torch.empty(x.shape[:-2] + (oh, ow), device=x.device,
                           dtype=torch.complex64 if cplx else torch.float32)
-    L.check(L.lib().mxr_conv2d(L.ref(L.desc(out)), L.ref(L.desc(x)), L.ref(L.desc(f)), m,
-                               L.stream_handle(stream)))
+    L.check(L.lib().mxr_conv2d(L.arg(out), L.arg(x), L.arg(f), m,
+                               L.raw_stream(stream)))
     return out

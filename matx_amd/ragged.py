@@ -47,7 +47,7 @@ class RaggedBatch:
         flags = (L.RAGGED_AUTOTUNE if autotune else 0) | (L.RAGGED_PERSISTENT if persistent else 0)
         h = ctypes.c_void_p()
         L.check(L.lib().mxr_ragged_plan_create(ctypes.byref(h), descs, len(jobs), flags,
-                                               L.stream_handle(stream)))
+                                               L.raw_stream(stream)))
         self._h = h
 
     def block_size(self, job: int) -> int:
@@ -56,7 +56,7 @@ class RaggedBatch:
         return m.value
 
     def execute(self, stream=None):
-        L.check(L.lib().mxr_ragged_execute(self._h, L.stream_handle(stream)))
+        L.check(L.lib().mxr_ragged_execute(self._h, L.raw_stream(stream)))
         return self.pw
 
     def graph(self, stream=None):

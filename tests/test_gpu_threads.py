@@ -90,3 +90,14 @@ def test_threads_bit_identical_to_single_thread(mx):
     for i in range(NTHREADS):
         for k, v in ref[i].items():
             assert torch.equal(results[i][k], v), (i, k)
+
+
+def test_raw_stream_is_the_current_stream():
+    """The handle the entry points get is torch's current stream's, inside and
+    outside a stream context, and a given stream's own."""
+    import matx_amd._lib as L
+    s = torch.cuda.Stream()
+    assert L.raw_stream() == torch.cuda.current_stream().cuda_stream == (L.stream_handle().value or 0)
+    with torch.cuda.stream(s):
+        assert L.raw_stream() == s.cuda_stream == L.stream_handle().value
+    assert L.raw_stream(s) == s.cuda_stream

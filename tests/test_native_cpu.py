@@ -367,3 +367,20 @@ def test_dlpack_export_descriptor(L):
     assert r == 6
     r, _ = status(L, lib.mxr_tensor_to_dlpack, ctypes.byref(s), 10, 0, rel, None, None)
     assert r == 2
+
+
+@pytest.mark.parametrize("shape", [(), (3,), (2, 0), (4, 5, 6), (1, 2, 3, 4, 5, 6, 7, 2)])
+def test_packed_descriptor(L, shape):
+    """arg()'s bytes are the mxr_tensor desc() fills, for every rank, on strided
+    and broadcast views; what desc() refuses, arg() refuses."""
+    torch = pytest.importorskip("torch")
+    for dt in (torch.complex64, torch.float32, torch.int32):
+        t = torch.zeros(shape, dtype=dt)
+        views = [t, t.permute(tuple(reversed(range(t.dim())))), t[..., None].expand(*shape, 7)[..., ::2] if t.dim() < 8 else t]
+        for v in views:
+            assert L.arg(v) == bytes(L.desc(v))
+    assert L.arg(None) is None
+    for bad in (torch.zeros(2, dtype=torch.float64), torch.zeros((1,) * 9)):
+        for f in (L.arg, L.desc):
+            with pytest.raises(L.MatxError):
+                f(bad)
