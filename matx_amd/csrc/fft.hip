@@ -39,6 +39,7 @@ struct FftArgs {
   int64_t istride, ostride;
   BatchIdx bi;     // batch dims: sa = input strides, sb = output strides
   int batch_fast;  // gather/scatter with lanes over the batch index
+  int small_batch; // nbatch below 2^31
   float scale;
   const float2 *tw;
 };
@@ -101,38 +102,98 @@ __device__ __forceinline__ void with_kind(int kind, F &&body) {
   else body(std::integral_constant<int, FFT_C2C>{});
 }
 
-template <int N>
+// Transforms per workgroup TB and threads NT (16 elements a thread).  Along a
+// strided axis (COL) the workgroup's transforms are neighbours in memory, and
+// 16 of them make the 128-byte runs of whole cache lines: 512 and 1024 points
+// take a 64 KiB tile for 16 and 8 of them.
+template <int N, bool COL>
 struct GenericCfg {
-  static constexpr int TB = N >= 4096 ? 1 : 4096 / N;
-  static constexpr int NT = N >= 4096 ? N / 16 : 256;
+  static constexpr int TB = COL && (N == 512 || N == 1024) ? 8192 / N : (N >= 4096 ? 1 : 4096 / N);
+  static constexpr int NT = TB * N / 16 < 256 ? 256 : TB * N / 16;
 };
 
-// COL: element i of transform t at i * TB + t (batch_fast calls, where the
-// workgroup's transforms are neighbours in memory and the gather and
-// scatter run lanes across them: consecutive lanes touch consecutive LDS
-// words, where the transform-major layout puts them a padded row apart).
+// COL: element i of transform t at i * TB + t (batch_fast calls: lanes run
+// across the transforms, so consecutive lanes touch consecutive LDS words,
+// where the transform-major layout puts them a padded row apart).
+// DIRECT: the first pass loads its butterflies' inputs from memory and the
+// last one stores its outputs there, in runs of at least 128 bytes (lanes
+// across transforms, or 16 butterflies and more of one transform side by
+// side); shorter contiguous transforms are staged through LDS instead, whole
+// rows at a time.  Bound by HBM: 16 x 8001 transforms of 256 points along a
+// strided axis
+// staged through LDS on both sides took 177 us, direct 130; 103 us is the copy
+// rate's.
 template <int N, bool INV, bool COL>
-__global__ __launch_bounds__(GenericCfg<N>::NT) void fft_generic_kernel(FftArgs a) {
-  constexpr int TB = GenericCfg<N>::TB;
-  constexpr int NT = GenericCfg<N>::NT;
-  using LY = Layout<N, TB, COL>;
+__global__ __launch_bounds__((GenericCfg<N, COL>::NT)) void fft_generic_kernel(FftArgs a) {
+  constexpr int TB = GenericCfg<N, COL>::TB;
+  constexpr int NT = GenericCfg<N, COL>::NT;
+  constexpr bool DIRECT = COL || N >= 256;
+  using LY = Layout<N, TB, COL, (COL && TB < 32 && N >= 32)>;
   using SQ = Seq<N, false>;
+  constexpr int K = SQ::n;
   __shared__ float2 lds[LY::LDS_ELEMS];
   __shared__ int64_t base_in[TB], base_out[TB];
 
-  const int64_t t0 = (int64_t)blockIdx.x * TB;
+  // neighbouring transforms along a strided axis share cache lines: one XCD
+  const int64_t t0 = (COL ? xcd_remap(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x) * TB;
   for (int t = threadIdx.x; t < TB; t += NT) {
     int64_t oi = 0, oo = 0;
-    if (t0 + t < a.nbatch) batch_offsets(a.bi, t0 + t, &oi, &oo);
+    if (t0 + t < a.nbatch) {
+      if (a.small_batch) batch_offsets32(a.bi, (uint32_t)(t0 + t), &oi, &oo);
+      else batch_offsets(a.bi, t0 + t, &oi, &oo);
+    }
     base_in[t] = oi;
     base_out[t] = oo;
   }
   __syncthreads();
 
+  if constexpr (DIRECT) {
+    constexpr int R0 = SQ::template R<0>, RL = SQ::template R<K - 1>;
+    using P0 = Pass<LY, R0, N, NT, TB>;
+    P0 p0;
+    if (a.in_len <= 0) {
+      p0.load([](int, int) { return make_float2(0.f, 0.f); });
+    } else if (a.kind == FFT_C2C && a.in_len == a.n) {
+#pragma unroll
+      for (int u = 0; u < P0::BPT; ++u) {
+        if (!P0::active(u)) continue;
+        int t, j;
+        LY::template bfly<R0>(threadIdx.x + u * NT, t, j);
+        // an idle transform reads its workgroup's first one
+        const float2 *src = a.in + base_in[t0 + t < a.nbatch ? t : 0] + (int64_t)j * a.istride;
+        const int64_t step = (int64_t)P0::NB * a.istride;
+#pragma unroll
+        for (int m = 0; m < R0; ++m, src += step) p0.v[u][m] = *src;
+      }
+    } else {
+      with_kind(a.kind, [&](auto kt) {
+        constexpr int KIND = decltype(kt)::value;
+        p0.load([&](int t, int i) { return fft_load<KIND>(a, base_in[t], i, t0 + t < a.nbatch); });
+      });
+    }
+    auto put = [&](int t, int k, float2 v) {
+      if (t0 + t < a.nbatch && k < a.out_len) fft_scatter(a, base_out[t], k, cscale(v, a.scale));
+    };
+    p0.template compute<1, INV>(nullptr);
+    if constexpr (K == 1) {
+      p0.template store<1>(put);
+    } else {
+      p0.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
+      wg_barrier();
+      lds_passes<LY, SQ, N, NT, TB, INV, 1, K - 1>(lds, a.tw);
+      constexpr int LSL = SQ::template LS<K - 1>;
+      Pass<LY, RL, N, NT, TB> pl;
+      pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
+      pl.template compute<LSL, INV>(a.tw + SQ::template TWOFF<K - 1>);
+      pl.template store<LSL>(put);
+    }
+    return;
+  }
+
   // gather: each thread's PER elements are loaded before any is stored, so
   // its loads are in flight together
   constexpr int PER = TB * N / NT;
-  static_assert(PER * NT == TB * N, "whole elements per thread");
+  static_assert(DIRECT || PER * NT == TB * N, "whole elements per thread");
   {
     float2 gv[PER];
 #pragma unroll
@@ -143,33 +204,21 @@ __global__ __launch_bounds__(GenericCfg<N>::NT) void fft_generic_kernel(FftArgs 
 #pragma unroll
         for (int m = 0; m < PER; ++m) {
           const int e = threadIdx.x + m * NT;
-          const int t = a.batch_fast ? e % TB : e / N;
-          const int i = a.batch_fast ? e / TB : e % N;
-          gv[m] = fft_load<KIND>(a, base_in[t], i, t0 + t < a.nbatch);
+          gv[m] = fft_load<KIND>(a, base_in[e / N], e % N, t0 + e / N < a.nbatch);
         }
       });
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
       const int e = threadIdx.x + m * NT;
-      const int t = a.batch_fast ? e % TB : e / N;
-      const int i = a.batch_fast ? e / TB : e % N;
-      lds[LY::addr(t, i)] = gv[m];
+      lds[LY::addr(e / N, e % N)] = gv[m];
     }
   }
   __syncthreads();
 
-  lds_passes<LY, SQ, N, NT, TB, INV, 0, SQ::n>(lds, a.tw);
+  lds_passes<LY, SQ, N, NT, TB, INV, 0, K>(lds, a.tw);
 
-  // scatter
   for (int e = threadIdx.x; e < TB * N; e += NT) {
-    int t, i;
-    if (a.batch_fast) {
-      t = e % TB;
-      i = e / TB;
-    } else {
-      t = e / N;
-      i = e % N;
-    }
+    const int t = e / N, i = e % N;
     if (t0 + t < a.nbatch && i < a.out_len) fft_scatter(a, base_out[t], i, cscale(lds[LY::addr(t, i)], a.scale));
   }
 }
@@ -183,25 +232,25 @@ __global__ void fft_n1_kernel(FftArgs a) {
   fft_scatter(a, oo, 0, cscale(fft_gather(a, oi, 0), a.scale));
 }
 
-template <int N>
-static mxr_status launch_generic(const FftArgs &a, bool inv, hipStream_t s) {
-  using C = GenericCfg<N>;
+template <int N, bool COL>
+static mxr_status launch_generic(FftArgs a, bool inv, hipStream_t s) {
+  using C = GenericCfg<N, COL>;
   const int64_t grid = (a.nbatch + C::TB - 1) / C::TB;
   if (grid == 0) return MXR_SUCCESS;
   MXR_REQUIRE(grid <= 0x7fffffff, MXR_INVALID_SIZE, "fft: batch too large");
+  a.small_batch = a.nbatch < (1ll << 31);
   ProfScope ps("fft_generic_kernel", s);
-  if constexpr (C::TB > 1) {
-    if (a.batch_fast) {
-      if (inv) fft_generic_kernel<N, true, true><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(a);
-      else fft_generic_kernel<N, false, true><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(a);
-      MXR_HIP_TRY(hipGetLastError());
-      return MXR_SUCCESS;
-    }
-  }
-  if (inv) fft_generic_kernel<N, true, false><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(a);
-  else fft_generic_kernel<N, false, false><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(a);
+  if (inv) fft_generic_kernel<N, true, COL><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(a);
+  else fft_generic_kernel<N, false, COL><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(a);
   MXR_HIP_TRY(hipGetLastError());
   return MXR_SUCCESS;
+}
+
+template <int N>
+static mxr_status launch_generic(const FftArgs &a, bool inv, hipStream_t s) {
+  if constexpr (N < 4096)
+    if (a.batch_fast) return launch_generic<N, true>(a, inv, s);
+  return launch_generic<N, false>(a, inv, s);
 }
 
 static mxr_status dispatch_generic(int64_t n, const FftArgs &a, bool inv, hipStream_t s) {
@@ -241,27 +290,118 @@ struct CztArgs {
   int n;               // transform size
   const float2 *chirp; // c[0..n)
   const float2 *spec;  // H[0..M), scaled by 1/M
+  const float2 *twi;   // table of the reversed sequence
 };
 
-template <int M, bool INV>
-__global__ __launch_bounds__(GenericCfg<M>::NT) void czt_kernel(CztArgs z) {
-  constexpr int TB = GenericCfg<M>::TB;
-  constexpr int NT = GenericCfg<M>::NT;
-  using LY = Layout<M, TB, false>;
+// DIRECT (as fft_generic_kernel's): the first pass loads x.c, the last forward
+// pass, the spectrum product and the first inverse pass (the inverse runs the
+// reversed radix sequence) share registers, and the last inverse pass stores
+// c.y.  M >= 2n, so the upper half of the inputs is zero and the upper half of
+// the outputs is not wanted: the first and the last pass do half the loads,
+// stores and sums.  8192 transforms of 1000 points: 77 us
+// with everything staged in LDS, 52 direct.
+template <int M, bool INV, bool COL>
+__global__ __launch_bounds__((GenericCfg<M, COL>::NT)) void czt_kernel(CztArgs z) {
+  constexpr int TB = GenericCfg<M, COL>::TB;
+  constexpr int NT = GenericCfg<M, COL>::NT;
+  constexpr bool DIRECT = COL || M >= 256;
+  using LY = Layout<M, TB, COL, (COL && TB < 32 && M >= 32)>;
   using SQ = Seq<M, false>;
   __shared__ float2 lds[LY::LDS_ELEMS];
   __shared__ int64_t base_in[TB], base_out[TB];
   const FftArgs &a = z.f;
   const int n = z.n;
 
-  const int64_t t0 = (int64_t)blockIdx.x * TB;
+  const int64_t t0 = (COL ? xcd_remap(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x) * TB;
   for (int t = threadIdx.x; t < TB; t += NT) {
     int64_t oi = 0, oo = 0;
-    if (t0 + t < a.nbatch) batch_offsets(a.bi, t0 + t, &oi, &oo);
+    if (t0 + t < a.nbatch) {
+      if (a.small_batch) batch_offsets32(a.bi, (uint32_t)(t0 + t), &oi, &oo);
+      else batch_offsets(a.bi, t0 + t, &oi, &oo);
+    }
     base_in[t] = oi;
     base_out[t] = oo;
   }
   __syncthreads();
+
+  if constexpr (DIRECT) {
+    using SI = Seq<M, true>;
+    constexpr int K = SQ::n;
+    constexpr int R0 = SQ::template R<0>, RL = SQ::template R<K - 1>, LSL = SQ::template LS<K - 1>;
+    using P0 = Pass<LY, R0, M, NT, TB>;
+    using PL = Pass<LY, RL, M, NT, TB>;
+    auto put = [&](int t, int k, float2 v) {
+      float2 y = cscale(cmul(v, z.chirp[k < n ? k : 0]), a.scale);
+      if (INV) y.y = -y.y;
+      if (t0 + t < a.nbatch && k < (int)a.out_len) fft_scatter(a, base_out[t], k, y);
+    };
+    P0 p0;
+    float2 cv[P0::BPT][R0 / 2];
+#pragma unroll
+    for (int u = 0; u < P0::BPT; ++u) {
+      int t, j;
+      LY::template bfly<R0>(threadIdx.x + u * NT, t, j);
+#pragma unroll
+      for (int m = 0; m < R0; ++m) p0.v[u][m] = make_float2(0.f, 0.f);
+#pragma unroll
+      for (int m = 0; m < R0 / 2; ++m) cv[u][m] = z.chirp[j + m * P0::NB < n ? j + m * P0::NB : 0];
+    }
+    if (a.in_len > 0)
+      with_kind(a.kind, [&](auto kt) {
+        constexpr int KIND = decltype(kt)::value;
+#pragma unroll
+        for (int u = 0; u < P0::BPT; ++u) {
+          if (!P0::active(u)) continue;
+          int t, j;
+          LY::template bfly<R0>(threadIdx.x + u * NT, t, j);
+#pragma unroll
+          for (int m = 0; m < R0 / 2; ++m) {
+            const int i = j + m * P0::NB;
+            p0.v[u][m] = fft_load<KIND>(a, base_in[t], i, t0 + t < a.nbatch && i < n);
+          }
+        }
+      });
+#pragma unroll
+    for (int u = 0; u < P0::BPT; ++u)
+#pragma unroll
+      for (int m = 0; m < R0 / 2; ++m) {
+        float2 x = p0.v[u][m];
+        if (INV) x.y = -x.y;
+        p0.v[u][m] = cmul(x, cv[u][m]);
+      }
+    p0.template compute<1, false>(nullptr);
+    PL pl;
+    if constexpr (K == 1) {
+      pl = p0;
+    } else {
+      p0.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
+      wg_barrier();
+      lds_passes<LY, SQ, M, NT, TB, false, 1, K - 1>(lds, a.tw);
+      pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
+      wg_barrier();
+      pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
+    }
+    PL::template outputs<LSL>([&](int u, int q, int, int k) { pl.v[u][q] = cmul(pl.v[u][q], z.spec[k]); });
+    pl.template compute<1, true>(nullptr);
+    if constexpr (K == 1) {
+      PL::template outputs<1>([&](int u, int q, int t, int k) {
+        if (q < RL / 2) put(t, k, pl.v[u][q]);
+      });
+    } else {
+      pl.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
+      wg_barrier();
+      lds_passes<LY, SI, M, NT, TB, true, 1, K - 1>(lds, z.twi);
+      constexpr int RI = SI::template R<K - 1>, LSI = SI::template LS<K - 1>;
+      using PI = Pass<LY, RI, M, NT, TB>;
+      PI pi;
+      pi.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
+      pi.template compute<LSI, true>(z.twi + SI::template TWOFF<K - 1>);
+      PI::template outputs<LSI>([&](int u, int q, int t, int k) {
+        if (q < RI / 2) put(t, k, pi.v[u][q]);
+      });
+    }
+    return;
+  }
 
   // gather x.c into the first n slots (x conjugated for the inverse; C2R
   // input extended to n first), zeros to M
@@ -269,7 +409,7 @@ __global__ __launch_bounds__(GenericCfg<M>::NT) void czt_kernel(CztArgs z) {
   // before the values are combined and stored)
   constexpr int PER = TB * M / NT;
   constexpr int CH = PER < 8 ? PER : 8;
-  static_assert(PER * NT == TB * M && PER % CH == 0, "whole chunks per thread");
+  static_assert(DIRECT || (PER * NT == TB * M && PER % CH == 0), "whole chunks per thread");
 #pragma unroll 1
   for (int m0 = 0; m0 < PER; m0 += CH) {
     float2 xv[CH], cv[CH];
@@ -281,22 +421,22 @@ __global__ __launch_bounds__(GenericCfg<M>::NT) void czt_kernel(CztArgs z) {
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
           const int e = threadIdx.x + (m0 + j) * NT;
-          const int t = a.batch_fast ? e % TB : e / M;
-          const int i = a.batch_fast ? e / TB : e % M;
+          const int t = e / M;
+          const int i = e % M;
           xv[j] = fft_load<KIND>(a, base_in[t], i, t0 + t < a.nbatch && i < n);
         }
       });
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const int e = threadIdx.x + (m0 + j) * NT;
-      const int i = a.batch_fast ? e / TB : e % M;
+      const int i = e % M;
       cv[j] = z.chirp[i < n ? i : 0];
     }
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const int e = threadIdx.x + (m0 + j) * NT;
-      const int t = a.batch_fast ? e % TB : e / M;
-      const int i = a.batch_fast ? e / TB : e % M;
+      const int t = e / M;
+      const int i = e % M;
       float2 x = xv[j];
       if (INV) x.y = -x.y;
       lds[LY::addr(t, i)] = cmul(x, cv[j]);
@@ -323,14 +463,7 @@ __global__ __launch_bounds__(GenericCfg<M>::NT) void czt_kernel(CztArgs z) {
   // the inverse)
   const int nout = (int)a.out_len;
   for (int e = threadIdx.x; e < TB * nout; e += NT) {
-    int t, k;
-    if (a.batch_fast) {
-      t = e % TB;
-      k = e / TB;
-    } else {
-      t = e / nout;
-      k = e % nout;
-    }
+    const int t = e / nout, k = e % nout;
     if (t0 + t >= a.nbatch) continue;
     float2 y = cscale(cmul(lds[LY::addr(t, k)], z.chirp[k]), a.scale);
     if (INV) y.y = -y.y;
@@ -413,17 +546,25 @@ static const float2 *czt_tables(int n, int M) {
   return d;
 }
 
-template <int M>
-static mxr_status launch_czt(const CztArgs &z, bool inv, hipStream_t s) {
-  using C = GenericCfg<M>;
+template <int M, bool COL>
+static mxr_status launch_czt(CztArgs z, bool inv, hipStream_t s) {
+  using C = GenericCfg<M, COL>;
+  z.f.small_batch = z.f.nbatch < (1ll << 31);
   const int64_t grid = (z.f.nbatch + C::TB - 1) / C::TB;
   if (grid == 0) return MXR_SUCCESS;
   MXR_REQUIRE(grid <= 0x7fffffff, MXR_INVALID_SIZE, "fft: batch too large");
   ProfScope ps("czt_kernel", s);
-  if (inv) czt_kernel<M, true><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(z);
-  else czt_kernel<M, false><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(z);
+  if (inv) czt_kernel<M, true, COL><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(z);
+  else czt_kernel<M, false, COL><<<dim3((unsigned)grid), dim3(C::NT), 0, s>>>(z);
   MXR_HIP_TRY(hipGetLastError());
   return MXR_SUCCESS;
+}
+
+template <int M>
+static mxr_status launch_czt(const CztArgs &z, bool inv, hipStream_t s) {
+  if constexpr (M < 4096)
+    if (z.f.batch_fast) return launch_czt<M, true>(z, inv, s);
+  return launch_czt<M, false>(z, inv, s);
 }
 
 // Largest size the Bluestein path takes (its convolution fits one 16384-point
@@ -437,8 +578,9 @@ static mxr_status dispatch_czt(int64_t n, FftArgs a, bool inv, hipStream_t s) {
   z.f = a;
   z.n = (int)n;
   z.f.tw = twiddles_device(M, false);
+  z.twi = twiddles_device(M, true);
   const float2 *tab = czt_tables((int)n, M);
-  MXR_REQUIRE(z.f.tw != nullptr && tab != nullptr, MXR_OUT_OF_MEMORY,
+  MXR_REQUIRE(z.f.tw != nullptr && z.twi != nullptr && tab != nullptr, MXR_OUT_OF_MEMORY,
               "fft: table allocation failed for size %lld", (long long)n);
   z.chirp = tab;
   z.spec = tab + n;

@@ -132,3 +132,30 @@ def test_conv1d_fft_errors(mx):
                   out=torch.empty((0,), dtype=torch.float32, device="cuda"))
     with pytest.raises(ValueError):
         mx.conv1d(f, f, "full", method="winograd")
+
+
+@pytest.mark.parametrize("n", [2, 16, 32, 64, 256, 512, 1024, 2048, 4096, 3, 7, 100, 129, 300, 700, 1025])
+@pytest.mark.parametrize("cols", [1, 15, 33])
+def test_fft_axes_direct(mx, n, cols):
+    """Transforms along a contiguous and along a strided axis, batches that do
+    not fill a workgroup, inputs shorter and longer than the transform, both
+    directions, real in and out, in place, against numpy in FP64."""
+    rng = np.random.default_rng(100 * n + cols)
+    for extent in {n, max(1, n - n // 3), n + 5}:
+        x = sig(rng, (2, extent, cols), True)
+        xt = np.ascontiguousarray(x.transpose(0, 2, 1))
+        r = sig(rng, (2, extent, cols), False)
+        ref, inv = np.fft.fft(x.astype(complex), n, axis=1), np.fft.ifft(x.astype(complex), n, axis=1)
+        assert rel(host(mx.fft(dev(x), n, 1)), ref) < RTOL
+        assert rel(host(mx.ifft(dev(x), n, 1)), inv) < RTOL
+        assert rel(host(mx.fft(dev(xt), n)), ref.transpose(0, 2, 1)) < RTOL
+        assert rel(host(mx.ifft(dev(xt), n)), inv.transpose(0, 2, 1)) < RTOL
+        rr = np.fft.rfft(r.astype(float), n, axis=1)
+        assert rel(host(mx.rfft(dev(r), n, 1)), rr) < RTOL
+        assert rel(host(mx.rfft(dev(np.ascontiguousarray(r.transpose(0, 2, 1))), n)), rr.transpose(0, 2, 1)) < RTOL
+        h = sig(rng, (2, n // 2 + 1, cols), True)
+        back = np.fft.irfft(h.astype(complex), n, axis=1)
+        assert rel(host(mx.irfft(dev(h), n, 1)), back) < RTOL
+    y = dev(x := sig(rng, (3, n, cols), True))
+    mx.fft(y, n, 1, out=y)
+    assert rel(host(y), np.fft.fft(x.astype(complex), axis=1)) < RTOL
