@@ -10,12 +10,13 @@
 //    M >= P in LDS, transforms, multiplies by the filter spectrum (computed
 //    once per call by fconv_spec_kernel), inverse transforms and writes only
 //    the mode's window.
-//  * longer rows (c64, one filter for every row): output k >= L-1 of the
-//    FULL convolution is lag k-(L-1) >= 0 of the correlation of x with
+//  * longer rows (c64, one filter for every row): output k of the FULL
+//    convolution is lag k-(L-1) of the correlation of x with
 //    g = reverse(conj(h)) (for corr: g = h), which the overlap-save
-//    pulse-compression kernels compute for rows of any length; the at most
-//    L-1 outputs before it read only x[0, L-1) and come from the fused kernel
-//    run on that prefix.
+//    pulse-compression kernels compute for rows of any length, starting at the
+//    mode's first lag (negative but for VALID; samples before the row are
+//    zero).  Two launches: the filter's spectrum (read reversed and
+//    conjugated in place) and the blocks.
 #include <algorithm>
 
 #include "fft_engine.hpp"
@@ -26,7 +27,7 @@ namespace mxr {
 
 mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, const mxr_tensor *w,
                      int64_t n, int window, int normalize, int writeback, int conj_w,
-                     hipStream_t stream);
+                     int64_t shift, int reverse_conj, hipStream_t stream);
 
 // TB rows per 256-thread workgroup below 4096 points, one row of M/16
 // threads from 4096 up (one radix-16 butterfly per thread per pass).
@@ -126,13 +127,6 @@ __global__ __launch_bounds__(FcCfg<M>::NT) void fconv_kernel(FcArgs a) {
     if (a.out_c) static_cast<float2 *>(a.out)[o] = v;
     else static_cast<float *>(a.out)[o] = v.x;
   }
-}
-
-__global__ void rev_conj_kernel(float2 *g, const float2 *h, int64_t L, int64_t hs) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= L) return;
-  const float2 v = h[(L - 1 - i) * hs];
-  g[i] = make_float2(v.x, -v.y);
 }
 
 // Largest transform of the fused path (one workgroup per row).
@@ -251,39 +245,18 @@ mxr_status conv1d_fft_impl(const mxr_tensor *out, const mxr_tensor *in, const mx
   if (numel(*out) == 0) return MXR_SUCCESS;
   if (P <= FCONV_MAX_M) return fconv_fused(out, in, N, filt, corr, s0, olen, s);
 
-  // long rows: overlap-save correlation for the outputs at or after L-1,
-  // the fused kernel on x[0, L-1) for the ones before
+  // long rows: overlap-save correlation with reverse(conj(h)), whose lag r is
+  // the FULL output r + L - 1; the outputs before FULL index L - 1 are negative
+  // lags (samples before the row are zero)
   MXR_REQUIRE(in->dtype == MXR_C64 && filt->dtype == MXR_C64, MXR_NOT_SUPPORTED,
               "%s: rows longer than %lld points (N + L - 1 = %lld) need c64 input and filter", fn,
               (long long)FCONV_MAX_M, (long long)P);
   MXR_REQUIRE(2 * L - 2 <= FCONV_MAX_M, MXR_NOT_SUPPORTED,
               "%s: filters longer than %lld taps need N + L - 1 <= %lld", fn,
               (long long)(FCONV_MAX_M / 2 + 1), (long long)FCONV_MAX_M);
-  const int64_t head = std::max<int64_t>(0, L - 1 - s0);  // outputs before FULL index L-1
-  if (head > 0) {
-    mxr_tensor oh = *out;
-    oh.shape[r - 1] = head;
-    if ((st = fconv_fused(&oh, in, std::min(N, L - 1), filt, corr, s0, head, s))) return st;
-  }
-  mxr_tensor ot = *out;
-  ot.shape[r - 1] = olen - head;
-  ot.data = static_cast<float2 *>(out->data) + head * out->stride[r - 1];
   int64_t n = 1;
   while (n < P) n <<= 1;
-  if (corr) return pc_common(fn, &ot, in, filt, n, 0, 0, 0, 1, s);
-  // the correlation filter g = reverse(conj(h))
-  float2 *g = static_cast<float2 *>(stream_workspace("conv1d_fft_rev", sizeof(float2) * L, s));
-  if (g == nullptr) return workspace_failure(fn);
-  rev_conj_kernel<<<dim3((unsigned)((L + 255) / 256)), dim3(256), 0, s>>>(
-      g, static_cast<const float2 *>(filt->data), L, filt->stride[0]);
-  MXR_HIP_TRY(hipGetLastError());
-  mxr_tensor gt{};
-  gt.data = g;
-  gt.dtype = MXR_C64;
-  gt.rank = 1;
-  gt.shape[0] = L;
-  gt.stride[0] = 1;
-  return pc_common(fn, &ot, in, &gt, n, 0, 0, 0, 1, s);
+  return pc_common(fn, out, in, filt, n, 0, 0, 0, 1, L - 1 - s0, !corr, s);
 }
 
 }  // namespace mxr

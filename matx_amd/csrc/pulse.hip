@@ -41,6 +41,7 @@ struct PcArgs {
   int64_t nblk;     // blocks per row
   int64_t bpw;      // blocks per workgroup (nblk when y aliases x)
   int64_t groups;   // total workgroups
+  int64_t shift;    // outputs start at lag -shift (samples before the row are zero)
   const float2 *wc; // M-point waveform spectrum, scaled by 1/M
   const float2 *twf, *twi;
 };
@@ -65,8 +66,9 @@ __device__ __forceinline__ OlsBlock pc_block(const PcArgs &a, int64_t g) {
   const uint32_t row = (uint32_t)g / (uint32_t)a.nblk, blk = (uint32_t)g - row * (uint32_t)a.nblk;
   int64_t ox, oy;
   batch_offsets32(a.bi, row, &ox, &oy);
-  return OlsBlock{a.x + ox, a.y + oy, (int)blk * (int)a.V, (int)a.n, (int)a.seff,
-                  (int)a.nout, (int)a.V, a.wc};
+  const int sh = (int)a.shift;
+  return OlsBlock{a.x + ox, a.y + oy + sh, (int)blk * (int)a.V - sh, (int)a.n, (int)a.seff,
+                  (int)a.nout - sh, (int)a.V, a.wc};
 }
 
 // Body shared by the per-call kernel and the ragged-batch kernels.  Pre: the
@@ -93,7 +95,8 @@ __device__ __forceinline__ void ols_block(const OlsBlock &ob, const float2 *twf,
     ps.load([&](int, int i) {
       int gi = lo + i;
       if (gi >= n32) gi -= n32;
-      return keep_if(xr[gi < seff32 ? gi : 0], gi < seff32);
+      const bool in = (uint32_t)gi < (uint32_t)seff32;
+      return keep_if(xr[in ? gi : 0], in);
     });
     ps.template compute<1, false>(nullptr);
     ps.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
@@ -137,10 +140,19 @@ __device__ __forceinline__ void ols_block(const OlsBlock &ob, const float2 *twf,
 // TB = 4096/M small blocks per 256-thread workgroup (M <= 2048): transform
 // t runs the block obs[t] (kept in LDS).  Same passes as ols_block; an
 // inactive transform has seff = 0 (reads nothing) and nout = lo (stores
-// nothing).
-template <int M>
-__device__ __forceinline__ void ols_multi(const OlsBlock *obs, const float2 *twf,
-                                          const float2 *twi, float2 *lds) {
+// nothing).  A wave's butterflies of the first and of the last pass (radix 16)
+// belong to one transform, so its samples and lags go through raw buffer
+// resources as in the 4096-point kernel, and those of the middle pass (radix
+// M/256) to transform u in round u.
+// WF: the last transform is the zero-padded waveform instead, whose spectrum
+// the others read from LDS (wf_out(bin) = what a spectrum buffer would hold).
+struct NoWf {
+  static constexpr bool on = false;
+};
+template <int M, class WfF>
+__device__ __forceinline__ void ols_multi(const OlsBlock *obs, const float2 *twf, const float2 *twi,
+                                          float2 *lds, bool wrap32, const WfF &wf) {
+  constexpr bool WF = WfF::on;
   constexpr int NT = 256, TB = 4096 / M;
   using LY = Layout<M, TB, false>;
   using SF = Seq<M, false>;
@@ -149,56 +161,90 @@ __device__ __forceinline__ void ols_multi(const OlsBlock *obs, const float2 *twf
   constexpr int R0 = SF::template R<0>;
   constexpr int RL = SF::template R<K - 1>;
   constexpr int LSL = SF::template LS<K - 1>;
-  constexpr int NBL = M / RL;
-  static_assert(K >= 2 && R0 == 16, "small-block kernel expects a radix-16 first pass");
+  constexpr int NB0 = M / 16;  // radix-16 butterflies per transform
+  static_assert(K == 3 && R0 == 16 && SF::template R<1> == 16 && RL == M / 256, "M in {1024, 2048}");
+  const int t = __builtin_amdgcn_readfirstlane(threadIdx.x / NB0), j0 = threadIdx.x % NB0;
+  const OlsBlock ob = obs[t];
+  const int lo = __builtin_amdgcn_readfirstlane(ob.lo), n32 = __builtin_amdgcn_readfirstlane(ob.n);
+  const int seff = __builtin_amdgcn_readfirstlane(ob.seff);
   {
     Pass<LY, R0, M, NT, TB> ps;
-    ps.load([&](int t, int i) {
-      const OlsBlock &ob = obs[t];
-      int gi = ob.lo + i;
-      if (gi >= ob.n) gi -= ob.n;
-      // sample 0 of the row (an idle transform's row is a real one) and a
-      // mask past seff: unconditional loads
-      return keep_if(ob.xr[gi < ob.seff ? gi : 0], gi < ob.seff);
-    });
+    float2(&v)[16] = ps.v[0];
+    bool mine = true;  // a block's wave (the waveform's loads itself)
+    if constexpr (WF) {
+      mine = t != TB - 1;
+      if (!mine) wf.load(v, j0, NB0);
+    }
+    if (!mine) {
+    } else if (lo >= 0 && lo + M <= n32) {
+      int avail = seff - lo;
+      avail = avail < 0 ? 0 : (avail > M ? M : avail);
+      const buf_rsrc rx = make_rsrc(ob.xr + lo, avail * 8);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) v[m] = buf_load2(rx, (j0 + m * NB0) * 8);
+    } else if (wrap32) {
+      const buf_rsrc rx = make_rsrc(ob.xr, seff * 8);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        const int gi = lo + j0 + m * NB0;
+        v[m] = buf_load2(rx, (int)min((uint32_t)gi, (uint32_t)(gi - n32)) * 8);
+      }
+    } else {  // rows past 32-bit byte offsets
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        int gi = lo + j0 + m * NB0;
+        if (gi >= n32) gi -= n32;
+        const bool in = (uint32_t)gi < (uint32_t)seff;
+        v[m] = keep_if(ob.xr[in ? gi : 0], in);
+      }
+    }
     ps.template compute<1, false>(nullptr);
-    ps.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
+    ps.template store<1>([&](int tt, int i, float2 x) { lds[LY::addr(tt, i)] = x; });
   }
   wg_barrier();
   lds_passes<LY, SF, M, NT, TB, false, 1, K - 1>(lds, twf);
   {
     Pass<LY, RL, M, NT, TB> ps;
-    ps.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
+    const int j = threadIdx.x;  // butterfly j of transform u in round u; k == j in the last pass
+    ps.load([&](int tt, int i) { return lds[LY::addr(tt, i)]; });
     wg_barrier();
     ps.template compute<LSL, false>(twf + SF::template TWOFF<K - 1>);
+    if constexpr (WF) {
 #pragma unroll
-    for (int u = 0; u < ps.BPT; ++u) {
-      if (!ps.active(u)) continue;
-      const int g = threadIdx.x + u * NT;
-      const int t = g / NBL, j = g % NBL;  // k == j in the last pass
-      const float2 *wc = obs[t].wc;
-#pragma unroll
-      for (int q = 0; q < RL; ++q) ps.v[u][q] = cmul(ps.v[u][q], wc[j + q * LSL]);
+      for (int q = 0; q < RL; ++q) lds[j + q * LSL] = wf.out(ps.v[TB - 1][q]);
+      wg_barrier();
     }
+#pragma unroll
+    for (int u = 0; u < (WF ? TB - 1 : TB); ++u) {
+#pragma unroll
+      for (int q = 0; q < RL; ++q) {
+        float2 w;
+        if constexpr (WF) w = lds[j + q * LSL];
+        else w = obs[u].wc[j + q * LSL];
+        ps.v[u][q] = cmul(ps.v[u][q], w);
+      }
+    }
+    if constexpr (WF) wg_barrier();  // the spectrum has been read
     ps.template compute<1, true>(nullptr);
-    ps.template store<1>([&](int t, int i, float2 v) { lds[LY::addr(t, i)] = v; });
+    ps.template store<1>([&](int tt, int i, float2 v) { lds[LY::addr(tt, i)] = v; });
   }
   wg_barrier();
   lds_passes<LY, SI, M, NT, TB, true, 1, K - 1>(lds, twi);
   {
     constexpr int RI = SI::template R<K - 1>;
     constexpr int LSI = SI::template LS<K - 1>;
+    static_assert(RI == 16 && LSI == NB0, "last inverse pass");
     Pass<LY, RI, M, NT, TB> ps;
-    ps.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
+    ps.load([&](int tt, int i) { return lds[LY::addr(tt, i)]; });
     ps.template compute<LSI, true>(twi + SI::template TWOFF<K - 1>);
-    ps.template store<LSI>([&](int t, int i, float2 v) {
-      const OlsBlock &ob = obs[t];
-      const int lim = (ob.nout - ob.lo) < ob.V ? (ob.nout - ob.lo) : ob.V;
-      if (i < lim) ob.yr[ob.lo + i] = v;  // the spectrum carries the 1/M
-    });
+    int lim = __builtin_amdgcn_readfirstlane(ob.nout) - lo;
+    const int V = __builtin_amdgcn_readfirstlane(ob.V);
+    lim = lim < V ? lim : V;
+    const buf_rsrc ry = make_rsrc(ob.yr + lo, lim * 8);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) buf_store2(ry, (j0 + q * NB0) * 8, ps.v[0][q]);
   }
 }
-
 // Per-call small blocks: 4096/M (row, block) groups per workgroup.
 template <int M>
 __global__ __launch_bounds__(256) void pc_ols_multi_kernel(PcArgs a) {
@@ -215,7 +261,50 @@ __global__ __launch_bounds__(256) void pc_ols_multi_kernel(PcArgs a) {
     obs[threadIdx.x] = ob;
   }
   __syncthreads();
-  ols_multi<M>(obs, a.twf, a.twi, lds);
+  ols_multi<M>(obs, a.twf, a.twi, lds, a.n <= PC_BUF_MAX_N, NoWf{});
+}
+
+// Small grids (as pc4096_wf_kernel): the last transform of every workgroup is
+// the waveform, so no spectrum launch precedes the filter.
+struct WfLoad {
+  static constexpr bool on = true;
+  const float2 *w;
+  int64_t wstride;
+  int L, conj_in, conj;
+  float out_scale;
+  __device__ __forceinline__ void load(float2 (&v)[16], int j, int step) const {
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      const int i = j + m * step;
+      v[m] = keep_if(w[(int64_t)(i < L ? i : 0) * wstride], i < L);
+    }
+    if (conj_in) {
+#pragma unroll
+      for (int m = 0; m < 16; ++m) v[m].y = -v[m].y;
+    }
+  }
+  __device__ __forceinline__ float2 out(float2 x) const {
+    x = cscale(x, out_scale);
+    return make_float2(x.x, conj ? -x.y : x.y);
+  }
+};
+
+template <int M>
+__global__ __launch_bounds__(256) void pc_ols_multi_wf_kernel(PcArgs a, WfLoad wf) {
+  constexpr int TB = 4096 / M;
+  __shared__ float2 lds[Layout<M, TB, false>::LDS_ELEMS];
+  __shared__ OlsBlock obs[TB];
+  if (threadIdx.x < TB) {
+    const int64_t g = (int64_t)blockIdx.x * (TB - 1) + threadIdx.x;
+    const bool idle = threadIdx.x == TB - 1 || g >= a.groups;
+    OlsBlock ob = pc_block(a, idle ? 0 : g);
+    if (idle) {
+      ob.lo = ob.seff = ob.nout = 0;
+    }
+    obs[threadIdx.x] = ob;
+  }
+  __syncthreads();
+  ols_multi<M>(obs, a.twf, a.twi, lds, a.n <= PC_BUF_MAX_N, wf);
 }
 
 // ROWLOOP: one workgroup walks blocks [b0, b1) of its row in order (needed
@@ -233,10 +322,11 @@ void pc_ols_kernel(PcArgs a) {
   const int64_t b1 = ROWLOOP ? (b0 + a.bpw < a.nblk ? b0 + a.bpw : a.nblk) : b0 + 1;
   int64_t ox, oy;
   batch_offsets(a.bi, row, &ox, &oy);
-  OlsBlock ob{a.x + ox, a.y + oy, 0, (int)a.n, (int)a.seff, (int)a.nout, (int)a.V, a.wc};
+  const int sh = (int)a.shift;
+  OlsBlock ob{a.x + ox, a.y + oy + sh, 0, (int)a.n, (int)a.seff, (int)a.nout - sh, (int)a.V, a.wc};
   for (int64_t b = b0; b < b1; ++b) {
     if (b != b0) wg_barrier();  // previous block's LDS reads are done
-    ob.lo = (int)(b * a.V);
+    ob.lo = (int)(b * a.V) - sh;
     ols_block<M>(ob, a.twf, a.twi, lds);
   }
 }
@@ -270,13 +360,14 @@ __device__ __forceinline__ void load_block4096(const OlsBlock &ob, float2 (&v)[N
   asm volatile("" : "+v"(j));  // the 16 offsets are formed here, not kept in registers by a caller's loop
   const float2 *__restrict__ xr = ob.xr;
   const int lo = ob.lo, n32 = ob.n, seff32 = ob.seff;
-  if (lo + 4096 <= n32) {
+  if (lo >= 0 && lo + 4096 <= n32) {
     int avail = seff32 - lo;
     avail = avail < 0 ? 0 : (avail > 4096 ? 4096 : avail);
     const buf_rsrc rx = make_rsrc(xr + lo, avail * 8);
 #pragma unroll
     for (int m = 0; m < NV; ++m) v[m] = buf_load2(rx, (j + (m0 + m) * NT) * 8);
-  } else {  // the block wraps around the circular period n (full fft_conv)
+  } else {  // the block starts before the row or wraps around the circular
+            // period n (full fft_conv); offsets outside the row read as zeros
     const buf_rsrc rx = make_rsrc(xr, seff32 * 8);
 #pragma unroll
     for (int m = 0; m < NV; ++m) {
@@ -380,6 +471,20 @@ void pc4096_kernel(Pc4096Args pa) {
   ols_block4096(pc_block(a, xcd_remap(blockIdx.x, a.groups)), pa.base1, pa.base2, lds);
 }
 
+// In place: one workgroup walks the blocks of its row in order (a block only
+// overwrites lags below the next block's first input).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void pc4096_row_kernel(Pc4096Args pa) {
+  using LY = Layout<4096, 1, false>;
+  __shared__ float2 lds[LY::LDS_ELEMS];
+  const PcArgs &a = pa.a;
+  const uint32_t row = (uint32_t)xcd_remap(blockIdx.x, a.groups);
+  for (int b = 0; b < (int)a.nblk; ++b) {
+    if (b) wg_barrier();  // previous block's LDS reads are done
+    ols_block4096(pc_block(a, (int64_t)row * a.nblk + b), opaque(pa.base1), opaque(pa.base2), lds);
+  }
+}
+
 // Small grids (fft_conv on a few hundred pulses, where one workgroup per
 // pulse leaves most CUs idle): every workgroup transforms the zero-padded
 // waveform itself instead of waiting for a one-workgroup spectrum launch.
@@ -394,7 +499,7 @@ struct Pc4096WfArgs {
   Pc4096Args p;
   const float2 *w;
   int64_t wstride;
-  int L, conj;
+  int L, conj_in, conj;
   float out_scale;
 };
 
@@ -430,6 +535,7 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
   for (int m = 0; m < 16; ++m) {
     const int i = j + m * NT;
     v[m] = keep_if(q.w[(int64_t)(i < q.L ? i : 0) * q.wstride], i < q.L);
+    if (q.conj_in) v[m].y = -v[m].y;
   }
   dft16<false>(v);
   TwRow<16> tw = load_tw<16>(q.p.base1, 16, j & 15);
@@ -494,7 +600,7 @@ __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *b
   // sample, zeros past it) and form sum and difference
   {
     const int i0 = (j >> 1) + (j & 1) * 4096;
-    if (lo + 8192 <= n32) {
+    if (lo >= 0 && lo + 8192 <= n32) {
       int avail = seff32 - lo;
       avail = avail < 0 ? 0 : (avail > 8192 ? 8192 : avail);
       const buf_rsrc rx = make_rsrc(xr + lo, avail * 8);
@@ -561,6 +667,18 @@ void pc8192_kernel(Pc8192Args pa) {
   ols_block8192(ob, pa.bA, pa.bB, pa.bC, lds);
 }
 
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
+void pc8192_row_kernel(Pc8192Args pa) {
+  using LY = Layout<8192, 1, false>;
+  __shared__ float2 lds[LY::LDS_ELEMS];
+  const PcArgs &a = pa.a;
+  const uint32_t row = (uint32_t)xcd_remap(blockIdx.x, a.groups);
+  for (int b = 0; b < (int)a.nblk; ++b) {
+    if (b) wg_barrier();
+    ols_block8192(pc_block(a, (int64_t)row * a.nblk + b), opaque(pa.bA), opaque(pa.bB), opaque(pa.bC), lds);
+  }
+}
+
 // One workgroup of M/16 threads.  Thread j loads samples j + m*M/16,
 // m < 16 (all loads in flight at once), which are exactly the inputs of
 // butterfly j of the first radix-16 Stockham pass, so the window, the
@@ -589,6 +707,7 @@ __device__ __forceinline__ void wfspec_body(const WfArgs &a, float2 *lds, double
   for (int m = 0; m < 16; ++m) {
     const int i = tid + m * NT;
     float2 v = p0.v[0][m];
+    if (a.conj_in) v.y = -v.y;
     if (a.window && i < a.L) v = cscale(v, hamming_f32(i, (int)a.L));
     acc += (double)v.x * v.x + (double)v.y * v.y;
     p0.v[0][m] = v;
@@ -704,7 +823,7 @@ __global__ __launch_bounds__(256) void pc_batch_multi_kernel(const PcJob *jobs, 
     obs[threadIdx.x] = ob;
   }
   __syncthreads();
-  ols_multi<M>(obs, twf, twi, lds);
+  ols_multi<M>(obs, twf, twi, lds, true, NoWf{});
 }
 
 template <bool PERSIST>
@@ -882,10 +1001,15 @@ mxr_status plan_pc(int64_t seff, int64_t L, int64_t n, int64_t nout, bool allow_
         if (last_lo + M > n && (last_lo + M - n) > 0 && seff > 0) return;
       }
     }
-    // relative cost per point: 1024..8192 have dedicated or multi-block
-    // kernels with several workgroups per CU; the 16384-point kernel holds
-    // one workgroup per CU and runs about half as fast per point (measured)
-    const double eff = M <= 8192 ? 1.0 : (M == 16384 ? 2.0 : 1e9);
+    // relative time per M log2 M, measured on 16 rows of 1048576 samples with
+    // filters of 30 to 513 taps (1024 and 2048: 0.33 to 0.35, 4096: 0.29 to
+    // 0.30, 8192: 0.38 ps a point and level) and on the radar cubes (4096:
+    // 0.245, 8192: 0.264); the 16384-point kernel holds one workgroup per CU
+    // and runs about half as fast per point
+    double eff = M <= 2048 ? 1.15 : (M == 4096 ? 1.0 : (M == 8192 ? 1.15 : (M == 16384 ? 2.0 : 1e9)));
+    // in place, the blocks of a row run one after another in its workgroup
+    // (385 rows of 5003 samples, 487 taps: three blocks of 2048 took 53 us, one of 8192 20)
+    if (in_place && p.nblk > 1) eff *= 2.0;
     const double cost = (double)p.nblk * M * ilog2(M) * eff;
     if (cost < best_cost || (cost == best_cost && M > best.M)) {
       best_cost = cost;
@@ -945,12 +1069,23 @@ constexpr int64_t PC_WF_FUSE_MAX_GROUPS = 512;
 
 template <int M>
 mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
+  // the spectrum in the same launch: plain waveforms, small grids
+  const bool fuse = wa && pa && pa->groups > 0 && pa->bpw == 1 && pa->groups <= PC_WF_FUSE_MAX_GROUPS &&
+                    !wa->window && !wa->normalize && !wa->writeback && wa->L >= 1 && wa->L <= M;
+  if constexpr (M <= 2048) {
+    if (fuse) {
+      constexpr int RB = 4096 / M - 1;  // blocks per workgroup beside the waveform
+      const WfLoad wf{wa->w, wa->wstride, (int)wa->L, wa->conj_in, wa->conj, wa->out_scale};
+      ProfScope ps("pc_ols_kernel", s);
+      pc_ols_multi_wf_kernel<M><<<dim3((unsigned)((pa->groups + RB - 1) / RB)), dim3(256), 0, s>>>(*pa, wf);
+      MXR_HIP_TRY(hipGetLastError());
+      return MXR_SUCCESS;
+    }
+  }
   if constexpr (M == 4096) {
-    if (wa && pa && pa->groups > 0 && pa->bpw == 1 && pa->n <= PC_BUF_MAX_N &&
-        pa->groups <= PC_WF_FUSE_MAX_GROUPS && !wa->window && !wa->normalize && !wa->writeback &&
-        wa->L >= 1 && wa->L <= 4096) {
+    if (fuse && pa->n <= PC_BUF_MAX_N) {
       Pc4096WfArgs q{{*pa, tw16_device(16), tw16_device(256)}, wa->w, wa->wstride,
-                     (int)wa->L, wa->conj, wa->out_scale};
+                     (int)wa->L, wa->conj_in, wa->conj, wa->out_scale};
       MXR_REQUIRE(q.p.base1 && q.p.base2, MXR_OUT_OF_MEMORY,
                   "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc4096_wf_kernel", s);
@@ -966,22 +1101,25 @@ mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
   MXR_HIP_TRY(hipGetLastError());
   if (!pa || pa->groups <= 0) return MXR_SUCCESS;
   if constexpr (M == 8192) {
-    if (pa->bpw == 1 && pa->n <= PC_BUF_MAX_N) {
+    // (a row's block numbers fit 32 bits too where one workgroup walks them)
+    if (pa->n <= PC_BUF_MAX_N && pa->groups * pa->bpw <= 0x7fffffff) {
       Pc8192Args p8{*pa, tw16_device(2), tw16_device(32), tw16_device(512)};
       MXR_REQUIRE(p8.bA && p8.bB && p8.bC, MXR_OUT_OF_MEMORY,
                   "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc8192_kernel", s);
-      pc8192_kernel<<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
+      if (pa->bpw > 1) pc8192_row_kernel<<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
+      else pc8192_kernel<<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
       MXR_HIP_TRY(hipGetLastError());
       return MXR_SUCCESS;
     }
   }
   if constexpr (M == 4096) {
-    if (pa->bpw == 1 && pa->n <= PC_BUF_MAX_N) {
+    if (pa->n <= PC_BUF_MAX_N && pa->groups * pa->bpw <= 0x7fffffff) {
       Pc4096Args p4{*pa, tw16_device(16), tw16_device(256)};
       MXR_REQUIRE(p4.base1 && p4.base2, MXR_OUT_OF_MEMORY, "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc4096_kernel", s);
-      pc4096_kernel<<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
+      if (pa->bpw > 1) pc4096_row_kernel<<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
+      else pc4096_kernel<<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
       MXR_HIP_TRY(hipGetLastError());
       return MXR_SUCCESS;
     }
@@ -1103,10 +1241,12 @@ static mxr_status pc_blocks(const char *fn, const PcPlan &plan, bool in_place, c
 mxr_status fft_conv_rows(const mxr_tensor *out, const mxr_tensor *x, const mxr_tensor *w,
                          int64_t n, int conj_w, hipStream_t s);
 
-// Shared body of mxr_pulse_compress and mxr_fft_conv.
+// Shared body of mxr_pulse_compress, mxr_fft_conv and the long rows of
+// mxr_conv1d_fft.  shift: the first output is lag -shift (0 <= shift < L, and
+// n covers every nonzero lag); reverse_conj: the waveform is reverse(conj(w)).
 mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, const mxr_tensor *w,
                      int64_t n, int window, int normalize, int writeback, int conj_w,
-                     hipStream_t stream) {
+                     int64_t shift, int reverse_conj, hipStream_t stream) {
   mxr_status st;
   if ((st = check_tensor(w, "waveform", MXR_C64, 1, 1))) return st;
   PcArgs pa{};
@@ -1115,7 +1255,8 @@ mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, c
   const int64_t L = w->shape[0];
   MXR_REQUIRE(L >= 1 && L <= n, MXR_INVALID_SIZE, "%s: waveform length %lld not in [1, n=%lld]", fn,
               (long long)L, (long long)n);
-  MXR_REQUIRE(!views_overlap(*w, *x) && !views_overlap(*w, *y), MXR_ALIAS_ERROR,
+  // (a filter that is part of the signal is only read: conv1d's is accepted)
+  MXR_REQUIRE((reverse_conj || !views_overlap(*w, *x)) && !views_overlap(*w, *y), MXR_ALIAS_ERROR,
               "%s: waveform aliases the signal", fn);
   PcPlan plan;
   if ((st = plan_pc(pa.seff, L, n, pa.nout, conj_w != 0, in_place, &plan))) return st;
@@ -1130,6 +1271,11 @@ mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, c
   WfArgs wa{};
   wa.w = (float2 *)w->data;
   wa.wstride = w->stride[0];
+  if (reverse_conj) {
+    wa.w += (L - 1) * wa.wstride;
+    wa.wstride = -wa.wstride;
+    wa.conj_in = 1;
+  }
   wa.L = L;
   wa.window = window;
   wa.normalize = normalize;
@@ -1139,6 +1285,7 @@ mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, c
   wa.tw = twf;
   wa.out_scale = (float)(1.0 / (double)plan.M);  // exact: a power of two
   if ((st = pc_blocks(fn, plan, in_place, wc, twf, twi, &pa))) return st;
+  pa.shift = shift;
   return dispatch_pc(plan.M, &wa, &pa, stream);
 }
 
@@ -1301,7 +1448,7 @@ mxr_status mxr_pulse_compress(const mxr_tensor *y, const mxr_tensor *x, const mx
   return mxr::guarded("mxr_pulse_compress", [&] {
     return mxr::pc_common("pulse_compress", y, x, w, n, (flags & MXR_PC_WINDOW) != 0,
                           (flags & MXR_PC_NORMALIZE) != 0, (flags & MXR_PC_WRITEBACK) != 0, 1,
-                          stream);
+                          0, 0, stream);
   });
 }
 
@@ -1309,7 +1456,7 @@ mxr_status mxr_fft_conv(const mxr_tensor *out, const mxr_tensor *x, const mxr_te
                         int conj_w, hipStream_t stream) {
   return mxr::guarded("mxr_fft_conv", [&] {
     if (w && w->rank > 1) return mxr::fft_conv_rows(out, x, w, n, conj_w ? 1 : 0, stream);
-    return mxr::pc_common("fft_conv", out, x, w, n, 0, 0, 0, conj_w ? 1 : 0, stream);
+    return mxr::pc_common("fft_conv", out, x, w, n, 0, 0, 0, conj_w ? 1 : 0, 0, 0, stream);
   });
 }
 

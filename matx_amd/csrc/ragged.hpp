@@ -43,6 +43,7 @@ struct WfArgs {
   int64_t wstride;
   int64_t L;
   int window, normalize, writeback, conj;
+  int conj_in;  // the waveform is conjugated on load
   float2 *wc;
   const float2 *tw;
   float out_scale;  // applied to the stored spectrum (the block kernels' 1/M)

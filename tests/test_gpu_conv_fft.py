@@ -159,3 +159,54 @@ def test_fft_axes_direct(mx, n, cols):
     y = dev(x := sig(rng, (3, n, cols), True))
     mx.fft(y, n, 1, out=y)
     assert rel(host(y), np.fft.fft(x.astype(complex), axis=1)) < RTOL
+
+
+@pytest.mark.parametrize("mode", ["full", "same", "valid"])
+@pytest.mark.parametrize("L", [2, 17, 210, 1300, 4001])
+def test_conv1d_long_rows_from_first_lag(mx, mode, L):
+    """Long rows start at the mode's first lag: outputs that reach before the
+    row, convolution and correlation, each block size, a filter that is part
+    of the signal, against numpy in FP64."""
+    rng = np.random.default_rng(L)
+    N = 20011
+    x, f = sig(rng, (2, N), True), sig(rng, (L,), True)
+    xd = dev(x)
+    X = np.fft.fft(x.astype(complex), 32768)
+    s0, num = {"full": (0, N + L - 1), "same": ((L - 1) // 2, N), "valid": (L - 1, N - L + 1)}[mode]
+    for corr in (False, True):
+        h = np.conj(f[::-1]) if corr else f
+        ref = np.fft.ifft(X * np.fft.fft(h.astype(complex), 32768))[:, s0:s0 + num]
+        got = (mx.corr if corr else mx.conv1d)(xd, dev(f), mode, method="fft")
+        assert rel(host(got), ref) < RTOL
+    part = xd[1, 5:5 + L]
+    ref = np.fft.ifft(X * np.fft.fft(x[1, 5:5 + L].astype(complex), 32768))[:, s0:s0 + num]
+    assert rel(host(mx.conv1d(xd, part, mode, method="fft")), ref) < RTOL
+
+
+@pytest.mark.parametrize("n,L", [(1024, 1), (1024, 100), (1024, 1024), (2048, 300), (16384, 100), (16384, 300)])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 7])
+@pytest.mark.parametrize("conj", [True, False])
+def test_fft_conv_waveform_beside_blocks(mx, n, L, rows, conj):
+    """Small calls whose workgroups transform the waveform beside one or three
+    blocks: rows that do not fill a workgroup, wrapping blocks, both forms."""
+    rng = np.random.default_rng(n + L + rows)
+    S = n - n // 5
+    x, w = sig(rng, (rows, S), True), sig(rng, (L,), True)
+    W = np.fft.fft(w.astype(complex), n)
+    ref = np.fft.ifft(np.fft.fft(x.astype(complex), n) * (np.conj(W) if conj else W))
+    assert rel(host(mx.fft_conv(dev(x), dev(w), n, conj=conj)), ref) < RTOL
+
+
+@pytest.mark.parametrize("S,L,n", [(9000, 1000, 16384), (20000, 900, 32768), (30000, 3000, 32768), (1500, 200, 2048)])
+def test_pulse_compress_in_place_rows(mx, S, L, n):
+    """In place: a row's blocks one after another in one workgroup, bit for bit
+    (same block size) or closely (another one) the out-of-place result."""
+    rng = np.random.default_rng(S)
+    x = dev(sig(rng, (3, n), True))
+    w = dev(sig(rng, (L,), True))
+    y = mx.pulse_compress(x[:, :S], w, n=n)
+    buf = x.clone()
+    out = buf[:, :S - L + 1]
+    mx.pulse_compress(buf[:, :S], w, n=n, out=out)
+    assert rel(host(out), host(y)) < 1e-6
+    assert np.array_equal(host(buf[:, S:]), host(x[:, S:]))
