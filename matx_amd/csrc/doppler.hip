@@ -172,7 +172,7 @@ __global__ __launch_bounds__(DopBatchCfg<ND>::NT) void doppler_batch_kernel(cons
     doppler_tile<ND, TR, DopBatchCfg<ND>::NT>(jb.a, (int)c, (int)(local - c * (uint32_t)jb.tiles) * TR, lds, win);
   };
   if constexpr (!PERSIST) {
-    item(blockIdx.x);
+    item(xcd_remap(blockIdx.x, items));
     return;
   }
   for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {

@@ -792,7 +792,7 @@ void pc_batch_kernel(const PcJob *jobs, const int *item_job, int64_t items, cons
                      const float2 *twi) {
   __shared__ float2 lds[Layout<M, 1, false>::LDS_ELEMS];
   if constexpr (!PERSIST) {
-    const int64_t it = blockIdx.x;
+    const int64_t it = xcd_remap(blockIdx.x, items);  // a row's overlapping blocks on one XCD
     ols_block<M>(job_block(uniform_copy(&jobs[item_job_of(item_job, it)]), it), twf, twi, lds);
     return;
   }
@@ -813,7 +813,7 @@ __global__ __launch_bounds__(256) void pc_batch_multi_kernel(const PcJob *jobs, 
   __shared__ float2 lds[Layout<M, TB, false>::LDS_ELEMS];
   __shared__ OlsBlock obs[TB];
   if (threadIdx.x < TB) {
-    const int64_t it0 = (int64_t)blockIdx.x * TB;
+    const int64_t it0 = xcd_remap(blockIdx.x, gridDim.x) * TB;
     const int64_t it = it0 + threadIdx.x < items ? it0 + threadIdx.x : it0;
     OlsBlock ob = job_block(jobs[item_job_lane(item_job, it)], it);
     if (it0 + threadIdx.x >= items) {  // past the last item: idle transform
@@ -832,7 +832,7 @@ void pc4096_batch_kernel(const PcJob *jobs, const int *item_job, int64_t items, 
                          const float4 *base2) {
   __shared__ float2 lds[Layout<4096, 1, false>::LDS_ELEMS];
   if constexpr (!PERSIST) {
-    const int64_t it = blockIdx.x;
+    const int64_t it = xcd_remap(blockIdx.x, items);  // a row's overlapping blocks on one XCD
     ols_block4096(job_block(uniform_copy(&jobs[item_job_of(item_job, it)]), it), base1, base2, lds);
     return;
   }
@@ -849,7 +849,7 @@ void pc8192_batch_kernel(const PcJob *jobs, const int *item_job, int64_t items, 
                          const float4 *bB, const float4 *bC) {
   __shared__ float2 lds[Layout<8192, 1, false>::LDS_ELEMS];
   if constexpr (!PERSIST) {
-    const int64_t it = blockIdx.x;
+    const int64_t it = xcd_remap(blockIdx.x, items);  // a row's overlapping blocks on one XCD
     ols_block8192(job_block(uniform_copy(&jobs[item_job_of(item_job, it)]), it), bA, bB, bC, lds);
     return;
   }
