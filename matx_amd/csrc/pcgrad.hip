@@ -122,33 +122,28 @@ __global__ __launch_bounds__(WgT<M>::NT) void pc_wgrad_kernel(WgArgs a) {
 }
 
 // M = 8192: the transforms of the 8192-point pulse-compression kernel
-// (radix 2 x 16 x 16 x 16, the radix-2 pass folded into the load).  Threads
-// 0-511 transform the block of x and threads 512-1023 that of gy, side by
-// side in an LDS buffer each (bins j + 512q of thread j); then each half
-// multiplies and accumulates one half of the bins, the other transform's
-// through LDS.
-// One 16-wave workgroup per CU at 128 VGPRs; with both transforms in the same
-// 512 threads one after the other, the two spectra and the running product
-// took 242 VGPRs, eight waves per CU: 2610 us against 2207 on 16 x 512 x 32768.
-// The next block's samples are loaded before the last pass (nothing is stored
-// in the walk, so no wait for a load waits for a store).
+// (radix 2 x 16 x 16 x 16, 512 threads, the radix-2 pass swapped between lanes
+// at the load).  A workgroup transforms the block of x, keeps its 16 bins a
+// thread, transforms the block of gy and accumulates the product: 128 VGPRs
+// hold the x bins, the running product and one pass, so two workgroups share
+// a CU, each in another phase.  16 x 512 x 32768: 2610 us at one workgroup per
+// CU (242 VGPRs), 2207 with the two transforms side by side in one 1024-thread
+// workgroup (every wave waits at the same barriers), 2003 like this.
 struct Wg8192Args {
   WgArgs a;
   const float4 *bA, *bB, *bC;  // factors of passes Ls = 2, 32, 512
 };
 
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void wgrad8192_kernel(Wg8192Args p) {
   using LY = Layout<8192, 1, false>;
-  __shared__ float2 lds2[2][LY::LDS_ELEMS];
+  __shared__ float2 lds[LY::LDS_ELEMS];
   const WgArgs &a = p.a;
-  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 9);
-  const int j = threadIdx.x & 511;
-  float2 *const lds = lds2[half];
+  const int j = threadIdx.x;
   const int rbase = lds_pad(j);
-  float2 acc[8], v[16];
+  float2 acc[16], X[16], v[16];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) acc[q] = make_float2(0.f, 0.f);
+  for (int q = 0; q < 16; ++q) acc[q] = make_float2(0.f, 0.f);
   auto xchg = [&](int ls_out) {
     const int k = j & (ls_out - 1), wbase = lds_pad((j - k) * 16 + k);
 #pragma unroll
@@ -159,8 +154,8 @@ void wgrad8192_kernel(Wg8192Args p) {
     wg_barrier();
   };
   // samples i0 + 256 m of item it's block of x (wrapping at n, zero from seff
-  // on) or of gy (zero from the block's last kept lag on)
-  auto fetch = [&](int64_t it, float2 (&u)[16]) {
+  // on) or, with half, of gy (zero from the block's last kept lag on)
+  auto fetch = [&](int64_t it, bool half, float2 (&u)[16]) {
     const uint32_t row = (uint32_t)it / (uint32_t)a.nblk;
     const int lo = (int)((uint32_t)it - row * (uint32_t)a.nblk) * a.V;
     int64_t ox, oy;
@@ -184,43 +179,34 @@ void wgrad8192_kernel(Wg8192Args p) {
       }
     }
   };
-  // the grid has at most one workgroup per item
-  int64_t it = blockIdx.x;
-  fetch(it, v);
-  for (;;) {
-    pair_dft2(v, (j & 1) != 0);
-    TwRow<16> tw = load_tw<16>(opaque(p.bA), 2, j & 1);
-    dft_tw<false>(v, tw);  // Ls = 2
-    tw = load_tw<16>(opaque(p.bB), 32, j & 31);
-    xchg(2);
-    dft_tw<false>(v, tw);  // Ls = 32
-    tw = load_tw<16>(opaque(p.bC), 512, j);
-    xchg(32);
-    it += gridDim.x;
-    float2 nx[16];
-    const bool more = it < a.items;
-    if (more) fetch(it, nx);
-    dft_tw<false>(v, tw);  // Ls = 512: bins j + 512q
-    // the x half takes bins q < 8, the gy half the others: each leaves the
-    // other's bins in its own buffer
+  for (int64_t it = blockIdx.x; it < a.items; it += gridDim.x) {
+#pragma unroll 1
+    for (int h = 0; h < 2; ++h) {  // x, then gy
+      fetch(it, h != 0, v);
+      pair_dft2(v, (j & 1) != 0);
+      TwRow<16> tw = load_tw<16>(opaque(p.bA), 2, j & 1);
+      dft_tw<false>(v, tw);
+      tw = load_tw<16>(opaque(p.bB), 32, j & 31);
+      xchg(2);
+      dft_tw<false>(v, tw);
+      tw = load_tw<16>(opaque(p.bC), 512, j);
+      xchg(32);
+      dft_tw<false>(v, tw);
+      if (h == 0) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) lds[j + 512 * q] = half ? v[q] : v[q + 8];
-    wg_barrier();
+        for (int q = 0; q < 16; ++q) X[q] = v[q];
+      } else {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const float2 o = lds2[half ^ 1][j + 512 * q];
-      const float2 x = half ? o : v[q], g = half ? v[q + 8] : o;
-      acc[q].x += x.x * g.x + x.y * g.y;  // X conj(G)
-      acc[q].y += x.y * g.x - x.x * g.y;
+        for (int q = 0; q < 16; ++q) {
+          acc[q].x += X[q].x * v[q].x + X[q].y * v[q].y;
+          acc[q].y += X[q].y * v[q].x - X[q].x * v[q].y;
+        }
+      }
     }
-    if (!more) break;
-    wg_barrier();  // the buffers are free again
-#pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = nx[q];
   }
-  float2 *pp = a.partial + (int64_t)blockIdx.x * 8192 + half * 4096;
+  float2 *pp = a.partial + (int64_t)blockIdx.x * 8192;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) pp[j + 512 * q] = acc[q];
+  for (int q = 0; q < 16; ++q) pp[j + 512 * q] = acc[q];
 }
 
 // spec[k] = sum over workgroups g of partial[g][k], in order, in double.
@@ -315,7 +301,7 @@ static mxr_status wgrad_run(const WgradJob &j, hipStream_t s) {
     // the dedicated kernel's 32-bit block numbers and byte offsets
     const bool w8 = M == 8192 && j.n <= PC_BUF_MAX_N && items < (1ll << 31);
     if (w8)
-      oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad8192_kernel, 1024, 0);
+      oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad8192_kernel, 512, 0);
     else
       oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pc_wgrad_kernel<M>, T::NT, 0);
     if (oe != hipSuccess || per_cu < 1) per_cu = 1;
@@ -343,7 +329,7 @@ static mxr_status wgrad_run(const WgradJob &j, hipStream_t s) {
       MXR_REQUIRE(p.bA && p.bB && p.bC, MXR_OUT_OF_MEMORY,
                   "pc waveform gradient: twiddle table allocation failed");
       ProfScope ps("wgrad8192_kernel", s);
-      wgrad8192_kernel<<<dim3((unsigned)grid), dim3(1024), 0, s>>>(p);
+      wgrad8192_kernel<<<dim3((unsigned)grid), dim3(512), 0, s>>>(p);
     } else {
       ProfScope ps("pc_wgrad_kernel", s);
       pc_wgrad_kernel<M><<<dim3((unsigned)grid), dim3(T::NT), 0, s>>>(a);
