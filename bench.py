@@ -448,8 +448,8 @@ def bench_conv(args):
                                        "wfspec_kernel", "fconv_kernel", "fconv_spec_kernel"])
     roof = kernel_roofline(kern, {"pc4096_kernel": B_ols, "pc8192_kernel": B_ols,
                                   "pc_ols_kernel": B_ols})
-    kfft = profiled_kernels(ftf, 10, ["czt_kernel"])
-    roof_fft = kernel_roofline(kfft, {"czt_kernel": B_fft})
+    kfft = profiled_kernels(ftf, 10, ["fft_mixed_kernel"])
+    roof_fft = kernel_roofline(kfft, {"fft_mixed_kernel": B_fft})
     sys.path.insert(0, ROOT)
     from oracle import oracle as orc
     orc.build()

@@ -9,6 +9,7 @@
 // innermost batch dim has unit stride (an FFT along a strided axis, e.g. the
 // pulse axis of a permuted view) the gather/scatter walk that dim fastest so
 // HBM accesses stay coalesced.
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <map>
@@ -275,8 +276,354 @@ static mxr_status dispatch_generic(int64_t n, const FftArgs &a, bool inv, hipStr
   return MXR_NOT_SUPPORTED;
 }
 
+// ------------------------------------- sizes without large primes: mixed radix
+// n = R0 R1 ... with every factor in MIX_RADIX: Stockham passes of those
+// radices over whole rows in LDS, one butterfly a thread and pass, so one
+// buffer serves a pass's loads and its stores.  The first pass loads from
+// memory, the last one stores there.  Pass p (Ls = product of the radices
+// before it, NB = n/R butterflies): inputs b + j NB, times w[j-1][b mod Ls],
+// outputs (b / Ls) Ls R + (b mod Ls) + q Ls.  The first pass's outputs are R0
+// apart from lane to lane: one unused element follows every R0 when R0 is even
+// (an odd distance in 8-byte elements meets every bank).
+// Every size and factorisation shares one kernel: the radices are uniform
+// branches, the divisions products with reciprocals.
+// Bound by HBM and the latency of the passes: 8192 transforms of 1000 points
+// (10 10 10) 32 us, 26 the copy rate's; 56 as a chirp-z transform, which does
+// two 2048-point transforms for each.  The same data as rows of other sizes,
+// chirp-z -> mixed, us: 24 points 73 -> 32, 100 48 -> 28, 360 62 -> 35, 1500
+// 68 -> 33, 2187 (9 9 9 3) 109 -> 49, 4500 134 -> 57, 7200 93 -> 53; along
+// a strided axis 100 54 -> 31, 1000 76 -> 41, 1500 191 -> 57, 4500 278 -> 214;
+// 7 rows of 1000 8.1 -> 6.5, of 7200 18 -> 10.  Smaller errors, too (1000
+// points: 1.2e-7 from 1.7e-7).  So every size with such factors that a
+// workgroup holds takes it, from MIX_MIN_N points (below, one pass or two
+// short ones); the others stay chirp-z.
+constexpr int MIX_RADIX[] = {16, 15, 12, 10, 9, 8, 6, 5, 4, 3};
+constexpr int MIX_MAX_PASSES = 8;
+constexpr int MIX_MAX_TB = 64;
+constexpr int MIX_MIN_N = 24;
+
+struct MixPass {
+  int R, Ls, NB;
+  uint32_t mNB, mLs;  // ceil(2^32 / NB), ceil(2^32 / Ls)
+  int tw;             // offset of the table rows [R - 1][Ls]
+};
+struct MixArgs {
+  FftArgs f;
+  int n, np, TB, lgTB;
+  int pad, row;  // 1 when R0 is even; elements of a row in LDS
+  const float2 *tw;
+  MixPass p[MIX_MAX_PASSES];
+};
+
+// cos and sin in double, |x| <= 2 pi, for the constants of composite radices
+constexpr double mix_series(double x, int first) {
+  double term = first ? x : 1.0, sum = 0.0;
+  for (int i = first; i < 48; i += 2) {
+    sum += term;
+    term = -term * x * x / ((i + 1) * (i + 2));
+  }
+  return sum;
+}
+constexpr double mix_angle(int k, int R) {  // -2 pi k / R in (-pi, pi]
+  const double x = -6.283185307179586476925286766559 * (k % R) / R;
+  return x <= -3.14159265358979323846264338327950288 ? x + 6.283185307179586476925286766559 : x;
+}
+
+template <bool INV>
+__device__ __forceinline__ void dft3(float2 &a, float2 &b, float2 &c) {
+  constexpr float S = INV ? 0.866025403784438646763723f : -0.866025403784438646763723f;
+  const float2 s = cadd(b, c), d = csub(b, c);
+  const float2 m = make_float2(fmaf(-0.5f, s.x, a.x), fmaf(-0.5f, s.y, a.y));
+  a = cadd(a, s);
+  b = make_float2(fmaf(-S, d.y, m.x), fmaf(S, d.x, m.y));
+  c = make_float2(fmaf(S, d.y, m.x), fmaf(-S, d.x, m.y));
+}
+
+template <bool INV>
+__device__ __forceinline__ void dft5(float2 (&a)[5]) {
+  constexpr float C1 = 0.309016994374947424102293f, C2 = -0.809016994374947424102293f;
+  constexpr float S1 = (INV ? 1.f : -1.f) * 0.951056516295153572116439f;
+  constexpr float S2 = (INV ? 1.f : -1.f) * 0.587785252292473129168706f;
+  const float2 p = cadd(a[1], a[4]), q = cadd(a[2], a[3]), d = csub(a[1], a[4]), e = csub(a[2], a[3]);
+  const float2 m1 = make_float2(fmaf(C2, q.x, fmaf(C1, p.x, a[0].x)), fmaf(C2, q.y, fmaf(C1, p.y, a[0].y)));
+  const float2 m2 = make_float2(fmaf(C1, q.x, fmaf(C2, p.x, a[0].x)), fmaf(C1, q.y, fmaf(C2, p.y, a[0].y)));
+  const float2 n1 = make_float2(fmaf(S2, e.x, S1 * d.x), fmaf(S2, e.y, S1 * d.y));
+  const float2 n2 = make_float2(fmaf(-S1, e.x, S2 * d.x), fmaf(-S1, e.y, S2 * d.y));
+  a[0] = cadd(a[0], cadd(p, q));
+  a[1] = make_float2(m1.x - n1.y, m1.y + n1.x);
+  a[4] = make_float2(m1.x + n1.y, m1.y - n1.x);
+  a[2] = make_float2(m2.x - n2.y, m2.y + n2.x);
+  a[3] = make_float2(m2.x + n2.y, m2.y - n2.x);
+}
+
+// y[k][i] *= exp(-+2 pi i k i / R), the constants by the compiler
+template <int R, int A, int B, bool INV, int... E>
+__device__ __forceinline__ void mix_twiddle(float2 (&y)[A][B], std::integer_sequence<int, E...>) {
+  (
+      [&] {
+        constexpr int k = E / B, i = E % B;
+        if constexpr (k > 0 && i > 0) {
+          constexpr double x = mix_angle(k * i, R);
+          constexpr float c = (float)mix_series(x, 0), s = (float)mix_series(INV ? -x : x, 1);
+          y[k][i] = cmul(y[k][i], make_float2(c, s));
+        }
+      }(),
+      ...);
+}
+
+template <int R, bool INV>
+__device__ __forceinline__ void mix_dft(float2 (&a)[R]) {
+  if constexpr (R == 3) {
+    dft3<INV>(a[0], a[1], a[2]);
+  } else if constexpr (R == 5) {
+    dft5<INV>(a);
+  } else if constexpr ((R & (R - 1)) == 0) {
+    dft<R, INV>(a);
+  } else {  // R = A B: B transforms of A points, twiddles, A transforms of B
+    constexpr int A = R % 5 == 0 ? 5 : 3, B = R / A;
+    float2 y[A][B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      float2 c[A];
+#pragma unroll
+      for (int j = 0; j < A; ++j) c[j] = a[j * B + i];
+      mix_dft<A, INV>(c);
+#pragma unroll
+      for (int k = 0; k < A; ++k) y[k][i] = c[k];
+    }
+    mix_twiddle<R, A, B, INV>(y, std::make_integer_sequence<int, R>{});
+#pragma unroll
+    for (int k = 0; k < A; ++k) {
+      mix_dft<B, INV>(y[k]);
+#pragma unroll
+      for (int q = 0; q < B; ++q) a[k + A * q] = y[k][q];
+    }
+  }
+}
+
+template <int R, bool INV, bool COL>
+__device__ __forceinline__ void mix_pass(const MixArgs &z, int ip, float2 *lds, const int64_t *base_in,
+                                         const int64_t *base_out, int64_t t0) {
+  const MixPass &p = z.p[ip];
+  const FftArgs &a = z.f;
+  const bool first = ip == 0, last = ip == z.np - 1;
+  const int idx = threadIdx.x;
+  const bool active = idx < z.TB * p.NB;
+  int t, b;
+  if constexpr (COL) {
+    t = idx & (z.TB - 1);
+    b = idx >> z.lgTB;
+  } else {
+    t = (int)__umulhi((uint32_t)idx, p.mNB);
+    b = idx - t * p.NB;
+  }
+  const int bq = first ? b : (int)__umulhi((uint32_t)b, p.mLs), k = b - bq * p.Ls;
+  const int es = COL ? z.TB : 1;  // distance of a row's elements
+  float2 *row = lds + (COL ? t : t * z.row);
+  float2 v[R];
+  if (active) {
+    if (first) {
+      if (a.in_len > 0) {
+        with_kind(a.kind, [&](auto kt) {
+#pragma unroll
+          for (int j = 0; j < R; ++j)
+            v[j] = fft_load<decltype(kt)::value>(a, base_in[t], b + j * p.NB, t0 + t < a.nbatch);
+        });
+      } else {
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[j] = make_float2(0.f, 0.f);
+      }
+    } else {
+      const int padded = ip == 1 ? z.pad : 0;  // the first pass's outputs
+      const int step = (p.NB + (padded ? (int)__umulhi((uint32_t)p.NB, p.mLs) : 0)) * es;
+      const float2 *src = row + (b + padded * bq) * es;
+#pragma unroll
+      for (int j = 0; j < R; ++j) v[j] = src[j * step];
+      const float2 *w = z.tw + p.tw + k;
+#pragma unroll
+      for (int j = 1; j < R; ++j) {
+        const float2 c = w[(j - 1) * p.Ls];
+        v[j] = INV ? cmulc(v[j], c) : cmul(v[j], c);
+      }
+    }
+    mix_dft<R, INV>(v);
+  }
+  if (last) {
+    if (active && t0 + t < a.nbatch) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int o = b + q * p.Ls;  // the last pass: Ls = NB, k = b
+        if (o < (int)a.out_len) fft_scatter(a, base_out[t], o, cscale(v[q], a.scale));
+      }
+    }
+    return;
+  }
+  if (!first) wg_barrier();  // the loads of this pass are done
+  if (active) {
+    float2 *dst = row + (first ? b * (R + z.pad) : bq * p.Ls * R + k) * es;
+    const int step = p.Ls * es;
+#pragma unroll
+    for (int q = 0; q < R; ++q) dst[q * step] = v[q];
+  }
+  wg_barrier();
+}
+
+template <bool INV, bool COL>
+__global__ __launch_bounds__(1024) void fft_mixed_kernel(MixArgs z) {
+  extern __shared__ float2 mix_lds[];
+  __shared__ int64_t base_in[MIX_MAX_TB], base_out[MIX_MAX_TB];
+  const FftArgs &a = z.f;
+  const int64_t t0 = (COL ? xcd_remap(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x) * z.TB;
+  for (int t = threadIdx.x; t < z.TB; t += blockDim.x) {
+    int64_t oi = 0, oo = 0;
+    if (t0 + t < a.nbatch) {
+      if (a.small_batch) batch_offsets32(a.bi, (uint32_t)(t0 + t), &oi, &oo);
+      else batch_offsets(a.bi, t0 + t, &oi, &oo);
+    }
+    base_in[t] = oi;
+    base_out[t] = oo;
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int ip = 0; ip < z.np; ++ip) {
+    switch (z.p[ip].R) {
+      case 16: mix_pass<16, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      case 15: mix_pass<15, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      case 12: mix_pass<12, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      case 10: mix_pass<10, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      case 9: mix_pass<9, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      case 8: mix_pass<8, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      case 6: mix_pass<6, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      case 5: mix_pass<5, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      case 4: mix_pass<4, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+      default: mix_pass<3, INV, COL>(z, ip, mix_lds, base_in, base_out, t0); break;
+    }
+  }
+}
+
+namespace {
+struct MixSeq {
+  int n = 0;
+  int r[MIX_MAX_PASSES] = {};
+};
+// Radices of an n-point transform, largest first: the fewest passes, among
+// those the one whose smallest radix (most threads) is largest.
+void mix_search(int n, int from, MixSeq &cur, MixSeq &best) {
+  if (n == 1) {
+    if (best.n == 0 || cur.n < best.n || (cur.n == best.n && cur.r[cur.n - 1] > best.r[best.n - 1])) best = cur;
+    return;
+  }
+  if (cur.n == MIX_MAX_PASSES || (best.n && cur.n >= best.n)) return;
+  for (int i = from; i < (int)(sizeof(MIX_RADIX) / sizeof(int)); ++i) {
+    if (n % MIX_RADIX[i]) continue;
+    cur.r[cur.n++] = MIX_RADIX[i];
+    mix_search(n / MIX_RADIX[i], i, cur, best);
+    --cur.n;
+  }
+}
+
+std::mutex g_mix_mu;
+std::map<std::pair<int, int>, float2 *> g_mix;  // (device, n) -> the passes' tables
+
+void clear_mix() {
+  std::lock_guard<std::mutex> g(g_mix_mu);
+  for (auto &kv : g_mix) {
+    int cur = 0;
+    (void)hipGetDevice(&cur);
+    (void)hipSetDevice(kv.first.first);
+    (void)hipFree(kv.second);
+    (void)hipSetDevice(cur);
+  }
+  g_mix.clear();
+}
+CacheClearRegistrar g_reg_mix(clear_mix);
+}  // namespace
+
+// Tables of an n-point transform, [R - 1][Ls] of exp(-2 pi i j k / (R Ls)) for
+// every pass but the first, built in double and rounded once.
+static const float2 *mix_tables(int n, const MixArgs &z) {
+  const auto key = std::make_pair(device_id(), n);
+  std::lock_guard<std::mutex> g(g_mix_mu);
+  auto it = g_mix.find(key);
+  if (it != g_mix.end()) return it->second;
+  const double two_pi = 6.283185307179586476925286766559;
+  std::vector<float2> host;
+  for (int p = 1; p < z.np; ++p)
+    for (int j = 1; j < z.p[p].R; ++j)
+      for (int k = 0; k < z.p[p].Ls; ++k) {
+        const double ang = -two_pi * (double)(j * k) / ((double)z.p[p].R * z.p[p].Ls);
+        host.push_back(make_float2((float)std::cos(ang), (float)std::sin(ang)));
+      }
+  float2 *d = nullptr;
+  if (hipMalloc(&d, sizeof(float2) * host.size()) != hipSuccess) return nullptr;
+  if (hipMemcpy(d, host.data(), sizeof(float2) * host.size(), hipMemcpyHostToDevice) != hipSuccess) {
+    (void)hipFree(d);
+    return nullptr;
+  }
+  g_mix[key] = d;
+  return d;
+}
+
+// Fills the passes of an n-point transform; false for sizes left to Bluestein:
+// a factor outside MIX_RADIX, one pass only, or more than a workgroup holds.
+static bool mix_plan(int64_t n, MixArgs &z) {
+  if (n < MIX_MIN_N || n > 8192) return false;
+  MixSeq cur, best;
+  mix_search((int)n, 0, cur, best);
+  if (best.n < 2) return false;
+  const int Rmin = best.r[best.n - 1];
+  z.n = (int)n;
+  z.np = best.n;
+  z.pad = best.r[0] % 2 == 0;
+  z.row = (int)n + (z.pad ? (int)n / best.r[0] : 0);
+  if (n / Rmin > 1024 || z.row > 8000) return false;
+  int Ls = 1, off = 0;
+  for (int p = 0; p < best.n; ++p) {
+    const int R = best.r[p];
+    z.p[p] = {R, Ls, (int)n / R, (uint32_t)(((1ull << 32) + n / R - 1) / (n / R)),
+              p ? (uint32_t)(((1ull << 32) + Ls - 1) / Ls) : 0u, off};
+    if (p) off += (R - 1) * Ls;
+    Ls *= R;
+  }
+  return true;
+}
+
+static mxr_status launch_mixed(MixArgs z, const FftArgs &f, bool inv, hipStream_t s) {
+  z.f = f;
+  z.f.small_batch = f.nbatch < (1ll << 31);
+  z.tw = mix_tables(z.n, z);
+  MXR_REQUIRE(z.tw != nullptr, MXR_OUT_OF_MEMORY, "fft: table allocation failed for size %d", z.n);
+  const int Rmin = z.p[z.np - 1].R, nb = z.n / Rmin;
+  const bool col = f.batch_fast && z.row <= 4096 && 2 * nb <= 1024;
+  int TB = 1;
+  z.lgTB = 0;
+  if (col) {
+    while (TB < 32 && 2 * TB * nb <= 1024 && 2 * TB * z.row <= 8000) {
+      TB *= 2;
+      ++z.lgTB;
+    }
+  } else {
+    TB = std::max(1, std::min({512 / nb, 5632 / z.row, MIX_MAX_TB}));
+    // few transforms: rather more workgroups
+    TB = (int)std::min<int64_t>(TB, std::max<int64_t>(1, f.nbatch / 512));
+  }
+  z.TB = TB;
+  const int64_t grid = (f.nbatch + TB - 1) / TB;
+  MXR_REQUIRE(grid <= 0x7fffffff, MXR_INVALID_SIZE, "fft: batch too large");
+  const int nt = (TB * nb + 63) / 64 * 64;
+  const size_t shm = sizeof(float2) * (size_t)TB * z.row;
+  ProfScope ps("fft_mixed_kernel", s);
+  const dim3 g((unsigned)grid), b((unsigned)nt);
+  if (col && inv) fft_mixed_kernel<true, true><<<g, b, shm, s>>>(z);
+  else if (col) fft_mixed_kernel<false, true><<<g, b, shm, s>>>(z);
+  else if (inv) fft_mixed_kernel<true, false><<<g, b, shm, s>>>(z);
+  else fft_mixed_kernel<false, false><<<g, b, shm, s>>>(z);
+  MXR_HIP_TRY(hipGetLastError());
+  return MXR_SUCCESS;
+}
+
 // ------------------------------------------------- other sizes: Bluestein
-// An n-point DFT of any n as a circular convolution of power-of-two length
+// An n-point DFT of any other n as a circular convolution of power-of-two length
 // M >= 2n - 1 (Bluestein's chirp-z identity nk = (n^2 + k^2 - (k - n)^2)/2):
 //   X[k] = c[k] * sum_j (x[j] c[j]) h[k - j],  c[j] = exp(-i pi j^2 / n),
 //   h[m] = conj(c[|m|]),
@@ -298,7 +645,7 @@ struct CztArgs {
 // reversed radix sequence) share registers, and the last inverse pass stores
 // c.y.  M >= 2n, so the upper half of the inputs is zero and the upper half of
 // the outputs is not wanted: the first and the last pass do half the loads,
-// stores and sums.  8192 transforms of 1000 points: 77 us
+// stores and sums.  8192 transforms of 1000 points (now mixed radix): 77 us
 // with everything staged in LDS, 52 direct.
 template <int M, bool INV, bool COL>
 __global__ __launch_bounds__((GenericCfg<M, COL>::NT)) void czt_kernel(CztArgs z) {
@@ -1029,6 +1376,8 @@ static mxr_status fft_impl(const char *fn, const mxr_tensor *out, const mxr_tens
     MXR_HIP_TRY(hipGetLastError());
     return MXR_SUCCESS;
   }
+  MixArgs z{};
+  if (!pow2 && mix_plan(n, z)) return launch_mixed(z, a, inv, stream);
   if (!pow2) return n <= CZT_MAX_N ? dispatch_czt(n, a, inv, stream) : dispatch_czt_big(n, a, inv, stream);
   if (n > 16384) return dispatch_big(n, a, inv, stream);
   a.tw = twiddles_device((int)n, false);

@@ -161,6 +161,17 @@ def test_fft_axes_direct(mx, n, cols):
     assert rel(host(y), np.fft.fft(x.astype(complex), axis=1)) < RTOL
 
 
+@pytest.mark.parametrize("n,cols", [(24, 33), (30, 300), (45, 15), (60, 1), (96, 33), (100, 70), (135, 15),
+                                    (225, 33), (360, 15), (1000, 33), (1000, 1200), (1152, 15), (1500, 33),
+                                    (2187, 3), (3000, 15), (3125, 3), (4500, 9), (5184, 2), (7200, 3)])
+def test_fft_mixed_radix(mx, n, cols):
+    """Sizes without large primes: every radix as a first, a middle and a last
+    pass, odd first radices and padded even ones, batches that do not fill a
+    workgroup and those that make it larger; the largest row a workgroup
+    holds."""
+    test_fft_axes_direct(mx, n, cols)
+
+
 @pytest.mark.parametrize("mode", ["full", "same", "valid"])
 @pytest.mark.parametrize("L", [2, 17, 210, 1300, 4001])
 def test_conv1d_long_rows_from_first_lag(mx, mode, L):
