@@ -67,7 +67,7 @@ def parse():
                          "loss forward + backward (grad steps/s); ragged: 256 uneven "
                          "pulse-compression + Doppler jobs, batched vs per-job launches; stage: "
                          "MatX's stage calls on the C++ front end; conv: conv1d by the FFT "
-                         "method on 16 x 1048576 c64 with 209 taps and 1000-point Bluestein "
+                         "method on 16 x 1048576 c64 with 209 taps and 1000-point "
                          "FFTs; ew: fused elementwise expressions at the radar cube's size")
     ap.add_argument("--streams", type=int, default=None,
                     help="pipelines run side by side as branches of the timed graph of the "
@@ -401,7 +401,7 @@ def bench_conv(args):
     """FFT-method conv1d at the size of MatX's CorrelationConvolutionLargeTest
     (test/00_transform/ConvCorr.cu:61-63: 8*122880 + 2*32768 samples, 209
     taps, FULL), batched over 16 rows of unit complex noise (sigma = 1), and
-    8192 Bluestein FFTs of 1000 points.  Timed as back-to-back calls with the
+    8192 FFTs of 1000 points.  Timed as back-to-back calls with the
     inputs resident; parity of row 0 (conv) and of 64 rows (FFT) against the
     FP64 oracle."""
     import numpy as np
@@ -439,13 +439,12 @@ def bench_conv(args):
     us_conv = timed(conv, k)
     us_fft = timed(ftf, k)
     # algorithmic bytes: read the signal, write the output (the filter is
-    # negligible); the overlap-save kernel writes outputs L-1 .. N+L-2, the
-    # fused head kernel the first L-1
+    # negligible); one launch of overlap-save blocks writes every output
     B_conv = 8 * rows * N + 8 * rows * (N + L - 1)
-    B_ols = 8 * rows * N + 8 * rows * N
+    B_ols = B_conv
     B_fft = 2 * 8 * rows2 * n2
     kern = profiled_kernels(conv, 10, ["pc4096_kernel", "pc8192_kernel", "pc_ols_kernel",
-                                       "wfspec_kernel", "fconv_kernel", "fconv_spec_kernel"])
+                                       "wfspec_kernel"])
     roof = kernel_roofline(kern, {"pc4096_kernel": B_ols, "pc8192_kernel": B_ols,
                                   "pc_ols_kernel": B_ols})
     kfft = profiled_kernels(ftf, 10, ["fft_mixed_kernel"])
@@ -473,7 +472,7 @@ def bench_conv(args):
                    "per_kernel_us": {kk: round(v[1], 2) for kk, v in kern.items()},
                    "rel_l2_vs_fp64_row0": rel_conv,
                    "bluestein_fft": {"workload": "fft of 8192 rows x 1000 points c64 "
-                                                 "(2048-point chirp-z convolution)",
+                                                 "(radices 10 10 10)",
                                      "us_per_call": round(us_fft, 2),
                                      "hbm_gbs": round(B_fft / (us_fft * 1e-6) / 1e9, 1),
                                      "roofline": roof_fft,
