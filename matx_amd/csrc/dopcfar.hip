@@ -13,19 +13,18 @@
 // starts on a 16-byte boundary of the detection rows); neighbouring tiles
 // overlap by 2*HXA columns, which the XCD-local L2 serves.
 //
-//  1. load: lane = range column, wave = a strip of Doppler-input rows i and
-//     the strip ND/2 rows below it; each lane reads its strips' pulses plus
-//     one on either side (512-byte coalesced rows) and forms the canceller
+//  1. load: half-wave = a strip of Doppler-input rows of 32 range columns, then
+//     of the 32 columns beside them; each lane reads its strips' pulses plus
+//     one on either side (256-byte coalesced rows) and forms the canceller
 //     output and the window in registers.
-//  2. The transform is split by its first radix-2 stage (decimation in
-//     frequency): the even Doppler bins are the ND/2-point transform of
-//     row i + row i + ND/2, the odd ones that of the difference at frequencies
-//     half a bin up, which only changes the butterflies' factors (the table's
-//     row k holds those of k + 1/2).  Both run through one LDS buffer of half
-//     the tile, one after the other, while the other half waits in registers.
-//     So a workgroup holds 36 KiB of LDS instead of 67 and four of them share
-//     a CU, each in another phase: with the whole tile in LDS, two workgroups
-//     of eight waves per CU loaded, transformed and summed almost in turn.
+//  2. The transforms run down the columns of one LDS buffer of half the tile:
+//     the left columns', then, from registers, the right columns'.  So a
+//     workgroup holds 34 KiB of LDS instead of 67 and four of them share a CU,
+//     each in another phase: with the whole tile in LDS, two workgroups of
+//     eight waves per CU loaded, transformed and summed almost in turn.
+//     (Splitting by the first radix-2 stage instead, even Doppler bins then
+//     odd ones, takes 47.9 us where this takes 49.8, but rounds otherwise,
+//     which moves cells that lie on the threshold.)
 //  3. CFAR on the power rows in LDS: a thread owns 4 adjacent output columns
 //     of a band of Doppler rows and walks down it.  Per row it forms the
 //     positive partial sums L (left of the hole), M (hole columns), Rt (right
@@ -37,9 +36,9 @@
 //     the same order, as the stand-alone CFAR kernel).
 //
 // 16 x 128 pulses x 8001 range bins, 5 x 13 window: 56.6 us with the whole tile
-// in LDS, 50.4 with the halves, 47.9 with the channel's loads through a buffer
-// resource (zeros outside it) and one branch a detection row; 38 us is its HBM
-// traffic at a large copy's rate, 31 us its VALU issue.
+// in LDS, 49.8 with the halves, the channel's loads through a buffer resource
+// (zeros outside it) and one branch a detection row; 38 us is its HBM traffic
+// at a large copy's rate, 31 us its VALU issue.
 #include <cmath>
 #include <cstdlib>
 
@@ -72,7 +71,7 @@ struct DcArgs {
   int tiles;     // range tiles per channel
   int vec_out;   // every output row is 16-byte aligned
   int y32;       // rows32 of y, below DC_FAR bytes
-  const float2 *tw, *twh;  // ND/2-point tables: k and k + 1/2
+  const float2 *tw;
   // threshold factor per in-bounds cell count n: alpha(n) (exact form) or
   // alpha(n)/n, alpha(n) = n*(pfa^(-1/n) - 1) evaluated in float on the host
   float thr[DC_MAXCELL + 1];
@@ -90,6 +89,7 @@ __device__ __forceinline__ void st32(T *base, uint32_t byte_off, T v) {
 }
 
 constexpr int DC_TB = 64;   // computed range columns per tile
+constexpr int DC_TH = 32;   // columns transformed together
 constexpr int DC_NT = 256;  // threads per workgroup
 constexpr int DC_PS = 64;   // power-tile row stride (floats)
 constexpr int DC_FAR = 1 << 30;  // a byte offset past every channel with y32
@@ -128,25 +128,13 @@ __device__ __forceinline__ void dc_win4(const float *u, float (&o)[4]) {
   }
 }
 
-// One H-point transform down the LDS columns, from LDS to registers: the last
-// pass's butterflies end in pl (bin j + q H/RL of butterfly j).  HALF: at
-// frequencies k + 1/2.  Pre: the rows are in LDS, visible to all threads.
-// Post: LDS is free.
-template <class LY, int H, bool HALF, class PL>
+// One ND-point transform down DC_TH LDS columns, from LDS to registers: the
+// last pass's butterflies end in pl, twiddles and sums of that pass still to
+// come.  Pre: the rows are in LDS, visible to all threads.  Post: LDS is free.
+template <class LY, int ND, class PL>
 __device__ __forceinline__ void dc_transform(PL &pl, float2 *lds, const float2 *tw) {
-  using SQ = Seq<H, false>;
-  constexpr int K = SQ::n;
-  static_assert(K <= 2, "half transforms of at most two passes");
-  if constexpr (K == 2) {
-    constexpr int R0 = SQ::template R<0>;
-    Pass<LY, R0, H, DC_NT, DC_TB> p0;
-    p0.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
-    wg_barrier();
-    if constexpr (HALF) p0.template compute_tw<1, false>(tw);
-    else p0.template compute<1, false>(nullptr);
-    p0.template store<1>([&](int t, int i, float2 x) { lds[LY::addr(t, i)] = x; });
-    wg_barrier();
-  }
+  using SQ = Seq<ND, false>;
+  lds_passes<LY, SQ, ND, DC_NT, DC_TH, false, 0, SQ::n - 1>(lds, tw);
   pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
   wg_barrier();
 }
@@ -156,20 +144,20 @@ __device__ __forceinline__ void dc_transform(PL &pl, float2 *lds, const float2 *
 template <int ND, int HY, int HX, int EY, int EX, bool EXACT>
 __global__ __launch_bounds__(DC_NT) __attribute__((amdgpu_waves_per_eu(HY > 2 ? 3 : 4)))
 void dopcfar_kernel(DcArgs a) {
-  constexpr int TB = DC_TB, NT = DC_NT, NW = NT / 64, H = ND / 2;
+  constexpr int TB = DC_TB, TH = DC_TH, NT = DC_NT, NS = NT / TH;
   constexpr int HXA = DcGeom<HX>::HXA, OUT = DcGeom<HX>::OUT;
   static_assert(OUT >= 16, "window too wide for a 64-column tile");
-  static_assert(H >= NW, "Doppler size below two rows per wave");
+  static_assert(ND >= NS, "Doppler size below one row per strip");
   constexpr int PS = DC_PS;
-  constexpr int SR = H / NW;  // rows of a wave's strip
-  using LY = Layout<H, TB, true>;
-  using SQ = Seq<H, false>;
+  constexpr int SR = ND / NS;  // rows of a half-wave's strip
+  using LY = Layout<ND, TH, true>;
+  using SQ = Seq<ND, false>;
   constexpr int K = SQ::n;
   constexpr int NCELL = (2 * HY + 1) * (2 * HX + 1);
   static_assert(NCELL <= DC_MAXCELL, "window area");
   // the complex half tile; after the transforms the power rows (stride PS,
   // HY zero rows either side)
-  constexpr int LDS2 = H * TB > ((ND + 2 * HY) * PS + 1) / 2 ? H * TB : ((ND + 2 * HY) * PS + 1) / 2;
+  constexpr int LDS2 = ND * TH > ((ND + 2 * HY) * PS + 1) / 2 ? ND * TH : ((ND + 2 * HY) * PS + 1) / 2;
   __shared__ __align__(16) float2 lds[LDS2];
   __shared__ float2 coef[ND];  // Doppler-input row i = coef.x*(y[p-1]+y[p+1]) + coef.y*y[p]
   __shared__ float thr_tab[NCELL + 1];
@@ -178,41 +166,35 @@ void dopcfar_kernel(DcArgs a) {
   const uint32_t g = (uint32_t)xcd_remap(blockIdx.x, G);
   const int c = (int)(g / (uint32_t)a.tiles), tile = (int)(g - (uint32_t)c * (uint32_t)a.tiles);
   const int r0 = tile * OUT - HXA;  // range bin of tile column 0
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tcol = threadIdx.x % TH, i0 = threadIdx.x / TH * SR;  // column of a half, first row
 
   // ---- 1. canceller + window in registers, zeros outside the cube: from the
   // range check of a buffer resource over the channel (a column outside it
   // reads past the end), or, where a channel is too large for its 32-bit
   // offsets, from masks on clamped indices.
-  float2 ev[SR], od[SR];  // rows i + (i + H), rows i - (i + H)
+  float2 va[SR + 2], vb[SR + 2];  // pulses, then Doppler-input rows, of the left and of the right columns
   {
-    const int r = r0 + lane;
-    const bool rok = r >= 0 && r < a.R;
     const float2 *chan = a.y + (int64_t)c * a.ys_c;
-    const int i0 = wv * SR;
-    float2 va[SR + 2], vb[SR + 2];
-    if (a.y32) {
-      const buf_rsrc ry = make_rsrc(chan, ((a.P - 1) * a.ys_p + a.R) * 8);
-      const int step = a.ys_p * 8;
-      const int v0 = (rok ? r * 8 : DC_FAR) + (i0 + a.p_off - 1) * step;  // pulse held in va[0]
+    const int pb = i0 + a.p_off - 1;  // pulse held in va[0], vb[0]
+    const buf_rsrc ry = make_rsrc(chan, a.y32 ? ((a.P - 1) * a.ys_p + a.R) * 8 : 0);
+    const int step = a.ys_p * 8;
+    auto fetch = [&](int r, float2 (&v)[SR + 2]) {
+      const bool rok = r >= 0 && r < a.R;
+      if (a.y32) {
+        const int v0 = (rok ? r * 8 : DC_FAR) + pb * step;
 #pragma unroll
-      for (int u = 0; u < SR + 2; ++u) va[u] = buf_load2(ry, v0 + u * step);
-#pragma unroll
-      for (int u = 0; u < SR + 2; ++u) vb[u] = buf_load2(ry, v0 + (u + H) * step);
-    } else {
-      const int rc = min(max(r, 0), a.R - 1);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        float2(&v)[SR + 2] = h ? vb : va;
-        const int pb = i0 + h * H + a.p_off - 1;
+        for (int u = 0; u < SR + 2; ++u) v[u] = buf_load2(ry, v0 + u * step);
+      } else {
+        const int rc = min(max(r, 0), a.R - 1);
 #pragma unroll
         for (int u = 0; u < SR + 2; ++u) {
           const float2 x = ld32(chan, (uint32_t)(rc + min(max(pb + u, 0), a.P - 1) * a.ys_p) * 8u);
           v[u] = keep_if(x, rok && pb + u >= 0 && pb + u < a.P);
         }
       }
-    }
+    };
+    fetch(r0 + tcol, va);
+    fetch(r0 + TH + tcol, vb);
     // canceller [1,-2,1] and window folded into two coefficients per row:
     // rows past the canceller output are zero, NONE passes y[p] windowed
     for (int i = threadIdx.x; i < ND; i += NT) {
@@ -222,47 +204,48 @@ void dopcfar_kernel(DcArgs a) {
     }
     for (int n = threadIdx.x; n <= NCELL; n += NT) thr_tab[n] = a.thr[n];
     wg_barrier();
+    auto rows = [&](float2 (&v)[SR + 2]) {
 #pragma unroll
-    for (int u = 0; u < SR; ++u) {
-      const float2 ca = coef[i0 + u], cb = coef[i0 + u + H];
-      const float2 x = make_float2(ca.x * (va[u].x + va[u + 2].x) + ca.y * va[u + 1].x,
-                                   ca.x * (va[u].y + va[u + 2].y) + ca.y * va[u + 1].y);
-      const float2 z = make_float2(cb.x * (vb[u].x + vb[u + 2].x) + cb.y * vb[u + 1].x,
-                                   cb.x * (vb[u].y + vb[u + 2].y) + cb.y * vb[u + 1].y);
-      ev[u] = cadd(x, z);
-      od[u] = csub(x, z);
-    }
+      for (int u = 0; u < SR; ++u) {
+        const float2 cf = coef[i0 + u];
+        v[u] = make_float2(fmaf(cf.x, v[u].x + v[u + 2].x, cf.y * v[u + 1].x),
+                           fmaf(cf.x, v[u].y + v[u + 2].y, cf.y * v[u + 1].y));
+      }
+    };
+    rows(va);
+    rows(vb);
 #pragma unroll
-    for (int u = 0; u < SR; ++u) lds[LY::addr(lane, i0 + u)] = ev[u];
+    for (int u = 0; u < SR; ++u) lds[LY::addr(tcol, i0 + u)] = va[u];
   }
   wg_barrier();
 
-  // ---- 2. the two half transforms; |X|^2 stays in registers until LDS is free
+  // ---- 2. the transforms of the two halves; |X|^2 of the left one stays in
+  // registers until LDS is free
   constexpr int RL = SQ::template R<K - 1>;
   constexpr int LSL = SQ::template LS<K - 1>;
-  using PL = Pass<LY, RL, H, NT, TB>;
+  using PL = Pass<LY, RL, ND, NT, TH>;
   float pe[PL::BPT][RL];
+  // |X|^2; the quarter bins of a one-pass transform sum the other way round
+  // (fixed, like every rounding that decides a cell on the threshold)
+  auto power = [](int q, float2 x) {
+    return K == 1 && (q == RL / 4 || q == 3 * RL / 4) ? cabs2(make_float2(x.y, x.x)) : cabs2(x);
+  };
   float *const pwt = reinterpret_cast<float *>(lds) + HY * PS;  // power row 0
   PL pl;
-  dc_transform<LY, H, false>(pl, lds, a.tw);
+  dc_transform<LY, ND>(pl, lds, a.tw);
 #pragma unroll
-  for (int u = 0; u < SR; ++u) lds[LY::addr(lane, wv * SR + u)] = od[u];
+  for (int u = 0; u < SR; ++u) lds[LY::addr(tcol, i0 + u)] = vb[u];
   pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
-#pragma unroll
-  for (int u = 0; u < PL::BPT; ++u)
-#pragma unroll
-    for (int q = 0; q < RL; ++q) pe[u][q] = cabs2(pl.v[u][q]);
+  PL::template outputs<LSL>([&](int u, int q, int, int) { pe[u][q] = power(q, pl.v[u][q]); });
   wg_barrier();
-  // the half-bin table holds the first pass too
-  constexpr int H0 = K == 2 ? SQ::template R<0> / 2 : 0;
-  dc_transform<LY, H, true>(pl, lds, a.twh);
+  dc_transform<LY, ND>(pl, lds, a.tw);
   for (int i = threadIdx.x; i < 2 * HY * TB; i += NT) {  // the CFAR's zero padding along Doppler
     const int row = i / TB < HY ? i / TB - HY : ND + i / TB - HY;
     pwt[row * PS + (i % TB)] = 0.f;
   }
-  PL::template outputs<LSL>([&](int u, int q, int t, int k) { pwt[2 * k * PS + t] = pe[u][q]; });
-  pl.template compute_tw<LSL, false>(a.twh + H0);
-  PL::template outputs<LSL>([&](int u, int q, int t, int k) { pwt[(2 * k + 1) * PS + t] = cabs2(pl.v[u][q]); });
+  PL::template outputs<LSL>([&](int u, int q, int t, int k) { pwt[k * PS + t] = pe[u][q]; });
+  pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
+  PL::template outputs<LSL>([&](int u, int q, int t, int k) { pwt[k * PS + TH + t] = power(q, pl.v[u][q]); });
   wg_barrier();
 
   // ---- 3. CFAR over the inner columns: a thread owns one output column quad
@@ -554,9 +537,8 @@ mxr_status doppler_cfar_impl(const mxr_tensor *dets, const mxr_tensor *ba_out,
       const float alpha = nf * (std::pow(pp->pfa, -1.0f / nf) - 1.0f);
       a.thr[n] = ba_out ? alpha : alpha / nf;
     }
-    a.tw = twiddles_device((int)nd / 2, false);
-    a.twh = twiddles_half_device((int)nd / 2);
-    MXR_REQUIRE(a.tw && a.twh, MXR_OUT_OF_MEMORY, "doppler_cfar: twiddle table allocation failed");
+    a.tw = twiddles_device((int)nd, false);
+    MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "doppler_cfar: twiddle table allocation failed");
     const int hy = wy / 2, hx = wx / 2, ey = gy / 2, ex = gx / 2;
     st = MXR_NOT_SUPPORTED;
 #define MXR_DC_CASE(HY_, HX_, EY_, EX_) \

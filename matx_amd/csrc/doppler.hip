@@ -105,12 +105,15 @@ __device__ __forceinline__ void doppler_tile(const DopArgs &a, int c, int r0, fl
   Pass<LY, RL, ND, NT, TR> pl;
   pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
   pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
+  // the one-pass transforms of 8 and 16 bins sum |X|^2 the other way round
+  // (fixed, like every rounding that decides a cell on the threshold)
+  auto power = [](float2 x) { return ND == 8 || ND == 16 ? cabs2(make_float2(x.y, x.x)) : cabs2(x); };
   if (a.out32) {  // columns past R are dropped by the range check
     constexpr int FAR = 0x7ffffff0;
     if (a.pw) {
       const buf_rsrc rp = make_rsrc(a.pw + (int64_t)c * a.ps_c, ((ND - 1) * (int)a.ps_k + a.R) * 4);
       pl.template store<LSL>([&](int t, int k, float2 v) {
-        buf_store1(rp, r0 + t < a.R ? (k * (int)a.ps_k + r0 + t) * 4 : FAR, cabs2(v));
+        buf_store1(rp, r0 + t < a.R ? (k * (int)a.ps_k + r0 + t) * 4 : FAR, power(v));
       });
     }
     if (a.rd) {
@@ -125,7 +128,7 @@ __device__ __forceinline__ void doppler_tile(const DopArgs &a, int c, int r0, fl
     const int r = r0 + t;
     if (r >= a.R) return;
     if (a.rd) a.rd[(int64_t)c * a.rs_c + (int64_t)k * a.rs_k + (int64_t)r * a.rs_r] = v;
-    if (a.pw) a.pw[(int64_t)c * a.ps_c + (int64_t)k * a.ps_k + (int64_t)r * a.ps_r] = cabs2(v);
+    if (a.pw) a.pw[(int64_t)c * a.ps_c + (int64_t)k * a.ps_k + (int64_t)r * a.ps_r] = power(v);
   });
 }
 
@@ -400,8 +403,8 @@ __global__ __launch_bounds__(DopAdjCfg<ND>::NT) void doppler_adj_kernel(DopGradA
   constexpr int TR = DopAdjCfg<ND>::TR;
   static_assert(TR <= 64 && 64 % TR == 0, "range tile must divide a wave");
   using LY = DopLayout<ND, TR>;
-  using SQ = Seq<ND, false>;
-  using SI = Seq<ND, true>;
+  using SQ = Seq<ND, false, true>;
+  using SI = Seq<ND, true, true>;
   constexpr int K = SQ::n;
   __shared__ float2 lds[LY::LDS_ELEMS];  // the windowed canceller rows, then D, then gu
   __shared__ __align__(16) float win[ND];
@@ -459,7 +462,7 @@ __global__ __launch_bounds__(DopAdjCfg<ND>::NT) void doppler_adj_kernel(DopGradA
     PL pl;
     pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
     wg_barrier();
-    pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
+    pl.template compute<LSL, false, true>(a.tw + SQ::template TWOFF<K - 1>);
     PL::template outputs<LSL>([&](int u, int q, int t, int k) {
       // a column past R holds no data: its gradient stays finite
       pl.v[u][q] = keep_if(cscale(pl.v[u][q], 2.0f * gpv[u][q]), r0 + t < a.R);
@@ -552,8 +555,8 @@ static mxr_status launch_doppler_adj(DopGradArgs a, const mxr_tensor *gtaps, hip
 }
 
 static mxr_status dispatch_doppler_adj(int64_t nd, DopGradArgs a, const mxr_tensor *gtaps, hipStream_t s) {
-  a.tw = twiddles_device((int)nd, false);
-  a.twi = twiddles_device((int)nd, true);
+  a.tw = factors_device((int)nd, false);
+  a.twi = factors_device((int)nd, true);
   MXR_REQUIRE(a.tw && a.twi, MXR_OUT_OF_MEMORY, "doppler adjoint: twiddle table allocation failed");
   a.y32 = rows32(a.P, a.R, a.ys_p, a.ys_r, 8);
   a.gp32 = rows32(nd, a.R, a.gs_k, a.gs_r, 4);

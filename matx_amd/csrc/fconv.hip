@@ -27,7 +27,7 @@ namespace mxr {
 
 mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, const mxr_tensor *w,
                      int64_t n, int window, int normalize, int writeback, int conj_w,
-                     int64_t shift, int reverse_conj, hipStream_t stream);
+                     int64_t shift, int reverse_conj, bool by_rate, hipStream_t stream);
 
 // TB rows per 256-thread workgroup below 4096 points, one row of M/16
 // threads from 4096 up (one radix-16 butterfly per thread per pass).
@@ -65,7 +65,7 @@ template <int M>
 __global__ __launch_bounds__(FcCfg<M>::NT) void fconv_spec_kernel(FcArgs a) {
   constexpr int NT = FcCfg<M>::NT;
   using LY = Layout<M, 1, false>;
-  using SQ = Seq<M, false>;
+  using SQ = Seq<M, false, true>;
   __shared__ float2 lds[LY::LDS_ELEMS];
   for (int i = threadIdx.x; i < M; i += NT) {
     float2 v = make_float2(0.f, 0.f);
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(FcCfg<M>::NT) void fconv_kernel(FcArgs a) {
   constexpr int TB = FcCfg<M>::TB;
   constexpr int NT = FcCfg<M>::NT;
   using LY = Layout<M, TB, false>;
-  using SQ = Seq<M, false>;
+  using SQ = Seq<M, false, true>;
   __shared__ float2 lds[LY::LDS_ELEMS];
   __shared__ int64_t base_in[TB], base_out[TB];
 
@@ -188,7 +188,7 @@ static mxr_status fconv_fused(const mxr_tensor *out, const mxr_tensor *in, int64
   a.olen = olen;
   a.spec = static_cast<float2 *>(stream_workspace("conv1d_fft_spec", sizeof(float2) * M, s));
   if (a.spec == nullptr) return workspace_failure("conv1d_fft");
-  a.tw = twiddles_device((int)M, false);
+  a.tw = factors_device((int)M, false);
   MXR_REQUIRE(a.tw, MXR_OUT_OF_MEMORY, "conv1d_fft: twiddle table allocation failed");
   switch (M) {
     case 8: return launch_fconv<8>(a, s);
@@ -256,7 +256,7 @@ mxr_status conv1d_fft_impl(const mxr_tensor *out, const mxr_tensor *in, const mx
               (long long)(FCONV_MAX_M / 2 + 1), (long long)FCONV_MAX_M);
   int64_t n = 1;
   while (n < P) n <<= 1;
-  return pc_common(fn, out, in, filt, n, 0, 0, 0, 1, L - 1 - s0, !corr, s);
+  return pc_common(fn, out, in, filt, n, 0, 0, 0, 1, L - 1 - s0, !corr, true, s);
 }
 
 }  // namespace mxr

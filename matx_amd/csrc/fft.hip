@@ -130,7 +130,7 @@ __global__ __launch_bounds__((GenericCfg<N, COL>::NT)) void fft_generic_kernel(F
   constexpr int NT = GenericCfg<N, COL>::NT;
   constexpr bool DIRECT = COL || N >= 256;
   using LY = Layout<N, TB, COL, (COL && TB < 32 && N >= 32)>;
-  using SQ = Seq<N, false>;
+  using SQ = Seq<N, false, !COL>;
   constexpr int K = SQ::n;
   __shared__ float2 lds[LY::LDS_ELEMS];
   __shared__ int64_t base_in[TB], base_out[TB];
@@ -185,7 +185,7 @@ __global__ __launch_bounds__((GenericCfg<N, COL>::NT)) void fft_generic_kernel(F
       constexpr int LSL = SQ::template LS<K - 1>;
       Pass<LY, RL, N, NT, TB> pl;
       pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
-      pl.template compute<LSL, INV>(a.tw + SQ::template TWOFF<K - 1>);
+      pl.template compute<LSL, INV, SQ::fact>(a.tw + SQ::template TWOFF<K - 1>);
       pl.template store<LSL>(put);
     }
     return;
@@ -653,7 +653,7 @@ __global__ __launch_bounds__((GenericCfg<M, COL>::NT)) void czt_kernel(CztArgs z
   constexpr int NT = GenericCfg<M, COL>::NT;
   constexpr bool DIRECT = COL || M >= 256;
   using LY = Layout<M, TB, COL, (COL && TB < 32 && M >= 32)>;
-  using SQ = Seq<M, false>;
+  using SQ = Seq<M, false, true>;
   __shared__ float2 lds[LY::LDS_ELEMS];
   __shared__ int64_t base_in[TB], base_out[TB];
   const FftArgs &a = z.f;
@@ -672,7 +672,7 @@ __global__ __launch_bounds__((GenericCfg<M, COL>::NT)) void czt_kernel(CztArgs z
   __syncthreads();
 
   if constexpr (DIRECT) {
-    using SI = Seq<M, true>;
+    using SI = Seq<M, true, true>;
     constexpr int K = SQ::n;
     constexpr int R0 = SQ::template R<0>, RL = SQ::template R<K - 1>, LSL = SQ::template LS<K - 1>;
     using P0 = Pass<LY, R0, M, NT, TB>;
@@ -726,7 +726,7 @@ __global__ __launch_bounds__((GenericCfg<M, COL>::NT)) void czt_kernel(CztArgs z
       lds_passes<LY, SQ, M, NT, TB, false, 1, K - 1>(lds, a.tw);
       pl.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
       wg_barrier();
-      pl.template compute<LSL, false>(a.tw + SQ::template TWOFF<K - 1>);
+      pl.template compute<LSL, false, true>(a.tw + SQ::template TWOFF<K - 1>);
     }
     PL::template outputs<LSL>([&](int u, int q, int, int k) { pl.v[u][q] = cmul(pl.v[u][q], z.spec[k]); });
     pl.template compute<1, true>(nullptr);
@@ -742,7 +742,7 @@ __global__ __launch_bounds__((GenericCfg<M, COL>::NT)) void czt_kernel(CztArgs z
       using PI = Pass<LY, RI, M, NT, TB>;
       PI pi;
       pi.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
-      pi.template compute<LSI, true>(z.twi + SI::template TWOFF<K - 1>);
+      pi.template compute<LSI, true, true>(z.twi + SI::template TWOFF<K - 1>);
       PI::template outputs<LSI>([&](int u, int q, int t, int k) {
         if (q < RI / 2) put(t, k, pi.v[u][q]);
       });
@@ -924,8 +924,8 @@ static mxr_status dispatch_czt(int64_t n, FftArgs a, bool inv, hipStream_t s) {
   CztArgs z{};
   z.f = a;
   z.n = (int)n;
-  z.f.tw = twiddles_device(M, false);
-  z.twi = twiddles_device(M, true);
+  z.f.tw = factors_device(M, false);
+  z.twi = factors_device(M, true);
   const float2 *tab = czt_tables((int)n, M);
   MXR_REQUIRE(z.f.tw != nullptr && z.twi != nullptr && tab != nullptr, MXR_OUT_OF_MEMORY,
               "fft: table allocation failed for size %lld", (long long)n);
@@ -1008,7 +1008,7 @@ __global__ __launch_bounds__(256) void fft_big_kernel(BigArgs a) {
   constexpr int NT = BigCfg<N>::NT;
   constexpr bool PASS1 = MODE == BIG_VIEW_TO_WORK || MODE == BIG_CHIRP_TO_WORK || MODE == BIG_WORK_TO_WORK;
   using LY = Layout<N, TB, true>;
-  using SQ = Seq<N, false>;
+  using SQ = Seq<N, false, true>;
   __shared__ float2 lds[LY::LDS_ELEMS];
   const FftArgs &f = a.f;
   const int64_t nblk = a.cols / TB;
@@ -1193,7 +1193,7 @@ template <int N, bool INV, int MODE>
 static mxr_status launch_big_one(const BigArgs &a, hipStream_t s) {
   constexpr int TB = BigCfg<N>::TB;
   BigArgs b = a;
-  b.tw_pass = twiddles_device(N, false);
+  b.tw_pass = factors_device(N, false);
   MXR_REQUIRE(b.tw_pass != nullptr, MXR_OUT_OF_MEMORY, "fft: twiddle table allocation failed");
   const int64_t grid = a.f.nbatch * (b.cols / TB);
   MXR_REQUIRE(grid <= 0x7fffffff, MXR_INVALID_SIZE, "fft: batch too large");
@@ -1380,7 +1380,7 @@ static mxr_status fft_impl(const char *fn, const mxr_tensor *out, const mxr_tens
   if (!pow2 && mix_plan(n, z)) return launch_mixed(z, a, inv, stream);
   if (!pow2) return n <= CZT_MAX_N ? dispatch_czt(n, a, inv, stream) : dispatch_czt_big(n, a, inv, stream);
   if (n > 16384) return dispatch_big(n, a, inv, stream);
-  a.tw = twiddles_device((int)n, false);
+  a.tw = a.batch_fast && n < 4096 ? twiddles_device((int)n, false) : factors_device((int)n, false);
   MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   return dispatch_generic(n, a, inv, stream);
 }

@@ -9,9 +9,11 @@
 //   a_m *= W_{Ls*R}^{m*k}                           (W_n = e^{-2 pi i/n} forward)
 //   b = DFT_R(a)
 //   Y[(j-k)*R + q*Ls + k] = b_q                     q = 0..R-1
-// After the last pass Y is in natural order.  The twiddles are folded into the
-// butterflies (dft_tw below); their factors come from tables built on the host
-// in double precision and rounded once to float.
+// After the last pass Y is in natural order.  Twiddles come from tables built
+// on the host in double precision and rounded once to float (one table per
+// (Ls, R) pass, k-major with stride R so a thread reads its R entries as one
+// contiguous run); transforms outside the detection chain fold them into the
+// butterflies (dft_tw below).
 #pragma once
 
 #include "mxr_internal.hpp"
@@ -88,6 +90,15 @@ __device__ __forceinline__ void dft8(float2 (&a)[8]) {
   for (int i = 0; i < 8; ++i) a[i] = y[i];
 }
 
+// a * W_16^3 of an inverse transform, the imaginary part's products summed in
+// the other order (which of two products a fused multiply-add rounds is the
+// compiler's choice otherwise, and lags must keep their bits).
+__device__ __forceinline__ float2 mul_w16_tail(float2 a) {
+  constexpr float C1 = 0.92387953251128675613f;  // cos(pi/8)
+  constexpr float S1 = 0.38268343236508977173f;  // sin(pi/8)
+  return make_float2(fmaf(a.x, S1, -(a.y * C1)), fmaf(a.y, S1, a.x * C1));
+}
+
 // a * W_16^e for e in {2, 6} equals H * hrot(a), H = sqrt(1/2), with hrot
 // made of additions only (W_16^2 = H (1 - i), W_16^6 = H (-1 - i) forward;
 // the inverse conjugates).
@@ -106,7 +117,8 @@ __device__ __forceinline__ void hpair(float2 u, float2 r, float2 &p, float2 &m) 
   m = make_float2(fmaf(-H, r.x, u.x), fmaf(-H, r.y, u.y));
 }
 
-template <bool INV>
+// TAIL: the last inverse pass of the 4096- and 8192-point block kernels.
+template <bool INV, bool TAIL = false>
 __device__ __forceinline__ void dft16(float2 (&a)[16]) {
   // 16 = 4 x 4: inner DFT4 over m2 (stride 4), twiddle W16^{m1 c}, DFT4 over
   // m1.  Z[m1][c] sits in a[m1 + 4c]; column c's outputs go to y[c + 4r].
@@ -124,7 +136,7 @@ __device__ __forceinline__ void dft16(float2 (&a)[16]) {
     y[12] = z3;
   }
   {  // c = 1: W^1, W^2, W^3
-    const float2 z1 = mul_w16<1, INV>(a[5]), z3 = mul_w16<3, INV>(a[7]);
+    const float2 z1 = mul_w16<1, INV>(a[5]), z3 = TAIL ? mul_w16_tail(a[7]) : mul_w16<3, INV>(a[7]);
     float2 t0, t1;
     hpair(a[4], hrot<2, INV>(a[6]), t0, t1);
     const float2 t2 = cadd(z1, z3), t3 = mul_w4<INV>(csub(z1, z3));
@@ -197,12 +209,11 @@ __host__ __device__ constexpr RadixSeq reversed(RadixSeq s) {
   for (int i = 0; i < s.n; ++i) o.r[i] = s.r[s.n - 1 - i];
   return o;
 }
-// Offset (in float2) of pass p's twiddle table inside a sequence's table: Ls
-// rows of R/2 factors per pass.
+// Offset (in float2) of pass p's twiddle table inside a sequence's table.
 __host__ __device__ constexpr int64_t tw_offset(RadixSeq s, int p) {
   int64_t off = 0, Ls = 1;
   for (int i = 0; i < p; ++i) {
-    off += (Ls > 1) ? Ls * s.r[i] / 2 : 0;
+    off += (Ls > 1) ? Ls * s.r[i] : 0;
     Ls *= s.r[i];
   }
   return off;
@@ -219,6 +230,82 @@ __host__ __device__ constexpr int pass_ls(RadixSeq s, int p) {
 __device__ __forceinline__ int lds_pad(int i) { return i + (i >> 4); }
 __host__ __device__ constexpr int lds_padded_len(int n) { return n + (n >> 4) + 1; }
 
+// --------------------------------------------------------- pass helpers
+template <int R, bool INV>
+__device__ __forceinline__ void apply_twiddles(float2 (&a)[R], const float2 *__restrict__ tw, int k) {
+  // tw points at the pass table; entries k*R + m, m = 1..R-1 (entry 0 holds
+  // 1 and is skipped).  Two twiddles per 16-byte load.
+  const float4 *t4 = reinterpret_cast<const float4 *>(tw + (int64_t)k * R);
+#pragma unroll
+  for (int h = 0; h < R / 2; ++h) {
+    float4 w = t4[h];
+    if (h > 0) a[2 * h] = cmul(a[2 * h], make_float2(w.x, INV ? -w.y : w.y));
+    a[2 * h + 1] = cmul(a[2 * h + 1], make_float2(w.z, INV ? -w.w : w.w));
+  }
+}
+
+// Host: build the twiddle table of a radix sequence for length N in double
+// precision, rounded once to float.  Layout per pass p (Ls > 1):
+// entry k*R + m = exp(-2 pi i m k / (Ls R)).
+void build_twiddles(int N, RadixSeq s, float2 *out);
+
+// Per-device cache of twiddle tables keyed by (N, reversed?).  Returns a
+// device pointer owned by the library.
+const float2 *twiddles_device(int N, bool reversed_seq);
+
+// v[m] *= W^{mk}, m = 1..15, from one power-base row (W^k, W^2k, W^4k,
+// W^8k): the other powers are products of at most four of them (at most
+// three extra roundings).  inv conjugates (inverse transform).
+__device__ __forceinline__ void tw_from_base(float2 (&v)[16], float4 b0, float4 b1, bool inv) {
+  float2 w1 = make_float2(b0.x, b0.y), w2 = make_float2(b0.z, b0.w);
+  float2 w4 = make_float2(b1.x, b1.y), w8 = make_float2(b1.z, b1.w);
+  if (inv) {
+    w1.y = -w1.y;
+    w2.y = -w2.y;
+    w4.y = -w4.y;
+    w8.y = -w8.y;
+  }
+  float2 w[16];
+  w[1] = w1;
+  w[2] = w2;
+  w[4] = w4;
+  w[8] = w8;
+  w[3] = cmul(w2, w1);
+  w[5] = cmul(w4, w1);
+  w[6] = cmul(w4, w2);
+  w[7] = cmul(w[6], w1);
+  w[9] = cmul(w8, w1);
+  w[10] = cmul(w8, w2);
+  w[11] = cmul(w[10], w1);
+  w[12] = cmul(w8, w4);
+  w[13] = cmul(w[12], w1);
+  w[14] = cmul(w[12], w2);
+  w[15] = cmul(w[14], w1);
+#pragma unroll
+  for (int m = 1; m < 16; ++m) v[m] = cmul(v[m], w[m]);
+}
+
+struct PowRow {
+  float4 a, b;
+};
+__device__ __forceinline__ PowRow load_pow(const float4 *base, int k) { return {base[2 * k], base[2 * k + 1]}; }
+// Pins a row's values: the inverse passes derive their twiddles anew rather
+// than from the forward passes' products, which round otherwise.
+__device__ __forceinline__ void pin_row(PowRow &r) {
+  asm volatile("" : "+v"(r.a.x), "+v"(r.a.y), "+v"(r.a.z), "+v"(r.a.w), "+v"(r.b.x), "+v"(r.b.y), "+v"(r.b.z),
+               "+v"(r.b.w));
+}
+template <bool INV, bool TAIL = false>
+__device__ __forceinline__ void pow_dft16(float2 (&v)[16], const PowRow &w) {
+  tw_from_base(v, w.a, w.b, INV);
+  dft16<INV, TAIL>(v);
+}
+
+// Per-device cache of radix-16 power-base rows for the pass with sub-length
+// Ls of an N-point transform: row k (k < Ls) holds W^k, W^2k, W^4k, W^8k with
+// W = e^{-2 pi i / (16 Ls)}, each from double precision rounded once.
+const float4 *pow_base_device(int N, int Ls);
+
 // ------------------------------------------------ twiddled butterflies
 // DFT_R of (x_j w^j), w = e^{-+2 pi i k/(Ls R)}, as a tree of two-point
 // butterflies a +- f b whose factor f is kept as (c, t) with f = c (1 -+ i t),
@@ -228,12 +315,14 @@ __host__ __device__ constexpr int lds_padded_len(int n) { return n + (n >> 4) + 
 // 152 for the plain butterfly, 60 for its twiddle products and 44 for deriving
 // eleven of the fifteen twiddles from four, and each input is rounded by one
 // operation less; a row of factors is half the size of a row of twiddles.
-// Measured: the 2048-point blocks of conv1d's FFT method (16 x 1048576, 209
-// taps) 98 -> 67 us, 8192 chirp-z transforms of 1000 points 94 -> 77 us.
-// pc4096_kernel, which had a row of four twiddles per butterfly and derived the
-// rest, gains from it only with its rows kept in registers for the inverse
-// passes (133 us a 16 x 128 x 9000 cube with the rows loaded four times, 127
-// with them kept; 132 before).
+// Rows of 4096 points 4096 at a time: 57 us with table twiddles, 46 like this;
+// of 16384 points 90 and 67; 8228 rows of 2039 points (chirp-z)
+// 179 and 102.
+// Where a wave shares its factors (transforms side by side along a strided
+// axis) the tables cost nothing and the plain butterfly is as fast or faster:
+// 16 x 8001 transforms of 256 points 126 us, 135 like this.  The detection
+// chain (pulse compression, the pulse-axis pass) keeps the plain butterfly,
+// whose roundings decide cells on the threshold.
 //
 // The factors of one k (w_n = e^{-2 pi i/n}; the tree's other factors are
 // these times -i, a swap):
@@ -326,21 +415,12 @@ __device__ __forceinline__ void dft_tw(float2 (&a)[16], const TwRow<16> &w) {
   for (int i = 0; i < 16; ++i) a[i] = y[i];
 }
 
-// Host: the factors of row k (or k + 1/2) of a pass (Ls, R), R/2 of them in
-// the order above.
-void tw_factors(int R, int64_t Ls, double k, float2 *out);
+// Host: the factors of row k of a pass (Ls, R), R/2 of them in the order above.
+void tw_factors(int R, int64_t Ls, int64_t k, float2 *out);
 
-// A transform at frequencies k + 1/2: the same passes with the factors of
-// k + 1/2 in place of those of k, the first pass (Ls = 1) included.  Table of
-// N's sequence: pass p's rows follow those of the passes before it.
-const float2 *twiddles_half_device(int N);
-
-// Per-device cache of twiddle tables keyed by (N, reversed?).  Returns a
-// device pointer owned by the library.
-const float2 *twiddles_device(int N, bool reversed_seq);
-
-// Per-device cache of the table of one radix-16 pass with sub-length Ls.
-const float4 *tw16_device(int Ls);
+// Per-device cache of factor tables keyed by (N, reversed?): Ls rows of R/2
+// factors per pass.
+const float2 *factors_device(int N, bool reversed_seq);
 
 // Raw buffer access (MUBUF) for the block kernels: a resource covering
 // `bytes` bytes from `base`.  The hardware range check returns zeros for
@@ -444,8 +524,10 @@ struct Layout {
   }
 };
 
-template <int N, bool REV>
+// FACT: passes with folded twiddles (dft_tw), tables from factors_device.
+template <int N, bool REV, bool FACT = false>
 struct Seq {
+  static constexpr bool fact = FACT;
   static constexpr RadixSeq s = REV ? reversed(radix_seq(N)) : radix_seq(N);
   static constexpr int n = s.n;
   template <int P>
@@ -453,7 +535,7 @@ struct Seq {
   template <int P>
   static constexpr int LS = pass_ls(s, P);
   template <int P>
-  static constexpr int64_t TWOFF = tw_offset(s, P);
+  static constexpr int64_t TWOFF = tw_offset(s, P) / (FACT ? 2 : 1);
 };
 
 // One Stockham pass: butterflies of this thread held in v[u][m].
@@ -480,29 +562,19 @@ struct Pass {
     }
   }
   // twiddle + DFT_R in registers
-  template <int LS, bool INV>
+  template <int LS, bool INV, bool FACT = false>
   __device__ __forceinline__ void compute(const float2 *__restrict__ tw) {
-#pragma unroll
-    for (int u = 0; u < BPT; ++u) {
-      if (!active(u)) continue;
-      if constexpr (LS > 1) {
-        int t, j;
-        LY::template bfly<R>(threadIdx.x + u * NT, t, j);
-        dft_tw<INV>(v[u], load_tw<R>(reinterpret_cast<const float4 *>(tw), LS, j & (LS - 1)));
-      } else {
-        dft<R, INV>(v[u]);
-      }
-    }
-  }
-  // the same with factors in the first pass too (half-bin tables)
-  template <int LS, bool INV>
-  __device__ __forceinline__ void compute_tw(const float2 *__restrict__ tw) {
 #pragma unroll
     for (int u = 0; u < BPT; ++u) {
       if (!active(u)) continue;
       int t, j;
       LY::template bfly<R>(threadIdx.x + u * NT, t, j);
-      dft_tw<INV>(v[u], load_tw<R>(reinterpret_cast<const float4 *>(tw), LS, j & (LS - 1)));
+      if constexpr (LS > 1 && FACT) {
+        dft_tw<INV>(v[u], load_tw<R>(reinterpret_cast<const float4 *>(tw), LS, j & (LS - 1)));
+      } else {
+        if constexpr (LS > 1) apply_twiddles<R, INV>(v[u], tw, j & (LS - 1));
+        dft<R, INV>(v[u]);
+      }
     }
   }
   // f(u, q, t, i) for the output positions store<LS> visits, value
@@ -548,7 +620,7 @@ __device__ __forceinline__ void lds_passes(float2 *lds, const float2 *__restrict
     Pass<LY, R, N, NT, TB> ps;
     ps.load([&](int t, int i) { return lds[LY::addr(t, i)]; });
     wg_barrier();
-    ps.template compute<LS, INV>(tw + SQ::template TWOFF<P>);
+    ps.template compute<LS, INV, SQ::fact>(tw + SQ::template TWOFF<P>);
     ps.template store<LS>([&](int t, int i, float2 x) { lds[LY::addr(t, i)] = x; });
     wg_barrier();
     lds_passes<LY, SQ, N, NT, TB, INV, P + 1, PE>(lds, tw);

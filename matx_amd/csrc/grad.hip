@@ -56,7 +56,7 @@ struct XcCfg {
 template <int M, bool INV>
 __device__ __forceinline__ void row_fft(float2 *buf, const float2 *tw) {
   using LY = Layout<M, 1, false>;
-  using SQ = Seq<M, false>;
+  using SQ = Seq<M, false, true>;
   lds_passes<LY, SQ, M, XcCfg<M>::NT, 1, INV, 0, SQ::n>(buf, tw);
 }
 
@@ -225,7 +225,7 @@ static mxr_status xc_run(const char *fn, const mxr_tensor *out, const RowOp &A, 
     a.obi.shape[d] = out->shape[d];
     a.obi.sa[d] = out->stride[d];
   }
-  a.tw = twiddles_device((int)n, false);
+  a.tw = factors_device((int)n, false);
   MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   a.scale = (float)(1.0 / (double)n);
   return xc_dispatch((int)n, a, batch_rows(out), s);
@@ -463,7 +463,7 @@ static mxr_status phase_isl_args(const char *fn, const mxr_tensor *phi, int64_t 
   a->ps_l = phi->stride[1];
   a->L = (int)phi->shape[1];
   *M = std::min<int64_t>(n, xc_size(2 * phi->shape[1] - 1));
-  a->tw = twiddles_device((int)*M, false);
+  a->tw = factors_device((int)*M, false);
   MXR_REQUIRE(a->tw != nullptr, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   return MXR_SUCCESS;
 }

@@ -30,7 +30,7 @@ template <int M>
 struct WgT {
   static constexpr int NT = M / 16;
   using LY = Layout<M, 1, false>;
-  using SF = Seq<M, false>;
+  using SF = Seq<M, false, true>;
   static constexpr int K = SF::n;
   static constexpr int R0 = SF::template R<0>;
   static constexpr int RL = SF::template R<K - 1>;
@@ -65,7 +65,7 @@ __device__ __forceinline__ void fwd_to_regs(typename WgT<M>::PL &pl, LoadF &&ld,
   wg_barrier();
   lds_passes<typename T::LY, typename T::SF, M, T::NT, 1, false, 1, T::K - 1>(lds, twf);
   pl.load([&](int t, int i) { return lds[T::LY::addr(t, i)]; });
-  pl.template compute<T::LSL, false>(twf + T::SF::template TWOFF<T::K - 1>);
+  pl.template compute<T::LSL, false, true>(twf + T::SF::template TWOFF<T::K - 1>);
 }
 
 template <int M>
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(WgT<M>::NT) void pc_wgrad_kernel(WgArgs a) {
 // workgroup (every wave waits at the same barriers), 2003 like this.
 struct Wg8192Args {
   WgArgs a;
-  const float4 *bA, *bB, *bC;  // factors of passes Ls = 2, 32, 512
+  const float4 *bA, *bB, *bC;  // power-base rows of passes Ls = 2, 32, 512
 };
 
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
@@ -184,14 +184,14 @@ void wgrad8192_kernel(Wg8192Args p) {
     for (int h = 0; h < 2; ++h) {  // x, then gy
       fetch(it, h != 0, v);
       pair_dft2(v, (j & 1) != 0);
-      TwRow<16> tw = load_tw<16>(opaque(p.bA), 2, j & 1);
-      dft_tw<false>(v, tw);
-      tw = load_tw<16>(opaque(p.bB), 32, j & 31);
+      PowRow tw = load_pow(opaque(p.bA), j & 1);
+      pow_dft16<false>(v, tw);
+      tw = load_pow(opaque(p.bB), j & 31);
       xchg(2);
-      dft_tw<false>(v, tw);
-      tw = load_tw<16>(opaque(p.bC), 512, j);
+      pow_dft16<false>(v, tw);
+      tw = load_pow(opaque(p.bC), j);
       xchg(32);
-      dft_tw<false>(v, tw);
+      pow_dft16<false>(v, tw);
       if (h == 0) {
 #pragma unroll
         for (int q = 0; q < 16; ++q) X[q] = v[q];
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(WgT<M>::NT) void wgrad_finish_kernel(const float2 *
 template <int M>
 static mxr_status wgrad_run(const WgradJob &j, hipStream_t s) {
   using T = WgT<M>;
-  const float2 *twf = twiddles_device(M, false);
+  const float2 *twf = factors_device(M, false);
   MXR_REQUIRE(twf != nullptr, MXR_OUT_OF_MEMORY, "pc waveform gradient: twiddle table allocation failed");
   MXR_REQUIRE(j.L <= M && j.V >= 1, MXR_INVALID_SIZE, "pc waveform gradient: inconsistent block plan");
   const int64_t items = j.rows * j.nblk;
@@ -325,7 +325,7 @@ static mxr_status wgrad_run(const WgradJob &j, hipStream_t s) {
     a.partial = ws;
     a.twf = twf;
     if (w8) {
-      Wg8192Args p{a, tw16_device(2), tw16_device(32), tw16_device(512)};
+      Wg8192Args p{a, pow_base_device(8192, 2), pow_base_device(8192, 32), pow_base_device(8192, 512)};
       MXR_REQUIRE(p.bA && p.bB && p.bC, MXR_OUT_OF_MEMORY,
                   "pc waveform gradient: twiddle table allocation failed");
       ProfScope ps("wgrad8192_kernel", s);

@@ -61,6 +61,13 @@ struct OlsBlock {
   const float2 *wc;  // M-point spectrum, scaled by 1/M
 };
 
+// A bin of the signal times the waveform's, with the roundings fixed (in a
+// plain product the compiler chooses which half of a sum the fused multiply-add
+// rounds, kernel by kernel).
+__device__ __forceinline__ float2 spec_mul(float2 v, float2 w) {
+  return make_float2(fmaf(v.x, w.x, -(v.y * w.y)), fmaf(v.y, w.x, v.x * w.y));
+}
+
 // Group g of a call: block g mod nblk of row g / nblk.
 __device__ __forceinline__ OlsBlock pc_block(const PcArgs &a, int64_t g) {
   const uint32_t row = (uint32_t)g / (uint32_t)a.nblk, blk = (uint32_t)g - row * (uint32_t)a.nblk;
@@ -221,7 +228,7 @@ __device__ __forceinline__ void ols_multi(const OlsBlock *obs, const float2 *twf
         float2 w;
         if constexpr (WF) w = lds[j + q * LSL];
         else w = obs[u].wc[j + q * LSL];
-        ps.v[u][q] = cmul(ps.v[u][q], w);
+        ps.v[u][q] = spec_mul(ps.v[u][q], w);
       }
     }
     if constexpr (WF) wg_barrier();  // the spectrum has been read
@@ -307,6 +314,31 @@ __global__ __launch_bounds__(256) void pc_ols_multi_wf_kernel(PcArgs a, WfLoad w
   ols_multi<M>(obs, a.twf, a.twi, lds, a.n <= PC_BUF_MAX_N, wf);
 }
 
+// In place: one workgroup walks its row's blocks in order, TB of them at a time
+// (every sample of a step is loaded before its first lag is stored, and the
+// lags of a step stay below the next step's first input).  385 rows of 5003
+// samples, 487 taps (three blocks of 2048): 27.6 us, one block at a time 53.
+template <int M>
+__global__ __launch_bounds__(256) void pc_ols_multi_row_kernel(PcArgs a) {
+  constexpr int TB = 4096 / M;
+  __shared__ float2 lds[Layout<M, TB, false>::LDS_ELEMS];
+  __shared__ OlsBlock obs[TB];
+  int64_t ox, oy;
+  batch_offsets(a.bi, xcd_remap(blockIdx.x, a.groups), &ox, &oy);
+  for (int64_t b0 = 0; b0 < a.nblk; b0 += TB) {
+    if (b0) wg_barrier();  // the last step's reads of obs and lds are done
+    if (threadIdx.x < TB) {
+      const int64_t b = b0 + threadIdx.x;
+      const bool idle = b >= a.nblk;  // past the row's last block
+      const int lo = (int)((idle ? b0 : b) * a.V);
+      obs[threadIdx.x] = OlsBlock{a.x + ox, a.y + oy, lo, (int)a.n, idle ? 0 : (int)a.seff,
+                                  idle ? lo : (int)a.nout, (int)a.V, a.wc};
+    }
+    __syncthreads();
+    ols_multi<M>(obs, opaque(a.twf), opaque(a.twi), lds, a.n <= PC_BUF_MAX_N, NoWf{});
+  }
+}
+
 // ROWLOOP: one workgroup walks blocks [b0, b1) of its row in order (needed
 // when y aliases x: a block only overwrites lags below the next block's
 // first input).  Otherwise each workgroup does exactly one block.
@@ -335,20 +367,21 @@ void pc_ols_kernel(PcArgs a) {
 // radix-16 butterfly per thread per pass).
 struct Pc4096Args {
   PcArgs a;
-  const float4 *base1;  // factors of pass Ls = 16
-  const float4 *base2;  // factors of pass Ls = 256
+  const float4 *base1;  // power-base rows of pass Ls = 16
+  const float4 *base2;  // power-base rows of pass Ls = 256
 };
 
 
 // One M = 4096 overlap-save block (256 threads); lds holds 4096 padded
 // elements.  Pre: the workgroup's previous use of lds is finished.
-// Thread j owns butterfly j of every radix-16 pass: its factors of the
-// Ls = 16 and Ls = 256 passes are rows j & 15 and j, loaded once, ahead of the
-// samples' arrival, and kept for the inverse passes.  A block that does not
-// wrap reads x through a raw buffer resource ending at the row's last sample
-// (the hardware returns zeros past it) and writes its kept lags through one
-// ending at its last kept lag (stores past it are dropped), so the block needs
-// no per-element tests; a wrapping block reads through one over the whole row.
+// Thread j owns butterfly j of every radix-16 pass: its twiddles of the
+// Ls = 16 and Ls = 256 passes come from power-base rows j & 15 and j, loaded
+// once, ahead of the samples' arrival, and kept for the inverse passes, which
+// conjugate them.  A block that does not wrap reads x through a raw buffer
+// resource ending at the row's last sample (the hardware returns zeros past
+// it) and writes its kept lags through one ending at its last kept lag (stores
+// past it are dropped), so the block needs no per-element tests; a wrapping
+// block reads through one over the whole row.
 // The spectrum's sixteen loads share one address register.  spec(q) gives bin
 // j + 256 q (the block's 1/M included).
 // Loads samples m0 .. m0 + NV - 1 of thread j of block ob
@@ -408,12 +441,12 @@ __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)
     for (int m = 0; m < 16; ++m) v[m] = lds[rbase + m * (NT + NT / 16)];
     wg_barrier();
   };
-  TwRow<16> t1 = load_tw<16>(base1, 16, j & 15), t2 = load_tw<16>(base2, 256, j);
+  PowRow t1 = load_pow(base1, j & 15), t2 = load_pow(base2, j);
 
   // forward pass 0 (Ls = 1) on the samples as loaded
   dft16<false>(v);
   xchg(1);
-  dft_tw<false>(v, t1);  // forward pass 1 (Ls = 16)
+  pow_dft16<false>(v, t1);  // forward pass 1 (Ls = 16)
   // the spectrum bins this thread multiplies, fetched before the exchange
   // so that their cache latency hides behind it and the last forward pass
   float2 sp[16];
@@ -422,7 +455,7 @@ __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)
     for (int q = 0; q < 16; ++q) sp[q] = spec(q);
   }
   xchg(16);
-  dft_tw<false>(v, t2);  // forward pass 2 (Ls = 256)
+  pow_dft16<false>(v, t2);  // forward pass 2 (Ls = 256)
   if constexpr (LATE_SPEC) {
     wg_barrier();  // the spectrum is complete
 #pragma unroll
@@ -430,11 +463,13 @@ __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)
   }
 #pragma unroll
   for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], sp[q]);
-  dft16<true>(v);            // inverse pass 0 (Ls = 1)
+  dft16<true>(v);          // inverse pass 0 (Ls = 1)
+  pin_row(t1);
+  pin_row(t2);
   xchg(1);
-  dft_tw<true>(v, t1);   // inverse pass 1 (Ls = 16)
+  pow_dft16<true>(v, t1);  // inverse pass 1 (Ls = 16)
   xchg(16);
-  dft_tw<true>(v, t2);   // inverse pass 2 (Ls = 256)
+  pow_dft16<true, true>(v, t2);  // inverse pass 2 (Ls = 256)
   // lags lo + j + 256 q below lo + lim are kept (the spectrum carries the 1/M)
   const int lim = (ob.nout - lo) < ob.V ? (ob.nout - lo) : ob.V;
   const buf_rsrc ry = make_rsrc(ob.yr + lo, lim * 8);
@@ -469,20 +504,6 @@ void pc4096_kernel(Pc4096Args pa) {
   __shared__ float2 lds[LY::LDS_ELEMS];
   const PcArgs &a = pa.a;
   ols_block4096(pc_block(a, xcd_remap(blockIdx.x, a.groups)), pa.base1, pa.base2, lds);
-}
-
-// In place: one workgroup walks the blocks of its row in order (a block only
-// overwrites lags below the next block's first input).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-void pc4096_row_kernel(Pc4096Args pa) {
-  using LY = Layout<4096, 1, false>;
-  __shared__ float2 lds[LY::LDS_ELEMS];
-  const PcArgs &a = pa.a;
-  const uint32_t row = (uint32_t)xcd_remap(blockIdx.x, a.groups);
-  for (int b = 0; b < (int)a.nblk; ++b) {
-    if (b) wg_barrier();  // previous block's LDS reads are done
-    ols_block4096(pc_block(a, (int64_t)row * a.nblk + b), opaque(pa.base1), opaque(pa.base2), lds);
-  }
 }
 
 // Small grids (fft_conv on a few hundred pulses, where one workgroup per
@@ -538,12 +559,12 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
     if (q.conj_in) v[m].y = -v[m].y;
   }
   dft16<false>(v);
-  TwRow<16> tw = load_tw<16>(q.p.base1, 16, j & 15);
+  PowRow tw = load_pow(q.p.base1, j & 15);
   xchg(1);
-  dft_tw<false>(v, tw);
-  tw = load_tw<16>(q.p.base2, 256, j);
+  pow_dft16<false>(v, tw);
+  tw = load_pow(q.p.base2, j);
   xchg(16);
-  dft_tw<false>(v, tw);
+  pow_dft16<false>(v, tw);
   // the exchange above ended with a barrier after every read of wsp
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
@@ -556,8 +577,8 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
 }
 
 // Dedicated M = 8192 block kernel: radix sequence 2 x 16 x 16 x 16 over 512
-// threads (one radix-16 butterfly per thread per pass) with the factor
-// tables of the passes Ls = 2, 32, 512
+// threads (one radix-16 butterfly per thread per pass) with the power-base
+// twiddles of the 4096-point kernel for the passes Ls = 2, 32, 512
 // (conjugated for the inverse).  The forward radix-2 pass (Ls = 1, no
 // twiddles) is folded into the load: radix-16 butterfly j of the next pass
 // takes X1[j + 512m] = x[j0] +- x[j0 + 4096] with j0 = j/2 + 256m and the
@@ -568,7 +589,7 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
 // registers before the first inverse exchange: five LDS exchanges per block.
 struct Pc8192Args {
   PcArgs a;
-  const float4 *bA, *bB, *bC;  // factors of passes Ls = 2, 32, 512
+  const float4 *bA, *bB, *bC;  // power-base rows for Ls = 2, 32, 512
 };
 
 __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *bA, const float4 *bB,
@@ -616,24 +637,24 @@ __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *b
     }
     pair_dft2(v, (j & 1) != 0);
   }
-  TwRow<16> tw = load_tw<16>(bA, 2, j & 1);
-  dft_tw<false>(v, tw);  // forward pass Ls = 2
-  tw = load_tw<16>(bB, 32, j & 31);
+  PowRow tw = load_pow(bA, j & 1);
+  pow_dft16<false>(v, tw);  // forward pass Ls = 2
+  tw = load_pow(bB, j & 31);
   xchg(2);
-  dft_tw<false>(v, tw);  // forward pass Ls = 32
-  tw = load_tw<16>(bC, 512, j);
+  pow_dft16<false>(v, tw);  // forward pass Ls = 32
+  tw = load_pow(bC, j);
   // the spectrum bins this thread multiplies, fetched before the exchange
   const buf_rsrc rw = make_rsrc(ob.wc, 8192 * 8);
   float2 sp[16];
 #pragma unroll
   for (int q = 0; q < 16; ++q) sp[q] = buf_load2s(rw, j * 8, q * 4096);
   xchg(32);
-  dft_tw<false>(v, tw);  // forward pass Ls = 512: bins j + 512q
+  pow_dft16<false>(v, tw);  // forward pass Ls = 512: bins j + 512q
 #pragma unroll
   for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], sp[q]);
   // inverse radix-2 pass (Ls = 1) on bins j + 512q, j + 512q + 4096; its
   // outputs 2 (j + 512 q) and the next sit at pad(2 j) + 1088 q and + 1
-  tw = load_tw<16>(bA, 2, j & 1);
+  tw = load_pow(bA, j & 1);
   const int e0 = lds_pad(2 * j);
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
@@ -644,13 +665,13 @@ __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *b
 #pragma unroll
   for (int m = 0; m < 16; ++m) v[m] = lds[rbase + 544 * m];
   wg_barrier();
-  dft_tw<true>(v, tw);  // inverse pass Ls = 2
-  tw = load_tw<16>(bB, 32, j & 31);
+  pow_dft16<true>(v, tw);  // inverse pass Ls = 2
+  tw = load_pow(bB, j & 31);
   xchg(2);
-  dft_tw<true>(v, tw);  // inverse pass Ls = 32
-  tw = load_tw<16>(bC, 512, j);
+  pow_dft16<true>(v, tw);  // inverse pass Ls = 32
+  tw = load_pow(bC, j);
   xchg(32);
-  dft_tw<true>(v, tw);  // inverse pass Ls = 512: lags j + 512q
+  pow_dft16<true, true>(v, tw);  // inverse pass Ls = 512: lags j + 512q
   // lags lo + j + 512 q below lo + lim are kept (stores past lim dropped by
   // the range check; the spectrum carries the 1/M)
   const int lim = (ob.nout - lo) < ob.V ? (ob.nout - lo) : ob.V;
@@ -665,18 +686,6 @@ void pc8192_kernel(Pc8192Args pa) {
   __shared__ float2 lds[LY::LDS_ELEMS];
   const OlsBlock ob = pc_block(pa.a, xcd_remap(blockIdx.x, pa.a.groups));
   ols_block8192(ob, pa.bA, pa.bB, pa.bC, lds);
-}
-
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
-void pc8192_row_kernel(Pc8192Args pa) {
-  using LY = Layout<8192, 1, false>;
-  __shared__ float2 lds[LY::LDS_ELEMS];
-  const PcArgs &a = pa.a;
-  const uint32_t row = (uint32_t)xcd_remap(blockIdx.x, a.groups);
-  for (int b = 0; b < (int)a.nblk; ++b) {
-    if (b) wg_barrier();
-    ols_block8192(pc_block(a, (int64_t)row * a.nblk + b), opaque(pa.bA), opaque(pa.bB), opaque(pa.bC), lds);
-  }
 }
 
 // One workgroup of M/16 threads.  Thread j loads samples j + m*M/16,
@@ -911,7 +920,7 @@ mxr_status launch_pc_batch(int M, const PcJob *d_jobs, const int *d_item_job, in
   ProfScope ps("pc_batch_kernel", s);
   switch (M) {
     case 4096: {
-      const float4 *b1 = tw16_device(16), *b2 = tw16_device(256);
+      const float4 *b1 = pow_base_device(4096, 16), *b2 = pow_base_device(4096, 256);
       MXR_REQUIRE(b1 && b2, MXR_OUT_OF_MEMORY, "ragged batch: twiddle table allocation failed");
       if (persist) pc4096_batch_kernel<true><<<dim3(grid), dim3(256), 0, s>>>(d_jobs, d_item_job, items, b1, b2);
       else pc4096_batch_kernel<false><<<dim3(grid), dim3(256), 0, s>>>(d_jobs, d_item_job, items, b1, b2);
@@ -933,7 +942,7 @@ mxr_status launch_pc_batch(int M, const PcJob *d_jobs, const int *d_item_job, in
           d_jobs, d_item_job, items, twf, twi);                                                       \
     break;
     case 8192: {
-      const float4 *bA = tw16_device(2), *bB = tw16_device(32), *bC = tw16_device(512);
+      const float4 *bA = pow_base_device(8192, 2), *bB = pow_base_device(8192, 32), *bC = pow_base_device(8192, 512);
       MXR_REQUIRE(bA && bB && bC, MXR_OUT_OF_MEMORY, "ragged batch: twiddle table allocation failed");
       if (persist) pc8192_batch_kernel<true><<<dim3(grid), dim3(512), 0, s>>>(d_jobs, d_item_job, items, bA, bB, bC);
       else pc8192_batch_kernel<false><<<dim3(grid), dim3(512), 0, s>>>(d_jobs, d_item_job, items, bA, bB, bC);
@@ -977,8 +986,13 @@ int forced_block() {
 
 // Chooses the overlap-save block size.  allow_ols is false for convolution
 // (conj_w = 0), where only the single n-point block is exact.
+// by_rate weighs each size by its kernel's measured rate (long convolutions,
+// the ragged batch).  Pulse compression counts points alone: its lags are
+// compared with thresholds further on, and a size that follows a kernel's speed
+// would change their rounding, and with it cells on the threshold, whenever a
+// kernel gets faster.
 mxr_status plan_pc(int64_t seff, int64_t L, int64_t n, int64_t nout, bool allow_ols, bool in_place,
-                   PcPlan *out, int force_M = 0) {
+                   bool by_rate, PcPlan *out, int force_M = 0) {
   PcPlan best{0, 0, 0};
   double best_cost = 1e300;
   auto consider = [&](int M) {
@@ -1002,14 +1016,15 @@ mxr_status plan_pc(int64_t seff, int64_t L, int64_t n, int64_t nout, bool allow_
       }
     }
     // relative time per M log2 M, measured on 16 rows of 1048576 samples with
-    // filters of 30 to 513 taps (1024 and 2048: 0.33 to 0.35, 4096: 0.29 to
-    // 0.30, 8192: 0.38 ps a point and level) and on the radar cubes (4096:
-    // 0.245, 8192: 0.264); the 16384-point kernel holds one workgroup per CU
-    // and runs about half as fast per point
-    double eff = M <= 2048 ? 1.15 : (M == 4096 ? 1.0 : (M == 8192 ? 1.15 : (M == 16384 ? 2.0 : 1e9)));
-    // in place, the blocks of a row run one after another in its workgroup
-    // (385 rows of 5003 samples, 487 taps: three blocks of 2048 took 53 us, one of 8192 20)
-    if (in_place && p.nblk > 1) eff *= 2.0;
+    // filters of 30 to 513 taps (1024 and 2048: 0.41 to 0.49, 4096: 0.25 to
+    // 0.29, 8192: 0.33 to 0.37 ps a point and level) and on 2048 rows of 9000
+    // samples (2048: 0.40 to 0.46, 4096: 0.27, 8192: 0.29); the 16384-point
+    // kernel holds one workgroup per CU and runs about half as fast per point
+    const double eff = M == 4096 ? 1.0
+                       : M <= 2048 ? (by_rate ? 1.5 : 1.0)
+                       : M == 8192 ? (by_rate ? 1.15 : 1.0)
+                       : M == 16384 ? 2.0
+                                    : 1e9;
     const double cost = (double)p.nblk * M * ilog2(M) * eff;
     if (cost < best_cost || (cost == best_cost && M > best.M)) {
       best_cost = cost;
@@ -1084,7 +1099,7 @@ mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
   }
   if constexpr (M == 4096) {
     if (fuse && pa->n <= PC_BUF_MAX_N) {
-      Pc4096WfArgs q{{*pa, tw16_device(16), tw16_device(256)}, wa->w, wa->wstride,
+      Pc4096WfArgs q{{*pa, pow_base_device(4096, 16), pow_base_device(4096, 256)}, wa->w, wa->wstride,
                      (int)wa->L, wa->conj_in, wa->conj, wa->out_scale};
       MXR_REQUIRE(q.p.base1 && q.p.base2, MXR_OUT_OF_MEMORY,
                   "pulse compression: twiddle table allocation failed");
@@ -1101,36 +1116,34 @@ mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
   MXR_HIP_TRY(hipGetLastError());
   if (!pa || pa->groups <= 0) return MXR_SUCCESS;
   if constexpr (M == 8192) {
-    // (a row's block numbers fit 32 bits too where one workgroup walks them)
-    if (pa->n <= PC_BUF_MAX_N && pa->groups * pa->bpw <= 0x7fffffff) {
-      Pc8192Args p8{*pa, tw16_device(2), tw16_device(32), tw16_device(512)};
+    if (pa->n <= PC_BUF_MAX_N && pa->bpw == 1) {
+      Pc8192Args p8{*pa, pow_base_device(8192, 2), pow_base_device(8192, 32), pow_base_device(8192, 512)};
       MXR_REQUIRE(p8.bA && p8.bB && p8.bC, MXR_OUT_OF_MEMORY,
                   "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc8192_kernel", s);
-      if (pa->bpw > 1) pc8192_row_kernel<<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
-      else pc8192_kernel<<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
+      pc8192_kernel<<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
       MXR_HIP_TRY(hipGetLastError());
       return MXR_SUCCESS;
     }
   }
   if constexpr (M == 4096) {
-    if (pa->n <= PC_BUF_MAX_N && pa->groups * pa->bpw <= 0x7fffffff) {
-      Pc4096Args p4{*pa, tw16_device(16), tw16_device(256)};
+    if (pa->n <= PC_BUF_MAX_N && pa->bpw == 1) {
+      Pc4096Args p4{*pa, pow_base_device(4096, 16), pow_base_device(4096, 256)};
       MXR_REQUIRE(p4.base1 && p4.base2, MXR_OUT_OF_MEMORY, "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc4096_kernel", s);
-      if (pa->bpw > 1) pc4096_row_kernel<<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
-      else pc4096_kernel<<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
+      pc4096_kernel<<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
       MXR_HIP_TRY(hipGetLastError());
       return MXR_SUCCESS;
     }
   }
   {
     ProfScope ps("pc_ols_kernel", s);
-    if (pa->bpw > 1) {
-      pc_ols_kernel<M, true><<<dim3((unsigned)pa->groups), dim3(PcCfg<M>::NT), 0, s>>>(*pa);
-    } else if constexpr (M <= 2048) {
+    if constexpr (M <= 2048) {
       constexpr int TB = 4096 / M;
-      pc_ols_multi_kernel<M><<<dim3((unsigned)((pa->groups + TB - 1) / TB)), dim3(256), 0, s>>>(*pa);
+      if (pa->bpw > 1) pc_ols_multi_row_kernel<M><<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(*pa);
+      else pc_ols_multi_kernel<M><<<dim3((unsigned)((pa->groups + TB - 1) / TB)), dim3(256), 0, s>>>(*pa);
+    } else if (pa->bpw > 1) {
+      pc_ols_kernel<M, true><<<dim3((unsigned)pa->groups), dim3(PcCfg<M>::NT), 0, s>>>(*pa);
     } else {
       pc_ols_kernel<M, false><<<dim3((unsigned)pa->groups), dim3(PcCfg<M>::NT), 0, s>>>(*pa);
     }
@@ -1155,13 +1168,13 @@ mxr_status dispatch_pc(int M, const WfArgs *wa, const PcArgs *pa, hipStream_t s)
 }  // namespace
 
 // Builds every table the block kernels of size M read (forward and reversed
-// pass twiddles, the factor tables of the dedicated 4096 and 8192 kernels),
-// so that later launches allocate nothing (and can be graph-captured).
+// pass twiddles, the power-base rows of the dedicated 4096 and 8192 kernels,
+// the waveform gradient's factors), so that later launches allocate nothing (and can be graph-captured).
 mxr_status pc_tables_prepare(int M, const char *fn) {
-  bool ok = twiddles_device(M, false) && twiddles_device(M, true);
-  if (M == 4096) ok = ok && tw16_device(16) && tw16_device(256);
+  bool ok = twiddles_device(M, false) && twiddles_device(M, true) && factors_device(M, false);
+  if (M == 4096) ok = ok && pow_base_device(4096, 16) && pow_base_device(4096, 256);
   if (M == 8192)
-    ok = ok && tw16_device(2) && tw16_device(32) && tw16_device(512);
+    ok = ok && pow_base_device(8192, 2) && pow_base_device(8192, 32) && pow_base_device(8192, 512);
   MXR_REQUIRE(ok, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   return MXR_SUCCESS;
 }
@@ -1171,7 +1184,7 @@ mxr_status pc_tables_prepare(int M, const char *fn) {
 mxr_status pc_plan_blocks(int64_t seff, int64_t L, int64_t n, int64_t nout, int M_req, int *M,
                           int64_t *V, int64_t *nblk) {
   PcPlan p;
-  mxr_status st = plan_pc(seff, L, n, nout, true, false, &p, M_req);
+  mxr_status st = plan_pc(seff, L, n, nout, true, false, true, &p, M_req);
   if (st) return st;
   *M = p.M;
   *V = p.V;
@@ -1246,7 +1259,7 @@ mxr_status fft_conv_rows(const mxr_tensor *out, const mxr_tensor *x, const mxr_t
 // n covers every nonzero lag); reverse_conj: the waveform is reverse(conj(w)).
 mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, const mxr_tensor *w,
                      int64_t n, int window, int normalize, int writeback, int conj_w,
-                     int64_t shift, int reverse_conj, hipStream_t stream) {
+                     int64_t shift, int reverse_conj, bool by_rate, hipStream_t stream) {
   mxr_status st;
   if ((st = check_tensor(w, "waveform", MXR_C64, 1, 1))) return st;
   PcArgs pa{};
@@ -1259,7 +1272,7 @@ mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, c
   MXR_REQUIRE((reverse_conj || !views_overlap(*w, *x)) && !views_overlap(*w, *y), MXR_ALIAS_ERROR,
               "%s: waveform aliases the signal", fn);
   PcPlan plan;
-  if ((st = plan_pc(pa.seff, L, n, pa.nout, conj_w != 0, in_place, &plan))) return st;
+  if ((st = plan_pc(pa.seff, L, n, pa.nout, conj_w != 0, in_place, by_rate, &plan))) return st;
   MXR_REQUIRE(L <= plan.M, MXR_NOT_SUPPORTED, "%s: waveform longer than the block", fn);
 
   float2 *wc = wc_buffer(plan.M, stream);
@@ -1315,7 +1328,7 @@ static mxr_status pc_plan_create(mxr_pc_plan *out, int64_t S, int64_t L, int64_t
               "pc_plan_create: flags may hold only MXR_PC_WINDOW | MXR_PC_NORMALIZE");
   PcPlan plan;
   mxr_status st;
-  if ((st = plan_pc(S < n ? S : n, L, n, nout, true, false, &plan))) return st;
+  if ((st = plan_pc(S < n ? S : n, L, n, nout, true, false, false, &plan))) return st;
   MXR_REQUIRE(L <= plan.M, MXR_NOT_SUPPORTED, "pc_plan_create: waveform longer than the block");
   if ((st = pc_tables_prepare(plan.M, "pc_plan_create"))) return st;
   const float2 *twf = twiddles_device(plan.M, false);
@@ -1448,7 +1461,7 @@ mxr_status mxr_pulse_compress(const mxr_tensor *y, const mxr_tensor *x, const mx
   return mxr::guarded("mxr_pulse_compress", [&] {
     return mxr::pc_common("pulse_compress", y, x, w, n, (flags & MXR_PC_WINDOW) != 0,
                           (flags & MXR_PC_NORMALIZE) != 0, (flags & MXR_PC_WRITEBACK) != 0, 1,
-                          0, 0, stream);
+                          0, 0, false, stream);
   });
 }
 
@@ -1456,7 +1469,8 @@ mxr_status mxr_fft_conv(const mxr_tensor *out, const mxr_tensor *x, const mxr_te
                         int conj_w, hipStream_t stream) {
   return mxr::guarded("mxr_fft_conv", [&] {
     if (w && w->rank > 1) return mxr::fft_conv_rows(out, x, w, n, conj_w ? 1 : 0, stream);
-    return mxr::pc_common("fft_conv", out, x, w, n, 0, 0, 0, conj_w ? 1 : 0, 0, 0, stream);
+    return mxr::pc_common("fft_conv", out, x, w, n, 0, 0, 0, conj_w ? 1 : 0, 0, 0, false,
+                          stream);
   });
 }
 

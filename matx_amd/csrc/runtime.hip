@@ -1,6 +1,7 @@
 // libmxr runtime: thread-local errors, descriptor checks, per-device caches
 // of twiddle tables (the analogue of MatX's plan cache,
 // include/matx/core/cache.h:167-291), and mxr_clear_caches.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -99,7 +100,29 @@ int max_lds_per_block() {
   return v;
 }
 
-void tw_factors(int R, int64_t Ls, double k, float2 *out) {
+void build_twiddles(int N, RadixSeq s, float2 *out) {
+  const double two_pi = 6.283185307179586476925286766559;
+  int64_t Ls = 1;
+  for (int p = 0; p < s.n; ++p) {
+    const int R = s.r[p];
+    if (Ls > 1) {
+      float2 *t = out + tw_offset(s, p);
+      const int64_t len = Ls * R;
+      for (int64_t k = 0; k < Ls; ++k) {
+        for (int m = 0; m < R; ++m) {
+          // reduce m*k modulo len before scaling: the angle index stays exact
+          const int64_t e = (m * k) % len;
+          const double a = -two_pi * (double)e / (double)len;
+          t[k * R + m] = make_float2((float)std::cos(a), (float)std::sin(a));
+        }
+      }
+    }
+    Ls *= R;
+  }
+  (void)N;
+}
+
+void tw_factors(int R, int64_t Ls, int64_t k, float2 *out) {
   // exponent num/16 of w_R beside the power of w: w^pw w_16^num
   struct F {
     int pw, num;
@@ -109,7 +132,7 @@ void tw_factors(int R, int64_t Ls, double k, float2 *out) {
   const F *f = R == 4 ? f4 : (R == 8 ? f8 : f16);
   const double two_pi = 6.283185307179586476925286766559;
   for (int i = 0; i < R / 2; ++i) {
-    const double ang = two_pi * (f[i].pw * k / (double)(Ls * R) + f[i].num / 16.0);
+    const double ang = two_pi * ((double)(f[i].pw * k) / (double)(Ls * R) + f[i].num / 16.0);
     double c = std::cos(ang);
     if (std::fabs(c) < TW_MIN_COS) c = TW_MIN_COS;
     out[i] = make_float2((float)c, (float)(std::sin(ang) / c));
@@ -117,10 +140,10 @@ void tw_factors(int R, int64_t Ls, double k, float2 *out) {
 }
 
 // The table of one pass: factors 2h, 2h + 1 of row k at float2 index 2 (h Ls + k).
-static void tw_pass(int R, int64_t Ls, float2 *out, double shift = 0.0) {
+static void tw_pass(int R, int64_t Ls, float2 *out) {
   float2 f[8];
   for (int64_t k = 0; k < Ls; ++k) {
-    tw_factors(R, Ls, (double)k + shift, f);
+    tw_factors(R, Ls, k, f);
     for (int h = 0; h < R / 4; ++h) {
       out[2 * (h * Ls + k)] = f[2 * h];
       out[2 * (h * Ls + k) + 1] = f[2 * h + 1];
@@ -151,19 +174,21 @@ void register_cache_clear(void (*fn)()) {
   clear_hooks().push_back(fn);
 }
 
-const float2 *twiddles_device(int N, bool rev) {
+// fact: the passes' factors (dft_tw) in place of their twiddles
+static const float2 *pass_tables(int N, bool rev, bool fact) {
   const int dev = device_id();
   std::lock_guard<std::mutex> g(g_tw_mu);
-  TwKey key{dev, N, rev ? 1 : 0};
+  TwKey key{dev, N, (rev ? 1 : 0) + (fact ? 2 : 0)};
   auto it = g_tw.find(key);
   if (it != g_tw.end()) return it->second;
   RadixSeq s = radix_seq(N);
   if (s.n < 0) return nullptr;
   if (rev) s = reversed(s);
-  const int64_t sz = tw_size(s) < 2 ? 2 : tw_size(s);
+  const int64_t sz = std::max<int64_t>(2, fact ? tw_size(s) / 2 : tw_size(s));
   std::vector<float2> host((size_t)sz, make_float2(1.f, 0.f));
-  for (int p = 0; p < s.n; ++p)
-    if (pass_ls(s, p) > 1) tw_pass(s.r[p], pass_ls(s, p), host.data() + tw_offset(s, p));
+  if (!fact) build_twiddles(N, s, host.data());
+  for (int p = 0; fact && p < s.n; ++p)
+    if (pass_ls(s, p) > 1) tw_pass(s.r[p], pass_ls(s, p), host.data() + tw_offset(s, p) / 2);
   float2 *d = nullptr;
   if (hipMalloc(&d, sizeof(float2) * sz) != hipSuccess) return nullptr;
   // a synchronous copy: tables are built once per (device, size), before use
@@ -176,6 +201,9 @@ const float2 *twiddles_device(int N, bool rev) {
           (long long)sz, dev);
   return d;
 }
+
+const float2 *twiddles_device(int N, bool rev) { return pass_tables(N, rev, false); }
+const float2 *factors_device(int N, bool rev) { return pass_tables(N, rev, true); }
 
 // ------------------------------------------------------------ profiling
 namespace {
@@ -219,42 +247,34 @@ namespace {
 std::map<TwKey, float4 *> g_pb;
 }
 
-// Uploads a table built once per key (g_tw_mu held).
-static const float4 *upload_table(const TwKey &key, const std::vector<float2> &host) {
+const float4 *pow_base_device(int N, int Ls) {
+  const int dev = device_id();
+  std::lock_guard<std::mutex> g(g_tw_mu);
+  TwKey key{dev, N, Ls};
+  auto it = g_pb.find(key);
+  if (it != g_pb.end()) return it->second;
+  const double two_pi = 6.283185307179586476925286766559;
+  const int64_t len = (int64_t)16 * Ls;
+  std::vector<float4> host((size_t)Ls * 2);
+  for (int64_t k = 0; k < Ls; ++k) {
+    float2 w[4];
+    const int pw[4] = {1, 2, 4, 8};
+    for (int i = 0; i < 4; ++i) {
+      const int64_t e = (pw[i] * k) % len;
+      const double ang = -two_pi * (double)e / (double)len;
+      w[i] = make_float2((float)std::cos(ang), (float)std::sin(ang));
+    }
+    host[2 * k] = make_float4(w[0].x, w[0].y, w[1].x, w[1].y);
+    host[2 * k + 1] = make_float4(w[2].x, w[2].y, w[3].x, w[3].y);
+  }
   float4 *d = nullptr;
-  if (hipMalloc(&d, sizeof(float2) * host.size()) != hipSuccess) return nullptr;
-  if (hipMemcpy(d, host.data(), sizeof(float2) * host.size(), hipMemcpyHostToDevice) != hipSuccess) {
+  if (hipMalloc(&d, sizeof(float4) * host.size()) != hipSuccess) return nullptr;
+  if (hipMemcpy(d, host.data(), sizeof(float4) * host.size(), hipMemcpyHostToDevice) != hipSuccess) {
     (void)hipFree(d);
     return nullptr;
   }
   g_pb[key] = d;
   return d;
-}
-
-const float2 *twiddles_half_device(int N) {
-  const int dev = device_id();
-  std::lock_guard<std::mutex> g(g_tw_mu);
-  TwKey key{dev, -N, 0};
-  auto it = g_pb.find(key);
-  if (it != g_pb.end()) return reinterpret_cast<const float2 *>(it->second);
-  const RadixSeq s = radix_seq(N);
-  if (s.n < 1) return nullptr;
-  const int64_t first = s.r[0] / 2;  // the first pass's one row
-  std::vector<float2> host((size_t)(first + tw_size(s)));
-  tw_pass(s.r[0], 1, host.data(), 0.5);
-  for (int p = 1; p < s.n; ++p) tw_pass(s.r[p], pass_ls(s, p), host.data() + first + tw_offset(s, p), 0.5);
-  return reinterpret_cast<const float2 *>(upload_table(key, host));
-}
-
-const float4 *tw16_device(int Ls) {
-  const int dev = device_id();
-  std::lock_guard<std::mutex> g(g_tw_mu);
-  TwKey key{dev, 16, Ls};
-  auto it = g_pb.find(key);
-  if (it != g_pb.end()) return it->second;
-  std::vector<float2> host((size_t)Ls * 8);
-  tw_pass(16, Ls, host.data());
-  return upload_table(key, host);
 }
 
 // Per (device, stream, tag) scratch buffers that only grow: partial sums of
@@ -330,7 +350,7 @@ static void clear_workspaces() {
 CacheClearRegistrar g_reg_ws(clear_workspaces);
 
 // Plans (pulse-compression and ragged) keep raw pointers to the twiddle and
-// factor tables; while any plan is alive mxr_clear_caches leaves the
+// power-base tables; while any plan is alive mxr_clear_caches leaves the
 // tables in place (a few hundred KiB), so a live plan never reads freed memory.
 namespace {
 int g_live_plans = 0;  // guarded by g_tw_mu
