@@ -308,32 +308,32 @@ const float4 *pow_base_device(int N, int Ls);
 
 // ------------------------------------------------ twiddled butterflies
 // DFT_R of (x_j w^j), w = e^{-+2 pi i k/(Ls R)}, as a tree of two-point
-// butterflies a +- f b whose factor f is kept as (c, t) with f = c (1 -+ i t),
-// c = cos, t = tan: u + i v = b (1 -+ i t) takes two fused multiply-adds and
-// a +- c (u + i v) four, where a complex product and two complex sums take
-// eight.  A radix-16 butterfly is 32 of them, 192 instructions in place of
-// 152 for the plain butterfly, 60 for its twiddle products and 44 for deriving
-// eleven of the fifteen twiddles from four, and each input is rounded by one
-// operation less; a row of factors is half the size of a row of twiddles.
-// Rows of 4096 points 4096 at a time: 57 us with table twiddles, 46 like this;
-// of 16384 points 90 and 67; 8228 rows of 2039 points (chirp-z)
-// 179 and 102.
-// Where a wave shares its factors (transforms side by side along a strided
-// axis) the tables cost nothing and the plain butterfly is as fast or faster:
-// 16 x 8001 transforms of 256 points 126 us, 135 like this.  The detection
-// chain (pulse compression, the pulse-axis pass) keeps the plain butterfly,
-// whose roundings decide cells on the threshold.
+// butterflies a +- f b.  A factor f = c -+ i s whose angle stays within pi/4 is
+// kept as (c, t = s/c), one between pi/4 and pi/2 as (s, k = c/s): u + i v =
+// b (1 -+ i t) or b (k -+ i) takes two fused multiply-adds and a +- c (u + i v)
+// four.  The factors that sweep more than that are kept as (c, s) and take
+// eight instructions: a tangent that grows towards pi/2 would overflow where
+// the transform does not.  A radix-16 butterfly is 32 of them, 224
+// instructions, where the plain butterfly takes 152 and its twiddle products
+// 60; each input is rounded by one operation less, and a row of factors is half
+// the size of a row of twiddles, which is what counts: 4096 rows of 4096 points
+// 57 us with table twiddles, 46 like this, 1024 of 16384 points 90 and 67, 8228
+// of 2039 points (chirp-z) 179 and 102.  Where a wave shares its factors
+// (transforms side by side along a strided axis) the tables cost nothing and
+// the plain butterfly is as fast or faster: 16 x 8001 transforms of 256 points
+// 126 us, 135 with factors.  The detection chain (pulse compression, the
+// pulse-axis pass) keeps the plain butterfly, whose roundings decide cells on
+// the threshold.
 //
 // The factors of one k (w_n = e^{-2 pi i/n}; the tree's other factors are
-// these times -i, a swap):
-//   R = 4:  w^2, w
-//   R = 8:  w^4, w^2; w, w w_8
-//   R = 16: w^8, w^4; w^2, w^2 w_8; w, w w_16; w w_8, w w_16^3
+// these times -i, a swap), with [0, pi) and [0, pi/2) swept by those in
+// brackets:
+//   R = 4:  (w^2), (w)
+//   R = 8:  (w^4), (w^2); w, w w_8
+//   R = 16: (w^8), (w^4); w^2, w^2 w_8; w, w w_16; w w_8, w w_16^3
 // stored two to a float4, group h of row k at [h * Ls + k], so that lanes with
-// neighbouring k read neighbouring 16-byte words.  All angles lie in [0, pi)
-// and only the first factor's reaches pi/2, where c is kept at TW_MIN_COS: the
-// factor is then off by that much, a sixteenth of a rounding.
-constexpr double TW_MIN_COS = 1.0 / (1 << 28);
+// neighbouring k read neighbouring 16-byte words.
+enum TwForm { TW_FULL, TW_TAN, TW_COT };
 
 template <int R>
 struct TwRow {
@@ -347,10 +347,25 @@ __device__ __forceinline__ TwRow<R> load_tw(const float4 *__restrict__ tw, int l
   return r;
 }
 
-// p = a + f b, m = a - f b; ROT: f times W_4 (-i forward, +i inverse)
-template <bool INV, bool ROT>
+// p = a + f b, m = a - f b, f kept as (c, t); ROT: f times W_4 (-i forward, +i
+// inverse)
+template <bool INV, bool ROT, TwForm F>
 __device__ __forceinline__ void tbf(float2 a, float2 b, float c, float t, float2 &p, float2 &m) {
-  const float u = fmaf(INV ? -t : t, b.y, b.x), v = fmaf(INV ? t : -t, b.x, b.y);
+  if constexpr (F == TW_FULL) {
+    const float2 u = make_float2(fmaf(INV ? -t : t, b.y, c * b.x), fmaf(INV ? t : -t, b.x, c * b.y));
+    const float2 r = ROT ? mul_w4<INV>(u) : u;
+    p = cadd(a, r);
+    m = csub(a, r);
+    return;
+  }
+  float u, v;
+  if constexpr (F == TW_TAN) {
+    u = fmaf(INV ? -t : t, b.y, b.x);
+    v = fmaf(INV ? t : -t, b.x, b.y);
+  } else {
+    u = fmaf(t, b.x, INV ? -b.y : b.y);
+    v = fmaf(t, b.y, INV ? b.x : -b.x);
+  }
   if constexpr (!ROT) {
     p = make_float2(fmaf(c, u, a.x), fmaf(c, v, a.y));
     m = make_float2(fmaf(-c, u, a.x), fmaf(-c, v, a.y));
@@ -365,19 +380,19 @@ __device__ __forceinline__ void tbf(float2 a, float2 b, float c, float t, float2
 
 // DFT_4 of (a0, f a1, f^2 a2, f^3 a3) in place; f^2 = (c2, t2), times W_4 with
 // ROT2, f = (c1, t1)
-template <bool INV, bool ROT2>
+template <bool INV, bool ROT2, TwForm F2, TwForm F1>
 __device__ __forceinline__ void dft4_tw(float2 &a0, float2 &a1, float2 &a2, float2 &a3, float c2, float t2,
                                         float c1, float t1) {
   float2 u0, u1, v0, v1;
-  tbf<INV, ROT2>(a0, a2, c2, t2, u0, u1);
-  tbf<INV, ROT2>(a1, a3, c2, t2, v0, v1);
-  tbf<INV, false>(u0, v0, c1, t1, a0, a2);
-  tbf<INV, true>(u1, v1, c1, t1, a1, a3);
+  tbf<INV, ROT2, F2>(a0, a2, c2, t2, u0, u1);
+  tbf<INV, ROT2, F2>(a1, a3, c2, t2, v0, v1);
+  tbf<INV, false, F1>(u0, v0, c1, t1, a0, a2);
+  tbf<INV, true, F1>(u1, v1, c1, t1, a1, a3);
 }
 
 template <bool INV>
 __device__ __forceinline__ void dft_tw(float2 (&a)[4], const TwRow<4> &w) {
-  dft4_tw<INV, false>(a[0], a[1], a[2], a[3], w.g[0].x, w.g[0].y, w.g[0].z, w.g[0].w);
+  dft4_tw<INV, false, TW_FULL, TW_FULL>(a[0], a[1], a[2], a[3], w.g[0].x, w.g[0].y, w.g[0].z, w.g[0].w);
 }
 
 template <bool INV>
@@ -386,12 +401,13 @@ __device__ __forceinline__ void dft_tw(float2 (&a)[8], const TwRow<8> &w) {
   // with w w_8^r
 #pragma unroll
   for (int q = 0; q < 2; ++q)
-    dft4_tw<INV, false>(a[q], a[q + 2], a[q + 4], a[q + 6], w.g[0].x, w.g[0].y, w.g[0].z, w.g[0].w);
+    dft4_tw<INV, false, TW_FULL, TW_FULL>(a[q], a[q + 2], a[q + 4], a[q + 6], w.g[0].x, w.g[0].y, w.g[0].z,
+                                          w.g[0].w);
   float2 y[8];
-  tbf<INV, false>(a[0], a[1], w.g[1].x, w.g[1].y, y[0], y[4]);
-  tbf<INV, false>(a[2], a[3], w.g[1].z, w.g[1].w, y[1], y[5]);
-  tbf<INV, true>(a[4], a[5], w.g[1].x, w.g[1].y, y[2], y[6]);
-  tbf<INV, true>(a[6], a[7], w.g[1].z, w.g[1].w, y[3], y[7]);
+  tbf<INV, false, TW_TAN>(a[0], a[1], w.g[1].x, w.g[1].y, y[0], y[4]);
+  tbf<INV, false, TW_COT>(a[2], a[3], w.g[1].z, w.g[1].w, y[1], y[5]);
+  tbf<INV, true, TW_TAN>(a[4], a[5], w.g[1].x, w.g[1].y, y[2], y[6]);
+  tbf<INV, true, TW_COT>(a[6], a[7], w.g[1].z, w.g[1].w, y[3], y[7]);
 #pragma unroll
   for (int i = 0; i < 8; ++i) a[i] = y[i];
 }
@@ -401,11 +417,12 @@ __device__ __forceinline__ void dft_tw(float2 (&a)[16], const TwRow<16> &w) {
   // 16 = 4 x 4: DFT_4 over inputs q + 4m with w^4, then over q with w w_16^r
 #pragma unroll
   for (int q = 0; q < 4; ++q)
-    dft4_tw<INV, false>(a[q], a[q + 4], a[q + 8], a[q + 12], w.g[0].x, w.g[0].y, w.g[0].z, w.g[0].w);
-  dft4_tw<INV, false>(a[0], a[1], a[2], a[3], w.g[1].x, w.g[1].y, w.g[2].x, w.g[2].y);
-  dft4_tw<INV, false>(a[4], a[5], a[6], a[7], w.g[1].z, w.g[1].w, w.g[2].z, w.g[2].w);
-  dft4_tw<INV, true>(a[8], a[9], a[10], a[11], w.g[1].x, w.g[1].y, w.g[3].x, w.g[3].y);
-  dft4_tw<INV, true>(a[12], a[13], a[14], a[15], w.g[1].z, w.g[1].w, w.g[3].z, w.g[3].w);
+    dft4_tw<INV, false, TW_FULL, TW_FULL>(a[q], a[q + 4], a[q + 8], a[q + 12], w.g[0].x, w.g[0].y, w.g[0].z,
+                                          w.g[0].w);
+  dft4_tw<INV, false, TW_TAN, TW_TAN>(a[0], a[1], a[2], a[3], w.g[1].x, w.g[1].y, w.g[2].x, w.g[2].y);
+  dft4_tw<INV, false, TW_COT, TW_TAN>(a[4], a[5], a[6], a[7], w.g[1].z, w.g[1].w, w.g[2].z, w.g[2].w);
+  dft4_tw<INV, true, TW_TAN, TW_COT>(a[8], a[9], a[10], a[11], w.g[1].x, w.g[1].y, w.g[3].x, w.g[3].y);
+  dft4_tw<INV, true, TW_COT, TW_COT>(a[12], a[13], a[14], a[15], w.g[1].z, w.g[1].w, w.g[3].z, w.g[3].w);
   float2 y[16];
 #pragma unroll
   for (int r = 0; r < 4; ++r)
@@ -421,6 +438,8 @@ void tw_factors(int R, int64_t Ls, int64_t k, float2 *out);
 // Per-device cache of factor tables keyed by (N, reversed?): Ls rows of R/2
 // factors per pass.
 const float2 *factors_device(int N, bool reversed_seq);
+// The same of one radix-16 pass with sub-length Ls.
+const float4 *factors16_device(int Ls);
 
 // Raw buffer access (MUBUF) for the block kernels: a resource covering
 // `bytes` bytes from `base`.  The hardware range check returns zeros for

@@ -128,10 +128,10 @@ __global__ __launch_bounds__(WgT<M>::NT) void pc_wgrad_kernel(WgArgs a) {
 // hold the x bins, the running product and one pass, so two workgroups share
 // a CU, each in another phase.  16 x 512 x 32768: 2610 us at one workgroup per
 // CU (242 VGPRs), 2207 with the two transforms side by side in one 1024-thread
-// workgroup (every wave waits at the same barriers), 2003 like this.
+// workgroup (every wave waits at the same barriers), 2040 like this.
 struct Wg8192Args {
   WgArgs a;
-  const float4 *bA, *bB, *bC;  // power-base rows of passes Ls = 2, 32, 512
+  const float4 *bA, *bB, *bC;  // factors of passes Ls = 2, 32, 512
 };
 
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
@@ -184,14 +184,14 @@ void wgrad8192_kernel(Wg8192Args p) {
     for (int h = 0; h < 2; ++h) {  // x, then gy
       fetch(it, h != 0, v);
       pair_dft2(v, (j & 1) != 0);
-      PowRow tw = load_pow(opaque(p.bA), j & 1);
-      pow_dft16<false>(v, tw);
-      tw = load_pow(opaque(p.bB), j & 31);
+      TwRow<16> tw = load_tw<16>(opaque(p.bA), 2, j & 1);
+      dft_tw<false>(v, tw);
+      tw = load_tw<16>(opaque(p.bB), 32, j & 31);
       xchg(2);
-      pow_dft16<false>(v, tw);
-      tw = load_pow(opaque(p.bC), j);
+      dft_tw<false>(v, tw);
+      tw = load_tw<16>(opaque(p.bC), 512, j);
       xchg(32);
-      pow_dft16<false>(v, tw);
+      dft_tw<false>(v, tw);
       if (h == 0) {
 #pragma unroll
         for (int q = 0; q < 16; ++q) X[q] = v[q];
@@ -325,7 +325,7 @@ static mxr_status wgrad_run(const WgradJob &j, hipStream_t s) {
     a.partial = ws;
     a.twf = twf;
     if (w8) {
-      Wg8192Args p{a, pow_base_device(8192, 2), pow_base_device(8192, 32), pow_base_device(8192, 512)};
+      Wg8192Args p{a, factors16_device(2), factors16_device(32), factors16_device(512)};
       MXR_REQUIRE(p.bA && p.bB && p.bC, MXR_OUT_OF_MEMORY,
                   "pc waveform gradient: twiddle table allocation failed");
       ProfScope ps("wgrad8192_kernel", s);

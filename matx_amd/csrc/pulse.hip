@@ -1174,7 +1174,8 @@ mxr_status pc_tables_prepare(int M, const char *fn) {
   bool ok = twiddles_device(M, false) && twiddles_device(M, true) && factors_device(M, false);
   if (M == 4096) ok = ok && pow_base_device(4096, 16) && pow_base_device(4096, 256);
   if (M == 8192)
-    ok = ok && pow_base_device(8192, 2) && pow_base_device(8192, 32) && pow_base_device(8192, 512);
+    ok = ok && pow_base_device(8192, 2) && pow_base_device(8192, 32) && pow_base_device(8192, 512) &&
+         factors16_device(2) && factors16_device(32) && factors16_device(512);
   MXR_REQUIRE(ok, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   return MXR_SUCCESS;
 }

@@ -123,19 +123,23 @@ void build_twiddles(int N, RadixSeq s, float2 *out) {
 }
 
 void tw_factors(int R, int64_t Ls, int64_t k, float2 *out) {
-  // exponent num/16 of w_R beside the power of w: w^pw w_16^num
+  // w^pw w_16^num, kept in form
   struct F {
     int pw, num;
+    TwForm form;
   };
-  static const F f4[] = {{2, 0}, {1, 0}}, f8[] = {{4, 0}, {2, 0}, {1, 0}, {1, 2}},
-                 f16[] = {{8, 0}, {4, 0}, {2, 0}, {2, 2}, {1, 0}, {1, 1}, {1, 2}, {1, 3}};
+  static const F f4[] = {{2, 0, TW_FULL}, {1, 0, TW_FULL}};
+  static const F f8[] = {{4, 0, TW_FULL}, {2, 0, TW_FULL}, {1, 0, TW_TAN}, {1, 2, TW_COT}};
+  static const F f16[] = {{8, 0, TW_FULL}, {4, 0, TW_FULL}, {2, 0, TW_TAN}, {2, 2, TW_COT},
+                          {1, 0, TW_TAN},  {1, 1, TW_TAN},  {1, 2, TW_COT}, {1, 3, TW_COT}};
   const F *f = R == 4 ? f4 : (R == 8 ? f8 : f16);
   const double two_pi = 6.283185307179586476925286766559;
   for (int i = 0; i < R / 2; ++i) {
     const double ang = two_pi * ((double)(f[i].pw * k) / (double)(Ls * R) + f[i].num / 16.0);
-    double c = std::cos(ang);
-    if (std::fabs(c) < TW_MIN_COS) c = TW_MIN_COS;
-    out[i] = make_float2((float)c, (float)(std::sin(ang) / c));
+    const double c = std::cos(ang), s = std::sin(ang);
+    out[i] = f[i].form == TW_FULL  ? make_float2((float)c, (float)s)
+             : f[i].form == TW_TAN ? make_float2((float)c, (float)(s / c))
+                                   : make_float2((float)s, (float)(c / s));
   }
 }
 
@@ -247,6 +251,18 @@ namespace {
 std::map<TwKey, float4 *> g_pb;
 }
 
+// Uploads a table built once per key (g_tw_mu held).
+static const float4 *upload_table(const TwKey &key, const std::vector<float4> &host) {
+  float4 *d = nullptr;
+  if (hipMalloc(&d, sizeof(float4) * host.size()) != hipSuccess) return nullptr;
+  if (hipMemcpy(d, host.data(), sizeof(float4) * host.size(), hipMemcpyHostToDevice) != hipSuccess) {
+    (void)hipFree(d);
+    return nullptr;
+  }
+  g_pb[key] = d;
+  return d;
+}
+
 const float4 *pow_base_device(int N, int Ls) {
   const int dev = device_id();
   std::lock_guard<std::mutex> g(g_tw_mu);
@@ -267,14 +283,18 @@ const float4 *pow_base_device(int N, int Ls) {
     host[2 * k] = make_float4(w[0].x, w[0].y, w[1].x, w[1].y);
     host[2 * k + 1] = make_float4(w[2].x, w[2].y, w[3].x, w[3].y);
   }
-  float4 *d = nullptr;
-  if (hipMalloc(&d, sizeof(float4) * host.size()) != hipSuccess) return nullptr;
-  if (hipMemcpy(d, host.data(), sizeof(float4) * host.size(), hipMemcpyHostToDevice) != hipSuccess) {
-    (void)hipFree(d);
-    return nullptr;
-  }
-  g_pb[key] = d;
-  return d;
+  return upload_table(key, host);
+}
+
+const float4 *factors16_device(int Ls) {
+  const int dev = device_id();
+  std::lock_guard<std::mutex> g(g_tw_mu);
+  TwKey key{dev, 16, Ls};
+  auto it = g_pb.find(key);
+  if (it != g_pb.end()) return it->second;
+  std::vector<float4> host((size_t)Ls * 4);
+  tw_pass(16, Ls, reinterpret_cast<float2 *>(host.data()));
+  return upload_table(key, host);
 }
 
 // Per (device, stream, tag) scratch buffers that only grow: partial sums of

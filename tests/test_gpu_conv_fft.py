@@ -221,3 +221,34 @@ def test_pulse_compress_in_place_rows(mx, S, L, n):
     mx.pulse_compress(buf[:, :S], w, n=n, out=out)
     assert rel(host(out), host(y)) < 1e-6
     assert np.array_equal(host(buf[:, S:]), host(x[:, S:]))
+
+
+@pytest.mark.parametrize("n", [32, 64, 128, 256, 512, 1024, 2048, 4096, 8192, 16384, 65536, 100, 29, 509, 2039])
+def test_fft_large_magnitudes(mx, n):
+    """Samples of 1e31: every intermediate of a transform is at most n times
+    that, far from the largest float, so nothing overflows on the way (both
+    directions, contiguous and strided, chirp-z and mixed radix too)."""
+    rng = np.random.default_rng(n)
+    x = (1e31 * (sig(rng, (3, n), True))).astype(np.complex64)
+    xs = np.ascontiguousarray(np.repeat(x[:, :, None], 5, axis=2))
+    for ref, f in ((np.fft.fft(x.astype(complex)), mx.fft), (np.fft.ifft(x.astype(complex)), mx.ifft)):
+        assert rel(host(f(dev(x), n)) / 1e31, ref / 1e31) < RTOL
+        assert rel(host(f(dev(xs), n, 1)) / 1e31, np.repeat(ref[:, :, None], 5, axis=2) / 1e31) < RTOL
+
+
+@pytest.mark.parametrize("N,L", [(20, 5), (300, 33), (3000, 500), (9000, 700), (20011, 210), (20011, 1300), (20011, 4001)])
+def test_conv_large_magnitudes(mx, N, L):
+    """The same for convolutions (one workgroup a row, overlap-save blocks) and
+    matched filters: signals of 1e31 under unit filters."""
+    rng = np.random.default_rng(N + L)
+    x, f = (1e31 * sig(rng, (2, N), True)).astype(np.complex64), sig(rng, (L,), True)
+    n = max(1024, 1 << (N + L - 1).bit_length())   # fft_conv's smallest transform
+    X = np.fft.fft(x.astype(complex) / 1e31, n)
+    full = np.fft.ifft(X * np.fft.fft(f.astype(complex), n))[:, :N + L - 1]
+    assert rel(host(mx.conv1d(dev(x), dev(f), "full", method="fft")) / 1e31, full) < RTOL
+    lags = np.fft.ifft(X * np.conj(np.fft.fft(f.astype(complex), n)))
+    assert rel(host(mx.fft_conv(dev(x), dev(f), n)) / 1e31, lags) < RTOL
+    buf = dev(x)
+    R = N - L + 1
+    mx.pulse_compress(buf, dev(f), n, window=False, normalize=False, out=buf[:, :R])
+    assert rel(host(buf[:, :R]) / 1e31, lags[:, :R]) < RTOL

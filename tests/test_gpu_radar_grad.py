@@ -284,3 +284,17 @@ def test_radar_gradient_sums_over_channels(mx):
     parts = sum(grad(Xd[c:c + 1]) for c in range(C))
     assert rel(g, parts) < 1e-5
     plan.close()
+
+
+@pytest.mark.parametrize("nd", [32, 64, 128, 256, 512, 1024])
+def test_doppler_large_magnitudes(mx, nd):
+    """Pulses of 1e31 through the pulse-axis pass (its map) and its adjoint: no
+    intermediate leaves the range of a float."""
+    rng = np.random.default_rng(nd)
+    y = (1e31 * crandn(rng, 2, nd, 37)).astype(np.complex64)
+    gp = rng.standard_normal((2, nd, 37)).astype(np.float32)
+    _, rd = mx.doppler(dev(y, torch.complex64), nd, tpc="none", want_rd=True, want_pow=False)
+    hw = hamming(nd)[None, :, None]
+    assert rel(host(rd) / 1e31, np.fft.fft(y.astype(complex) / 1e31 * hw, nd, axis=1)) < RTOL
+    gy = mx.ops.doppler_adjoint(dev(gp, torch.float32), dev(y, torch.complex64), nd, tpc="none")
+    assert rel(host(gy) / 1e31, np_doppler_adjoint(gp, y / 1e31, nd, "none", nd)) < RTOL
