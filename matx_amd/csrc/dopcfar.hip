@@ -184,6 +184,9 @@ void dopcfar_kernel(DcArgs a) {
         const int v0 = (rok ? r * 8 : DC_FAR) + pb * step;
 #pragma unroll
         for (int u = 0; u < SR + 2; ++u) v[u] = buf_load2(ry, v0 + u * step);
+      } else if (a.P == 0) {  // no pulse to clamp to
+#pragma unroll
+        for (int u = 0; u < SR + 2; ++u) v[u] = make_float2(0.f, 0.f);
       } else {
         const int rc = min(max(r, 0), a.R - 1);
 #pragma unroll

@@ -59,13 +59,16 @@ __device__ __forceinline__ void load_canceller(const A &a, int c, int r0, float2
     int off = pb * step + (r0 + t) * 8;
 #pragma unroll
     for (int u = 0; u < SR + 2; ++u, off += step) v[u] = buf_load2(ry, off);
-  } else {
+  } else if (a.P > 0) {
     const float2 *col = a.y + (int64_t)c * a.ys_c + (int64_t)min(r0 + t, a.R - 1) * a.ys_r;
 #pragma unroll
     for (int u = 0; u < SR + 2; ++u) {
       const int p = pb + u;
       v[u] = keep_if(col[(int64_t)min(max(p, 0), a.P - 1) * a.ys_p], p >= 0 && p < a.P);
     }
+  } else {  // no pulse to clamp to
+#pragma unroll
+    for (int u = 0; u < SR + 2; ++u) v[u] = make_float2(0.f, 0.f);
   }
 #pragma unroll
   for (int u = 0; u < SR; ++u) {

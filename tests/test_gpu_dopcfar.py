@@ -233,3 +233,20 @@ def test_pulse_compression_long_period(mx, L, log2n):
         y.append(host(plan(x)))
         plan.close()
     assert rel(y[1], y[0]) < RTOL
+
+
+@pytest.mark.parametrize("nd", [2, 8, 64, 256])
+def test_no_pulses(mx, nd):
+    """A cube without pulses (a null pointer) is a zero Doppler input: every
+    output is written, as zeros, and nothing is read."""
+    C, R = 2, 70
+    y = torch.empty((C, 0, R), dtype=torch.complex64, device="cuda")
+    pw = torch.full((C, nd, R), 7.0, device="cuda")
+    rd = torch.full((C, nd, R), 7.0, dtype=torch.complex64, device="cuda")
+    mx.doppler(y, nd, tpc="none", pw=pw, rd=rd)
+    assert not pw.any() and not rd.any()
+    pw, rd = mx.ops.doppler_taps(y, torch.empty(0, device="cuda"), nd, want_rd=True)
+    assert not pw.any() and not rd.any()
+    dets = torch.full((C, nd, R), 7, dtype=torch.int32, device="cuda")
+    dets, ba, pw = mx.doppler_cfar(y, nd, tpc="none", dets=dets, want_ba=True, want_pow=True)
+    assert not dets.any() and not pw.any() and not ba.any()
