@@ -313,8 +313,10 @@ void cfar_strip_kernel(CfarArgs a) {
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // wave -> (channel, band, strip), strips fastest: a workgroup's waves are
   // neighbours along the rows and meet in their halo columns
-  const uint32_t g = (uint32_t)xcd_remap(blockIdx.x, gridDim.x) * CS_NW + wv;
-  if (g >= (uint32_t)a.C * a.bands * a.strips) return;  // no barrier follows
+  const uint32_t waves = (uint32_t)a.C * a.bands * a.strips, groups = (waves + CS_NW - 1) / CS_NW;
+  if (block_id() >= groups) return;
+  const uint32_t g = (uint32_t)xcd_remap(block_id(), groups) * CS_NW + wv;
+  if (g >= waves) return;  // no barrier follows
   const int strip = (int)(g % a.strips), gb = (int)(g / a.strips);
   const int band = gb % a.bands, c = gb / a.bands;
   const int y0 = band * a.band_rows;
@@ -507,7 +509,7 @@ static mxr_status launch_cfar(CfarArgs a, hipStream_t s) {
       a.bands = (a.Ny + a.band_rows - 1) / a.band_rows;
       const int64_t G = (waves() + CS_NW - 1) / CS_NW;
       MXR_REQUIRE(G * CS_NW < (1ll << 31), MXR_INVALID_SIZE, "cfar: too many tiles");
-      const dim3 grid((unsigned)G);
+      const dim3 grid = linear_grid(G);
       ProfScope ps("cfar_strip_kernel", s);
       auto go = [&]<bool CIN>() {
         if (ex) wp ? cfar_strip_kernel<HY, HX, EY, EX, CIN, true, true><<<grid, dim3(CS_NT), 0, s>>>(a)

@@ -142,7 +142,9 @@ __global__ __launch_bounds__(DopCfg<ND>::NT) void doppler_kernel(DopArgs a) {
   __shared__ float2 lds[DopLayout<ND, DopCfg<ND>::TR>::LDS_ELEMS];
   __shared__ __align__(16) float win[ND];
   const uint32_t tiles = (uint32_t)(a.R + DopCfg<ND>::TR - 1) / DopCfg<ND>::TR;
-  const uint32_t g = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t G = (int64_t)tiles * a.C;
+  if (block_id() >= G) return;
+  const uint32_t g = (uint32_t)xcd_remap(block_id(), G);
   const uint32_t c = g / tiles;
   doppler_tile<ND>(a, (int)c, (int)(g - c * tiles) * DopCfg<ND>::TR, lds, win);
 }
@@ -242,7 +244,7 @@ static mxr_status launch_doppler(const DopArgs &a, hipStream_t s) {
   MXR_REQUIRE(G < (1ll << 31), MXR_INVALID_SIZE, "doppler: too many tiles");
   {
     ProfScope ps("doppler_kernel", s);
-    doppler_kernel<ND><<<dim3((unsigned)G), dim3(DopCfg<ND>::NT), 0, s>>>(a);
+    doppler_kernel<ND><<<linear_grid(G), dim3(DopCfg<ND>::NT), 0, s>>>(a);
   }
   MXR_HIP_TRY(hipGetLastError());
   return MXR_SUCCESS;
@@ -411,7 +413,9 @@ __global__ __launch_bounds__(DopAdjCfg<ND>::NT) void doppler_adj_kernel(DopGradA
   constexpr int K = SQ::n;
   __shared__ float2 lds[LY::LDS_ELEMS];  // the windowed canceller rows, then D, then gu
   __shared__ __align__(16) float win[ND];
-  const uint32_t g0 = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t G = (int64_t)a.tiles * a.C;
+  if (block_id() >= G) return;
+  const uint32_t g0 = (uint32_t)xcd_remap(block_id(), G);
   const int c = (int)(g0 / (uint32_t)a.tiles), tile = (int)(g0 - (uint32_t)c * (uint32_t)a.tiles);
   const int r0 = tile * TR;
   float *part = a.partial ? a.partial + ((int64_t)c * a.tiles + tile) * a.P : nullptr;
@@ -536,7 +540,8 @@ template <int ND>
 static mxr_status launch_doppler_adj(DopGradArgs a, const mxr_tensor *gtaps, hipStream_t s) {
   constexpr int TR = DopAdjCfg<ND>::TR;
   a.tiles = (a.R + TR - 1) / TR;
-  MXR_REQUIRE((int64_t)a.tiles * a.C < (1ll << 31), MXR_INVALID_SIZE, "doppler adjoint: too many tiles");
+  const int64_t G = (int64_t)a.tiles * a.C;
+  MXR_REQUIRE(G < (1ll << 31), MXR_INVALID_SIZE, "doppler adjoint: too many tiles");
   a.partial = nullptr;
   if (gtaps) {
     a.partial = (float *)stream_workspace("doppler_taps_partial",
@@ -545,7 +550,7 @@ static mxr_status launch_doppler_adj(DopGradArgs a, const mxr_tensor *gtaps, hip
   }
   {
     ProfScope ps("doppler_adj_kernel", s);
-    doppler_adj_kernel<ND><<<dim3((unsigned)(a.tiles * a.C)), dim3(DopAdjCfg<ND>::NT), 0, s>>>(a);
+    doppler_adj_kernel<ND><<<linear_grid(G), dim3(DopAdjCfg<ND>::NT), 0, s>>>(a);
   }
   MXR_HIP_TRY(hipGetLastError());
   if (gtaps) {

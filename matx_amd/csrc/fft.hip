@@ -310,6 +310,7 @@ struct MixPass {
 struct MixArgs {
   FftArgs f;
   int n, np, TB, lgTB;
+  int64_t groups;  // workgroups
   int pad, row;  // 1 when R0 is even; elements of a row in LDS
   const float2 *tw;
   MixPass p[MIX_MAX_PASSES];
@@ -473,7 +474,8 @@ __global__ __launch_bounds__(1024) void fft_mixed_kernel(MixArgs z) {
   extern __shared__ float2 mix_lds[];
   __shared__ int64_t base_in[MIX_MAX_TB], base_out[MIX_MAX_TB];
   const FftArgs &a = z.f;
-  const int64_t t0 = (COL ? xcd_remap(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x) * z.TB;
+  if (block_id() >= z.groups) return;
+  const int64_t t0 = (COL ? xcd_remap(block_id(), z.groups) : block_id()) * z.TB;
   for (int t = threadIdx.x; t < z.TB; t += blockDim.x) {
     int64_t oi = 0, oo = 0;
     if (t0 + t < a.nbatch) {
@@ -610,10 +612,11 @@ static mxr_status launch_mixed(MixArgs z, const FftArgs &f, bool inv, hipStream_
   z.TB = TB;
   const int64_t grid = (f.nbatch + TB - 1) / TB;
   MXR_REQUIRE(grid <= 0x7fffffff, MXR_INVALID_SIZE, "fft: batch too large");
+  z.groups = grid;
   const int nt = (TB * nb + 63) / 64 * 64;
   const size_t shm = sizeof(float2) * (size_t)TB * z.row;
   ProfScope ps("fft_mixed_kernel", s);
-  const dim3 g((unsigned)grid), b((unsigned)nt);
+  const dim3 g = linear_grid(grid), b((unsigned)nt);
   if (col && inv) fft_mixed_kernel<true, true><<<g, b, shm, s>>>(z);
   else if (col) fft_mixed_kernel<false, true><<<g, b, shm, s>>>(z);
   else if (inv) fft_mixed_kernel<true, false><<<g, b, shm, s>>>(z);

@@ -147,6 +147,16 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t g, int64_t G) {
   return (g % NX) * q + g / NX;
 }
 
+// A grid of G workgroups of up to 1024 threads: the launch counts a dimension's
+// threads in 32 bits (and silently runs what is left modulo 2^32), so long ones
+// fold into rows.  block_id() is the workgroup's number; those from G on, in the
+// last row, have nothing to do.
+inline dim3 linear_grid(int64_t G) {
+  constexpr int64_t ROW = 1 << 21;
+  return G <= ROW ? dim3((unsigned)G) : dim3((unsigned)ROW, (unsigned)((G + ROW - 1) / ROW));
+}
+__device__ __forceinline__ int64_t block_id() { return (int64_t)blockIdx.y * gridDim.x + blockIdx.x; }
+
 int device_id();
 int cu_count();  // compute units of the current device (cached)
 int max_lds_per_block();

@@ -323,8 +323,9 @@ __global__ __launch_bounds__(256) void pc_ols_multi_row_kernel(PcArgs a) {
   constexpr int TB = 4096 / M;
   __shared__ float2 lds[Layout<M, TB, false>::LDS_ELEMS];
   __shared__ OlsBlock obs[TB];
+  if (block_id() >= a.groups) return;
   int64_t ox, oy;
-  batch_offsets(a.bi, xcd_remap(blockIdx.x, a.groups), &ox, &oy);
+  batch_offsets(a.bi, xcd_remap(block_id(), a.groups), &ox, &oy);
   for (int64_t b0 = 0; b0 < a.nblk; b0 += TB) {
     if (b0) wg_barrier();  // the last step's reads of obs and lds are done
     if (threadIdx.x < TB) {
@@ -1140,7 +1141,7 @@ mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
     ProfScope ps("pc_ols_kernel", s);
     if constexpr (M <= 2048) {
       constexpr int TB = 4096 / M;
-      if (pa->bpw > 1) pc_ols_multi_row_kernel<M><<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(*pa);
+      if (pa->bpw > 1) pc_ols_multi_row_kernel<M><<<linear_grid(pa->groups), dim3(256), 0, s>>>(*pa);
       else pc_ols_multi_kernel<M><<<dim3((unsigned)((pa->groups + TB - 1) / TB)), dim3(256), 0, s>>>(*pa);
     } else if (pa->bpw > 1) {
       pc_ols_kernel<M, true><<<dim3((unsigned)pa->groups), dim3(PcCfg<M>::NT), 0, s>>>(*pa);

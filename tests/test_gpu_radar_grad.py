@@ -298,3 +298,20 @@ def test_doppler_large_magnitudes(mx, nd):
     assert rel(host(rd) / 1e31, np.fft.fft(y.astype(complex) / 1e31 * hw, nd, axis=1)) < RTOL
     gy = mx.ops.doppler_adjoint(dev(gp, torch.float32), dev(y, torch.complex64), nd, tpc="none")
     assert rel(host(gy) / 1e31, np_doppler_adjoint(gp, y / 1e31, nd, "none", nd)) < RTOL
+
+
+def test_doppler_launch_past_32_bit_threads(mx):
+    """More range tiles than a launch dimension counts threads for (2^32 over
+    256 a workgroup): every tile of the pulse-axis pass and of its adjoint
+    runs, the first and the last included."""
+    C, R = 32768, 16416   # 513 tiles of 32 bins a channel
+    y = torch.zeros((C, 1, R), dtype=torch.complex64, device="cuda")
+    y[0, 0, 0], y[C - 1, 0, R - 1] = 2, 3
+    pw = torch.full((C, 2, R), 5.0, device="cuda")
+    mx.doppler(y, 2, tpc="none", pw=pw)
+    assert float(pw[0, 1, 0]) == 4 and float(pw[C - 1, 1, R - 1]) == 9
+    assert int(torch.count_nonzero(pw)) == 4
+    gy = torch.full_like(y, 5)
+    mx.ops.doppler_adjoint(torch.ones(1, 1, 1, device="cuda").expand(C, 2, R), y, 2, tpc="none", gy=gy)
+    assert gy[0, 0, 0] == 8 and gy[C - 1, 0, R - 1] == 12    # 2 sum_k conj(F) F y
+    assert int(torch.count_nonzero(gy)) == 2
