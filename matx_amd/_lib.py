@@ -84,6 +84,23 @@ class mxr_cfar_params(ctypes.Structure):
                 ("pfa", ctypes.c_float)]
 
 
+_TENSOR_SIZE = ctypes.sizeof(mxr_tensor)
+_TENSOR_PTR = ctypes.POINTER(mxr_tensor)
+
+
+class _TensorArg:
+    """The argument type `const mxr_tensor *`: the packed bytes arg() makes, or
+    what POINTER(mxr_tensor) takes (an mxr_tensor, a reference to one, None)."""
+
+    @staticmethod
+    def from_param(v):
+        if type(v) is bytes:
+            if len(v) != _TENSOR_SIZE:
+                raise TypeError(f"expected an mxr_tensor of {_TENSOR_SIZE} bytes, got {len(v)}")
+            return v
+        return _TENSOR_PTR.from_param(v)
+
+
 _lib = None
 
 
@@ -108,7 +125,8 @@ def lib():
             f"{LIB_PATH} is missing: build the HIP library with "
             "`python -m matx_amd.build` (there is no CPU fallback)")
     L = ctypes.CDLL(LIB_PATH)
-    T = V = ctypes.c_void_p  # an mxr_tensor as bytes (arg), by reference, or None
+    T = _TensorArg
+    V = ctypes.c_void_p
     I64 = ctypes.c_int64
     I = ctypes.c_int
     L.mxr_last_error.restype = ctypes.c_char_p
@@ -236,11 +254,11 @@ def arg(t):
         return None
     dt = _DTYPES.get(t.dtype)
     if dt is None:
-        if not _DTYPES:
-            import torch
-            _DTYPES.update({torch.complex64: C64, torch.float32: F32, torch.int32: I32})
-            return arg(t)
-        raise MatxError(6, f"unsupported dtype {t.dtype}")
+        import torch
+        _DTYPES.update({torch.complex64: C64, torch.float32: F32, torch.int32: I32})
+        dt = _DTYPES.get(t.dtype)
+        if dt is None:
+            raise MatxError(6, f"unsupported dtype {t.dtype}")
     r = t.dim()
     if r > MXR_MAX_RANK:
         raise MatxError(3, f"rank {r} > {MXR_MAX_RANK}")

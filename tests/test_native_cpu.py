@@ -384,3 +384,20 @@ def test_packed_descriptor(L, shape):
         for f in (L.arg, L.desc):
             with pytest.raises(L.MatxError):
                 f(bad)
+
+
+def test_tensor_argument_types(L):
+    """A tensor argument is packed bytes of the structure's size, an mxr_tensor,
+    a reference to one, or None; anything else is refused before the call."""
+    torch = pytest.importorskip("torch")
+    lib = L.lib()
+    x = torch.zeros((2, 8), dtype=torch.complex64)
+    good = L.arg(x)
+    assert len(good) == ctypes.sizeof(L.mxr_tensor)
+    for t in (good, L.desc(x), L.ref(L.desc(x)), ctypes.pointer(L.desc(x)), None):
+        # a transform of no points: refused by the library itself
+        assert lib.mxr_fft_c2c(t, t, -1, 0, 0, 0, None) != 0
+    for bad in (good[:-1], good + b"\0", b"", 0, 4096, ctypes.c_void_p(0), "x", L.mxr_cfar_params(), [good]):
+        for args in ((bad, good), (good, bad)):
+            with pytest.raises(ctypes.ArgumentError):
+                lib.mxr_fft_c2c(*args, 8, 0, 0, 0, None)
