@@ -252,3 +252,31 @@ def test_conv_large_magnitudes(mx, N, L):
     R = N - L + 1
     mx.pulse_compress(buf, dev(f), n, window=False, normalize=False, out=buf[:, :R])
     assert rel(host(buf[:, :R]) / 1e31, lags[:, :R]) < RTOL
+
+
+@pytest.mark.parametrize("n", [7, 11, 29, 59, 101, 251, 509, 1021, 2039, 4093, 8191])
+@pytest.mark.parametrize("cols", [1, 15])
+def test_fft_chirp_z_lengths(mx, n, cols):
+    """Primes, one for every convolution length of the chirp-z kernels (16 to
+    16384 points): contiguous and strided, both directions, real in and out."""
+    test_fft_axes_direct(mx, n, cols)
+
+
+@pytest.mark.parametrize("L", [700, 3000])   # blocks of 4096 and 8192 points
+@pytest.mark.parametrize("over", [0, 1])
+def test_conv1d_longest_rows(mx, L, over):
+    """FULL outputs of rows that just fit a period of 2^27 samples, the largest
+    of the block kernels' 32-bit byte offsets, and of rows one longer (general
+    addressing): the first blocks start before the row, the last end past it.
+    Noise at either end of the row, zeros between."""
+    rng = np.random.default_rng(L)
+    N, K = (1 << 27) - L + 1 + over, 5000
+    a, b, f = sig(rng, (K,), True), sig(rng, (K,), True), sig(rng, (L,), True)
+    x = torch.zeros((1, N), dtype=torch.complex64, device="cuda")
+    x[0, :K], x[0, N - K:] = dev(a), dev(b)
+    y = mx.conv1d(x, dev(f), "full", method="fft")
+    f64 = lambda u: np.fft.fft(u.astype(complex), 16384)  # noqa: E731
+    lo, hi = (np.fft.ifft(f64(u) * f64(f))[:K + L - 1] for u in (a, b))
+    assert rel(host(y[0, :K + L - 1]), lo) < RTOL
+    assert rel(host(y[0, N - K:]), hi) < RTOL
+    assert not y[0, K + L + 16384:N - K - 16384].any()

@@ -219,9 +219,11 @@ def test_pulse_compression_wrapping_blocks(mx, S, L, n, C):
 @pytest.mark.parametrize("L", [700, 3000])
 @pytest.mark.parametrize("log2n", [27, 28])
 def test_pulse_compression_long_period(mx, L, log2n):
-    """The largest period of the block kernels' 32-bit byte offsets and the one
-    past it (the general kernel), on short rows: both give the lags of a short
-    period that already covers every nonzero one."""
+    """A period of 2^27 samples (the block kernels) and one past it (the general
+    kernel) on short rows, blocks that start in the row: both give the lags of
+    a short period that already covers every nonzero one.  Blocks at the far
+    end of such a period, where the offsets are large: test_long_period_ends
+    and test_conv1d_longest_rows."""
     rng = np.random.default_rng(L)
     S, nout = 9001, 9001 - L + 1
     x = dev((rng.standard_normal((2, S)) + 1j * rng.standard_normal((2, S))).astype(np.complex64))
@@ -250,3 +252,21 @@ def test_no_pulses(mx, nd):
     dets = torch.full((C, nd, R), 7, dtype=torch.int32, device="cuda")
     dets, ba, pw = mx.doppler_cfar(y, nd, tpc="none", dets=dets, want_ba=True, want_pow=True)
     assert not dets.any() and not pw.any() and not ba.any()
+
+
+@pytest.mark.parametrize("L", [64, 200, 700, 3000])   # blocks of 1024, 2048, 4096, 8192
+@pytest.mark.parametrize("log2n", [27, 28])
+def test_long_period_ends(mx, L, log2n):
+    """All n lags of a short row: the last blocks run past the period, at byte
+    offsets up to 2^30 (the largest the block kernels take) and past it (the
+    general addressing).  First lags, wrapped (negative) lags and the zeros
+    between them are those of a short period."""
+    rng = np.random.default_rng(L)
+    S, n = 9001, 1 << log2n
+    x = dev((rng.standard_normal((1, S)) + 1j * rng.standard_normal((1, S))).astype(np.complex64))
+    w = dev((rng.standard_normal(L) + 1j * rng.standard_normal(L)).astype(np.complex64))
+    short = host(mx.fft_conv(x, w, 16384))
+    y = mx.fft_conv(x, w, n)
+    assert rel(host(y[:, :S]), short[:, :S]) < RTOL
+    assert rel(host(y[:, n - L + 1:]), short[:, 16384 - L + 1:]) < RTOL
+    assert not y[:, S + 16384:n - L - 16384].any()

@@ -648,3 +648,40 @@ def test_sum(mx):
     r = rng.standard_normal((7, 333)).astype(np.float32)
     sr = host(E.sum(dev(r, torch.float32)[:, ::2]))
     assert abs(sr - r[:, ::2].astype(np.float64).sum()) < 1e-4 * np.abs(r).sum()
+
+
+@pytest.mark.parametrize("win,guard", [((5, 13), (3, 3)), ((7, 21), (3, 5))])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_cfar_strips_not_finite(mx, win, guard, cplx):
+    """Infinities, NaN and the largest and smallest floats in the map, at
+    corners, edges and inside: the strip kernel gives the register-only
+    kernel's bits (columns two apart take it), an average is NaN where a
+    training cell is, and a NaN average or cell detects nothing."""
+    rng = np.random.default_rng(win[0])
+    C, Ny, Nx = 2, 140, 517
+    m = np.abs(rng.standard_normal((C, Ny, Nx))).astype(np.float32)
+    special = [np.inf, np.nan, np.finfo(np.float32).max, np.finfo(np.float32).tiny, 0.0]
+    spots = [(0, 0), (0, Nx - 1), (Ny - 1, 0), (Ny - 1, Nx - 1), (70, 255), (63, 240), (64, 31), (100, 300)]
+    for i, (y, x) in enumerate(spots):
+        m[i % C, y, x] = special[i % 2]
+        m[(i + 1) % C, y, x] = special[2 + i % 3]
+    src = np.sqrt(m).astype(np.complex64) if cplx else m
+    dt = torch.complex64 if cplx else torch.float32
+    wide = torch.zeros((C, Ny, Nx, 2), dtype=dt, device="cuda")
+    wide[..., 0] = dev(src, dt)
+    args = dict(win=win, guard=guard, pfa=1e-2, want_ba=True)
+    dets, ba, _ = mx.cfar(dev(src, dt), **args)
+    dets2, ba2, _ = mx.cfar(wide[..., 0], **args)
+    assert torch.equal(dets, dets2)
+    assert torch.equal(ba.view(torch.int32)[~ba.isnan()], ba2.view(torch.int32)[~ba2.isnan()])
+    assert torch.equal(ba.isnan(), ba2.isnan())
+    bad = np.zeros((C, Ny, Nx), bool)
+    nan = np.isnan(m)
+    for dy in range(-(win[0] // 2), win[0] // 2 + 1):
+        for dx in range(-(win[1] // 2), win[1] // 2 + 1):
+            if abs(dy) <= guard[0] // 2 and abs(dx) <= guard[1] // 2:
+                continue
+            y0, y1, x0, x1 = max(0, -dy), Ny - max(0, dy), max(0, -dx), Nx - max(0, dx)
+            bad[:, y0:y1, x0:x1] |= nan[:, y0 + dy:y1 + dy, x0 + dx:x1 + dx]
+    assert np.array_equal(host(ba.isnan()), bad)
+    assert not host(dets)[bad | nan].any()

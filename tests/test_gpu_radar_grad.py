@@ -315,3 +315,17 @@ def test_doppler_launch_past_32_bit_threads(mx):
     mx.ops.doppler_adjoint(torch.ones(1, 1, 1, device="cuda").expand(C, 2, R), y, 2, tpc="none", gy=gy)
     assert gy[0, 0, 0] == 8 and gy[C - 1, 0, R - 1] == 12    # 2 sum_k conj(F) F y
     assert int(torch.count_nonzero(gy)) == 2
+
+
+@pytest.mark.parametrize("L", [700, 3000])   # blocks of 4096 and 8192 points
+@pytest.mark.parametrize("log2n", [27, 28])
+def test_pc_waveform_grad_long_period(mx, L, log2n):
+    """Periods of 2^27 samples (the dedicated 8192-point kernel) and past it
+    (the general kernel): the gradient is that of a short period."""
+    rng = np.random.default_rng(L)
+    S, R = 9001, 9001 - L + 1
+    x, gy, w = crandn(rng, 3, S), crandn(rng, 3, R), crandn(rng, L)
+    plan = mx.ops.PulseCompressionPlan(S, L, 1 << log2n, R)
+    plan.set_waveform(dev(w))
+    assert rel(host(plan.waveform_grad(dev(gy), dev(x), dev(w))), np_waveform_grad(gy, x, w, 16384)) < RTOL
+    plan.close()
