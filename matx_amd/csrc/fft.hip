@@ -1,14 +1,18 @@
 // Generic batched 1-D C2C FFT over arbitrary strided views
 // (replaces fft_impl/ifft_impl, include/matx/transforms/fft/fft_cuda.h:680-774).
 //
-// One workgroup owns TB whole transforms in LDS: a gather phase reads them
-// with the view's strides (zero-padding or truncating to n, the size rule of
-// include/matx/transforms/fft/fft_common.h:39-140), the Stockham passes run
-// LDS->LDS, and a scatter phase writes the output view with the norm scale
-// folded in (fft_cuda.h:126-188 does it as a separate pass).  When the
-// innermost batch dim has unit stride (an FFT along a strided axis, e.g. the
-// pulse axis of a permuted view) the gather/scatter walk that dim fastest so
-// HBM accesses stay coalesced.
+// One workgroup owns TB whole transforms.  The first Stockham pass loads its
+// butterflies' inputs from memory with the view's strides (zero-padding or
+// truncating to n, the size rule of
+// include/matx/transforms/fft/fft_common.h:39-140), the passes between run
+// LDS->LDS, and the last one stores to the output view with the norm scale
+// folded in (fft_cuda.h:126-188 does it as a separate pass); contiguous rows
+// under 256 points are gathered into and scattered from LDS instead, whole rows
+// at a time.  When the innermost batch dim has unit stride (an FFT along a
+// strided axis, e.g. the pulse axis of a permuted view) lanes walk that dim so
+// HBM accesses stay coalesced.  Sizes: powers of two up to 16384 by
+// fft_generic_kernel, sizes with factors 2, 3 and 5 by fft_mixed_kernel, others
+// up to 8192 by czt_kernel, larger ones in several launches (fft_big_kernel).
 #include <algorithm>
 #include <cmath>
 #include <complex>
@@ -567,7 +571,11 @@ static const float2 *mix_tables(int n, const MixArgs &z) {
 }
 
 // Fills the passes of an n-point transform; false for sizes left to Bluestein:
-// a factor outside MIX_RADIX, one pass only, or more than a workgroup holds.
+// a factor outside MIX_RADIX, one pass only, or more than a workgroup holds at
+// one butterfly a thread (1024) and 8000 elements (64000 bytes; a kernel's LDS
+// without opting in is 64 KiB and the rows' offsets take 1 KiB).  Of the sizes
+// with factors 2, 3 and 5 from 24 to 8192 these are 5625, 6075, 6250, 6750,
+// 7290, 7500, 7776, 8000 and 8100.
 static bool mix_plan(int64_t n, MixArgs &z) {
   if (n < MIX_MIN_N || n > 8192) return false;
   MixSeq cur, best;
@@ -597,6 +605,14 @@ static mxr_status launch_mixed(MixArgs z, const FftArgs &f, bool inv, hipStream_
   MXR_REQUIRE(z.tw != nullptr, MXR_OUT_OF_MEMORY, "fft: table allocation failed for size %d", z.n);
   const int Rmin = z.p[z.np - 1].R, nb = z.n / Rmin;
   const bool col = f.batch_fast && z.row <= 4096 && 2 * nb <= 1024;
+  // Transforms per workgroup.  Along a strided axis as many (a power of two)
+  // as 1024 threads and 8000 elements hold: their rows are the memory's runs.
+  // 1000 points 43.6 us, 73 with a quarter of the elements; 1500 points 53 and
+  // 75; 360 points would rather have 256 threads (45 and 36).  Contiguous ones
+  // fill 512 threads and 5632 elements (three workgroups' LDS a CU): 256
+  // threads are 0 to 13 % faster on 8 Mi elements, 1024 up to 33 % slower,
+  // 2816 to 8000 elements within 8 %; and no more than leave two workgroups a
+  // CU (300 rows of 1000 points 7.0 us, in one workgroup's worth each 7.9).
   int TB = 1;
   z.lgTB = 0;
   if (col) {
@@ -606,7 +622,6 @@ static mxr_status launch_mixed(MixArgs z, const FftArgs &f, bool inv, hipStream_
     }
   } else {
     TB = std::max(1, std::min({512 / nb, 5632 / z.row, MIX_MAX_TB}));
-    // few transforms: rather more workgroups
     TB = (int)std::min<int64_t>(TB, std::max<int64_t>(1, f.nbatch / 512));
   }
   z.TB = TB;

@@ -159,6 +159,5 @@ __device__ __forceinline__ int64_t block_id() { return (int64_t)blockIdx.y * gri
 
 int device_id();
 int cu_count();  // compute units of the current device (cached)
-int max_lds_per_block();
 
 }  // namespace mxr

@@ -87,19 +87,6 @@ int cu_count() {
   return v;
 }
 
-int max_lds_per_block() {
-  static std::mutex mu;
-  static std::map<int, int> cache;
-  std::lock_guard<std::mutex> g(mu);
-  int d = device_id();
-  auto it = cache.find(d);
-  if (it != cache.end()) return it->second;
-  int v = 65536;
-  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, d) != hipSuccess) v = 65536;
-  cache[d] = v;
-  return v;
-}
-
 void build_twiddles(int N, RadixSeq s, float2 *out) {
   const double two_pi = 6.283185307179586476925286766559;
   int64_t Ls = 1;
