@@ -237,6 +237,15 @@ int doppler_batch_tile(int nd) {
   return 0;
 }
 
+// The tables of an nd-point pass and of its adjoint, built together, so that
+// after either call the other one's first can be captured.
+static bool doppler_tables(int nd, const float2 **tw, const float2 **fwd, const float2 **inv) {
+  *tw = twiddles_device(nd, false);
+  *fwd = factors_device(nd, false);
+  *inv = factors_device(nd, true);
+  return *tw && *fwd && *inv;
+}
+
 template <int ND>
 static mxr_status launch_doppler(const DopArgs &a, hipStream_t s) {
   constexpr int TR = DopCfg<ND>::TR;
@@ -320,8 +329,9 @@ static mxr_status doppler_run(const mxr_tensor *pow_out, const mxr_tensor *rd_ou
   a.y32 = rows32(P, R, y->stride[1], y->stride[2], 8);
   a.out32 = (!rd_out || rows32(nd, R, rd_out->stride[1], rd_out->stride[2], 8)) &&
             (!pow_out || rows32(nd, R, pow_out->stride[1], pow_out->stride[2], 4));
-  a.tw = twiddles_device((int)nd, false);
-  MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "doppler: twiddle table allocation failed");
+  const float2 *fwd, *inv;
+  MXR_REQUIRE(doppler_tables((int)nd, &a.tw, &fwd, &inv), MXR_OUT_OF_MEMORY,
+              "doppler: twiddle table allocation failed");
   switch (nd) {
     case 2: return launch_doppler<2>(a, stream);
     case 4: return launch_doppler<4>(a, stream);
@@ -563,9 +573,9 @@ static mxr_status launch_doppler_adj(DopGradArgs a, const mxr_tensor *gtaps, hip
 }
 
 static mxr_status dispatch_doppler_adj(int64_t nd, DopGradArgs a, const mxr_tensor *gtaps, hipStream_t s) {
-  a.tw = factors_device((int)nd, false);
-  a.twi = factors_device((int)nd, true);
-  MXR_REQUIRE(a.tw && a.twi, MXR_OUT_OF_MEMORY, "doppler adjoint: twiddle table allocation failed");
+  const float2 *plain;
+  MXR_REQUIRE(doppler_tables((int)nd, &plain, &a.tw, &a.twi), MXR_OUT_OF_MEMORY,
+              "doppler adjoint: twiddle table allocation failed");
   a.y32 = rows32(a.P, a.R, a.ys_p, a.ys_r, 8);
   a.gp32 = rows32(nd, a.R, a.gs_k, a.gs_r, 4);
   a.gy32 = a.gy && rows32(a.P, a.R, a.gys_p, a.gys_r, 8);

@@ -1398,7 +1398,11 @@ static mxr_status fft_impl(const char *fn, const mxr_tensor *out, const mxr_tens
   if (!pow2 && mix_plan(n, z)) return launch_mixed(z, a, inv, stream);
   if (!pow2) return n <= CZT_MAX_N ? dispatch_czt(n, a, inv, stream) : dispatch_czt_big(n, a, inv, stream);
   if (n > 16384) return dispatch_big(n, a, inv, stream);
-  a.tw = a.batch_fast && n < 4096 ? twiddles_device((int)n, false) : factors_device((int)n, false);
+  a.tw = factors_device((int)n, false);
+  if (n < 4096) {  // both forms, so that after one axis the other's first call can be captured
+    const float2 *plain = twiddles_device((int)n, false);
+    if (a.batch_fast || !plain) a.tw = plain;
+  }
   MXR_REQUIRE(a.tw != nullptr, MXR_OUT_OF_MEMORY, "%s: twiddle table allocation failed", fn);
   return dispatch_generic(n, a, inv, stream);
 }

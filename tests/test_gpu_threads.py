@@ -101,3 +101,37 @@ def test_raw_stream_is_the_current_stream():
     with torch.cuda.stream(s):
         assert L.raw_stream() == s.cuda_stream == L.stream_handle().value
     assert L.raw_stream(s) == s.cuda_stream
+
+
+@pytest.mark.parametrize("first", ["forward", "backward"])
+def test_sibling_call_captures_without_a_warm_up(first):
+    """After one of a pair of calls (pulse-axis pass and adjoint, a transform
+    along either axis) the other's first call of the size can be captured: the
+    pair's tables are built together."""
+    import matx_amd as mx
+    import matx_amd._lib as L
+    L.check(L.lib().mxr_clear_caches())
+    g = torch.Generator(device="cuda").manual_seed(3)
+    y = torch.randn((2, 64, 100), dtype=torch.complex64, device="cuda", generator=g)
+    gp = torch.randn((2, 64, 100), device="cuda", generator=g)
+    yt = y.transpose(1, 2).contiguous()
+    pw, gy, rt, c = torch.empty_like(gp), torch.empty_like(y), torch.empty_like(yt), torch.empty_like(y)
+    pair = [(lambda: mx.doppler(y, 64, pw=pw), lambda: mx.ops.doppler_adjoint(gp, y, 64, gy=gy)),
+            (lambda: mx.fft(y, 64, 1, out=c), lambda: mx.fft(yt, 64, 2, out=rt))]
+    for fwd, bwd in pair:
+        warm, cold = (fwd, bwd) if first == "forward" else (bwd, fwd)
+        warm()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            cold()
+        for t in (pw, gy, rt, c):
+            t.fill_(-1)
+        for _ in range(3):
+            graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in (pw, gy, rt, c)]
+        for t in (pw, gy, rt, c):
+            t.fill_(-1)
+        cold()
+        assert all(torch.equal(u, v) for u, v in zip(got, (pw, gy, rt, c)))
