@@ -441,6 +441,29 @@ const float2 *factors_device(int N, bool reversed_seq);
 // The same of one radix-16 pass with sub-length Ls.
 const float4 *factors16_device(int Ls);
 
+// The twiddled radix-16 butterflies of a block kernel's passes: power-base rows,
+// or folded factors.
+template <bool FOLD>
+struct Row16 {
+  using T = PowRow;
+  __device__ static __forceinline__ T load(const float4 *tab, int, int k) { return load_pow(tab, k); }
+  __device__ static __forceinline__ void pin(T &r) { pin_row(r); }
+  template <bool INV, bool TAIL = false>
+  __device__ static __forceinline__ void dft(float2 (&v)[16], const T &w) {
+    pow_dft16<INV, TAIL>(v, w);
+  }
+};
+template <>
+struct Row16<true> {
+  using T = TwRow<16>;
+  __device__ static __forceinline__ T load(const float4 *tab, int ls, int k) { return load_tw<16>(tab, ls, k); }
+  __device__ static __forceinline__ void pin(T &) {}
+  template <bool INV, bool TAIL = false>
+  __device__ static __forceinline__ void dft(float2 (&v)[16], const T &w) {
+    dft_tw<INV>(v, w);
+  }
+};
+
 // Raw buffer access (MUBUF) for the block kernels: a resource covering
 // `bytes` bytes from `base`.  The hardware range check returns zeros for
 // loads at offsets at or past `bytes` and drops such stores, so a block that

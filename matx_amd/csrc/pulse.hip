@@ -42,6 +42,7 @@ struct PcArgs {
   int64_t bpw;      // blocks per workgroup (nblk when y aliases x)
   int64_t groups;   // total workgroups
   int64_t shift;    // outputs start at lag -shift (samples before the row are zero)
+  int fold;         // 4096 and 8192 points: folded factors (long convolutions)
   const float2 *wc; // M-point waveform spectrum, scaled by 1/M
   const float2 *twf, *twi;
 };
@@ -368,8 +369,8 @@ void pc_ols_kernel(PcArgs a) {
 // radix-16 butterfly per thread per pass).
 struct Pc4096Args {
   PcArgs a;
-  const float4 *base1;  // power-base rows of pass Ls = 16
-  const float4 *base2;  // power-base rows of pass Ls = 256
+  const float4 *base1;  // power-base rows (FOLD: factors) of pass Ls = 16
+  const float4 *base2;  // and of pass Ls = 256
 };
 
 
@@ -384,7 +385,10 @@ struct Pc4096Args {
 // past it are dropped), so the block needs no per-element tests; a wrapping
 // block reads through one over the whole row.
 // The spectrum's sixteen loads share one address register.  spec(q) gives bin
-// j + 256 q (the block's 1/M included).
+// j + 256 q (the block's 1/M included).  FOLD: folded factors instead of
+// power-base rows, for long convolutions, whose outputs are compared with
+// nothing: 16 x 1048576, 209 taps: 52.3 us, 52.4 with power-base rows, error
+// against FP64 2.15e-7, 2.5e-7.
 // Loads samples m0 .. m0 + NV - 1 of thread j of block ob
 // (x[lo + j + 256 m]) into v[0 .. NV).
 template <int NV>
@@ -416,7 +420,7 @@ __device__ __forceinline__ void load_block4096(const OlsBlock &ob, float2 (&v)[N
 // LATE_SPEC: the spectrum is written by other threads of the workgroup
 // while the forward passes run (pc4096_wf_kernel); it is read after one more
 // barrier, following the last forward pass, instead of being prefetched.
-template <class Spec, bool LATE_SPEC = false>
+template <bool FOLD, class Spec, bool LATE_SPEC = false>
 __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)[16],
                                                  const float4 *base1, const float4 *base2,
                                                  float2 *lds, Spec spec) {
@@ -442,12 +446,13 @@ __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)
     for (int m = 0; m < 16; ++m) v[m] = lds[rbase + m * (NT + NT / 16)];
     wg_barrier();
   };
-  PowRow t1 = load_pow(base1, j & 15), t2 = load_pow(base2, j);
+  using RW = Row16<FOLD>;
+  typename RW::T t1 = RW::load(base1, 16, j & 15), t2 = RW::load(base2, 256, j);
 
   // forward pass 0 (Ls = 1) on the samples as loaded
   dft16<false>(v);
   xchg(1);
-  pow_dft16<false>(v, t1);  // forward pass 1 (Ls = 16)
+  RW::template dft<false>(v, t1);  // forward pass 1 (Ls = 16)
   // the spectrum bins this thread multiplies, fetched before the exchange
   // so that their cache latency hides behind it and the last forward pass
   float2 sp[16];
@@ -456,7 +461,7 @@ __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)
     for (int q = 0; q < 16; ++q) sp[q] = spec(q);
   }
   xchg(16);
-  pow_dft16<false>(v, t2);  // forward pass 2 (Ls = 256)
+  RW::template dft<false>(v, t2);  // forward pass 2 (Ls = 256)
   if constexpr (LATE_SPEC) {
     wg_barrier();  // the spectrum is complete
 #pragma unroll
@@ -464,13 +469,13 @@ __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)
   }
 #pragma unroll
   for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], sp[q]);
-  dft16<true>(v);          // inverse pass 0 (Ls = 1)
-  pin_row(t1);
-  pin_row(t2);
+  dft16<true>(v);  // inverse pass 0 (Ls = 1)
+  RW::pin(t1);
+  RW::pin(t2);
   xchg(1);
-  pow_dft16<true>(v, t1);  // inverse pass 1 (Ls = 16)
+  RW::template dft<true>(v, t1);  // inverse pass 1 (Ls = 16)
   xchg(16);
-  pow_dft16<true, true>(v, t2);  // inverse pass 2 (Ls = 256)
+  RW::template dft<true, true>(v, t2);  // inverse pass 2 (Ls = 256)
   // lags lo + j + 256 q below lo + lim are kept (the spectrum carries the 1/M)
   const int lim = (ob.nout - lo) < ob.V ? (ob.nout - lo) : ob.V;
   const buf_rsrc ry = make_rsrc(ob.yr + lo, lim * 8);
@@ -480,31 +485,33 @@ __device__ __forceinline__ void filter_block4096(const OlsBlock &ob, float2 (&v)
 
 // One block, loaded and filtered.  Pre: the workgroup's previous use of lds
 // is finished.
-template <class Spec>
+template <bool FOLD, class Spec>
 __device__ __forceinline__ void ols_block4096(const OlsBlock ob, const float4 *base1,
                                               const float4 *base2, float2 *lds, Spec spec) {
   float2 v[16];
   load_block4096(ob, v, 0);
-  filter_block4096(ob, v, base1, base2, lds, spec);
+  filter_block4096<FOLD>(ob, v, base1, base2, lds, spec);
 }
 
 // The block's spectrum from its buffer (ob.wc).
+template <bool FOLD = false>
 __device__ __forceinline__ void ols_block4096(const OlsBlock ob, const float4 *base1,
                                               const float4 *base2, float2 *lds) {
   const buf_rsrc rw = make_rsrc(ob.wc, 4096 * 8);
-  ols_block4096(ob, base1, base2, lds, [&](int q) { return buf_load2s(rw, (int)threadIdx.x * 8, q * 2048); });
+  ols_block4096<FOLD>(ob, base1, base2, lds, [&](int q) { return buf_load2s(rw, (int)threadIdx.x * 8, q * 2048); });
 }
 
 // One workgroup per block.  (Resident workgroups that load the next block's
 // samples during the last inverse pass measure 5 to 10 % slower: the memory
 // counter is shared by loads and stores, so the next block's first wait for a
 // load also waits for this block's stores to land.)
+template <bool FOLD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void pc4096_kernel(Pc4096Args pa) {
   using LY = Layout<4096, 1, false>;
   __shared__ float2 lds[LY::LDS_ELEMS];
   const PcArgs &a = pa.a;
-  ols_block4096(pc_block(a, xcd_remap(blockIdx.x, a.groups)), pa.base1, pa.base2, lds);
+  ols_block4096<FOLD>(pc_block(a, xcd_remap(blockIdx.x, a.groups)), pa.base1, pa.base2, lds);
 }
 
 // Small grids (fft_conv on a few hundred pulses, where one workgroup per
@@ -525,6 +532,7 @@ struct Pc4096WfArgs {
   float out_scale;
 };
 
+template <bool FOLD>
 __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
   using LY = Layout<4096, 1, false>;
   __shared__ float2 lds[LY::LDS_ELEMS];   // the block's exchanges
@@ -538,7 +546,7 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
     // barriers: 4 in the forward exchanges, 1 for the spectrum, 4 in the
     // inverse exchanges
     auto spec = [&](int q) { return wsp[(int)threadIdx.x + q * 256]; };
-    filter_block4096<decltype(spec), true>(ob, v, q.p.base1, q.p.base2, lds, spec);
+    filter_block4096<FOLD, decltype(spec), true>(ob, v, q.p.base1, q.p.base2, lds, spec);
     return;
   }
   // the waveform: the same three forward passes, exchanged through wsp
@@ -560,12 +568,13 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
     if (q.conj_in) v[m].y = -v[m].y;
   }
   dft16<false>(v);
-  PowRow tw = load_pow(q.p.base1, j & 15);
+  using RW = Row16<FOLD>;
+  typename RW::T tw = RW::load(q.p.base1, 16, j & 15);
   xchg(1);
-  pow_dft16<false>(v, tw);
-  tw = load_pow(q.p.base2, j);
+  RW::template dft<false>(v, tw);
+  tw = RW::load(q.p.base2, 256, j);
   xchg(16);
-  pow_dft16<false>(v, tw);
+  RW::template dft<false>(v, tw);
   // the exchange above ended with a barrier after every read of wsp
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
@@ -590,9 +599,10 @@ __global__ __launch_bounds__(512) void pc4096_wf_kernel(Pc4096WfArgs q) {
 // registers before the first inverse exchange: five LDS exchanges per block.
 struct Pc8192Args {
   PcArgs a;
-  const float4 *bA, *bB, *bC;  // power-base rows for Ls = 2, 32, 512
+  const float4 *bA, *bB, *bC;  // power-base rows (FOLD: factors) for Ls = 2, 32, 512
 };
 
+template <bool FOLD = false>
 __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *bA, const float4 *bB,
                                               const float4 *bC, float2 *lds) {
   constexpr int NT = 512;
@@ -638,24 +648,25 @@ __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *b
     }
     pair_dft2(v, (j & 1) != 0);
   }
-  PowRow tw = load_pow(bA, j & 1);
-  pow_dft16<false>(v, tw);  // forward pass Ls = 2
-  tw = load_pow(bB, j & 31);
+  using RW = Row16<FOLD>;
+  typename RW::T tw = RW::load(bA, 2, j & 1);
+  RW::template dft<false>(v, tw);  // forward pass Ls = 2
+  tw = RW::load(bB, 32, j & 31);
   xchg(2);
-  pow_dft16<false>(v, tw);  // forward pass Ls = 32
-  tw = load_pow(bC, j);
+  RW::template dft<false>(v, tw);  // forward pass Ls = 32
+  tw = RW::load(bC, 512, j);
   // the spectrum bins this thread multiplies, fetched before the exchange
   const buf_rsrc rw = make_rsrc(ob.wc, 8192 * 8);
   float2 sp[16];
 #pragma unroll
   for (int q = 0; q < 16; ++q) sp[q] = buf_load2s(rw, j * 8, q * 4096);
   xchg(32);
-  pow_dft16<false>(v, tw);  // forward pass Ls = 512: bins j + 512q
+  RW::template dft<false>(v, tw);  // forward pass Ls = 512: bins j + 512q
 #pragma unroll
   for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], sp[q]);
   // inverse radix-2 pass (Ls = 1) on bins j + 512q, j + 512q + 4096; its
   // outputs 2 (j + 512 q) and the next sit at pad(2 j) + 1088 q and + 1
-  tw = load_pow(bA, j & 1);
+  tw = RW::load(bA, 2, j & 1);
   const int e0 = lds_pad(2 * j);
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
@@ -666,13 +677,13 @@ __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *b
 #pragma unroll
   for (int m = 0; m < 16; ++m) v[m] = lds[rbase + 544 * m];
   wg_barrier();
-  pow_dft16<true>(v, tw);  // inverse pass Ls = 2
-  tw = load_pow(bB, j & 31);
+  RW::template dft<true>(v, tw);  // inverse pass Ls = 2
+  tw = RW::load(bB, 32, j & 31);
   xchg(2);
-  pow_dft16<true>(v, tw);  // inverse pass Ls = 32
-  tw = load_pow(bC, j);
+  RW::template dft<true>(v, tw);  // inverse pass Ls = 32
+  tw = RW::load(bC, 512, j);
   xchg(32);
-  pow_dft16<true, true>(v, tw);  // inverse pass Ls = 512: lags j + 512q
+  RW::template dft<true, true>(v, tw);  // inverse pass Ls = 512: lags j + 512q
   // lags lo + j + 512 q below lo + lim are kept (stores past lim dropped by
   // the range check; the spectrum carries the 1/M)
   const int lim = (ob.nout - lo) < ob.V ? (ob.nout - lo) : ob.V;
@@ -681,12 +692,13 @@ __device__ __forceinline__ void ols_block8192(const OlsBlock ob, const float4 *b
   for (int q = 0; q < 16; ++q) buf_store2(ry, (j + q * 512) * 8, v[q]);
 }
 
+template <bool FOLD>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void pc8192_kernel(Pc8192Args pa) {
   using LY = Layout<8192, 1, false>;
   __shared__ float2 lds[LY::LDS_ELEMS];
   const OlsBlock ob = pc_block(pa.a, xcd_remap(blockIdx.x, pa.a.groups));
-  ols_block8192(ob, pa.bA, pa.bB, pa.bC, lds);
+  ols_block8192<FOLD>(ob, pa.bA, pa.bB, pa.bC, lds);
 }
 
 // One workgroup of M/16 threads.  Thread j loads samples j + m*M/16,
@@ -1085,6 +1097,7 @@ constexpr int64_t PC_WF_FUSE_MAX_GROUPS = 512;
 
 template <int M>
 mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
+  auto table16 = [&](int N, int Ls) { return pa->fold ? factors16_device(Ls) : pow_base_device(N, Ls); };
   // the spectrum in the same launch: plain waveforms, small grids
   const bool fuse = wa && pa && pa->groups > 0 && pa->bpw == 1 && pa->groups <= PC_WF_FUSE_MAX_GROUPS &&
                     !wa->window && !wa->normalize && !wa->writeback && wa->L >= 1 && wa->L <= M;
@@ -1100,12 +1113,13 @@ mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
   }
   if constexpr (M == 4096) {
     if (fuse && pa->n <= PC_BUF_MAX_N) {
-      Pc4096WfArgs q{{*pa, pow_base_device(4096, 16), pow_base_device(4096, 256)}, wa->w, wa->wstride,
+      Pc4096WfArgs q{{*pa, table16(4096, 16), table16(4096, 256)}, wa->w, wa->wstride,
                      (int)wa->L, wa->conj_in, wa->conj, wa->out_scale};
       MXR_REQUIRE(q.p.base1 && q.p.base2, MXR_OUT_OF_MEMORY,
                   "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc4096_wf_kernel", s);
-      pc4096_wf_kernel<<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(q);
+      if (pa->fold) pc4096_wf_kernel<true><<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(q);
+      else pc4096_wf_kernel<false><<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(q);
       MXR_HIP_TRY(hipGetLastError());
       return MXR_SUCCESS;
     }
@@ -1118,21 +1132,23 @@ mxr_status launch_pc(const WfArgs *wa, const PcArgs *pa, hipStream_t s) {
   if (!pa || pa->groups <= 0) return MXR_SUCCESS;
   if constexpr (M == 8192) {
     if (pa->n <= PC_BUF_MAX_N && pa->bpw == 1) {
-      Pc8192Args p8{*pa, pow_base_device(8192, 2), pow_base_device(8192, 32), pow_base_device(8192, 512)};
+      Pc8192Args p8{*pa, table16(8192, 2), table16(8192, 32), table16(8192, 512)};
       MXR_REQUIRE(p8.bA && p8.bB && p8.bC, MXR_OUT_OF_MEMORY,
                   "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc8192_kernel", s);
-      pc8192_kernel<<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
+      if (pa->fold) pc8192_kernel<true><<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
+      else pc8192_kernel<false><<<dim3((unsigned)pa->groups), dim3(512), 0, s>>>(p8);
       MXR_HIP_TRY(hipGetLastError());
       return MXR_SUCCESS;
     }
   }
   if constexpr (M == 4096) {
     if (pa->n <= PC_BUF_MAX_N && pa->bpw == 1) {
-      Pc4096Args p4{*pa, pow_base_device(4096, 16), pow_base_device(4096, 256)};
+      Pc4096Args p4{*pa, table16(4096, 16), table16(4096, 256)};
       MXR_REQUIRE(p4.base1 && p4.base2, MXR_OUT_OF_MEMORY, "pulse compression: twiddle table allocation failed");
       ProfScope ps("pc4096_kernel", s);
-      pc4096_kernel<<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
+      if (pa->fold) pc4096_kernel<true><<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
+      else pc4096_kernel<false><<<dim3((unsigned)pa->groups), dim3(256), 0, s>>>(p4);
       MXR_HIP_TRY(hipGetLastError());
       return MXR_SUCCESS;
     }
@@ -1301,6 +1317,7 @@ mxr_status pc_common(const char *fn, const mxr_tensor *y, const mxr_tensor *x, c
   wa.out_scale = (float)(1.0 / (double)plan.M);  // exact: a power of two
   if ((st = pc_blocks(fn, plan, in_place, wc, twf, twi, &pa))) return st;
   pa.shift = shift;
+  pa.fold = by_rate;
   return dispatch_pc(plan.M, &wa, &pa, stream);
 }
 

@@ -280,3 +280,15 @@ def test_conv1d_longest_rows(mx, L, over):
     assert rel(host(y[0, :K + L - 1]), lo) < RTOL
     assert rel(host(y[0, N - K:]), hi) < RTOL
     assert not y[0, K + L + 16384:N - K - 16384].any()
+
+
+def test_conv1d_long_rows_error(mx):
+    """Rows of 1048576 samples through 4096-point blocks lose no accuracy to
+    2048-point ones, which erred by 2.12e-7 here: a radix-16 block of twice the
+    points has 12 / 11 = 1.09 times the levels, so 1.1 times that is allowed."""
+    rng = np.random.default_rng(209)
+    N, L = 1048576, 209
+    x, f = sig(rng, (4, N), True), sig(rng, (L,), True)
+    n = 1 << 21
+    ref = np.fft.ifft(np.fft.fft(x.astype(complex), n) * np.fft.fft(f.astype(complex), n))[:, (L - 1) // 2:(L - 1) // 2 + N]
+    assert rel(host(mx.conv1d(dev(x), dev(f), "same", method="fft")), ref) < 1.1 * 2.12e-7
